@@ -137,13 +137,18 @@ int axc_quint8_zero_point(float range_min, float range_max, int32_t *zero_point)
 int axc_qint32_range_for_multiplication(float min_a, float max_a, float min_b, float max_b, float *min_c,
                                         float *max_c);
 
-/* How the dense kernel would cut this layer on the current device (for tools and tests; the reference has no
- * counterpart, its launch shapes are fixed in cuda/approx_nn_conv_kernels.cu:296-627):
+/* How the dense kernels whose sums the vector ALUs make would cut this layer on the current device (for tools and tests;
+ * the reference has no counterpart, its launch shapes are fixed in cuda/approx_nn_conv_kernels.cu:296-627):
  * plan = { columns per tile (16/32/64), rows per tile, row tiles, column tiles, K splits, workgroups,
  *          fills of 64 filter entries per K split, how the layer runs given a workspace of the size
  *          axc_conv2d_workspace_bytes reports: 0 = table rows expanded inside every tile, 1 = out of pre-expanded
  *          rows, 2 = out of pre-expanded rows by the kernel whose wavefronts do not meet at a barrier between fills }. */
 int axc_conv2d_tile_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
+/* Whether the layer runs the kernel whose sums the matrix cores make instead (given a workspace of the size
+ * axc_conv2d_workspace_bytes reports, and neither axc_set_preexpand nor axc_set_tile_columns pinning another), and how
+ * that cuts it: plan = { 1 or 0 (then the rest is 0 too), units of 64 pixels per wavefront (the kernel's variant), units
+ * per tile, row tiles, column tiles (8 columns), K splits, workgroups, fills of 16 filter elements per K split }. */
+int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
 /* Pins the tile width the planner uses (16, 32 or 64 columns; 0 = its own choice, the default), process-wide, for
  * tests and timing of the wider-tile kernel variants.  The environment variable AXC_TILE_COLUMNS gives the initial
  * value and is read once, when the library is loaded.  Like axc_set_preexpand it is process-wide; a workspace query and

@@ -7,7 +7,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libaxconv_hip.so")
-SOURCES = ["axconv_api.hip", "lutgemm_kernel.hip", "lutgemm_px_kernel.hip", "prepass_kernels.hip", "depthwise_kernel.hip"]
+SOURCES = ["axconv_api.hip", "lutgemm_kernel.hip", "lutgemm_px_kernel.hip", "lutgemm_mx_kernel.hip", "prepass_kernels.hip", "depthwise_kernel.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -19,11 +19,12 @@ FLAGS = [
 
 
 def generate():
-    """Writes csrc/lookup_asm.inc, the generated inline assembly of the lookup phase."""
-    gen = os.path.join(CSRC, "gen_lookup_asm.py")
-    text = subprocess.run([sys.executable, gen], stdout=subprocess.PIPE, text=True, check=True).stdout
-    with open(os.path.join(CSRC, "lookup_asm.inc"), "w") as f:
-        f.write(text)
+    """Writes csrc/lookup_asm.inc and csrc/lookup_mx.inc, the generated inline assembly of the lookup phases."""
+    for name in ("lookup_asm", "lookup_mx"):
+        gen = os.path.join(CSRC, "gen_%s.py" % name)
+        text = subprocess.run([sys.executable, gen], stdout=subprocess.PIPE, text=True, check=True).stdout
+        with open(os.path.join(CSRC, name + ".inc"), "w") as f:
+            f.write(text)
 
 
 def build(verbose=False, extra=()):

@@ -573,6 +573,121 @@ DensePlan make_plan(const ConvGeom &g, int cus, int px_mode = kPxModeGlobal)
     return plan;
 }
 
+// ---- lutgemm_mx_kernel: lookups summed by the matrix cores, out of pre-expanded rows of its own form ----
+MxDiv mx_div(uint32_t d)
+{
+    if (d <= 1)
+        return {0u, 0u};
+    uint32_t s = 1;
+    while (s < 31 && (1u << s) < d)
+        ++s;
+    return {(uint32_t)((((uint64_t)1 << (31 + s)) + d - 1) / d), s - 1};
+}
+
+// Tiles of 64-pixel units x 8 columns: how many row tiles, which kernel variant, how many K splits.  Microseconds,
+// measured by running 3x3 layers of 9 and of 36 fills in every variant (U units per wavefront):
+//   a fill    0.30 + 0.138 U, at least 1.05 + 0.03 U (64 KiB of rows into LDS with every CU doing so: U = 2 takes 1.11, 8 1.45,
+//             13 2.1, 25 3.75); with four loads per unit instead of one (pixels that are no neighbouring dwords)
+//             0.35 + 0.243 U, at least 1.3
+//   a tile    1.3 + 0.70 U: geometry, the sums' start values, the outputs (for the most part the stores of 32-byte pieces)
+// K splits and the rows cost what they cost the other kernels (compute_plan).
+MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, bool one_load, int cus, double clock_hz)
+{
+    MxPlan best{};
+    double best_cost = 1e300;
+    const int n_col = (co + kMxCols - 1) / kMxCols;
+    const int fills = (int)((quads + kMxFillQuads - 1) / kMxFillQuads);
+    const int max_units = kMxUnits[sizeof(kMxUnits) / sizeof(kMxUnits[0]) - 1];
+    const int64_t total_units = (groups + 15) / 16;
+    const int64_t cap = (int64_t)kMxWaves * max_units;
+    const int64_t min_tiles = (total_units + cap - 1) / cap;
+    const double rows_bytes = (double)n_col * fills * 65536.0;
+    const double rows_us = rows_bytes <= 400e6 ? 1.5 + rows_bytes / 7e6 : 6.5 + rows_bytes / 4.5e6;
+    for (int ks : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        const int fps = (fills + ks - 1) / ks;
+        if (ks > 1 && (fps < 4 || (int64_t)(ks - 1) * fps >= fills))
+            continue;
+        std::vector<int64_t> cands{min_tiles};
+        for (int64_t rounds = 1; rounds <= 64; ++rounds)
+            for (int64_t n_row : {rounds * cus / ((int64_t)n_col * ks), rounds * cus / ((int64_t)n_col * ks) + 1})
+                if (n_row > min_tiles && n_row <= total_units)
+                    cands.push_back(n_row);
+        for (int64_t n_row : cands) {
+            const int64_t upt = (total_units + n_row - 1) / n_row;
+            int units = 0;
+            for (int u : kMxUnits)
+                if (!units && (int64_t)u * kMxWaves >= upt)
+                    units = u;
+            if (!units)
+                continue;
+            const int64_t rows = (total_units + upt - 1) / upt;
+            const int64_t tiles = rows * n_col * ks, rounds = (tiles + cus - 1) / cus;
+            const double fill = one_load ? std::max(1.05 + 0.03 * units, 0.30 + 0.138 * units)
+                                         : std::max(1.3, 0.35 + 0.243 * units);
+            double us = std::max((double)rounds * (fps * fill + 1.3 + 0.70 * units), rows_bytes / 3e6);
+            if (ks > 1)
+                us += 7.1 + (double)(ks + 1) * (double)outputs * 4.0 * 1.46e-7;
+            const double cost = (us + rows_us) * 1e-6 * clock_hz;
+            if (cost < best_cost) {
+                best_cost = cost;
+                best.units = units;
+                best.units_per_tile = (int)upt;
+                best.n_row_tiles = (int)rows;
+                best.n_col_tiles = n_col;
+                best.fills = fills;
+                best.k_splits = ks;
+                best.fills_per_split = fps;
+                best.grid = (int)(tiles < cus ? tiles : cus);
+                best.cost = (float)cost;
+            }
+        }
+    }
+    return best;
+}
+
+MxPlan make_mx_plan(const ConvGeom &g, bool one_load, int cus)
+{
+    typedef std::tuple<int64_t, int, int64_t, int64_t, bool, int> Key;
+    static std::mutex mu;
+    static std::map<Key, MxPlan> cache;
+    const int64_t quads = (int64_t)g.KH * g.KW * g.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
+    const Key key{quads, g.Co, groups, g.M * g.Co, one_load, cus};
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        auto it = cache.find(key);
+        if (it != cache.end())
+            return it->second;
+    }
+    const MxPlan plan = compute_mx_plan(quads, g.Co, groups, g.M * g.Co, one_load, cus, device_clock_hz());
+    std::lock_guard<std::mutex> lock(mu);
+    if (cache.size() >= 4096)
+        cache.clear();
+    cache[key] = plan;
+    return plan;
+}
+
+XqLayout plain_layout(const ConvGeom &g) { return {g.H, g.W, 0, 0}; }
+
+// The layout with the padding written out: as many rows / columns in front as the larger of the two paddings.
+XqLayout padded_layout(const ConvGeom &g, bool flat)
+{
+    const int below = (g.OH - 1) * g.sh - g.ph + (g.KH - 1) * g.dh + 1 - g.H;
+    const int right = (g.OW - 1) * g.sw - g.pw + (g.KW - 1) * g.dw + 1 - g.W;
+    XqLayout l;
+    l.row0 = std::max(0, std::max(g.ph, below));
+    l.col0 = flat ? 0 : std::max(0, std::max(g.pw, right));
+    l.Hp = g.H + l.row0;
+    l.Wp = g.W + l.col0;
+    return l;
+}
+
+// Bytes of xq: its rows and those behind the last image (a group of four pixels may reach a few bytes past its row).
+size_t xq_bytes_of(const ConvGeom &g, const XqLayout &l, int flat_row_bytes)
+{
+    const size_t rows = (size_t)g.N * l.Hp + l.tail_rows();
+    return rows * (flat_row_bytes ? (size_t)flat_row_bytes : (size_t)g.C4 * l.Wp * 4) + 16;
+}
+
 inline size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct DenseWorkspace {
@@ -581,28 +696,32 @@ struct DenseWorkspace {
     size_t total_no_px;  // what a launch needs that does without them
 };
 
-// sub_bytes: room for the pixels a strided 1x1 filter reads, gathered into a dense tensor (see prepare_dense)
-DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, size_t sub_bytes, int flat_row_bytes)
+// sub_bytes: room for the pixels a strided 1x1 filter reads, gathered into a dense tensor (see prepare_dense).  mx: the
+// plan of lutgemm_mx_kernel where the layer runs that one, else null.
+DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, const MxPlan *mx, const XqLayout &lay,
+                               size_t sub_bytes, int flat_row_bytes)
 {
     DenseWorkspace w;
     size_t off = 0;
     w.sub_off = off; off += align_up(sub_bytes);
-    w.xq_off = off;   // + the zero-point row; the flat layout's last quad may reach a few bytes past its row
-    off += align_up(flat_row_bytes ? ((size_t)g.N * g.H + 1) * flat_row_bytes + 16
-                                   : ((size_t)g.N * g.H + 1) * g.C4 * g.W * 4);
+    w.xq_off = off; off += align_up(xq_bytes_of(g, lay, flat_row_bytes));   // + the zero-point row(s)
     w.psum_off = off; off += align_up((size_t)g.M * 4); // patch sums: one float per output pixel
-    w.wq_off = off; off += align_up((size_t)plan.n_col_tiles * plan.fills * 64 * 2);
+    w.wq_off = off; off += mx ? 0 : align_up((size_t)plan.n_col_tiles * plan.fills * 64 * 2);
     w.fsum_off = off; off += align_up((size_t)g.Co * 4);
     w.layer_off = off;  // layer entry point: partial (min, max) pairs of both tensors, then the LayerQuant
     off += align_up((size_t)4 * kMinMaxBlocks * sizeof(float)) + align_up(sizeof(LayerQuant));
     w.part_off = off;   // int32 partial sums of the K splits
-    if (plan.k_splits > 1)
-        off += align_up((size_t)plan.k_splits * (size_t)g.M * g.Co * 4);
+    const int k_splits = mx ? mx->k_splits : plan.k_splits;
+    if (k_splits > 1)
+        off += align_up((size_t)k_splits * (size_t)g.M * g.Co * 4);
     w.total_no_px = off;
     w.px_off = off;
-    w.px_bytes = plan.px ? (size_t)plan.n_col_tiles * (size_t)(plan.fills / 2) * 65536 : 0;
+    w.px_bytes = mx ? (size_t)mx->n_col_tiles * (size_t)mx->fills * 65536
+                    : plan.px ? (size_t)plan.n_col_tiles * (size_t)(plan.fills / 2) * 65536 : 0;
     off += align_up(w.px_bytes);
     w.total = off;
+    if (mx)
+        w.total_no_px = off;   // its kernel has no form without the rows
     return w;
 }
 
@@ -614,19 +733,51 @@ struct PreparedDense {
     int flat_row_bytes;  // > 0: xq in the flat layout, rows of this many bytes
     bool subsample;
     DensePlan plan;
+    bool mx;             // the layer runs lutgemm_mx_kernel, cut as mxp says (plan then only describes the other kernels)
+    MxPlan mxp;
+    XqLayout lay;
     DenseWorkspace ws;
     bool empty;
 };
+
+// Decides whether the layer runs lutgemm_mx_kernel: where the two cost models, fitted to the launch times of each, say
+// that it is the faster one.  ResNet-50's and the CIFAR network's layers, forced both ways (whole op, us): 3x3 64->64 @56x56
+// 289.8 -> 194.3, 1x1 64->256 @56x56 173.8 -> 153.9, 3x3 128->128 @28x28 309.1 -> 202.2, 3x3 16->16 @32x32x128 42.4 -> 32.4;
+// not 1x1 32->192 @112x112, two fills under the stores of a whole tile (331 against 401).
+void prepare_mx(PreparedDense *pd)
+{
+    const ConvGeom &g = pd->g;
+    const XqLayout lay = padded_layout(g, pd->flat_row_bytes > 0);
+    const size_t padded = xq_bytes_of(g, lay, pd->flat_row_bytes), plain = xq_bytes_of(g, plain_layout(g), pd->flat_row_bytes);
+    if (padded >= ((size_t)1 << 31) || padded > plain + plain / 2 + 65536)   // padding larger than the image: not worth it
+        return;
+    if (g.M >= ((int64_t)1 << 31) - 4096 || g.Co > 65536)   // pixel numbers and a tile's output offsets in 31 bits
+        return;
+    ConvGeom gq = pd->gk;
+    gq.OW = g.OW;
+    const MxPlan plan = make_mx_plan(gq, (pd->flat_row_bytes ? g.sw * g.C : g.sw * 4) == 4, device_cus());
+    if (plan.units == 0 || (size_t)plan.n_col_tiles * (size_t)plan.fills * 65536 > kPxMaxBytes)
+        return;
+    if (plan.cost > pd->plan.cost)
+        return;
+    pd->mx = true;
+    pd->mxp = plan;
+    pd->lay = lay;
+}
 
 // A 1x1 filter with a stride only ever reads every stride-th pixel, and never needs padding: the op equals the 1x1
 // stride-1 op on the subsampled input.  Those pixels are gathered into the workspace first (element_bytes each:
 // floats, or bytes for the codes entry point), and every kernel then sees a dense, unpadded stride-1 layer with a
 // quarter (stride 2) of the pixels to quantize and sum.  allow_subsample = false keeps the layer as given (callers
-// with their own padding origin).
-int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, bool allow_subsample = true, int element_bytes = 4,
-                  int px_mode = kPxModeGlobal)
+// with their own padding origin: `pads`, rows and columns).  allow_mx = false: the layer as the other kernels run it.
+int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
+                  int px_mode = kPxModeGlobal, bool allow_mx = true)
 {
+    const bool allow_subsample = pads == nullptr;
     const bool allow_flat = allow_subsample;   // both are for callers that leave the padding origin to the library
+    pd->mx = false;
+    pd->mxp = MxPlan{};
+    pd->lay = XqLayout{};
     int rc = geometry(desc, &pd->dims);
     if (rc != AXC_OK)
         return rc;
@@ -634,6 +785,10 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, bool allow_sub
     if (rc != AXC_OK)
         return rc;
     pd->g = pd->g_full = make_geom(pd->dims);
+    if (pads) {
+        pd->g.ph = pd->g_full.ph = pads[0];
+        pd->g.pw = pd->g_full.pw = pads[1];
+    }
     pd->subsample = false;
     pd->empty = pd->g.M * pd->g.Co == 0; // approx_nn_conv_ops.cpp:449
     if (pd->empty || pd->g.K == 0) {
@@ -688,11 +843,45 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, bool allow_sub
         }
     }
     pd->plan = make_plan(pd->gk, device_cus(), px_mode);
-    pd->ws = dense_workspace(pd->g, pd->plan, sub_bytes, pd->flat_row_bytes);
+    pd->lay = plain_layout(pd->g);
+    if (allow_mx && px_mode == kPxModeGlobal && g_px_mode.load(std::memory_order_relaxed) == 0 &&
+        g_forced_nt.load(std::memory_order_relaxed) == 0 && pd->plan.px)
+        prepare_mx(pd);
+    pd->ws = dense_workspace(pd->g, pd->plan, pd->mx ? &pd->mxp : nullptr, pd->lay, sub_bytes, pd->flat_row_bytes);
     return AXC_OK;
 }
 
-enum class DenseOut { Float, AccI32 };
+// tf1 AxConv2D: filter origin offsets of ReferenceAxConvFunctor (tf1/axqconv/axqconv.cc:153-163), C integer division
+void axconv_tf1_pads(const ConvGeom &g, int padding, int pads[2])
+{
+    const int extra = padding == AXC_PAD_VALID ? 1 : 0;
+    pads[0] = ((g.OH - 1) * g.sh + g.KH - g.H + extra) / 2;
+    pads[1] = ((g.OW - 1) * g.sw + g.KW - g.W + extra) / 2;
+}
+
+// The layer as it runs with this much workspace: in the form the planner prefers if that fits, else in the next one.
+// Without room for the pre-expanded rows it runs the kernel that expands inside its tiles, with the tile shape and K
+// split the planner prices for THAT kernel, if the workspace holds what that plan needs (its K split may ask for partial
+// sums the other plan has none of); otherwise with the plan at hand.
+int prepare_dense_for(const axc_conv2d_desc *desc, size_t workspace_bytes, const int *pads, int element_bytes,
+                      PreparedDense *pd)
+{
+    int rc = prepare_dense(desc, pd, pads, element_bytes);
+    if (rc != AXC_OK || pd->empty)
+        return rc;
+    if (pd->mx && workspace_bytes < pd->ws.total) {
+        rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, false);
+        if (rc != AXC_OK)
+            return rc;
+    }
+    if (!pd->mx && pd->plan.px && workspace_bytes < pd->ws.total) {
+        PreparedDense alt;
+        rc = prepare_dense(desc, &alt, pads, element_bytes, -1);
+        if (rc == AXC_OK && workspace_bytes >= alt.ws.total)
+            *pd = alt;
+    }
+    return AXC_OK;
+}
 
 int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *input, const float *filter,
               const uint8_t *input_codes, const uint8_t *filter_codes, int input_zero_code,
@@ -711,24 +900,11 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     if (int rc_wait = wait_error_check(&wait_word))
         return rc_wait;
     PreparedDense pd;
-    int rc = prepare_dense(desc, &pd, pad_before_override == nullptr, codes_mode ? 1 : 4);
+    int rc = prepare_dense_for(desc, workspace_bytes, pad_before_override, codes_mode ? 1 : 4, &pd);
     if (rc != AXC_OK)
         return rc;
     if (pd.empty)
         return AXC_OK;
-    if (pd.plan.px && workspace_bytes < pd.ws.total) {
-        // No room for the pre-expanded rows: the layer runs the kernel that expands inside its tiles, with the tile
-        // shape and K split the planner prices for THAT kernel, if the workspace holds what that plan needs (its K
-        // split may ask for partial sums the other plan has none of); otherwise with the plan at hand.
-        PreparedDense alt;
-        rc = prepare_dense(desc, &alt, pad_before_override == nullptr, codes_mode ? 1 : 4, -1);
-        if (rc == AXC_OK && workspace_bytes >= alt.ws.total)
-            pd = alt;
-    }
-    if (pad_before_override) { // a caller with its own padding rule (tf1 AxConv2D); the plan does not depend on it
-        pd.g.ph = pad_before_override[0];
-        pd.g.pw = pad_before_override[1];
-    }
     if ((!codes_mode && (!input || !filter)) || (codes_mode && !filter_codes) || (!out_f && !out_i))
         return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
     hipStream_t stream = static_cast<hipStream_t>(stream_v);
@@ -752,7 +928,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         return AXC_OK;
     }
     // a workspace without room for the pre-expanded rows still serves: the layer then runs without them
-    const bool use_px = pd.plan.px && workspace_bytes >= pd.ws.total;
+    const bool use_px = (pd.mx || pd.plan.px) && workspace_bytes >= pd.ws.total;
+    const MxPlan *const mx = pd.mx ? &pd.mxp : nullptr;
     if (workspace_bytes < pd.ws.total_no_px || (!workspace && pd.ws.total_no_px))
         return fail(AXC_INVALID_ARGUMENT, "workspace too small (see axc_conv2d_workspace_bytes)");
     if (((uintptr_t)workspace & 255) != 0)
@@ -795,30 +972,30 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     if (out_f && !codes_mode) {
         // carries the filter pre-pass, and with it the pre-expanded rows, along when it can
         ProfScope ps(flat ? "patch_sums_flat" : "patch_sums", stream);
-        const FilterJob job = {filter, filter_codes, &pd.plan, tq_f, wq, fsum, table->dev_tableT, px_rows};
+        const FilterJob job = {filter, filter_codes, &pd.plan, tq_f, wq, fsum, table->dev_tableT, px_rows, mx};
         if (flat)   // the patch sums write the flat layout where they hold the rows anyway, else the pass below does
-            AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, xq, &quantized_by_patch_sums, nullptr,
+            AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, pd.lay, xq, &quantized_by_patch_sums, nullptr,
                                       nullptr, pd.flat_row_bytes));
         else
-            AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, xq, &quantized_by_patch_sums, &job,
+            AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, pd.lay, xq, &quantized_by_patch_sums, &job,
                                       &filter_done, 0, &px_done));
     }
     if (flat && !quantized_by_patch_sums) {
         ProfScope ps("quantize_flat_rows", stream);
-        AXC_HIP(launch_quantize_flat_rows(input, codes_mode ? input_codes : nullptr, g, g.pw, pd.flat_row_bytes, tq_in,
+        AXC_HIP(launch_quantize_flat_rows(input, codes_mode ? input_codes : nullptr, g, pd.lay, g.pw, pd.flat_row_bytes, tq_in,
                                           lq_dev, reinterpret_cast<uint8_t *>(xq), stream));
     } else if (flat) {
         // written by the patch-sum launch
     } else if (codes_mode) {
         ProfScope ps("codes_relayout", stream);
-        AXC_HIP(launch_codes_relayout(input_codes, g, zp4, xq, stream));
+        AXC_HIP(launch_codes_relayout(input_codes, g, pd.lay, zp4, xq, stream));
     } else if (!quantized_by_patch_sums) {
         ProfScope ps("quantize_relayout", stream);
-        AXC_HIP(launch_quantize_relayout(input, g, tq_in, lq_dev, xq, nullptr, stream));
+        AXC_HIP(launch_quantize_relayout(input, g, tq_in, lq_dev, pd.lay, xq, nullptr, stream));
     }
     if (!filter_done) {
         ProfScope ps("filter_pack", stream);
-        AXC_HIP(launch_filter_pack(codes_mode ? nullptr : filter, filter_codes, gk, pd.plan, tq_f, lq_dev, wq,
+        AXC_HIP(launch_filter_pack(codes_mode ? nullptr : filter, filter_codes, gk, pd.plan, mx, tq_f, lq_dev, wq,
                                    (out_f && !codes_mode) ? fsum : nullptr, stream, table->dev_tableT, px_rows, &px_done));
     }
 
@@ -858,10 +1035,87 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     if (use_px) {
         if (!px_done) {
             ProfScope ps("px_expand_rows", stream);
-            AXC_HIP(launch_px_expand_rows(wq, table->dev_tableT, pd.plan, px_rows, stream));
+            if (mx)
+                AXC_HIP(launch_mx_expand_rows(codes_mode ? nullptr : filter, filter_codes, gk, *mx, tq_f, lq_dev,
+                                              table->dev_tableT, px_rows, stream));
+            else
+                AXC_HIP(launch_px_expand_rows(wq, table->dev_tableT, pd.plan, px_rows, stream));
         }
         p.px_rows = px_rows;
         p.px_bytes = (uint32_t)pd.ws.px_bytes;
+    }
+    if (mx) {
+        MxParams m = {};
+        m.plan = *mx;
+        m.xq = xq;
+        m.xq_bytes = (uint32_t)xq_bytes_of(g, pd.lay, pd.flat_row_bytes);
+        m.rows = px_rows;
+        m.rows_bytes = (uint32_t)pd.ws.px_bytes;
+        m.psum = psum;
+        m.fsum = fsum;
+        m.bias = bias;
+        m.out_f = out_f;
+        m.out_i = out_i;
+        m.lq_dev = lq_dev;
+        m.s1xs2 = p.s1xs2;
+        m.m1 = p.m1;
+        m.m2 = p.m2;
+        m.k_m1xm2 = p.k_m1xm2;
+        m.relu = p.relu;
+        m.M = g.M;
+        m.Co = g.Co;
+        m.oh = g.OH;
+        m.ow = g.OW;
+        m.groups_per_row = (g.OW + 3) / 4;
+        m.groups = (int)((int64_t)g.N * g.OH * m.groups_per_row);
+        m.linear = (g.OW & 3) == 0;
+        m.div_groups = mx_div((uint32_t)m.groups_per_row);
+        m.div_oh = mx_div((uint32_t)g.OH);
+        m.div_c4 = mx_div((uint32_t)gk.C4);
+        m.div_kw = mx_div((uint32_t)gk.KW);
+        const uint32_t row = flat ? (uint32_t)pd.flat_row_bytes : (uint32_t)g.C4 * (uint32_t)pd.lay.Wp * 4u;
+        m.pitch = flat ? (uint32_t)(g.sw * g.C) : (uint32_t)g.sw * 4u;
+        m.origin = (uint32_t)(pd.lay.row0 - g.ph) * row + (flat ? 0u : (uint32_t)(pd.lay.col0 - g.pw) * 4u);
+        m.img_step = (uint32_t)pd.lay.Hp * row;
+        m.orow_step = (uint32_t)g.sh * row;
+        m.group_step = 4u * m.pitch;
+        m.kh_step = (uint32_t)g.dh * row;
+        m.kw_step = (uint32_t)g.dw * 4u;   // (the flat layout has one tap per filter row)
+        m.quad_step = flat ? 4u : (uint32_t)pd.lay.Wp * 4u;
+        m.c4 = gk.C4;
+        m.kw = gk.KW;
+        // four quads on = `taps` whole taps and dq quads
+        const int taps = kMxFillQuads / gk.C4;
+        m.dq = kMxFillQuads % gk.C4;
+        m.dkw = taps % gk.KW;
+        m.doff = (uint32_t)m.dq * m.quad_step + (uint32_t)m.dkw * m.kw_step + (uint32_t)(taps / gk.KW) * m.kh_step;
+        m.qoff = m.kw_step - (uint32_t)gk.C4 * m.quad_step;
+        m.kwoff = m.kh_step - (uint32_t)gk.KW * m.kw_step;
+        {
+            const uint32_t step = kMxWaves * 16u, rows = step / (uint32_t)m.groups_per_row;
+            m.step_groups = step % (uint32_t)m.groups_per_row;
+            m.step_rows = rows % (uint32_t)g.OH;
+            m.step_bytes = rows / (uint32_t)g.OH * m.img_step + m.step_rows * m.orow_step + m.step_groups * m.group_step;
+            m.carry_row = m.orow_step - (uint32_t)m.groups_per_row * m.group_step;
+            m.carry_img = m.img_step - (uint32_t)g.OH * m.orow_step;
+        }
+        m.spin_limit = p.spin_limit;
+        m.wait_error = p.wait_error;
+        int32_t *const part = reinterpret_cast<int32_t *>(ws + pd.ws.part_off);
+        if (mx->k_splits > 1) {
+            m.out_f = nullptr;
+            m.out_i = part;
+        }
+        {
+            ProfScope ps("lutgemm_px", stream);
+            AXC_HIP(launch_dense_mx(m, stream));
+        }
+        if (mx->k_splits > 1) {
+            p.plan.k_splits = mx->k_splits;
+            ProfScope ps("splitk_epilogue", stream);
+            AXC_HIP(launch_splitk_epilogue(p, part, out_f, out_i, stream));
+        }
+        return AXC_OK;
     }
     if (flat) {
         p.xq_bytes = (uint32_t)((size_t)g.N * g.H * pd.flat_row_bytes);
@@ -1143,7 +1397,9 @@ int axc_conv2d_workspace_bytes(const axc_conv2d_desc *desc, size_t *bytes)
     int rc = prepare_dense(desc, &pd);
     if (rc != AXC_OK)
         return rc;
-    rc = prepare_dense(desc, &pd_plain, false);
+    int pads[2];
+    axconv_tf1_pads(pd.g_full, desc->padding, pads);
+    rc = prepare_dense(desc, &pd_plain, pads);
     if (rc != AXC_OK)
         return rc;
     *bytes = pd.ws.total > pd_plain.ws.total ? pd.ws.total : pd_plain.ws.total;
@@ -1170,14 +1426,6 @@ int axc_fake_approx_depthwise_conv2d(const axc_table *table, const axc_conv2d_de
                          workspace_bytes, stream, true, bias, activation);
 }
 
-// tf1 AxConv2D: filter origin offsets of ReferenceAxConvFunctor (tf1/axqconv/axqconv.cc:153-163), C integer division
-static void axconv_tf1_pads(const ConvGeom &g, int padding, int pads[2])
-{
-    const int extra = padding == AXC_PAD_VALID ? 1 : 0;
-    pads[0] = ((g.OH - 1) * g.sh + g.KH - g.H + extra) / 2;
-    pads[1] = ((g.OW - 1) * g.sw + g.KW - g.W + extra) / 2;
-}
-
 int axc_axconv2d_quint8(const axc_table *table, const axc_conv2d_desc *desc, const uint8_t *input,
                         const uint8_t *filter, int32_t offset_input, int32_t offset_filter, int32_t *output,
                         void *workspace, size_t workspace_bytes, void *stream)
@@ -1195,22 +1443,27 @@ int axc_axconv2d_quint8(const axc_table *table, const axc_conv2d_desc *desc, con
         return fail(AXC_INVALID_ARGUMENT, "padding must be SAME or VALID");
     if (offset_input < 0 || offset_input > 255) // the reference stores it in a quint8 for taps outside the image (:215)
         return fail(AXC_INVALID_ARGUMENT, "offset_input must be in [0, 255]");
+    axc_conv2d_dims dims;
+    int rc = geometry(desc, &dims);
+    if (rc != AXC_OK)
+        return rc;
+    rc = validate_for_launch(desc, dims, false);
+    if (rc != AXC_OK)
+        return rc;
+    int pads[2];
+    axconv_tf1_pads(make_geom(dims), desc->padding, pads);
     PreparedDense pd;
-    int rc = prepare_dense(desc, &pd, false);
+    rc = prepare_dense_for(desc, workspace_bytes, pads, 1, &pd);   // the form run_dense gives it: where its sums may go
     if (rc != AXC_OK)
         return rc;
     if (pd.empty)
         return AXC_OK;
     if (!input || !filter || !output)
         return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
-    int pads[2];
-    axconv_tf1_pads(pd.g, desc->padding, pads);
     rc = run_dense(table, desc, nullptr, nullptr, input, filter, offset_input, 0.0f, 0.0f, 0.0f, 0.0f, nullptr, output,
                    workspace, workspace_bytes, stream, false, nullptr, AXC_ACT_NONE, pads);
     if (rc != AXC_OK || pd.g.K == 0)
         return rc;
-    pd.g.ph = pads[0];
-    pd.g.pw = pads[1];
     char *ws = static_cast<char *>(workspace);
     ProfScope ps("axconv_correction", static_cast<hipStream_t>(stream));
     AXC_HIP(launch_axconv_correction(input, filter, pd.g, offset_input, offset_filter,
@@ -1312,6 +1565,22 @@ int axc_conv2d_tile_plan(const axc_conv2d_desc *desc, int32_t plan[8])
     return AXC_OK;
 }
 
+int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8])
+{
+    if (!plan)
+        return fail(AXC_INVALID_ARGUMENT, "null argument");
+    PreparedDense pd;
+    int rc = prepare_dense(desc, &pd);
+    if (rc != AXC_OK)
+        return rc;
+    const MxPlan &m = pd.mxp;
+    const int32_t v[8] = {pd.mx ? 1 : 0, m.units, m.units_per_tile, m.n_row_tiles, m.n_col_tiles, m.k_splits, m.grid,
+                          m.k_splits > 1 ? m.fills_per_split : m.fills};
+    for (int i = 0; i < 8; ++i)
+        plan[i] = pd.mx ? v[i] : 0;
+    return AXC_OK;
+}
+
 int axc_set_wait_limit(uint32_t polls)
 {
     g_wait_limit.store(polls, std::memory_order_relaxed);
@@ -1397,11 +1666,16 @@ int axc_conv2d_minmax_static(const axc_table *table, const axc_conv2d_desc *desc
     int rc = prepare_dense(desc, &pd);
     if (rc != AXC_OK)
         return rc;
-    size_t needed = pd.plan.px ? pd.ws.total : pd.ws.total_no_px;
-    if (pd.plan.px && needed > kStaticScratchBytes) {
+    if (pd.mx && pd.ws.total > kStaticScratchBytes) {   // without the room it would run as the other kernels do
+        rc = prepare_dense(desc, &pd, nullptr, 4, kPxModeGlobal, false);
+        if (rc != AXC_OK)
+            return rc;
+    }
+    size_t needed = (pd.mx || pd.plan.px) ? pd.ws.total : pd.ws.total_no_px;
+    if (!pd.mx && pd.plan.px && needed > kStaticScratchBytes) {
         // without room for pre-expanded rows the layer runs as run_dense re-plans it, or as planned minus the rows
         PreparedDense alt;
-        rc = prepare_dense(desc, &alt, true, 4, -1);
+        rc = prepare_dense(desc, &alt, nullptr, 4, -1);
         if (rc != AXC_OK)
             return rc;
         needed = std::min(alt.ws.total, pd.ws.total_no_px);

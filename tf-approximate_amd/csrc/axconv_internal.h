@@ -124,6 +124,67 @@ struct DenseParams {
     uint32_t *wait_error;
 };
 
+// ---- lutgemm_mx_kernel.hip: lookups summed by the matrix cores ----
+constexpr int kMxThreads = 256;                // four wavefronts, one per SIMD, 512 registers each
+constexpr int kMxWaves = kMxThreads / 64;
+constexpr int kMxCols = 8;                     // columns per tile
+constexpr int kMxFillQuads = 4;                // channel quads (of any taps) per fill
+constexpr int kMxUnits[] = {2, 3, 4, 6, 8, 10, 13, 16, 20, 25};   // 64-pixel units per wavefront: the kernel's variants
+
+struct MxPlan {
+    int units;             // units per wavefront, one of kMxUnits
+    int units_per_tile;    // units in a tile, at most kMxWaves * units
+    int n_row_tiles, n_col_tiles;
+    int fills;             // fills of kMxFillQuads quads over the whole K
+    int k_splits, fills_per_split;
+    int grid;
+    float cost;            // cycles the planner's model expects
+};
+
+// Quantized input with its padding written out, as lutgemm_mx_kernel reads it: dwords [n][Hp][C4][Wp], pixel (h, w) in
+// row h + row0, column w + col0.  The rows and columns in front of an image double as those behind the one before it,
+// so row0 and col0 are the larger of the two paddings; behind the last image follow row0 more rows and, where there is
+// column padding too, one for the columns behind the last of those.  Without padding (and always for the other kernels)
+// Hp = H, Wp = W, row0 = col0 = 0, and one row follows the last image.
+struct XqLayout {
+    int Hp, Wp, row0, col0;
+    __host__ __device__ int tail_rows() const { return row0 == 0 ? 1 : row0 + (col0 > 0 ? 1 : 0); }
+};
+
+struct MxDiv {             // division by a constant for 31-bit numbers: mulhi(n, mul) >> shift; mul = 0: n itself
+    uint32_t mul, shift;
+};
+
+struct MxParams {
+    MxPlan plan;
+    const void *xq;
+    uint32_t xq_bytes;
+    const uint16_t *rows;
+    uint32_t rows_bytes;
+    const float *psum, *fsum, *bias;
+    float *out_f;
+    int32_t *out_i;        // with k_splits > 1: [k_splits][M][Co] partial sums
+    const LayerQuant *lq_dev;
+    float s1xs2, m1, m2, k_m1xm2;
+    int relu;
+    int64_t M;
+    int Co, oh, ow;
+    int groups, groups_per_row;    // groups of four neighbouring pixels of an output row: of the layer, per row
+    int linear;                    // output rows are whole groups: pixel = 4 * group + position
+    MxDiv div_groups, div_oh, div_c4, div_kw;
+    // bytes in xq: of output pixel 0's tap (0, 0); between images, output rows, pixel groups, pixels of a group; between
+    // tap rows, tap columns and quads
+    uint32_t origin, img_step, orow_step, group_step, pitch, kh_step, kw_step, quad_step;
+    int c4, kw;                    // quads per tap, taps per filter row
+    int dq, dkw;                   // four quads on: quads and taps to add, and the bytes they are; then what a carry
+    uint32_t doff, qoff, kwoff;    // of the quad into the tap and of the tap into the tap row adds
+    // 64 groups on (a wavefront's next unit): output rows and groups to add (and images), the bytes they are; what a carry
+    // of the groups into the row and of the rows into the image adds to those
+    uint32_t step_rows, step_groups, step_bytes, carry_row, carry_img;
+    uint32_t spin_limit;
+    uint32_t *wait_error;
+};
+
 struct DepthwiseParams {
     int N, H, W, C, KH, KW, OH, OW, sh, sw, dh, dw, ph, pw;
     int64_t M;
@@ -194,7 +255,7 @@ double device_clock_hz();  // shader clock of the current device (cached)
 
 // ---- launchers (each enqueues on `stream`; returns hipError_t of the launch) -----------------
 hipError_t launch_quantize_relayout(const float *x, const ConvGeom &g, const TensorQuant &tq, const LayerQuant *lq_dev,
-                                    uint32_t *xq, float *chsum, hipStream_t stream);
+                                    const XqLayout &lay, uint32_t *xq, float *chsum, hipStream_t stream);
 // With xq_fused / fused given, 1x1 stride-1 layers also get their quantized activations from this pass
 // (*fused = true); the caller then skips launch_quantize_relayout.
 // The filter pre-pass of the same layer (what launch_filter_pack would do), for a launch that can take it along.
@@ -207,12 +268,14 @@ struct FilterJob {
     float *fsum;
     const uint16_t *tableT;   // with px_rows: the transposed table the pre-expanded rows are built from
     uint16_t *px_rows;        // nullptr: the layer does not run out of pre-expanded rows
+    const MxPlan *mx;         // not null: the layer runs lutgemm_mx_kernel, whose rows those are; no packed filter
 };
 // xq_fused / fused: the launch may also quantize the input into xq (then *fused is set);
 // filter_job / filter_done: it may also do the filter pre-pass (then *filter_done is set), and with it build the
 // pre-expanded rows that filter_job names (then *px_done is set).
 hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuant &tq, const LayerQuant *lq_dev,
-                             float *psum, hipStream_t stream, uint32_t *xq_fused = nullptr, bool *fused = nullptr,
+                             float *psum, hipStream_t stream, const XqLayout &lay, uint32_t *xq_fused = nullptr,
+                             bool *fused = nullptr,
                              const FilterJob *filter_job = nullptr, bool *filter_done = nullptr,
                              int flat_row_bytes = 0,   // > 0: a fused xq is written in the flat layout
                              bool *px_done = nullptr);
@@ -222,16 +285,16 @@ constexpr int kMinMaxBlocks = 2048;   // partial (min, max) pairs per tensor in 
 // out[n][oh][ow][:] = in[n][oh * sh][ow * sw][:] for tensors of element_bytes-wide elements (C per pixel)
 hipError_t launch_subsample(const void *in, int element_bytes, int N, int H, int W, int C, int sh, int sw, int OH, int OW,
                             void *out, hipStream_t stream);
-hipError_t launch_codes_relayout(const uint8_t *codes, const ConvGeom &g, uint32_t zp4, uint32_t *xq,
+hipError_t launch_codes_relayout(const uint8_t *codes, const ConvGeom &g, const XqLayout &lay, uint32_t zp4, uint32_t *xq,
                                  hipStream_t stream);
 // Flat layout of xq: rows of row_bytes bytes, pad_left pixels of the zero-point code, the W pixels' codes, zero-point
 // codes up to the end of the row; one more row of zero-point codes behind the last image.  From floats (x) or codes.
-hipError_t launch_quantize_flat_rows(const float *x, const uint8_t *codes, const ConvGeom &g, int pad_left,
-                                     int row_bytes, const TensorQuant &tq, const LayerQuant *lq_dev, uint8_t *xq,
+hipError_t launch_quantize_flat_rows(const float *x, const uint8_t *codes, const ConvGeom &g, const XqLayout &lay,
+                                     int pad_left, int row_bytes, const TensorQuant &tq, const LayerQuant *lq_dev, uint8_t *xq,
                                      hipStream_t stream);
 // tableT / px_rows / px_done: the launch may also build the pre-expanded rows of the layer (then *px_done is set)
 hipError_t launch_filter_pack(const float *filter, const uint8_t *filter_codes, const ConvGeom &g,
-                              const DensePlan &plan, const TensorQuant &tq, const LayerQuant *lq_dev,
+                              const DensePlan &plan, const MxPlan *mx, const TensorQuant &tq, const LayerQuant *lq_dev,
                               uint16_t *wq, float *fsum, hipStream_t stream, const uint16_t *tableT = nullptr,
                               uint16_t *px_rows = nullptr, bool *px_done = nullptr);
 hipError_t launch_quantize_flat(const float *v, int64_t n, float offset, float inv_scale, uint8_t *codes,
@@ -242,6 +305,10 @@ hipError_t launch_px_expand_rows(const uint16_t *wq, const uint16_t *tableT, con
                                  hipStream_t stream);
 hipError_t launch_dense_px(const DenseParams &p, bool out_i32, hipStream_t stream);
 bool px_free_running(const DensePlan &plan, int taps);   // the plan runs lutgemm_pxf_kernel (no barrier between fills)
+hipError_t launch_mx_expand_rows(const float *filter, const uint8_t *filter_codes, const ConvGeom &g, const MxPlan &plan,
+                                 const TensorQuant &tq, const LayerQuant *lq_dev, const uint16_t *tableT, uint16_t *rows,
+                                 hipStream_t stream);
+hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream);
 hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials, float *out_f, int32_t *out_i,
                                   hipStream_t stream);
 hipError_t launch_axconv_correction(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,

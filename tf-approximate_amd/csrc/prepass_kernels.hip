@@ -23,30 +23,70 @@ __device__ __forceinline__ void wait_lds_reads()
     __builtin_amdgcn_s_waitcnt(0xC07F | (PENDING << 8)); // vmcnt and expcnt left at their maxima
 }
 
+// Dword index of channel quad c4 of pixel (n, h, w) in xq, and of the first quad's row of image row nh = n * H + h.
+__device__ __forceinline__ int64_t xq_row(const XqLayout &lay, int64_t n, int h, int C4)
+{
+    return (n * lay.Hp + h + lay.row0) * C4 * lay.Wp + lay.col0;
+}
+__device__ __forceinline__ int64_t xq_row_nh(const XqLayout &lay, int64_t nh, int H, int C4)
+{
+    if (lay.Hp != H) {
+        const int64_t n = nh / H;
+        return xq_row(lay, n, (int)(nh - n * H), C4);
+    }
+    return nh * C4 * lay.Wp + lay.col0;
+}
+
+// Everything in xq that is not a pixel, every dword of it the zero-point code x4: the row(s) behind the last image, and
+// where the padding is written out the rows in front of every image and the columns in front of every row.  The
+// workgroups that write xq each take a share: thread `first` of `step`.
+__device__ __forceinline__ void xq_fill_padding(uint32_t *__restrict__ xq, const XqLayout &lay, int N, int H, int C4,
+                                                uint32_t zp4, int64_t first, int64_t step)
+{
+    const int64_t row = (int64_t)C4 * lay.Wp;
+    const int64_t rows_total = ((int64_t)N * lay.row0 + lay.tail_rows()) * row;
+    for (int64_t i = first; i < rows_total; i += step) {
+        const int64_t k = i / row;
+        int64_t r = (int64_t)N * lay.Hp + (k - (int64_t)N * lay.row0);
+        if (k < (int64_t)N * lay.row0) {
+            const int64_t n = k / lay.row0;
+            r = n * lay.Hp + (k - n * lay.row0);
+        }
+        xq[r * row + (i - k * row)] = zp4;
+    }
+    if (lay.col0 == 0)
+        return;
+    const int64_t cols_total = (int64_t)N * H * C4 * lay.col0;
+    for (int64_t i = first; i < cols_total; i += step) {
+        const int64_t pl = i / lay.col0, nh = pl / C4, n = nh / H;   // plane, image row
+        const int c4 = (int)(pl - nh * C4), h = (int)(nh - n * H);
+        xq[((n * lay.Hp + h + lay.row0) * C4 + c4) * lay.Wp + (i - pl * lay.col0)] = zp4;
+    }
+}
+
 // Input pre-pass.  Restates the quantize and the channel part of the patch sum of
 // ApproxConvIm2ColKernel (tf2/src/approx_nn_conv_kernels.cpp:288-294) once per input element
 // instead of once per patch element.
-//   xq   [N][H][C4][W]  one dword = codes of channels 4*c4 .. 4*c4+3 of one pixel, each code stored as
+//   xq   [N][H][C4][W]  (or as XqLayout says) one dword = codes of channels 4*c4 .. 4*c4+3 of one pixel, each code stored as
 //                       its expanded-row index phys_row(code)
 //   chsum[N][H][W]      sum over channels of the raw floats, c ascending
 // One thread per pixel: the channel loop is sequential so the sum has the reference's order within a pixel.
 __global__ void __launch_bounds__(256) quantize_relayout_kernel(const float *__restrict__ x, int64_t pixels,
-                                                                 int H, int W, int C, int C4, const TensorQuant tq,
+                                                                 int H, int W, int C, int C4, const XqLayout lay,
+                                                                 const TensorQuant tq,
                                                                  const LayerQuant *__restrict__ lq_dev,
                                                                  uint32_t *__restrict__ xq,
                                                                  float *__restrict__ chsum)
 {
     const TensorQuant q = lq_dev ? lq_dev->in : tq;
-    const uint32_t zp4 = q.zp4;
     const int64_t pix = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    // the extra [C4][W] row behind the image rows: every dword is the zero-point code x4
-    for (int64_t i = pix; i < (int64_t)C4 * W; i += (int64_t)gridDim.x * blockDim.x)
-        xq[pixels * C4 + i] = zp4;
+    xq_fill_padding(xq, lay, (int)(pixels / ((int64_t)H * W)), H, C4, q.zp4, pix, (int64_t)gridDim.x * blockDim.x);
     if (pix >= pixels)
         return;
     const int w = (int)(pix % W);
     const int64_t nh = pix / W; // n * H + h
     const float *src = x + pix * C;
+    uint32_t *const dst = xq + xq_row_nh(lay, nh, H, C4) + w;
     float sum = 0.0f;
     for (int c4 = 0; c4 < C4; ++c4) {
         uint32_t packed = 0;
@@ -59,7 +99,7 @@ __global__ void __launch_bounds__(256) quantize_relayout_kernel(const float *__r
                 packed |= phys_row(quantize_code(v, q.offset, q.inv_scale)) << (8 * i);
             }
         }
-        xq[(nh * C4 + c4) * W + w] = packed;
+        dst[(int64_t)c4 * lay.Wp] = packed;
     }
     if (chsum)
         chsum[pix] = sum;
@@ -68,16 +108,15 @@ __global__ void __launch_bounds__(256) quantize_relayout_kernel(const float *__r
 // Same result as quantize_relayout_kernel for C % 4 == 0, with fully coalesced reads: consecutive lanes
 // read consecutive float4 of the NHWC input (one float4 = the four channels of one xq dword).
 __global__ void __launch_bounds__(256) quantize_relayout_vec4_kernel(const float4 *__restrict__ x4, int64_t quads,
-                                                                      int W, int C4, const TensorQuant tq,
+                                                                      int H, int W, int C4, const XqLayout lay,
+                                                                      const TensorQuant tq,
                                                                       const LayerQuant *__restrict__ lq_dev,
                                                                       uint32_t *__restrict__ xq)
 {
     const TensorQuant q = lq_dev ? lq_dev->in : tq;
-    const uint32_t zp4 = q.zp4;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    // the extra [C4][W] row behind the image rows: every dword is the zero-point code x4
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (int64_t)C4 * W; i += stride)
-        xq[quads + i] = zp4;
+    xq_fill_padding(xq, lay, (int)(quads / ((int64_t)H * W * C4)), H, C4, q.zp4,
+                    (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += stride) {
         const float4 v = x4[i];
         const int64_t pix = i / C4;
@@ -88,7 +127,7 @@ __global__ void __launch_bounds__(256) quantize_relayout_vec4_kernel(const float
                                 (phys_row(quantize_code(fake_quant_value(v.y, q), q.offset, q.inv_scale)) << 8) |
                                 (phys_row(quantize_code(fake_quant_value(v.z, q), q.offset, q.inv_scale)) << 16) |
                                 (phys_row(quantize_code(fake_quant_value(v.w, q), q.offset, q.inv_scale)) << 24);
-        xq[(nh * C4 + c4) * W + w] = packed;
+        xq[xq_row_nh(lay, nh, H, C4) + (int64_t)c4 * lay.Wp + w] = packed;
     }
 }
 
@@ -256,6 +295,7 @@ struct FilterWork {
     int expand_blocks;
     const uint16_t *tableT;
     uint16_t *px_rows;
+    int mx_fills;     // > 0: rows in the form lutgemm_mx_kernel.hip reads, this many fills per column tile
 };
 
 __device__ __forceinline__ void filter_pack_element(const int64_t i, const float *__restrict__ filter,
@@ -277,16 +317,16 @@ template <bool SEG>
 __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x, const ConvGeom &g, const int rb,
                                                      const int in_rows, const int wseg, const TensorQuant &tq,
                                                      const LayerQuant *__restrict__ lq_dev, float *__restrict__ psum,
-                                                     uint32_t *__restrict__ xq, const int bid_in, const int nblocks,
+                                                     uint32_t *__restrict__ xq, const XqLayout &lay, const int bid_in, const int nblocks,
                                                      const int nthreads, const FilterWork &fw)
 {
     // xq != nullptr: the block also quantizes the input rows it owns among those it copies (the rows under its
     // own band of output rows; the launcher has checked that these lie inside every block's window and together
     // cover the image), which saves the separate quantize pass over the input.
     const TensorQuant qt = lq_dev ? lq_dev->in : tq;
-    if (xq && bid_in == 0)
-        for (int i = threadIdx.x; i < g.C4 * g.W; i += blockDim.x)
-            xq[(int64_t)g.N * g.H * g.C4 * g.W + i] = qt.zp4;
+    if (xq)
+        xq_fill_padding(xq, lay, g.N, g.H, g.C4, qt.zp4, (int64_t)bid_in * blockDim.x + threadIdx.x,
+                        (int64_t)nblocks * blockDim.x);
     extern __shared__ __align__(16) unsigned char ps_lds[];
     float *const rows = reinterpret_cast<float *>(ps_lds);
     const int t = threadIdx.x;
@@ -363,7 +403,7 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
                     *reinterpret_cast<float4 *>(&rows[(rr[u] * wc + ww[u]) * pitch + q * 4]) = f;
                     const int iw = iw_lo + ww[u];
                     if (xq && in_image && ih >= own_lo && ih < own_hi && (!SEG || (iw >= own_clo && iw < own_chi)))
-                        xq[(((int64_t)n * g.H + ih) * g.C4 + q) * g.W + iw] =
+                        xq[xq_row(lay, n, ih, g.C4) + q * lay.Wp + iw] =
                             phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
                             (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
                             (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
@@ -513,14 +553,20 @@ __global__ void __launch_bounds__(1024) patch_sums_smallc_kernel(const float *__
                                                                   const int rb, const int in_rows, const TensorQuant tq,
                                                                   const LayerQuant *__restrict__ lq_dev,
                                                                   float *__restrict__ psum, uint32_t *__restrict__ xq,
-                                                                  const int flat_row_bytes, const int pad_left)
+                                                                  const XqLayout lay, const int flat_row_bytes,
+                                                                  const int pad_left)
 {
     // flat_row_bytes > 0: xq in the flat layout (see quantize_flat_rows_kernel), rows of that many bytes
     const TensorQuant qt = lq_dev ? lq_dev->in : tq;
-    const int zp_row_dwords = flat_row_bytes ? flat_row_bytes / 4 : g.C4 * g.W;
-    if (xq && blockIdx.x == 0)
-        for (int i = threadIdx.x; i < zp_row_dwords; i += blockDim.x)
-            xq[(int64_t)g.N * g.H * zp_row_dwords + i] = qt.zp4;
+    if (xq) {   // a row of the flat layout is one "quad" of that many dwords, its horizontal padding written below
+        XqLayout l = lay;
+        if (flat_row_bytes) {
+            l.Wp = flat_row_bytes / 4;
+            l.col0 = 0;
+        }
+        xq_fill_padding(xq, l, g.N, g.H, flat_row_bytes ? 1 : g.C4, qt.zp4, (int64_t)blockIdx.x * blockDim.x + threadIdx.x,
+                        (int64_t)gridDim.x * blockDim.x);
+    }
     extern __shared__ __align__(16) unsigned char ps_lds[];
     float *const rows = reinterpret_cast<float *>(ps_lds);
     const int t = threadIdx.x;
@@ -575,7 +621,7 @@ __global__ void __launch_bounds__(1024) patch_sums_smallc_kernel(const float *__
                     ++px;
                 }
             }
-            xq[((int64_t)n * g.H + ih) * per_row + d] = packed;
+            xq[((int64_t)n * lay.Hp + ih + lay.row0) * per_row + d] = packed;
         }
     } else if (xq) {
         const int own_lo = oh0 * g.sh;           // owned input rows: [own_lo, own_hi)
@@ -591,7 +637,7 @@ __global__ void __launch_bounds__(1024) patch_sums_smallc_kernel(const float *__
             for (int k = 0; k < 4; ++k)
                 if (c4 * 4 + k < g.C)
                     packed |= phys_row(quantize_code(src[k], qt.offset, qt.inv_scale)) << (8 * k);
-            xq[(((int64_t)n * g.H + ih) * g.C4 + c4) * g.W + w] = packed;
+            xq[xq_row(lay, n, ih, g.C4) + c4 * lay.Wp + w] = packed;
         }
     }
     const int ohl = t / g.OW, ow = t - ohl * g.OW;
@@ -628,14 +674,17 @@ __global__ void __launch_bounds__(1024) patch_sums_smallc_kernel(const float *__
 
 // Same relayout for caller-supplied codes (uint8 NHWC).
 __global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__restrict__ codes, int64_t pixels,
-                                                              int W, int C, int C4, uint32_t *__restrict__ xq)
+                                                              int H, int W, int C, int C4, const XqLayout lay,
+                                                              uint32_t zp4, uint32_t *__restrict__ xq)
 {
     const int64_t pix = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    xq_fill_padding(xq, lay, (int)(pixels / ((int64_t)H * W)), H, C4, zp4, pix, (int64_t)gridDim.x * blockDim.x);
     if (pix >= pixels)
         return;
     const int w = (int)(pix % W);
     const int64_t nh = pix / W;
     const uint8_t *src = codes + pix * C;
+    uint32_t *const dst = xq + xq_row_nh(lay, nh, H, C4) + w;
     for (int c4 = 0; c4 < C4; ++c4) {
         uint32_t packed = 0;
 #pragma unroll
@@ -644,7 +693,7 @@ __global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__re
             if (c < C)
                 packed |= phys_row(src[c]) << (8 * i);
         }
-        xq[(nh * C4 + c4) * W + w] = packed;
+        dst[(int64_t)c4 * lay.Wp] = packed;
     }
 }
 
@@ -678,6 +727,23 @@ __device__ __forceinline__ uint16_t filter_code_at(const int64_t i, const float 
                             : (uint16_t)quantize_code(fake_quant_value(filter[idx], qf), qf.offset, qf.inv_scale);
     }
     return code;
+}
+
+// The filter code of one of the 128 slots of a fill of lutgemm_mx_kernel: slot = filter element * 8 + column, the fill's
+// 16 filter elements being quads 4 f .. 4 f + 3 of the K order (tap, quad).
+__device__ __forceinline__ uint16_t mx_filter_code_at(const int ct, const int f, const int slot,
+                                                      const float *__restrict__ filter,
+                                                      const uint8_t *__restrict__ filter_codes, int taps, int C, int C4,
+                                                      int Co, const TensorQuant &qf)
+{
+    const int quad = f * kMxFillQuads + (slot >> 5);
+    const int tap = quad / C4, c = (quad - tap * C4) * 4 + ((slot >> 3) & 3);
+    const int col = ct * kMxCols + (slot & 7);
+    if (tap >= taps || c >= C || col >= Co)
+        return kNullWeight;
+    const int64_t idx = ((int64_t)tap * C + c) * Co + col;
+    return filter_codes ? (uint16_t)filter_codes[idx]
+                        : (uint16_t)quantize_code(fake_quant_value(filter[idx], qf), qf.offset, qf.inv_scale);
 }
 
 __device__ __forceinline__ void filter_pack_element(const int64_t i, const float *__restrict__ filter,
@@ -801,25 +867,52 @@ __device__ __forceinline__ void filter_sums_block(const int block, const float *
 // fsum is null), the others pack the codes.
 // One (column tile, pair of fills) of the pre-expanded rows (px_expand.h) by a workgroup of 4 * CB threads that is
 // not the one that packs the pair's filter codes: it computes the 128 codes itself, into LDS behind the stage.
+// mx_fills > 0: the fill's slots and entries in lutgemm_mx_kernel's form (mx_filter_code_at, top bits flipped).
 template <int CB>
 __device__ __forceinline__ void px_expand_own_codes(const int eb, const float *__restrict__ filter,
                                                     const uint8_t *__restrict__ filter_codes, int taps, int C, int C4,
                                                     int Co, const TensorQuant &q, const uint16_t *__restrict__ tableT,
-                                                    uint16_t *__restrict__ px_rows)
+                                                    uint16_t *__restrict__ px_rows, const int mx_fills)
 {
     extern __shared__ __align__(16) unsigned char px_lds[];
     uint32_t *const stage = reinterpret_cast<uint32_t *>(px_lds);
     constexpr int kParts = 256 / CB;
-    const int fills = taps * C4, px_fills = fills / 2;   // 16-column tiles: a fill is one channel quad of a tap
+    const int fills = taps * C4, px_fills = mx_fills ? mx_fills : fills / 2;   // 16-column tiles: a fill is one channel quad of a tap
     const int part = eb % kParts, cf = eb / kParts;      // cf = ct * px_fills + f
     const int ct = cf / px_fills, f = cf - ct * px_fills;
     uint16_t *const codes = reinterpret_cast<uint16_t *>(stage + px_expand_stage_dwords<CB>());
     if (threadIdx.x < 128)
-        codes[threadIdx.x] = filter_code_at(((int64_t)ct * fills + 2 * (int64_t)f) * 64 + threadIdx.x, filter, filter_codes,
-                                            taps, C, C4, Co, 16, q);
+        codes[threadIdx.x] = mx_fills ? mx_filter_code_at(ct, f, (int)threadIdx.x, filter, filter_codes, taps, C, C4, Co, q)
+                                      : filter_code_at(((int64_t)ct * fills + 2 * (int64_t)f) * 64 + threadIdx.x, filter,
+                                                       filter_codes, taps, C, C4, Co, 16, q);
     __syncthreads();
     px_expand_part<CB>(stage, part, [&](const int sl) { return codes[sl]; }, tableT,
-                       reinterpret_cast<uint32_t *>(px_rows + (size_t)cf * (kPxFillBytes / 2)));
+                       reinterpret_cast<uint32_t *>(px_rows + (size_t)cf * (kPxFillBytes / 2)), mx_fills ? 0x80808080u : 0u);
+}
+
+// The rows of lutgemm_mx_kernel in a launch of their own, where they are too many to ride in another one.
+__global__ void __launch_bounds__(512) mx_expand_rows_kernel(const float *__restrict__ filter,
+                                                             const uint8_t *__restrict__ filter_codes, int taps, int C,
+                                                             int C4, int Co, const TensorQuant tq,
+                                                             const LayerQuant *__restrict__ lq_dev,
+                                                             const uint16_t *__restrict__ tableT,
+                                                             uint16_t *__restrict__ rows, const int mx_fills)
+{
+    px_expand_own_codes<128>((int)blockIdx.x, filter, filter_codes, taps, C, C4, Co, lq_dev ? lq_dev->flt : tq, tableT, rows,
+                             mx_fills);
+}
+
+hipError_t launch_mx_expand_rows(const float *filter, const uint8_t *filter_codes, const ConvGeom &g, const MxPlan &plan,
+                                 const TensorQuant &tq, const LayerQuant *lq_dev, const uint16_t *tableT, uint16_t *rows,
+                                 hipStream_t stream)
+{
+    const size_t lds = (size_t)px_expand_stage_dwords<128>() * 4 + 256;
+    const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(mx_expand_rows_kernel), (int)lds);
+    if (e != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(mx_expand_rows_kernel, dim3((unsigned)((int64_t)plan.n_col_tiles * plan.fills * 2)), dim3(512), lds,
+                       stream, filter, filter_codes, g.KH * g.KW, g.C, g.C4, g.Co, tq, lq_dev, tableT, rows, plan.fills);
+    return hipGetLastError();
 }
 
 // One launch for the whole filter pre-pass: the first sum_blocks workgroups compute the column sums (skipped when
@@ -832,7 +925,7 @@ __global__ void __launch_bounds__(kFsThreads) filter_prep_kernel(const float *__
                                                                   uint16_t *__restrict__ wq, int sum_blocks,
                                                                   float *__restrict__ fsum, int pack_blocks,
                                                                   const uint16_t *__restrict__ tableT,
-                                                                  uint16_t *__restrict__ px_rows)
+                                                                  uint16_t *__restrict__ px_rows, const int mx_fills)
 {
     const TensorQuant q = lq_dev ? lq_dev->flt : tq;
     if ((int)blockIdx.x < sum_blocks) {
@@ -845,7 +938,7 @@ __global__ void __launch_bounds__(kFsThreads) filter_prep_kernel(const float *__
         filter_pack_element(i, filter, filter_codes, taps, C, C4, Co, nt, n_col_tiles, q, wq);
         return;
     }
-    px_expand_own_codes<kFsThreads / 4>(pb - pack_blocks, filter, filter_codes, taps, C, C4, Co, q, tableT, px_rows);
+    px_expand_own_codes<kFsThreads / 4>(pb - pack_blocks, filter, filter_codes, taps, C, C4, Co, q, tableT, px_rows, mx_fills);
 }
 
 // Patch sums of a 1x1, stride-1, unpadded layer: the patch of an output pixel is the pixel itself, so the pixels
@@ -861,13 +954,14 @@ constexpr int kFlatPer = kFlatPixels * (kFlatChunk / 4) / kFlatThreads; // 16-by
 __device__ __forceinline__ void patch_sums_flat_body(const float *__restrict__ x, const ConvGeom &g,
                                                      const TensorQuant &tq, const LayerQuant *__restrict__ lq_dev,
                                                      float *__restrict__ psum, uint32_t *__restrict__ xq,
-                                                     const int bid, const int pixels)
+                                                     const XqLayout &lay, const int bid, const int nblocks,
+                                                     const int pixels)
 {
     // pixels: pixels per workgroup, 64 / 128 / 256 (fewer when the layer has few pixels, for enough workgroups)
     const TensorQuant qt = lq_dev ? lq_dev->in : tq;
-    if (xq && bid == 0)
-        for (int i = threadIdx.x; i < g.C4 * g.W; i += blockDim.x)
-            xq[(int64_t)g.N * g.H * g.C4 * g.W + i] = qt.zp4;
+    if (xq)
+        xq_fill_padding(xq, lay, g.N, g.H, g.C4, qt.zp4, (int64_t)bid * blockDim.x + threadIdx.x,
+                        (int64_t)nblocks * blockDim.x);
     extern __shared__ __align__(16) unsigned char pf_lds[];
     float *const rows = reinterpret_cast<float *>(pf_lds);
     const int t = threadIdx.x;
@@ -890,7 +984,7 @@ __device__ __forceinline__ void patch_sums_flat_body(const float *__restrict__ x
     {
         const int64_t m = m0 + (code_px < npx ? code_px : 0);
         const int64_t nh = m / g.W;
-        code_idx = (uint32_t)(nh * g.C4 * g.W + (m - nh * g.W));
+        code_idx = (uint32_t)(xq_row_nh(lay, nh, g.H, g.C4) + (m - nh * g.W));
     }
     const int chunks = (g.C + kFlatChunk - 1) / kFlatChunk;
     float4 v[kFlatPer];
@@ -926,7 +1020,7 @@ __device__ __forceinline__ void patch_sums_flat_body(const float *__restrict__ x
             const int nq = (g.C - c0 < kFlatChunk ? g.C - c0 : kFlatChunk) / 4;
             for (int qq = code_q0; qq < nq; qq += code_qstep) {
                 const float4 f = *reinterpret_cast<const float4 *>(&rows[code_px * kFlatPitch + qq * 4]);
-                xq[code_idx + (uint32_t)(c0 / 4 + qq) * (uint32_t)g.W] =
+                xq[code_idx + (uint32_t)(c0 / 4 + qq) * (uint32_t)lay.Wp] =
                     phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
                     (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
                     (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
@@ -967,14 +1061,14 @@ template <int PIXELS>
 __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x, const ConvGeom &g,
                                                      const TensorQuant &tq, const LayerQuant *__restrict__ lq_dev,
                                                      float *__restrict__ psum, uint32_t *__restrict__ xq,
-                                                     const int bid)
+                                                     const XqLayout &lay, const int bid, const int nblocks)
 {
     constexpr int pixels = PIXELS, kDeepMaxPixels = PIXELS;
     constexpr int kDeepPer = PIXELS * (kDeepChunk / 4) / kDeepThreads; // 16-byte loads per thread and pass
     const TensorQuant qt = lq_dev ? lq_dev->in : tq;
-    if (xq && bid == 0)
-        for (int i = threadIdx.x; i < g.C4 * g.W; i += blockDim.x)
-            xq[(int64_t)g.N * g.H * g.C4 * g.W + i] = qt.zp4;
+    if (xq)
+        xq_fill_padding(xq, lay, g.N, g.H, g.C4, qt.zp4, (int64_t)bid * blockDim.x + threadIdx.x,
+                        (int64_t)nblocks * blockDim.x);
     extern __shared__ __align__(16) unsigned char pd_lds[];
     float *const stage = reinterpret_cast<float *>(pd_lds);
     const int t = threadIdx.x;
@@ -994,7 +1088,7 @@ __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x
         const int64_t m = m0 + (px < npx ? px : npx - 1);
         const int64_t nh = m / g.W;
         const int w = (int)(m - nh * g.W);
-        xq_idx[k] = (uint32_t)((nh * g.C4 + q) * g.W + w);
+        xq_idx[k] = (uint32_t)(xq_row_nh(lay, nh, g.H, g.C4) + (int64_t)q * lay.Wp + w);
         src[k] = x + m * g.C;
     }
     float4 v[kDeepAhead][kDeepPer];
@@ -1017,7 +1111,7 @@ __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x
             if (loader && px < kDeepMaxPixels)
                 *reinterpret_cast<float4 *>(&half[px * kDeepPitch + q * 4]) = f;
             if (xq && px_ok[k] && c_ok)
-                xq[xq_idx[k] + (uint32_t)(pass * (kDeepChunk / 4)) * (uint32_t)g.W] =
+                xq[xq_idx[k] + (uint32_t)(pass * (kDeepChunk / 4)) * (uint32_t)lay.Wp] =
                     phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
                     (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
                     (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
@@ -1115,9 +1209,11 @@ __device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const La
     // pre-expanded rows: blockDim.x / 4 activation codes of a pair of fills per workgroup
     const int eb = pb - fw.pack_blocks;
     if (blockDim.x == 512)
-        px_expand_own_codes<128>(eb, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, q, fw.tableT, fw.px_rows);
+        px_expand_own_codes<128>(eb, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, q, fw.tableT, fw.px_rows,
+                                 fw.mx_fills);
     else
-        px_expand_own_codes<256>(eb, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, q, fw.tableT, fw.px_rows);
+        px_expand_own_codes<256>(eb, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, q, fw.tableT, fw.px_rows,
+                                 fw.mx_fills);
     return true;
 }
 
@@ -1127,35 +1223,35 @@ __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *
                                                                     const TensorQuant tq,
                                                                     const LayerQuant *__restrict__ lq_dev,
                                                                     float *__restrict__ psum, uint32_t *__restrict__ xq,
-                                                                    const FilterWork fw)
+                                                                    const XqLayout lay, const FilterWork fw)
 {
     int bid;
     if (filter_work_block(fw, lq_dev, &bid))
         return;
-    patch_sums_rows_body<true>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, bid, fw.work_blocks, nthreads, fw);
+    patch_sums_rows_body<true>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw);
 }
 
 __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__restrict__ x, const ConvGeom g, int rb,
                                                                 int in_rows, int nthreads, const TensorQuant tq,
                                                                 const LayerQuant *__restrict__ lq_dev,
                                                                 float *__restrict__ psum, uint32_t *__restrict__ xq,
-                                                                const FilterWork fw)
+                                                                const XqLayout lay, const FilterWork fw)
 {
     int bid;
     if (filter_work_block(fw, lq_dev, &bid))
         return;
     if (rb < 0) { // 1x1, stride 1, many channels, few pixels
         if (in_rows == 8)
-            patch_sums_deep_body<8>(x, g, tq, lq_dev, psum, xq, bid);
+            patch_sums_deep_body<8>(x, g, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks);
         else
-            patch_sums_deep_body<16>(x, g, tq, lq_dev, psum, xq, bid);
+            patch_sums_deep_body<16>(x, g, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks);
         return;
     }
     if (rb == 0) { // 1x1, stride 1: flat pixel list
-        patch_sums_flat_body(x, g, tq, lq_dev, psum, xq, bid, in_rows);
+        patch_sums_flat_body(x, g, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, in_rows);
         return;
     }
-    patch_sums_rows_body<false>(x, g, rb, in_rows, g.OW, tq, lq_dev, psum, xq, bid, fw.work_blocks, nthreads, fw);
+    patch_sums_rows_body<false>(x, g, rb, in_rows, g.OW, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw);
 }
 
 __global__ void __launch_bounds__(256) quantize_flat_kernel(const float *__restrict__ v, int64_t n, float offset,
@@ -1483,16 +1579,8 @@ hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials,
     return hipGetLastError();
 }
 
-static hipError_t launch_zero_point_row(const ConvGeom &g, uint32_t zp4, uint32_t *xq, hipStream_t stream)
-{
-    const int n = g.C4 * g.W;
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream,
-                       xq + (size_t)g.N * g.H * g.C4 * g.W, n, zp4);
-    return hipGetLastError();
-}
-
 hipError_t launch_quantize_relayout(const float *x, const ConvGeom &g, const TensorQuant &tq, const LayerQuant *lq_dev,
-                                    uint32_t *xq, float *chsum, hipStream_t stream)
+                                    const XqLayout &lay, uint32_t *xq, float *chsum, hipStream_t stream)
 {
     const int64_t pixels = (int64_t)g.N * g.H * g.W;
     if ((g.C & 3) == 0 && !chsum && ((uintptr_t)x & 15) == 0) {
@@ -1500,11 +1588,11 @@ hipError_t launch_quantize_relayout(const float *x, const ConvGeom &g, const Ten
         int64_t blocks = (quads + 256 * 4 - 1) / (256 * 4);
         if (blocks > 65536) blocks = 65536;
         hipLaunchKernelGGL(quantize_relayout_vec4_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
-                           reinterpret_cast<const float4 *>(x), quads, g.W, g.C4, tq, lq_dev, xq);
+                           reinterpret_cast<const float4 *>(x), quads, g.H, g.W, g.C4, lay, tq, lq_dev, xq);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(quantize_relayout_kernel, dim3(blocks_for(pixels, 256)), dim3(256), 0, stream, x, pixels,
-                       g.H, g.W, g.C, g.C4, tq, lq_dev, xq, chsum);
+                       g.H, g.W, g.C, g.C4, lay, tq, lq_dev, xq, chsum);
     return hipGetLastError();
 }
 
@@ -1627,7 +1715,7 @@ static void choose_band(const ConvGeom &g, int sum_blocks, int *rb_out, int *in_
 }
 
 hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuant &tq, const LayerQuant *lq_dev,
-                             float *psum, hipStream_t stream, uint32_t *xq_fused, bool *fused,
+                             float *psum, hipStream_t stream, const XqLayout &lay, uint32_t *xq_fused, bool *fused,
                              const FilterJob *filter_job, bool *filter_done, int flat_row_bytes, bool *px_done)
 {
     if (fused)
@@ -1701,7 +1789,8 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             int block_threads = threads;
             if (filter_job && filter_done) {
                 const DensePlan &plan = *filter_job->plan;
-                const int64_t total = (int64_t)plan.n_col_tiles * plan.fills * 64;
+                const MxPlan *const mx = filter_job->mx;   // its kernel reads rows only: nothing to pack
+                const int64_t total = mx ? 0 : (int64_t)plan.n_col_tiles * plan.fills * 64;
                 fw.filter = filter_job->filter;
                 fw.filter_codes = filter_job->filter_codes;
                 fw.taps = g.KH * g.KW;
@@ -1727,9 +1816,10 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                 *filter_done = true;
                 // ... and so do the pre-expanded rows where the layer runs out of them: blockDim.x / 4 activation
                 // codes of a pair of fills per workgroup, the stage and the pair's 128 filter codes in LDS
-                if (px_done && filter_job->px_rows && plan.nt == 16 && plan.fills == fw.taps * fw.C4 &&
-                    (plan.fills & 1) == 0) {
-                    const int64_t eb = (int64_t)plan.n_col_tiles * (plan.fills / 2) * (1024 / block_threads);
+                const int64_t row_fills = mx ? (int64_t)mx->n_col_tiles * mx->fills : (int64_t)plan.n_col_tiles * (plan.fills / 2);
+                if (px_done && filter_job->px_rows &&
+                    (mx || (plan.nt == 16 && plan.fills == fw.taps * fw.C4 && (plan.fills & 1) == 0))) {
+                    const int64_t eb = row_fills * (1024 / block_threads);
                     const size_t need = (size_t)(block_threads / 4) * kPxExpandPitch * 4 + 256;
                     // Every workgroup of a launch takes the same LDS.  Where the patch sums take so much that a CU
                     // holds fewer of these workgroups than its wavefront slots allow (2048 threads), the rows are
@@ -1737,12 +1827,13 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                     // @28x28 -3.1 %) until the rows are many (1.2 GB: 0.26 -> 0.33 ms, +2.3 % on the layer).
                     const size_t lds_with = lds < need ? need : lds;
                     const bool slow = lds_with * (size_t)(2048 / block_threads) > (size_t)device_lds_bytes();
-                    const size_t row_bytes = (size_t)plan.n_col_tiles * (size_t)(plan.fills / 2) * kPxFillBytes;
+                    const size_t row_bytes = (size_t)row_fills * kPxFillBytes;
                     if (eb + fw.sum8 + work_blocks + fw.pack_blocks < ((int64_t)1 << 31) &&
                         lds_with <= (size_t)device_lds_bytes() && !(slow && row_bytes > ((size_t)512 << 20))) {
                         fw.expand_blocks = (int)eb;
                         fw.tableT = filter_job->tableT;
                         fw.px_rows = filter_job->px_rows;
+                        fw.mx_fills = mx ? mx->fills : 0;
                         lds = lds < need ? need : lds;
                         *px_done = true;
                     }
@@ -1756,14 +1847,14 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                 if (e != hipSuccess)
                     return e;
                 hipLaunchKernelGGL(patch_sums_segments_kernel, dim3(grid), dim3(block_threads), lds, stream, x, g, rb, in_rows, threads, wseg, tq, lq_dev, psum,
-                                   fuse ? xq_fused : nullptr, fw);
+                                   fuse ? xq_fused : nullptr, lay, fw);
                 return hipGetLastError();
             }
             const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(patch_sums_rows_kernel), device_lds_bytes());
             if (e != hipSuccess)
                 return e;
             hipLaunchKernelGGL(patch_sums_rows_kernel, dim3(grid), dim3(block_threads),
-                               lds, stream, x, g, rb, in_rows, threads, tq, lq_dev, psum, fuse ? xq_fused : nullptr, fw);
+                               lds, stream, x, g, rb, in_rows, threads, tq, lq_dev, psum, fuse ? xq_fused : nullptr, lay, fw);
             return hipGetLastError();
         }
     }
@@ -1793,7 +1884,7 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             const int bands = (g.OH + rb - 1) / rb;
             hipLaunchKernelGGL(patch_sums_smallc_kernel, dim3((unsigned)((int64_t)g.N * bands)), dim3(threads),
                                (size_t)in_rows * row_bytes, stream, x, g, rb, in_rows, tq, lq_dev, psum,
-                               fuse ? xq_fused : nullptr, flat_row_bytes, g.pw);
+                               fuse ? xq_fused : nullptr, lay, flat_row_bytes, g.pw);
             return hipGetLastError();
         }
     }
@@ -1846,38 +1937,38 @@ hipError_t launch_subsample(const void *in, int element_bytes, int N, int H, int
     return hipGetLastError();
 }
 
-hipError_t launch_codes_relayout(const uint8_t *codes, const ConvGeom &g, uint32_t zp4, uint32_t *xq,
+hipError_t launch_codes_relayout(const uint8_t *codes, const ConvGeom &g, const XqLayout &lay, uint32_t zp4, uint32_t *xq,
                                  hipStream_t stream)
 {
-    hipError_t ez = launch_zero_point_row(g, zp4, xq, stream);
-    if (ez != hipSuccess)
-        return ez;
     const int64_t pixels = (int64_t)g.N * g.H * g.W;
-    hipLaunchKernelGGL(codes_relayout_kernel, dim3(blocks_for(pixels, 256)), dim3(256), 0, stream, codes, pixels,
-                       g.W, g.C, g.C4, xq);
+    hipLaunchKernelGGL(codes_relayout_kernel, dim3(blocks_for(pixels, 256)), dim3(256), 0, stream, codes, pixels, g.H,
+                       g.W, g.C, g.C4, lay, zp4, xq);
     return hipGetLastError();
 }
 
 hipError_t launch_filter_pack(const float *filter, const uint8_t *filter_codes, const ConvGeom &g,
-                              const DensePlan &plan, const TensorQuant &tq, const LayerQuant *lq_dev, uint16_t *wq,
+                              const DensePlan &plan, const MxPlan *mx, const TensorQuant &tq, const LayerQuant *lq_dev, uint16_t *wq,
                               float *fsum, hipStream_t stream, const uint16_t *tableT, uint16_t *px_rows, bool *px_done)
 {
     if (px_done)
         *px_done = false;
-    const int64_t total = (int64_t)plan.n_col_tiles * plan.fills * 64;
+    const int64_t total = mx ? 0 : (int64_t)plan.n_col_tiles * plan.fills * 64;   // lutgemm_mx_kernel reads rows only
     const int sum_blocks = (fsum && filter) ? (int)blocks_for(g.Co, kFsCols) : 0;
     const int pack_blocks = (int)blocks_for(total, kFsThreads);
     size_t lds = sum_blocks ? kFsLdsBytes : 0;
     // the pre-expanded rows ride along as in launch_patch_sums: a whole pair of fills per workgroup of 1024
     int64_t expand_blocks = 0;
-    const size_t row_bytes = (size_t)plan.n_col_tiles * (size_t)(plan.fills / 2) * kPxFillBytes;
-    if (px_done && px_rows && plan.nt == 16 && plan.fills == g.KH * g.KW * g.C4 && (plan.fills & 1) == 0 &&
+    const int64_t row_fills = mx ? (int64_t)mx->n_col_tiles * mx->fills : (int64_t)plan.n_col_tiles * (plan.fills / 2);
+    const size_t row_bytes = (size_t)row_fills * kPxFillBytes;
+    if (px_done && px_rows && (mx || (plan.nt == 16 && plan.fills == g.KH * g.KW * g.C4 && (plan.fills & 1) == 0)) &&
         row_bytes <= ((size_t)512 << 20)) {
-        expand_blocks = (int64_t)plan.n_col_tiles * (plan.fills / 2);
+        expand_blocks = row_fills;
         const size_t need = (size_t)(kFsThreads / 4) * kPxExpandPitch * 4 + 256;
         lds = lds < need ? need : lds;
         *px_done = true;
     }
+    if (sum_blocks + pack_blocks + expand_blocks == 0)   // rows in a launch of their own, nothing else to do
+        return hipSuccess;
     if (lds) {
         const hipError_t ea = set_max_dynamic_lds_once(reinterpret_cast<const void *>(filter_prep_kernel),
                                                        (int)(lds > (size_t)kFsLdsBytes ? lds : (size_t)kFsLdsBytes));
@@ -1886,17 +1977,17 @@ hipError_t launch_filter_pack(const float *filter, const uint8_t *filter_codes, 
     }
     hipLaunchKernelGGL(filter_prep_kernel, dim3((unsigned)(sum_blocks + pack_blocks + expand_blocks)), dim3(kFsThreads), lds,
                        stream, filter, filter_codes, g.KH * g.KW, g.C, g.C4, g.Co, plan.nt, plan.n_col_tiles, tq, lq_dev,
-                       wq, sum_blocks, fsum, pack_blocks, tableT, px_rows);
+                       wq, sum_blocks, fsum, pack_blocks, tableT, px_rows, mx ? mx->fills : 0);
     return hipGetLastError();
 }
 
 // Flat layout of the quantized input for channel counts that are no multiple of four: one thread per dword of xq.
-// Byte b of row r (r = image * H + input row; row N * H is the zero-point row that taps outside the image read)
-// is the code of channel b % C of pixel b / C - pad_left, the zero-point code where that pixel lies outside the
+// Byte b of row r (r = image * Hp + row0 + input row; the other rows are zero-point rows that taps outside the image
+// read) is the code of channel b % C of pixel b / C - pad_left, the zero-point code where that pixel lies outside the
 // image or b lies behind the last pixel.
 __global__ void __launch_bounds__(256) quantize_flat_rows_kernel(const float *__restrict__ x,
-                                                                 const uint8_t *__restrict__ codes, int64_t rows,
-                                                                 int W, int C, int pad_left, int row_bytes,
+                                                                 const uint8_t *__restrict__ codes, int N, int H,
+                                                                 const XqLayout lay, int W, int C, int pad_left, int row_bytes,
                                                                  const TensorQuant tq,
                                                                  const LayerQuant *__restrict__ lq_dev,
                                                                  uint32_t *__restrict__ xq)
@@ -1904,9 +1995,10 @@ __global__ void __launch_bounds__(256) quantize_flat_rows_kernel(const float *__
     const TensorQuant qt = lq_dev ? lq_dev->in : tq;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;   // dword index
     const int dwords_per_row = row_bytes / 4;
-    if (i >= (rows + 1) * dwords_per_row)
+    if (i >= ((int64_t)N * lay.Hp + lay.tail_rows()) * dwords_per_row)
         return;
-    const int64_t r = i / dwords_per_row;
+    const int64_t r = i / dwords_per_row, n = r / lay.Hp;
+    const int h = (int)(r - n * lay.Hp) - lay.row0;
     const int b0 = (int)(i - r * dwords_per_row) * 4;
     const uint32_t zp = qt.zp4 & 0xffu;
     uint32_t word = 0;
@@ -1915,8 +2007,8 @@ __global__ void __launch_bounds__(256) quantize_flat_rows_kernel(const float *__
         const int b = b0 + k;
         const int px = b / C, c = b - px * C, w = px - pad_left;
         uint32_t code = zp;
-        if (r < rows && (unsigned)w < (unsigned)W) {
-            const int64_t src = (r * W + w) * C + c;
+        if (n < N && h >= 0 && (unsigned)w < (unsigned)W) {
+            const int64_t src = ((n * H + h) * W + w) * C + c;
             code = codes ? phys_row(codes[src])
                          : phys_row(quantize_code(fake_quant_value(x[src], qt), qt.offset, qt.inv_scale));
         }
@@ -1925,13 +2017,12 @@ __global__ void __launch_bounds__(256) quantize_flat_rows_kernel(const float *__
     xq[i] = word;
 }
 
-hipError_t launch_quantize_flat_rows(const float *x, const uint8_t *codes, const ConvGeom &g, int pad_left,
+hipError_t launch_quantize_flat_rows(const float *x, const uint8_t *codes, const ConvGeom &g, const XqLayout &lay, int pad_left,
                                      int row_bytes, const TensorQuant &tq, const LayerQuant *lq_dev, uint8_t *xq,
                                      hipStream_t stream)
 {
-    const int64_t rows = (int64_t)g.N * g.H;
-    const int64_t dwords = (rows + 1) * (row_bytes / 4);
-    hipLaunchKernelGGL(quantize_flat_rows_kernel, dim3(blocks_for(dwords, 256)), dim3(256), 0, stream, x, codes, rows,
+    const int64_t dwords = ((int64_t)g.N * lay.Hp + lay.tail_rows()) * (row_bytes / 4);
+    hipLaunchKernelGGL(quantize_flat_rows_kernel, dim3(blocks_for(dwords, 256)), dim3(256), 0, stream, x, codes, g.N, g.H, lay,
                        g.W, g.C, pad_left, row_bytes, tq, lq_dev, reinterpret_cast<uint32_t *>(xq));
     return hipGetLastError();
 }

@@ -26,10 +26,11 @@ constexpr int px_expand_stage_dwords() { return CB * kPxExpandPitch; }
 // stage: CB * kPxExpandPitch dwords of LDS; code_of(s): filter code of slot s (0..127) of the fill; dst: the fill's
 // 64 KiB in memory; part: which CB activation codes.  All 4 * CB threads of the workgroup's first wavefronts call it
 // (threadIdx.x < 4 * CB); contains a barrier that every thread of the workgroup must reach: threads beyond 4 * CB
-// call px_expand_idle() instead.
+// call px_expand_idle() instead.  flip: exclusive-or'd into every pair of entries.
 template <int CB, typename CodeOf>
 __device__ __forceinline__ void px_expand_part(uint32_t *__restrict__ stage, const int part, CodeOf code_of,
-                                               const uint16_t *__restrict__ tableT, uint32_t *__restrict__ dst)
+                                               const uint16_t *__restrict__ tableT, uint32_t *__restrict__ dst,
+                                               const uint32_t flip = 0u)
 {
     const uint32_t al = threadIdx.x % CB, a = (uint32_t)part * CB + al;
     const int quarter = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / CB));
@@ -37,7 +38,7 @@ __device__ __forceinline__ void px_expand_part(uint32_t *__restrict__ stage, con
     for (int d = 0; d < 16; ++d) {
         const uint32_t lo = tableT[(uint32_t)code_of(quarter * 32 + 2 * d) * 256u + a];
         const uint32_t hi = tableT[(uint32_t)code_of(quarter * 32 + 2 * d + 1) * 256u + a];
-        stage[al * kPxExpandPitch + quarter * 16 + d] = lo | (hi << 16);
+        stage[al * kPxExpandPitch + quarter * 16 + d] = (lo | (hi << 16)) ^ flip;
     }
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;

@@ -332,6 +332,18 @@ def conv2d_tile_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding="S
     return dict(zip(keys, [int(v) for v in plan]))
 
 
+def conv2d_matrix_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding="SAME", dilations=(1, 1, 1, 1)):
+    """How the kernel whose sums the matrix cores make cuts a layer on the current device, as a dict; None for a layer
+    that does not run it."""
+    lib = _lib.load()
+    desc = make_desc(tuple(input_shape), tuple(filter_shape), list(strides), padding, (), "NHWC", list(dilations), 8)
+    plan = (ctypes.c_int32 * 8)()
+    _check(lib.axc_conv2d_matrix_plan(ctypes.byref(desc), plan))
+    keys = ("units_per_wavefront", "units_per_tile", "row_tiles", "column_tiles", "k_splits", "workgroups",
+            "fills_per_split")
+    return dict(zip(keys, [int(v) for v in plan[1:]])) if plan[0] else None
+
+
 def set_tile_columns(columns):
     """Pins the dense kernel's tile width (16 / 32 / 64 columns; 0 = the planner's choice) for the whole process."""
     _check(_lib.load().axc_set_tile_columns(int(columns)))
