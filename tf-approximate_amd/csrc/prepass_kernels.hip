@@ -1807,7 +1807,10 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                 // A block of pack work would hold a patch-sum block's worth of LDS for nothing: with bands of rows
                 // (large LDS, most threads idle while the chains run) idle wavefronts of the patch-sum blocks pack,
                 // those on SIMDs that hold no chain, so at most three chain wavefronts per block.
-                if (!flat && rb * wseg <= 3 * 64)
+                // Only while each of them has a few elements to pack: under few patch-sum blocks the packing would outlast
+                // everything else (3x3 512->512 on one 7x7 image: 880 elements a thread, 505 us of a launch of 41).
+                const int64_t packers = work_blocks * (block_threads / 4) * (4 - (rb * wseg + 63) / 64);
+                if (!flat && rb * wseg <= 3 * 64 && total <= 16 * packers)
                     fw.pack_total = total;
                 fw.sum8 = (fw.sum_blocks + 7) & ~7;
                 fw.pack_blocks = fw.pack_total > 0 ? 0 : (int)blocks_for(total, block_threads);
