@@ -887,7 +887,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
               const uint8_t *input_codes, const uint8_t *filter_codes, int input_zero_code,
               float in_min, float in_max, float f_min, float f_max, float *out_f, int32_t *out_i,
               void *workspace, size_t workspace_bytes, void *stream_v, bool layer_mode = false,
-              const float *bias = nullptr, int activation = AXC_ACT_NONE, const int *pad_before_override = nullptr)
+              const float *bias = nullptr, int activation = AXC_ACT_NONE, const int *pad_before_override = nullptr,
+              const int32_t *tf1_offset_filter = nullptr)
 {
     if (!table || !desc)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
@@ -999,6 +1000,15 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
                                    (out_f && !codes_mode) ? fsum : nullptr, stream, table->dev_tableT, px_rows, &px_done));
     }
 
+    // tf1 op (codes in, int32 out: neither patch nor filter sums of floats): the terms of its zero points, in their place
+    int32_t *const pixel_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(psum) : nullptr;
+    int32_t *const column_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(fsum) : nullptr;
+    if (tf1_offset_filter) {
+        ProfScope ps("axconv_terms", stream);
+        AXC_HIP(launch_axconv_terms(input_codes, filter_codes, g, input_zero_code, *tf1_offset_filter, pixel_term, column_term,
+                                    stream));
+    }
+
     DenseParams p;
     p.g = gk;
     p.g.ph = g.ph;   // a caller's own padding origin (never with the flat layout)
@@ -1054,6 +1064,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         m.psum = psum;
         m.fsum = fsum;
         m.bias = bias;
+        m.pixel_term = pixel_term;
+        m.column_term = column_term;
         m.out_f = out_f;
         m.out_i = out_i;
         m.lq_dev = lq_dev;
@@ -1157,29 +1169,26 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             p.stagger_sleeps = sleeps < 1 ? 1 : (sleeps > 8 ? 8 : sleeps);
         }
     }
-    if (pd.plan.k_splits > 1) {
-        int32_t *part = reinterpret_cast<int32_t *>(ws + pd.ws.part_off);
+    const bool splits = pd.plan.k_splits > 1;
+    int32_t *const part = reinterpret_cast<int32_t *>(ws + pd.ws.part_off);
+    if (splits) {
         p.out_f = nullptr;
         p.out_i = part;
-        if (use_px) {
-            ProfScope ps("lutgemm_px", stream);
-            AXC_HIP(launch_dense_px(p, true, stream));
-        } else {
-            ProfScope ps("lutgemm_expand", stream);
-            AXC_HIP(launch_dense(p, true, stream));
-        }
-        ProfScope ps("splitk_epilogue", stream);
-        AXC_HIP(launch_splitk_epilogue(p, part, out_f, out_i, stream));
-        return AXC_OK;
     }
     if (use_px) {
         ProfScope ps("lutgemm_px", stream);
-        AXC_HIP(launch_dense_px(p, out_i != nullptr, stream));
-        return AXC_OK;
-    }
-    {
+        AXC_HIP(launch_dense_px(p, p.out_i != nullptr, stream));
+    } else {
         ProfScope ps("lutgemm_expand", stream);
-        AXC_HIP(launch_dense(p, out_i != nullptr, stream));
+        AXC_HIP(launch_dense(p, p.out_i != nullptr, stream));
+    }
+    if (splits) {
+        ProfScope ps("splitk_epilogue", stream);
+        AXC_HIP(launch_splitk_epilogue(p, part, out_f, out_i, stream));
+    }
+    if (tf1_offset_filter) {
+        ProfScope ps("axconv_correction", stream);
+        AXC_HIP(launch_axconv_correction(g, pixel_term, column_term, out_i, stream));
     }
     return AXC_OK;
 }
@@ -1460,17 +1469,8 @@ int axc_axconv2d_quint8(const axc_table *table, const axc_conv2d_desc *desc, con
         return AXC_OK;
     if (!input || !filter || !output)
         return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
-    rc = run_dense(table, desc, nullptr, nullptr, input, filter, offset_input, 0.0f, 0.0f, 0.0f, 0.0f, nullptr, output,
-                   workspace, workspace_bytes, stream, false, nullptr, AXC_ACT_NONE, pads);
-    if (rc != AXC_OK || pd.g.K == 0)
-        return rc;
-    char *ws = static_cast<char *>(workspace);
-    ProfScope ps("axconv_correction", static_cast<hipStream_t>(stream));
-    AXC_HIP(launch_axconv_correction(input, filter, pd.g, offset_input, offset_filter,
-                                     reinterpret_cast<int32_t *>(ws + pd.ws.psum_off),
-                                     reinterpret_cast<int32_t *>(ws + pd.ws.fsum_off), output,
-                                     static_cast<hipStream_t>(stream)));
-    return AXC_OK;
+    return run_dense(table, desc, nullptr, nullptr, input, filter, offset_input, 0.0f, 0.0f, 0.0f, 0.0f, nullptr, output,
+                     workspace, workspace_bytes, stream, false, nullptr, AXC_ACT_NONE, pads, &offset_filter);
 }
 
 // AxTune of ApproximateSelector::init (tf1/axqconv/approximate_selector.h:52-85): weight column w is replaced by

@@ -162,6 +162,7 @@ struct MxParams {
     const uint16_t *rows;
     uint32_t rows_bytes;
     const float *psum, *fsum, *bias;
+    const int32_t *pixel_term, *column_term;   // not null (tf1 op): added to the integer outputs, by the first K split
     float *out_f;
     int32_t *out_i;        // with k_splits > 1: [k_splits][M][Co] partial sums
     const LayerQuant *lq_dev;
@@ -311,8 +312,12 @@ hipError_t launch_mx_expand_rows(const float *filter, const uint8_t *filter_code
 hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream);
 hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials, float *out_f, int32_t *out_i,
                                   hipStream_t stream);
-hipError_t launch_axconv_correction(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,
-                                    int offset_filter, int32_t *asum, int32_t *bsum, int32_t *out, hipStream_t stream);
+// tf1 AxConv2D: what the zero points add to the sums of products, per output pixel and per output column; and the pass
+// that adds them to finished sums (lutgemm_mx_kernel does so as it stores)
+hipError_t launch_axconv_terms(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,
+                               int offset_filter, int32_t *pixel_term, int32_t *column_term, hipStream_t stream);
+hipError_t launch_axconv_correction(const ConvGeom &g, const int32_t *pixel_term, const int32_t *column_term, int32_t *out,
+                                    hipStream_t stream);
 hipError_t launch_fill_u32(uint32_t *dst, int64_t n, uint32_t value, hipStream_t stream);
 hipError_t launch_depthwise_filter(const float *filter, int taps, int C, const TensorQuant &tq,
                                    const LayerQuant *lq_dev, uint8_t *wcodes, float *fsum, hipStream_t stream);

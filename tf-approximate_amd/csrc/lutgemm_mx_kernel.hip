@@ -292,14 +292,19 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         const bool quads = (p.Co & 3) == 0;
         const float e_s1xs2 = p.lq_dev ? p.lq_dev->s1xs2 : p.s1xs2, e_m1 = p.lq_dev ? p.lq_dev->m1 : p.m1;
         const float e_m2 = p.lq_dev ? p.lq_dev->m2 : p.m2, e_km = p.lq_dev ? p.lq_dev->k_m1xm2 : p.k_m1xm2;
+        const bool terms = ints && p.column_term != nullptr && ksi == 0;
         float t3[4], bias[4];   // no bias: -0.0f, which changes no value
+        uint32_t term[4];       // integer outputs: what the column adds
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int c = col0 + e < p.Co ? col0 + e : p.Co - 1;
             t3[e] = ints ? 0.0f : __fmul_rn(e_m1, p.fsum[c]);
             bias[e] = (!ints && p.bias) ? p.bias[c] : -0.0f;
+            term[e] = terms ? (uint32_t)p.column_term[c] : 0u;
         }
-        const rsrc_t ps_rsrc = make_rsrc(ints ? static_cast<const void *>(p.xq) : p.psum + m_first, ints ? 0u : tile_pixels * 4u);
+        // a dword per pixel: the patch sum, or what the pixel adds to integer outputs (nothing: an empty buffer reads as zeros)
+        const void *const per_pixel = terms ? static_cast<const void *>(p.pixel_term + m_first) : p.psum + m_first;
+        const rsrc_t ps_rsrc = ints && !terms ? make_rsrc(p.xq, 0u) : make_rsrc(per_pixel, tile_pixels * 4u);
         auto join = [&](const int32_t lo, const int32_t hi) __attribute__((always_inline)) {
             return (uint32_t)lo + ((uint32_t)hi << 8);
         };
@@ -309,14 +314,14 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             constexpr int kAhead = 6;   // units whose patch sums are loaded together, ahead of their stores
 #pragma unroll
             for (int u0 = 0; u0 < U; u0 += kAhead) {
-                float ps[kAhead][2];
+                uint32_t ps[kAhead][2];
 #pragma unroll
-                for (int k = 0; k < kAhead && !kInts; ++k)
+                for (int k = 0; k < kAhead; ++k)
                     if (u0 + k < U) {
                         uint32_t px[2];
                         pixels_of(u0 + k, px);
-                        ps[k][0] = __uint_as_float(ld_u32(ps_rsrc, px[0] * 4u, 0u));
-                        ps[k][1] = __uint_as_float(ld_u32(ps_rsrc, px[1] * 4u, 0u));
+                        ps[k][0] = ld_u32(ps_rsrc, px[0] * 4u, 0u);
+                        ps[k][1] = ld_u32(ps_rsrc, px[1] * 4u, 0u);
                     }
 #pragma unroll
                 for (int k = 0; k < kAhead; ++k) {
@@ -339,8 +344,12 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                         const auto s1 = __builtin_amdgcn_permlane16_swap(join(a[8 * jp + 2], a[8 * jp + 3]),
                                                                          join(a[8 * jp + 6], a[8 * jp + 7]), false, false);
                         mx_u32x4 d = {s0[0], s1[0], s0[1], s1[1]};
-                        if (!kInts) {
-                            const float t1 = __fmul_rn(e_m2, ps[k][jp]);
+                        if (kInts) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                d[e] += ps[k][jp] + term[e];
+                        } else {
+                            const float t1 = __fmul_rn(e_m2, __uint_as_float(ps[k][jp]));
 #pragma unroll
                             for (int e = 0; e < 4; ++e) {
                                 float v = __fadd_rn(__fmul_rn((float)(int32_t)d[e], e_s1xs2), t1);

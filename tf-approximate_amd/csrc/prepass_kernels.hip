@@ -1426,10 +1426,101 @@ hipError_t launch_layer_quant(const float *input, int64_t n_input, const float *
 
 // ---- integer zero-point correction of the tf1 AxConv2D op (tf1/axqconv/axqconv.cc:228-247) ----
 // total = sum(T[a][b] - a*offset_filter - b*offset_input + offset_input*offset_filter) over the patch, where a tap
-// outside the image has a = offset_input.  The LUT-GEMM gives sum(T); these kernels give sum(a) per output pixel and
-// sum(b) per output column, and the last one combines them.
-__global__ void __launch_bounds__(256) code_patch_sums_kernel(const uint8_t *__restrict__ codes, ConvGeom g,
-                                                               int offset_input, int32_t *__restrict__ asum)
+// outside the image has a = offset_input.  The LUT-GEMM gives sum(T); one launch makes the rest, in arithmetic modulo
+// 2^32 (as the reference's int32 sums wrap):
+//   pixel_term[m]    = -offset_filter * sum(a)                             per output pixel
+//   column_term[col] = -offset_input * sum(b) + K * offset_input * offset_filter   per output column
+// lutgemm_mx_kernel adds both as it stores; the other LUT-GEMM kernels leave them to axconv_correct_kernel.
+//
+// Pixels: a workgroup sums the channels of the input rows under a few output rows into LDS, chunks of V bytes per thread
+// (coalesced; the sum of four bytes is one v_sad_u8), and then every output pixel its window of those.  Bound by the
+// latency of its two short phases: 128 images of 32x32x32 under 3x3, 64 -> 6 us for one thread per pixel reading its
+// patch byte by byte before.  Columns: 16 columns x 32 slices of K per workgroup, joined in LDS (one thread per column
+// before: 43 us at K = 288).
+constexpr int kAxSumThreads = 512, kAxSumCols = 16;
+constexpr int kAxSumLdsBytes = 64 * 1024;
+constexpr int kAxSumSlices = kAxSumThreads / kAxSumCols;
+
+template <int V>
+__device__ __forceinline__ uint32_t sum_of_bytes(const uint8_t *__restrict__ src)
+{
+    uint32_t s = 0;
+    if constexpr (V == 16) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(src);
+        s = __builtin_amdgcn_sad_u8(v.x, 0u, s);
+        s = __builtin_amdgcn_sad_u8(v.y, 0u, s);
+        s = __builtin_amdgcn_sad_u8(v.z, 0u, s);
+        s = __builtin_amdgcn_sad_u8(v.w, 0u, s);
+    } else if constexpr (V == 4) {
+        s = __builtin_amdgcn_sad_u8(*reinterpret_cast<const uint32_t *>(src), 0u, 0u);
+    } else {
+        s = *src;
+    }
+    return s;
+}
+
+// Workgroups below `filter_blocks` make column terms, the others pixel terms of `rows_out` output rows each.
+template <int V>
+__global__ void __launch_bounds__(kAxSumThreads) axconv_terms_kernel(const uint8_t *__restrict__ codes,
+                                                                     const uint8_t *__restrict__ fcodes, const ConvGeom g,
+                                                                     const int rows_out, const int filter_blocks,
+                                                                     const uint32_t offset_input,
+                                                                     const uint32_t offset_filter,
+                                                                     uint32_t *__restrict__ pixel_term,
+                                                                     uint32_t *__restrict__ column_term)
+{
+    extern __shared__ uint32_t ax_lds[];
+    const int t = (int)threadIdx.x;
+    if ((int)blockIdx.x < filter_blocks) {
+        const int cl = t % kAxSumCols, slice = t / kAxSumCols, col = (int)blockIdx.x * kAxSumCols + cl;
+        uint32_t s = 0;
+        if (col < g.Co)
+            for (int k = slice; k < g.K; k += kAxSumSlices)
+                s += fcodes[(int64_t)k * g.Co + col];
+        ax_lds[t] = s;
+        __syncthreads();
+        if (slice == 0 && col < g.Co) {
+            for (int i = 1; i < kAxSumSlices; ++i)
+                s += ax_lds[i * kAxSumCols + cl];
+            column_term[col] = (uint32_t)g.K * offset_input * offset_filter - offset_input * s;
+        }
+        return;
+    }
+    const int blocks_per_image = (g.OH + rows_out - 1) / rows_out;
+    const int b = (int)blockIdx.x - filter_blocks, n = b / blocks_per_image;
+    const int oh0 = (b - n * blocks_per_image) * rows_out;
+    const int rows = (g.OH - oh0 < rows_out ? g.OH - oh0 : rows_out);
+    const int ih0 = oh0 * g.sh - g.ph, rows_in = (rows - 1) * g.sh + (g.KH - 1) * g.dh + 1;
+    const uint32_t outside = offset_input * (uint32_t)g.C;
+    for (int i = t; i < rows_in * g.W; i += kAxSumThreads) {
+        const int ih = ih0 + i / g.W;
+        ax_lds[i] = (unsigned)ih < (unsigned)g.H ? 0u : outside;
+    }
+    __syncthreads();
+    // the rows inside the image are one run of memory
+    const int first = ih0 < 0 ? -ih0 : 0, last = g.H - ih0 < rows_in ? g.H - ih0 : rows_in;   // [first, last) of rows_in
+    const int chunks = g.C / V;   // of a pixel
+    const uint8_t *const src = codes + ((int64_t)n * g.H + ih0 + first) * g.W * g.C;
+    const int total = last > first ? (last - first) * g.W * chunks : 0;
+    for (int i = t; i < total; i += kAxSumThreads)
+        atomicAdd(&ax_lds[first * g.W + i / chunks], sum_of_bytes<V>(src + (int64_t)i * V));
+    __syncthreads();
+    for (int i = t; i < rows * g.OW; i += kAxSumThreads) {
+        const int r = i / g.OW, ow = i - r * g.OW;
+        uint32_t s = 0;
+        for (int kh = 0; kh < g.KH; ++kh)
+            for (int kw = 0; kw < g.KW; ++kw) {
+                const int iw = ow * g.sw - g.pw + kw * g.dw;
+                s += (unsigned)iw < (unsigned)g.W ? ax_lds[(r * g.sh + kh * g.dh) * g.W + iw] : outside;
+            }
+        pixel_term[((int64_t)n * g.OH + oh0) * g.OW + i] = 0u - offset_filter * s;
+    }
+}
+
+// The same pixel terms, one thread per pixel: for images of which the rows under one output row do not fit the LDS.
+__global__ void __launch_bounds__(256) axconv_pixel_terms_kernel(const uint8_t *__restrict__ codes, ConvGeom g,
+                                                                 const uint32_t offset_input, const uint32_t offset_filter,
+                                                                 uint32_t *__restrict__ pixel_term)
 {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= g.M)
@@ -1438,7 +1529,7 @@ __global__ void __launch_bounds__(256) code_patch_sums_kernel(const uint8_t *__r
     const int rem = (int)(m - (int64_t)n * g.OH * g.OW);
     const int oh = rem / g.OW, ow = rem - oh * g.OW;
     const int ih0 = oh * g.sh - g.ph, iw0 = ow * g.sw - g.pw;
-    int32_t s = 0;
+    uint32_t s = 0;
     for (int kh = 0; kh < g.KH; ++kh)
         for (int kw = 0; kw < g.KW; ++kw) {
             const int ih = ih0 + kh * g.dh, iw = iw0 + kw * g.dw;
@@ -1447,50 +1538,59 @@ __global__ void __launch_bounds__(256) code_patch_sums_kernel(const uint8_t *__r
                 for (int c = 0; c < g.C; ++c)
                     s += src[c];
             } else {
-                s += offset_input * g.C;
+                s += offset_input * (uint32_t)g.C;
             }
         }
-    asum[m] = s;
+    pixel_term[m] = 0u - offset_filter * s;
 }
 
-__global__ void __launch_bounds__(256) code_filter_sums_kernel(const uint8_t *__restrict__ fcodes, int K, int Co,
-                                                                int32_t *__restrict__ bsum)
-{
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= Co)
-        return;
-    int32_t s = 0;
-    for (int k = 0; k < K; ++k)
-        s += fcodes[(int64_t)k * Co + col];
-    bsum[col] = s;
-}
-
-__global__ void __launch_bounds__(256) axconv_correct_kernel(int32_t *__restrict__ out, int64_t mc, int Co,
-                                                              const int32_t *__restrict__ asum,
-                                                              const int32_t *__restrict__ bsum, int offset_input,
-                                                              int offset_filter, int K)
+__global__ void __launch_bounds__(256) axconv_correct_kernel(uint32_t *__restrict__ out, int64_t mc, int Co,
+                                                              const uint32_t *__restrict__ pixel_term,
+                                                              const uint32_t *__restrict__ column_term)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= mc)
         return;
     const int64_t m = i / Co;
-    const int col = (int)(i - m * Co);
-    // wraps like the reference's int32 arithmetic would
-    const int64_t t = (int64_t)out[i] - (int64_t)asum[m] * offset_filter - (int64_t)bsum[col] * offset_input +
-                      (int64_t)K * offset_input * offset_filter;
-    out[i] = (int32_t)t;
+    out[i] += pixel_term[m] + column_term[i - m * Co];
 }
 
-hipError_t launch_axconv_correction(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,
-                                    int offset_filter, int32_t *asum, int32_t *bsum, int32_t *out, hipStream_t stream)
+hipError_t launch_axconv_terms(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,
+                               int offset_filter, int32_t *pixel_term, int32_t *column_term, hipStream_t stream)
 {
-    hipLaunchKernelGGL(code_patch_sums_kernel, dim3(blocks_for(g.M, 256)), dim3(256), 0, stream, codes, g, offset_input,
-                       asum);
-    hipLaunchKernelGGL(code_filter_sums_kernel, dim3(blocks_for(g.Co, 256)), dim3(256), 0, stream, fcodes, g.K, g.Co,
-                       bsum);
+    const uint32_t oi = (uint32_t)offset_input, of = (uint32_t)offset_filter;
+    uint32_t *const pt = reinterpret_cast<uint32_t *>(pixel_term), *const ct = reinterpret_cast<uint32_t *>(column_term);
+    const int filter_blocks = (g.Co + kAxSumCols - 1) / kAxSumCols;
+    // output rows per workgroup: about a thousand workgroups, at most 32 KiB of LDS; one row may take 64 KiB
+    const int64_t under = (int64_t)(g.KH - 1) * g.dh + 1;
+    auto lds_of = [&](int64_t rows) { return ((rows - 1) * g.sh + under) * g.W * 4; };
+    int64_t rows = (int64_t)g.N * g.OH / 1024;
+    rows = rows < 1 ? 1 : rows > g.OH ? g.OH : rows;
+    while (rows > 1 && lds_of(rows) > kAxSumLdsBytes / 2)
+        rows = (rows + 1) / 2;
+    const bool in_lds = lds_of(rows) <= kAxSumLdsBytes && (int64_t)g.C * g.W * ((rows - 1) * g.sh + under) < (1 << 30) &&
+                        (int64_t)g.N * g.OH + filter_blocks < ((int64_t)1 << 31);
+    const unsigned pixel_blocks = in_lds ? (unsigned)((int64_t)g.N * ((g.OH + rows - 1) / rows)) : 0u;
+    size_t lds = kAxSumThreads * 4;
+    if (in_lds && (size_t)lds_of(rows) > lds)
+        lds = (size_t)lds_of(rows);
+    // wide loads where a pixel is whole chunks and the tensor begins on one
+    const int v = (g.C % 16 == 0 && ((uintptr_t)codes & 15) == 0) ? 16 : (g.C % 4 == 0 && ((uintptr_t)codes & 3) == 0) ? 4 : 1;
+    auto kernel = v == 16 ? axconv_terms_kernel<16> : v == 4 ? axconv_terms_kernel<4> : axconv_terms_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)filter_blocks + pixel_blocks), dim3(kAxSumThreads), lds, stream, codes, fcodes, g,
+                       (int)rows, filter_blocks, oi, of, pt, ct);
+    if (!in_lds)
+        hipLaunchKernelGGL(axconv_pixel_terms_kernel, dim3(blocks_for(g.M, 256)), dim3(256), 0, stream, codes, g, oi, of, pt);
+    return hipGetLastError();
+}
+
+hipError_t launch_axconv_correction(const ConvGeom &g, const int32_t *pixel_term, const int32_t *column_term, int32_t *out,
+                                    hipStream_t stream)
+{
     const int64_t mc = g.M * g.Co;
-    hipLaunchKernelGGL(axconv_correct_kernel, dim3(blocks_for(mc, 256)), dim3(256), 0, stream, out, mc, g.Co, asum, bsum,
-                       offset_input, offset_filter, g.K);
+    hipLaunchKernelGGL(axconv_correct_kernel, dim3(blocks_for(mc, 256)), dim3(256), 0, stream,
+                       reinterpret_cast<uint32_t *>(out), mc, g.Co, reinterpret_cast<const uint32_t *>(pixel_term),
+                       reinterpret_cast<const uint32_t *>(column_term));
     return hipGetLastError();
 }
 
