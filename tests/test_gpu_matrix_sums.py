@@ -38,6 +38,12 @@ CASES = [
     ((64, 56, 56, 64), (3, 3, 64), 1, 1, "SAME", 25, False),
     ((61, 57, 59, 32), (3, 3, 72), 1, 1, "SAME", None, None),    # ragged everything, nine column tiles
     ((32, 56, 56, 256), (1, 1, 512), 1, 1, "SAME", None, None),  # several tiles per workgroup
+    # odd numbers of channel quads, whose other kernel expands the rows inside its tiles
+    ((8, 57, 55, 4), (5, 5, 40), 1, 1, "SAME", 2, False),        # one quad: four taps to a step of the filter position
+    ((4, 40, 31, 12), (5, 5, 40), 1, 1, "SAME", 2, True),        # three
+    ((9, 40, 31, 9), (5, 3, 50), 1, 1, "SAME", 2, False),        # nine channels in three quads, fifty columns
+    ((7, 61, 45, 20), (3, 3, 75), 2, 1, "VALID", 3, True),       # five
+    ((5, 57, 29, 36), (3, 3, 40), 1, 1, "VALID", 4, True),       # nine
 ]
 
 

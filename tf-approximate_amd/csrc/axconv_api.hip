@@ -758,7 +758,11 @@ void prepare_mx(PreparedDense *pd)
     const MxPlan plan = make_mx_plan(gq, (pd->flat_row_bytes ? g.sw * g.C : g.sw * 4) == 4, device_cus());
     if (plan.units == 0 || (size_t)plan.n_col_tiles * (size_t)plan.fills * 65536 > kPxMaxBytes)
         return;
-    if (plan.cost > pd->plan.cost)
+    // Against the kernel that expands inside its tiles, which writes no rows, it must promise 2 %: predicted to be equal,
+    // 1x1 128->512 on one 28x28 image took 42 us against 28 (33 MB of rows for 784 pixels), 5x5 19->224 @12x28x52 95.4 / 94.4.
+    // Predicted 4 to 32 % faster, measured (whole op, us): 3x3/2 20->75 @61x45x7 45.2 -> 37.1, 3x3 256->256 @14x14x64 349.6
+    // -> 330.7, 1x1 1024->512 @14x14x64 320.8 -> 280.9, 1x1 256->128 on one 56x56 image 35.7 -> 31.7.
+    if (plan.cost > pd->plan.cost * (pd->plan.px ? 1.0f : 0.98f))
         return;
     pd->mx = true;
     pd->mxp = plan;
@@ -845,7 +849,7 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     pd->plan = make_plan(pd->gk, device_cus(), px_mode);
     pd->lay = plain_layout(pd->g);
     if (allow_mx && px_mode == kPxModeGlobal && g_px_mode.load(std::memory_order_relaxed) == 0 &&
-        g_forced_nt.load(std::memory_order_relaxed) == 0 && pd->plan.px)
+        g_forced_nt.load(std::memory_order_relaxed) == 0)
         prepare_mx(pd);
     pd->ws = dense_workspace(pd->g, pd->plan, pd->mx ? &pd->mxp : nullptr, pd->lay, sub_bytes, pd->flat_row_bytes);
     return AXC_OK;
