@@ -35,7 +35,10 @@ extern __shared__ __align__(16) unsigned char lds_mx[];
 // grows, by one per wavefront and event: four arrivals of the buffer's fill j, then its four readers, then the
 // arrivals of fill j + 1, ...
 constexpr uint32_t kMxCb = 2 * kPxFillBytes;
-constexpr int kMxLdsBytes = 2 * kPxFillBytes + 32;
+// Behind that the values the wavefronts' pixels add (patch sums, or the zero-point terms of integer outputs): a dword per
+// pixel of the tile, 256 bytes per unit.
+constexpr uint32_t kMxPixelValues = kMxCb + 32;
+constexpr int mx_lds_bytes(const int units) { return (int)kMxPixelValues + kMxWaves * units * 256; }
 constexpr uint32_t kMxWaveBytes = kPxFillBytes / kMxWaves;   // a wavefront's share of a fill
 constexpr int kMxBlockCols = 8;   // column tiles (of 8) that the workgroups of an XCD walk side by side
 
@@ -56,6 +59,7 @@ __device__ __forceinline__ int mx_lane()
     return lane;
 }
 
+typedef __attribute__((address_space(3))) uint32_t *mx_lds_u32;   // from an LDS address (dynamic LDS starts at 0)
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t mx_u32x4 __attribute__((ext_vector_type(4)));
 
@@ -95,13 +99,18 @@ __device__ __forceinline__ void mx_fills(i32x16 (&acc)[U], uint32_t &ch0, uint32
     (void)ev;
 }
 
-template <int U, bool VEC>
+// SIMPLE: output rows of whole groups of four pixels (p.linear) and columns in fours.  Its stores need no branch: their
+// descriptor ends behind the tile's last unit, and lanes beyond the last column start at an offset that no descriptor
+// reaches (2^31; 24 * 256 pixels of at most 2^18 bytes stay below 2^32).  An instantiation of its own, because the sums
+// leave no registers for both forms side by side (of U = 2, whose stores are few, the compiler makes none).
+template <int U, bool VEC, bool SIMPLE>
 __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParams p)
 {
+    const bool linear = SIMPLE || p.linear;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 
     if (threadIdx.x < 8)
-        reinterpret_cast<volatile uint32_t *>(lds_mx + kMxCb)[threadIdx.x] = 0u;
+        ((mx_lds_u32)(lds_mx + kMxCb))[threadIdx.x] = 0u;
     __syncthreads();   // the only barrier of the kernel
 
     const int n_col = p.plan.n_col_tiles * p.plan.k_splits, n_row = p.plan.n_row_tiles;
@@ -171,6 +180,47 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         const int f0 = ksi * Fs;                            // its fills: [f0, f0 + Ft)
         const int Ft = F - f0 < Fs ? F - f0 : Fs;
         const int unit0 = rt * p.plan.units_per_tile;
+
+        // What every pixel adds, fetched into LDS under the lookups, 64 pixels of this wavefront per instruction.  Loaded
+        // by the epilogue instead, a batch of them waited for the stores of the batch before (the vector-memory counter
+        // goes down in order), a round trip through the stores' queue for every six units: 5.3 us a tile of 25 (whole op,
+        // us: 1x1 256->1024 @56x56x32 682 -> 640, 3x3 64->64 @56x56x64 184 -> 181).  A pixel that does not exist fetches the
+        // tile's first one's.
+        struct Pixels {   // the tile's first output row (not linear), first pixel, and how many pixels lie behind that
+            uint32_t row_first, count;
+            int64_t m_first;
+        };
+        auto tile_pixels_of = [&](const int unit) __attribute__((always_inline)) {
+            Pixels t;
+            t.row_first = linear ? 0u : mx_quotient((uint32_t)unit * 16u, p.div_groups);
+            t.m_first = linear ? (int64_t)unit * 64 : (int64_t)t.row_first * p.ow;
+            t.count = (uint32_t)(p.M - t.m_first < 1 << 20 ? p.M - t.m_first : 1 << 20);
+            return t;
+        };
+        const uint32_t values_at = kMxPixelValues + (uint32_t)wave * (U * 256u);
+        if (p.out_i == nullptr || (p.column_term != nullptr && ksi == 0)) {
+            const Pixels t = tile_pixels_of(unit0);
+            const uint32_t row_first = t.row_first, tile_pixels = t.count;
+            const void *const per_pixel = p.out_i ? static_cast<const void *>(p.pixel_term + t.m_first) : p.psum + t.m_first;
+            const rsrc_t pp_rsrc = make_rsrc(per_pixel, tile_pixels * 4u);
+            const uint32_t lane = (uint32_t)mx_lane();
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                uint32_t at;
+                if (linear) {
+                    at = (uint32_t)(wave + u * kMxWaves) * 64u + lane;
+                    at = at < tile_pixels ? at : 0u;
+                } else {
+                    const uint32_t grp = (uint32_t)(unit0 + wave + u * kMxWaves) * 16u + (lane >> 2);
+                    const uint32_t row = mx_quotient(grp, p.div_groups);
+                    const uint32_t ow = (grp - row * (uint32_t)p.groups_per_row) * 4u + (lane & 3u);
+                    at = (row - row_first) * (uint32_t)p.ow + ow;
+                    at = ow < (uint32_t)p.ow && at < tile_pixels ? at : 0u;
+                }
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(pp_rsrc, (__attribute__((address_space(3))) void *)(uintptr_t)(values_at + u * 256u),
+                                                         4, (int)(at * 4u), 0, 0, 0);
+            }
+        }
 
         i32x16 acc[U];
         uint32_t fail;
@@ -245,7 +295,7 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         }
         if (fail) {   // a wait that ran out: tell the host and the other wavefronts, and leave
             if (mx_lane() == 0) {
-                reinterpret_cast<volatile uint32_t *>(lds_mx + kMxCb)[2] = 1u;
+                *(mx_lds_u32)(uintptr_t)(kMxCb + 8u) = 1u;
                 if (p.wait_error)
                     __hip_atomic_store(p.wait_error, fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             }
@@ -261,15 +311,18 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         // descriptor reaches) is not stored.
         const int lane = mx_lane();
         const uint32_t g = (uint32_t)lane >> 4, i = (uint32_t)lane & 15u;
-        const bool ints = p.out_i != nullptr;
         const int col0 = ct * 8 + (int)(g >> 1) * 4;
-        const uint32_t row_first = p.linear ? 0u : mx_quotient((uint32_t)unit0 * 16u, p.div_groups);
-        const int64_t m_first = p.linear ? (int64_t)unit0 * 64 : (int64_t)row_first * p.ow;
-        const uint32_t tile_pixels = (uint32_t)(p.M - m_first < 1 << 20 ? p.M - m_first : 1 << 20);
+        const bool ints = p.out_i != nullptr, terms = ints && p.column_term != nullptr && ksi == 0;
+        int unit_first = unit0;
+        asm volatile("" : "+s"(unit_first));   // worked out again, not kept: the fill loop leaves few scalar registers
+        const Pixels tile_px = tile_pixels_of(unit_first);
+        const uint32_t row_first = tile_px.row_first, tile_pixels = tile_px.count;
+        const int64_t m_first = tile_px.m_first;
         const uint32_t pixel_bytes = (uint32_t)p.Co * 4u;
         uint32_t *const out = (ints ? reinterpret_cast<uint32_t *>(p.out_i) + (int64_t)ksi * p.M * p.Co
                                     : reinterpret_cast<uint32_t *>(p.out_f)) + m_first * p.Co;
-        const uint64_t out_bytes = (uint64_t)tile_pixels * pixel_bytes;
+        const uint32_t own_pixels = (uint32_t)p.plan.units_per_tile * 64u;
+        const uint64_t out_bytes = (uint64_t)(SIMPLE && own_pixels < tile_pixels ? own_pixels : tile_pixels) * pixel_bytes;
         const rsrc_t out_rsrc = make_rsrc(out, out_bytes < 0x80000000u ? (uint32_t)out_bytes : 0x80000000u);
         constexpr uint32_t kNowhere = 0x80000000u;
         // This lane's pixels of the wavefront's unit u (in each pair of neighbours the even or the odd one), counted from
@@ -277,22 +330,21 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         // pixels follow each other (those beyond the layer's last are left to the descriptors).
         const uint32_t j0 = g & 1u, px0 = ((uint32_t)wave * 16u + i) * 4u + j0;
         auto pixels_of = [&](const int u, uint32_t (&px)[2]) __attribute__((always_inline)) {
-            if (p.linear) {
+            if (linear) {
                 px[0] = px0 + (uint32_t)u * (kMxWaves * 64u);
                 px[1] = px[0] + 2u;
             } else {
-                const uint32_t grp = (uint32_t)(unit0 + wave + u * kMxWaves) * 16u + i;
+                const uint32_t grp = (uint32_t)(unit_first + wave + u * kMxWaves) * 16u + i;
                 const uint32_t row = mx_quotient(grp, p.div_groups), ow = (grp - row * (uint32_t)p.groups_per_row) * 4u + j0;
                 const uint32_t at = (row - row_first) * (uint32_t)p.ow + ow;
                 px[0] = ow < (uint32_t)p.ow && at < tile_pixels ? at : kNowhere;
                 px[1] = ow + 2u < (uint32_t)p.ow && at + 2u < tile_pixels ? at + 2u : kNowhere;
             }
         };
-        const uint32_t at0 = px0 * pixel_bytes + (uint32_t)col0 * 4u;   // bytes of px0 (linear)
+        const uint32_t at0 = SIMPLE && col0 >= p.Co ? kNowhere : px0 * pixel_bytes + (uint32_t)col0 * 4u;   // bytes of px0 (linear)
         const bool quads = (p.Co & 3) == 0;
         const float e_s1xs2 = p.lq_dev ? p.lq_dev->s1xs2 : p.s1xs2, e_m1 = p.lq_dev ? p.lq_dev->m1 : p.m1;
         const float e_m2 = p.lq_dev ? p.lq_dev->m2 : p.m2, e_km = p.lq_dev ? p.lq_dev->k_m1xm2 : p.k_m1xm2;
-        const bool terms = ints && p.column_term != nullptr && ksi == 0;
         float t3[4], bias[4];   // no bias: -0.0f, which changes no value
         uint32_t term[4];       // integer outputs: what the column adds
 #pragma unroll
@@ -302,36 +354,34 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             bias[e] = (!ints && p.bias) ? p.bias[c] : -0.0f;
             term[e] = terms ? (uint32_t)p.column_term[c] : 0u;
         }
-        // a dword per pixel: the patch sum, or what the pixel adds to integer outputs (nothing: an empty buffer reads as zeros)
-        const void *const per_pixel = terms ? static_cast<const void *>(p.pixel_term + m_first) : p.psum + m_first;
-        const rsrc_t ps_rsrc = ints && !terms ? make_rsrc(p.xq, 0u) : make_rsrc(per_pixel, tile_pixels * 4u);
+        // the values fetched before the lookups, of this lane's pixels of unit 0 (integer outputs without terms: masked out)
+        const mx_lds_u32 values = (mx_lds_u32)(uintptr_t)(values_at + i * 16u + j0 * 4u);
+        const uint32_t value_mask = ints && !terms ? 0u : 0xffffffffu;
         auto join = [&](const int32_t lo, const int32_t hi) __attribute__((always_inline)) {
             return (uint32_t)lo + ((uint32_t)hi << 8);
         };
-        // INTS: int32 sums; RELU: the activation
+        // kInts: int32 sums; kRelu: the activation
         auto store_tile = [&](auto ints_t, auto relu_t) __attribute__((always_inline)) {
             constexpr bool kInts = decltype(ints_t)::value, kRelu = decltype(relu_t)::value;
-            constexpr int kAhead = 6;   // units whose patch sums are loaded together, ahead of their stores
+            constexpr int kAhead = 6;   // units whose values are read together
 #pragma unroll
             for (int u0 = 0; u0 < U; u0 += kAhead) {
                 uint32_t ps[kAhead][2];
 #pragma unroll
                 for (int k = 0; k < kAhead; ++k)
                     if (u0 + k < U) {
-                        uint32_t px[2];
-                        pixels_of(u0 + k, px);
-                        ps[k][0] = ld_u32(ps_rsrc, px[0] * 4u, 0u);
-                        ps[k][1] = ld_u32(ps_rsrc, px[1] * 4u, 0u);
+                        ps[k][0] = values[(u0 + k) * 64] & value_mask;
+                        ps[k][1] = values[(u0 + k) * 64 + 2] & value_mask;
                     }
 #pragma unroll
                 for (int k = 0; k < kAhead; ++k) {
                     const int u = u0 + k;
-                    if (u >= U || u * kMxWaves + wave >= p.plan.units_per_tile)
+                    if (u >= U || (!SIMPLE && u * kMxWaves + wave >= p.plan.units_per_tile))
                         continue;
                     const i32x16 &a = acc[u < U ? u : 0];
                     uint32_t at[2] = {at0 + (uint32_t)u * (kMxWaves * 64u) * pixel_bytes, 0u};
                     at[1] = at[0] + 2u * pixel_bytes;
-                    if (!p.linear) {
+                    if (!linear) {
                         uint32_t px[2];
                         pixels_of(u, px);
                         at[0] = px[0] == kNowhere ? kNowhere : px[0] * pixel_bytes + (uint32_t)col0 * 4u;
@@ -357,7 +407,9 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                                 d[e] = __float_as_uint(kRelu ? fmaxf(v, 0.0f) : v);
                             }
                         }
-                        if (quads) {
+                        if (SIMPLE) {
+                            __builtin_amdgcn_raw_buffer_store_b128(d, out_rsrc, (int)at[jp], 0, 0);
+                        } else if (quads) {
                             __builtin_amdgcn_raw_buffer_store_b128(d, out_rsrc, (int)(col0 < p.Co ? at[jp] : kNowhere), 0, 0);
                         } else {
 #pragma unroll
@@ -376,27 +428,29 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             store_tile(no(), yes());
         else
             store_tile(no(), no());
+        asm volatile("" ::: "memory");   // the values are read before the next tile's are fetched into their place
     }
 }
 
-template <int U, bool VEC>
+template <int U, bool VEC, bool SIMPLE>
 static hipError_t launch_mx_one(const MxParams &p, hipStream_t stream)
 {
-    auto kernel = lutgemm_mx_kernel<U, VEC>;
-    const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(kernel), kMxLdsBytes, true);
+    auto kernel = lutgemm_mx_kernel<U, VEC, SIMPLE>;
+    const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(kernel), mx_lds_bytes(U), true);
     if (e != hipSuccess)
         return e;
-    hipLaunchKernelGGL(kernel, dim3(p.plan.grid), dim3(kMxThreads), kMxLdsBytes, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(p.plan.grid), dim3(kMxThreads), mx_lds_bytes(U), stream, p);
     return hipGetLastError();
 }
 
 hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream)
 {
-    const bool vec = p.pitch == 4;
+    const bool vec = p.pitch == 4, simple = p.linear && (p.Co & 3) == 0;
     switch (p.plan.units) {
 #define AXC_MX_LAUNCH(N)                                                                                               \
     case N:                                                                                                            \
-        return vec ? launch_mx_one<N, true>(p, stream) : launch_mx_one<N, false>(p, stream);
+        return simple && N > 2 ? (vec ? launch_mx_one<N, true, (N > 2)>(p, stream) : launch_mx_one<N, false, (N > 2)>(p, stream)) \
+                               : (vec ? launch_mx_one<N, true, false>(p, stream) : launch_mx_one<N, false, false>(p, stream));
         AXC_MX_LAUNCH(2)
         AXC_MX_LAUNCH(3)
         AXC_MX_LAUNCH(4)
