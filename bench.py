@@ -84,6 +84,8 @@ CPU_SAMPLE_S = 0.5      # single-thread reference sample per `layers` record
 # device copy of known size inside the same run.  Keyed by (workload, kernel); not measured in the run that prints
 # them: the bench line says which profile they come from.
 PROFILED_TRAFFIC = {
+    ("conv3x3_b64_56x56x64_to_64_s1_same", "lutgemm_mx"): (2.000 * 84123.2 * 1024 + 1.000 * 50210.9 * 1024,
+                                                           "profiles/lutgemm_mx_conv3x3_b64_56x56x64.md"),
     ("conv3x3_b64_56x56x64_to_64_s1_same", "lutgemm_px"): (2.000 * 81258.0 * 1024 + 1.000 * 64419.8 * 1024,
                                                            "profiles/lutgemm_px_conv3x3_b64_56x56x64.md"),
     ("conv3x3_b64_56x56x64_to_64_s1_same", "lutgemm_expand"): (2.000 * 8312.5 * 1024 + 1.000 * 61656.5 * 1024,
@@ -147,17 +149,18 @@ class Ceilings:
         self.valu_nominal = self.cus * 64.0 * self.clock_hz     # 4 SIMDs x 16 lanes per clock and CU
         self.port_nominal = self.cus * 256.0 * self.clock_hz    # 64 banks x 4 bytes per clock and CU
 
-    def fractions(self, lookups_per_s):
+    def fractions(self, lookups_per_s, kernel):
         valu_ceiling = max(self.valu_nominal, self.valu_lane_ops)
         port_ceiling = max(self.port_nominal, self.port_bytes)
         f_port = 2.0 * lookups_per_s / port_ceiling
-        f_valu = lookups_per_s * self.ops_per_lookup / valu_ceiling
+        ops_per_lookup = 0.0 if kernel == "lutgemm_mx" else self.ops_per_lookup   # the matrix cores make those sums
+        f_valu = lookups_per_s * ops_per_lookup / valu_ceiling
         bound = "lds" if f_port >= f_valu else "valu"
-        peak = port_ceiling / 2.0 if bound == "lds" else valu_ceiling / self.ops_per_lookup
+        peak = port_ceiling / 2.0 if bound == "lds" else valu_ceiling / ops_per_lookup
         return {"bound": bound, "frac": round(max(f_port, f_valu), 4), "frac_lds_port": round(f_port, 4),
                 "frac_valu": round(f_valu, 4),
                 "frac_lds_port_measured": round(2.0 * lookups_per_s / self.port_bytes, 4),
-                "frac_valu_measured": round(lookups_per_s * self.ops_per_lookup / self.valu_lane_ops, 4),
+                "frac_valu_measured": round(lookups_per_s * ops_per_lookup / self.valu_lane_ops, 4),
                 "frac_lookup_mix_measured": round(lookups_per_s / self.mix, 4),
                 "frac_nominal_gather": round(lookups_per_s / NOMINAL_LDS_LOOKUPS_PER_S, 4)}, peak
 
@@ -297,9 +300,15 @@ def sampled_oracle_check(oracle, table, op, xd, fd, strides, depthwise, y, n_sam
     return bit_exact, linf
 
 
-def dense_kernel_name(kernels_ms):
-    """The LUT-GEMM kernel a dense layer ran: out of pre-expanded rows, or expanding inside every tile."""
-    return "lutgemm_px" if "lutgemm_px" in kernels_ms else "lutgemm_expand"
+def dense_kernel_name(ops, kernels_ms, xs, fs, strides):
+    """The LUT-GEMM kernel a dense layer ran: out of pre-expanded rows with the sums on the matrix cores or on the vector
+    ALUs, or expanding inside every tile.  The library times the first two under one name."""
+    if "lutgemm_px" not in kernels_ms:
+        return "lutgemm_expand"
+    if ops.conv2d_matrix_plan(tuple(xs), tuple(fs), (1, strides[0], strides[1], 1)) is None:
+        return "lutgemm_px"
+    kernels_ms["lutgemm_mx"] = kernels_ms.pop("lutgemm_px")
+    return "lutgemm_mx"
 
 
 def cpu_reference_sample(oracle, table, xd, fd, strides, depthwise, seconds=CPU_SAMPLE_S):
@@ -343,7 +352,7 @@ def measure_layer(pkg, ops, oracle, ceil, spec, steps=None, preroll_s=0.08):
     N, OH, OW, Cout = y.shape
     taps_c = fs[0] * fs[1] * (1 if depthwise else fs[2])
     lookups = N * OH * OW * Cout * taps_c
-    main = "depthwise_lut" if depthwise else dense_kernel_name(kms)
+    main = "depthwise_lut" if depthwise else dense_kernel_name(ops, kms, xs, fs, strides)
     kernel_ms = kms[main]
     rec = {"config": config, "layer": name, "input": list(xs), "filter": list(fs), "strides": list(strides),
            "codes": codes, "table": tkind, "M": N * OH * OW, "K": taps_c, "N": Cout, "lookups": lookups,
@@ -355,7 +364,7 @@ def measure_layer(pkg, ops, oracle, ceil, spec, steps=None, preroll_s=0.08):
         rec.update({"bound": "hbm", "frac": round(gbps / HBM_PEAK_GBPS, 4), "hbm_algorithmic_gbytes_per_s": round(gbps, 1),
                     "frac_of_device_copy": round(gbps * 1e9 / ceil.copy_bytes, 4), "algorithmic_bytes": nbytes})
     else:
-        fr, _ = ceil.fractions(lookups / (kernel_ms * 1e-3))
+        fr, _ = ceil.fractions(lookups / (kernel_ms * 1e-3), main)
         rec.update(fr)
     if oracle is not None:
         exact, linf = sampled_oracle_check(oracle, table, op, xd, fd, strides, depthwise, y)
@@ -547,7 +556,7 @@ def main():
     lookups = n * oh * ow * co * taps_c
     gmacs = lookups / (ms_per_step * 1e-3) / 1e9
 
-    main_kernel = "depthwise_lut" if depthwise else dense_kernel_name(kms)
+    main_kernel = "depthwise_lut" if depthwise else dense_kernel_name(ops, kms, xs, fs, strides)
     main_ms = kms[main_kernel]
     achieved = lookups / (main_ms * 1e-3)
     ceil = Ceilings(ops)
@@ -572,7 +581,7 @@ def main():
             "glookups_per_s": round(achieved / 1e9, 1),
         }
     else:
-        fr, peak = ceil.fractions(achieved)
+        fr, peak = ceil.fractions(achieved, main_kernel)
         roofline = {
             "bound": fr["bound"],
             "kernel": main_kernel,
