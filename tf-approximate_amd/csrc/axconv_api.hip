@@ -589,7 +589,8 @@ MxDiv mx_div(uint32_t d)
 //   a fill    0.30 + 0.138 U, at least 1.05 + 0.03 U (64 KiB of rows into LDS with every CU doing so: U = 2 takes 1.11, 8 1.45,
 //             13 2.1, 25 3.75); with four loads per unit instead of one (pixels that are no neighbouring dwords)
 //             0.35 + 0.243 U, at least 1.3
-//   a tile    1.3 + 0.70 U: geometry, the sums' start values, the outputs (for the most part the stores of 32-byte pieces)
+//   a tile    1.3 + 0.70 U up to U = 6, then 0.42 a unit (18.8 at U = 25 while batches of six units waited for each other's
+//             stores, 13.5 without): geometry, the sums' start values, the outputs, stored in 32-byte pieces
 // K splits and the rows cost what they cost the other kernels (compute_plan).
 MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, bool one_load, int cus, double clock_hz)
 {
@@ -624,7 +625,8 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, b
             const int64_t tiles = rows * n_col * ks, rounds = (tiles + cus - 1) / cus;
             const double fill = one_load ? std::max(1.05 + 0.03 * units, 0.30 + 0.138 * units)
                                          : std::max(1.3, 0.35 + 0.243 * units);
-            double us = std::max((double)rounds * (fps * fill + 1.3 + 0.70 * units), rows_bytes / 3e6);
+            const double tile = 1.3 + 0.70 * std::min(units, 6) + 0.42 * std::max(units - 6, 0);
+            double us = std::max((double)rounds * (fps * fill + tile), rows_bytes / 3e6);
             if (ks > 1)
                 us += 7.1 + (double)(ks + 1) * (double)outputs * 4.0 * 1.46e-7;
             const double cost = (us + rows_us) * 1e-6 * clock_hz;
@@ -762,7 +764,11 @@ void prepare_mx(PreparedDense *pd)
     // 1x1 128->512 on one 28x28 image took 42 us against 28 (33 MB of rows for 784 pixels), 5x5 19->224 @12x28x52 95.4 / 94.4.
     // Predicted 4 to 32 % faster, measured (whole op, us): 3x3/2 20->75 @61x45x7 45.2 -> 37.1, 3x3 256->256 @14x14x64 349.6
     // -> 330.7, 1x1 1024->512 @14x14x64 320.8 -> 280.9, 1x1 256->128 on one 56x56 image 35.7 -> 31.7.
-    if (plan.cost > pd->plan.cost * (pd->plan.px ? 1.0f : 0.98f))
+    // Rows beyond some 20 MB for few pixels cost up to 0.2 us a MB more than the plan says (1x1/2 64->1712 @54x13x22, 56 MB:
+    // 56.7 us against 48.5).
+    const double rows_bytes = (double)plan.n_col_tiles * plan.fills * 65536.0;
+    const double slow_rows = std::max(0.0, rows_bytes - 22e6) / 5e12 * device_clock_hz();
+    if (pd->plan.px ? plan.cost > pd->plan.cost : plan.cost + slow_rows > pd->plan.cost * 0.98)
         return;
     pd->mx = true;
     pd->mxp = plan;
