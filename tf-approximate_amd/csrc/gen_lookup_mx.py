@@ -313,10 +313,15 @@ def emit(units, vec):
     st.ins("s_add_u32 %[whole], %[tmp], 4")
     st.ins("s_cmp_eq_u32 %[left], 1")
     st.ins("s_cselect_b32 %[whole], 0, %[whole]")
-    # the rows that follow: the tile's next fill, or the first one of the workgroup's next tile
+    # the rows that follow: the tile's next fill, or the first one of the workgroup's next tile, or none: then ENEXT has bit
+    # 31 set, which moves into the vector offset.  That one is what a descriptor's bounds check covers; the scalar offset
+    # must stay inside the rows by itself.
     st.ins("s_add_u32 %[eoff], %[eoff], 0x10000")
     st.ins("s_cmp_eq_u32 %[left], 1")
     st.ins("s_cselect_b32 %[eoff], %[enext], %[eoff]")
+    st.ins("s_and_b32 %[tmp], %[eoff], 0x80000000")
+    st.ins("s_xor_b32 %[eoff], %[eoff], %[tmp]")
+    st.ins("v_or_b32 v%d, %%[tmp], v%d" % (V_L16, V_L16))
     # the state the loop was entered with: W reads and D units of activations in flight, nothing else that counts
     # (operations older than those only make a wait stricter)
     assert st.vm_q == [op for x in range(1, d) for op in acts[x]][-len(st.vm_q):] or not st.vm_q
@@ -335,13 +340,13 @@ def emit(units, vec):
         lo = acc_reg(units, u, 0)
         b = int(lo[2:lo.index(":")])
         outs.append('"={%s[%d:%d]}"(ACC[%d])' % (lo[0], b, b + 15, u))
-    inouts = [("CH0", V_CH0), ("CH1", V_CH1), ("KOFF", V_KOFF), ("QL", V_Q), ("KWL", V_KW), ("CINIT", V_POLL)]
+    inouts = [("CH0", V_CH0), ("CH1", V_CH1), ("KOFF", V_KOFF), ("QL", V_Q), ("KWL", V_KW), ("CINIT", V_POLL), ("L16", V_L16)]
     outs += ['"+{v%d}"(%s)' % (r, name) for name, r in inouts]
     scalars = [("cbcur", "CBCUR"), ("cboth", "CBOTH"), ("edst", "EDST"), ("gf", "GF"), ("left", "LEFT"), ("free", "FREE"),
                ("whole", "WHOLE"), ("eoff", "EOFF")]
     outs += ['[%s] "+&s"(%s)' % s for s in scalars]
     outs += ['[fail] "=&s"(FAIL)', '[tmp] "=&s"(TMP)', '[ev] "=&s"(EV)']
-    ins = ['"{v[%d:%d]}"(AOP)' % (V_A, V_A + 3), '"{v%d}"(IDX)' % V_IDX, '"{v%d}"(L16)' % V_L16]
+    ins = ['"{v[%d:%d]}"(AOP)' % (V_A, V_A + 3), '"{v%d}"(IDX)' % V_IDX]
     ins += ['"{v%d}"(SEL[%d])' % (V_SEL + c, c) for c in range(4)]
     ins += ['"{v%d}"(BASE[%d])' % (V_BASE + u, u) for u in range(units)]
     ins += ['[%s] "s"(%s)' % x for x in [("xq", "XQ"), ("erc", "ERC"), ("enext", "ENEXT"), ("cb0", "CB0"), ("spin", "SPIN"), ("whole0", "WHOLE0"),
@@ -351,8 +356,8 @@ def emit(units, vec):
         ins += ['[p%d] "s"(KS.pitch[%d])' % (j, j - 1) for j in (1, 2, 3)]
     clob = ['"v%d"' % r for r in list(range(V_ADDR, V_ADDR + 4)) + [V_TMP, V_CB] + list(range(ring, end))]
     clob += ['"m0"', '"scc"', '"vcc"', '"memory"']
-    args = ("ACC, CH0, CH1, KOFF, QL, KWL, CINIT, CBCUR, CBOTH, EDST, GF, LEFT, FREE, WHOLE, EOFF, FAIL, TMP, EV, AOP, IDX, "
-            "L16, SEL, BASE, XQ, ERC, ENEXT, CB0, SPIN, WHOLE0, KS")
+    args = ("ACC, CH0, CH1, KOFF, QL, KWL, CINIT, L16, CBCUR, CBOTH, EDST, GF, LEFT, FREE, WHOLE, EOFF, FAIL, TMP, EV, AOP, "
+            "IDX, SEL, BASE, XQ, ERC, ENEXT, CB0, SPIN, WHOLE0, KS")
     text = " \\\n        ".join('"%s\\n\\t"' % line for line in st.lines)
     return ("#define MX_FILLS_U%d_%s(%s) \\\n    asm volatile( \\\n        %s \\\n        : %s \\\n        : %s \\\n        : %s)\n"
             % (units, "V" if vec else "S", args, text, ", ".join(outs), ", ".join(ins), ", ".join(clob)))

@@ -69,9 +69,9 @@ struct MxKStep {   // how a lane's filter position moves on by four quads (scala
 
 template <int U, bool VEC>
 __device__ __forceinline__ void mx_fills(i32x16 (&acc)[U], uint32_t &ch0, uint32_t &ch1, uint32_t &koff, uint32_t &ql,
-                                         uint32_t &kwl, uint32_t &cinit, uint32_t &cbcur, uint32_t &cboth, uint32_t &edst,
-                                         uint32_t &gf, uint32_t &left, uint32_t &free_at, uint32_t &whole, uint32_t &eoff,
-                                         uint32_t &fail, const mx_u32x4 aop, const uint32_t idx, const uint32_t l16,
+                                         uint32_t &kwl, uint32_t &cinit, uint32_t &l16, uint32_t &cbcur, uint32_t &cboth,
+                                         uint32_t &edst, uint32_t &gf, uint32_t &left, uint32_t &free_at, uint32_t &whole, uint32_t &eoff,
+                                         uint32_t &fail, const mx_u32x4 aop, const uint32_t idx,
                                          const uint32_t (&sel)[4], const uint32_t (&base)[U], const rsrc_t xq,
                                          const rsrc_t erc, const uint32_t enext, const uint32_t spin, const uint32_t whole0,
                                          const MxKStep &ks)
@@ -79,11 +79,11 @@ __device__ __forceinline__ void mx_fills(i32x16 (&acc)[U], uint32_t &ch0, uint32
     uint32_t tmp, ev;
 #define AXC_MX_CASE(N)                                                                                                  \
     if constexpr (U == N && VEC)                                                                                        \
-        MX_FILLS_U##N##_V(acc, ch0, ch1, koff, ql, kwl, cinit, cbcur, cboth, edst, gf, left, free_at, whole, eoff, fail, tmp, \
-                          ev, aop, idx, l16, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks);                      \
+        MX_FILLS_U##N##_V(acc, ch0, ch1, koff, ql, kwl, cinit, l16, cbcur, cboth, edst, gf, left, free_at, whole, eoff, fail, \
+                          tmp, ev, aop, idx, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks);                      \
     if constexpr (U == N && !VEC)                                                                                       \
-        MX_FILLS_U##N##_S(acc, ch0, ch1, koff, ql, kwl, cinit, cbcur, cboth, edst, gf, left, free_at, whole, eoff, fail, tmp, \
-                          ev, aop, idx, l16, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks);
+        MX_FILLS_U##N##_S(acc, ch0, ch1, koff, ql, kwl, cinit, l16, cbcur, cboth, edst, gf, left, free_at, whole, eoff, fail, \
+                          tmp, ev, aop, idx, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks);
     AXC_MX_CASE(2)
     AXC_MX_CASE(3)
     AXC_MX_CASE(4)
@@ -168,7 +168,8 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         int rt, ctv;
         decode(tile, rt, ctv);
         const bool has_next = tile + tile_step < tile_end;
-        // rows to fetch behind this tile's last fill: the next tile's first fill, or (past the end: nothing moves) none
+        // rows to fetch behind this tile's last fill: the next tile's first fill, or none (bit 31: the fill loop's loads then
+        // lie behind the descriptor's end, and nothing moves)
         uint32_t enext = 0x80000000u;
         if (has_next) {
             int rt_next, ctv_next;
@@ -288,10 +289,11 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             uint32_t left = (uint32_t)Ft;
             // the other buffer is free once fill gf - 1 is read (fill 1 goes into a buffer never used)
             uint32_t free_at = gf == 0u ? 0u : mx_free(gf - 1u), whole = Ft > 1 ? mx_whole(gf + 1u) : 0u;
-            uint32_t eoff = Ft > 1 ? ((uint32_t)(ct * F + f0) + 1u) * (uint32_t)kPxFillBytes + wofs : enext;
+            const uint32_t after = Ft > 1 ? ((uint32_t)(ct * F + f0) + 1u) * (uint32_t)kPxFillBytes + wofs : enext;
+            uint32_t eoff = after & 0x7fffffffu, l16 = (uint32_t)lane * 16u | (after & 0x80000000u);
             const uint32_t whole0 = mx_whole(gf);
-            mx_fills<U, VEC>(acc, ch0, ch1, koff, ql, kwl, cinit, cbcur, cboth, edst, gf, left, free_at, whole, eoff, fail, aop,
-                             idx, (uint32_t)lane * 16u, sel, base, xq_rsrc, e_rsrc, enext, p.spin_limit, whole0, ks);
+            mx_fills<U, VEC>(acc, ch0, ch1, koff, ql, kwl, cinit, l16, cbcur, cboth, edst, gf, left, free_at, whole, eoff, fail,
+                             aop, idx, sel, base, xq_rsrc, e_rsrc, enext, p.spin_limit, whole0, ks);
         }
         if (fail) {   // a wait that ran out: tell the host and the other wavefronts, and leave
             if (mx_lane() == 0) {
