@@ -185,6 +185,20 @@ def test_tile_plans_fit_the_kernels(ops, lib):
     assert seen_px > 50 and seen_split > 50 and seen_px_split > 5 and seen_free > 5
 
 
+def test_strided_pixel_groups_stay_in_the_workspace(ops):
+    """lutgemm_mx_kernel reads the missing pixels of a group of four as well, up to three pixel pitches behind the last one
+    that exists; what is certain to lie behind the quantized input is one fill of rows (64 KiB)."""
+    seen = 0
+    for stride in (1, 2, 3, 100, 3000, 5461, 5462, 16383, 32766):
+        for xs, fs in [((1, 1, 40, 7), (3, 3, 7, 8)), ((64, 28, 28, 64), (3, 3, 64, 64)), ((1, 1, 9000, 32), (1, 2, 32, 8)),
+                       ((16, 1, 3, 7), (3, 3, 7, 8)), ((64, 112, 112, 2), (5, 5, 2, 64))]:
+            plan = ops.conv2d_matrix_plan(xs, fs, (1, 1, stride, 1))
+            if plan is not None:
+                seen += 1
+                assert 3 * stride * (4 if xs[3] % 4 == 0 else min(xs[3], 4)) <= 65536, (xs, fs, stride, plan)
+    assert seen > 10
+
+
 def test_workspace_sizes(ops, lib):
     desc = ops.make_desc((64, 56, 56, 64), (3, 3, 64, 64), (1, 1, 1, 1), "SAME")
     rc, n = _ws(lib, desc)

@@ -755,9 +755,14 @@ void prepare_mx(PreparedDense *pd)
         return;
     if (g.M >= ((int64_t)1 << 31) - 4096 || g.Co > 65536)   // pixel numbers and a tile's output offsets in 31 bits
         return;
+    // Pixels of a group that do not exist are read too, up to three pitches behind the input by a scalar offset, which a
+    // descriptor's bounds check need not cover: that must still be the workspace (a fill of rows, 64 KiB, lies behind).
+    const int64_t pitch = (int64_t)g.sw * (pd->flat_row_bytes ? g.C : 4);
+    if (3 * pitch > 65536)
+        return;
     ConvGeom gq = pd->gk;
     gq.OW = g.OW;
-    const MxPlan plan = make_mx_plan(gq, (pd->flat_row_bytes ? g.sw * g.C : g.sw * 4) == 4, device_cus());
+    const MxPlan plan = make_mx_plan(gq, pitch == 4, device_cus());
     if (plan.units == 0 || (size_t)plan.n_col_tiles * (size_t)plan.fills * 65536 > kPxMaxBytes)
         return;
     // Against the kernel that expands inside its tiles, which writes no rows, it must promise 2 %: predicted to be equal,
