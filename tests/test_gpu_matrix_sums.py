@@ -123,3 +123,22 @@ def test_layer_entry_and_integer_op(pkg, oracle):
         off_in = ops.float_to_quantized_unclamped_quint8(0.0, MM[0], MM[1])
         off_f = ops.float_to_quantized_unclamped_quint8(0.0, MM[2], MM[3])
         assert np.array_equal(out.cpu().numpy(), oracle.axconv2d_tf1(table, xc, fc, off_in, off_f, stride, padding)), xs
+
+
+@pytest.mark.parametrize("xs,fs", [((1, 1, 30001, 32), (1, 3, 32, 20000)), ((2, 1, 20001, 32), (1, 1, 32, 32774))])
+def test_output_rows_beyond_2_gib(pkg, xs, fs):
+    """One output row takes more bytes than a store's 31-bit offset counts, and tiles begin anywhere in it."""
+    print("case", xs, fs, flush=True)
+    ops = pkg.ops
+    assert ops.conv2d_matrix_plan(xs, fs) is not None and xs[2] % 4 != 0 and xs[2] * fs[3] * 4 > 1 << 31
+    table = pkg.synth.table_random(3)
+    xd, fd = bench.device_tensors(pkg, xs, fs, "uniform", seed=3)
+    op = pkg.ApproxConv2DWithMinMaxVars([1, 1, 1, 1], 8, table, "SAME")
+    for run in (lambda: op.accumulators(xd, fd, *MM), lambda: op(xd, fd, *MM, activation="relu").view(torch.int32)):
+        got = run()
+        try:
+            ops.set_preexpand(-1)
+            want = run()
+        finally:
+            ops.set_preexpand(0)
+        assert torch.equal(got, want), "%d of %d differ" % (int((got != want).sum()), got.numel())

@@ -187,21 +187,23 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         // goes down in order), a round trip through the stores' queue for every six units: 5.3 us a tile of 25 (whole op,
         // us: 1x1 256->1024 @56x56x32 682 -> 640, 3x3 64->64 @56x56x64 184 -> 181).  A pixel that does not exist fetches the
         // tile's first one's.
-        struct Pixels {   // the tile's first output row (not linear), first pixel, and how many pixels lie behind that
-            uint32_t row_first, count;
+        struct Pixels {   // the tile's first pixel, its output row and the pixels of that row before it (not linear), and how
+            uint32_t row_first, before, count;   // many pixels the layer has from the first one on
             int64_t m_first;
         };
         auto tile_pixels_of = [&](const int unit) __attribute__((always_inline)) {
             Pixels t;
-            t.row_first = linear ? 0u : mx_quotient((uint32_t)unit * 16u, p.div_groups);
-            t.m_first = linear ? (int64_t)unit * 64 : (int64_t)t.row_first * p.ow;
+            const uint32_t grp = (uint32_t)unit * 16u;
+            t.row_first = linear ? 0u : mx_quotient(grp, p.div_groups);
+            t.before = linear ? 0u : (grp - t.row_first * (uint32_t)p.groups_per_row) * 4u;
+            t.m_first = linear ? (int64_t)unit * 64 : (int64_t)t.row_first * p.ow + t.before;
             t.count = (uint32_t)(p.M - t.m_first < 1 << 20 ? p.M - t.m_first : 1 << 20);
             return t;
         };
         const uint32_t values_at = kMxPixelValues + (uint32_t)wave * (U * 256u);
         if (p.out_i == nullptr || (p.column_term != nullptr && ksi == 0)) {
             const Pixels t = tile_pixels_of(unit0);
-            const uint32_t row_first = t.row_first, tile_pixels = t.count;
+            const uint32_t row_first = t.row_first, before = t.before, tile_pixels = t.count;
             const void *const per_pixel = p.out_i ? static_cast<const void *>(p.pixel_term + t.m_first) : p.psum + t.m_first;
             const rsrc_t pp_rsrc = make_rsrc(per_pixel, tile_pixels * 4u);
             const uint32_t lane = (uint32_t)mx_lane();
@@ -215,7 +217,7 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                     const uint32_t grp = (uint32_t)(unit0 + wave + u * kMxWaves) * 16u + (lane >> 2);
                     const uint32_t row = mx_quotient(grp, p.div_groups);
                     const uint32_t ow = (grp - row * (uint32_t)p.groups_per_row) * 4u + (lane & 3u);
-                    at = (row - row_first) * (uint32_t)p.ow + ow;
+                    at = (row - row_first) * (uint32_t)p.ow + ow - before;
                     at = ow < (uint32_t)p.ow && at < tile_pixels ? at : 0u;
                 }
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(pp_rsrc, (__attribute__((address_space(3))) void *)(uintptr_t)(values_at + u * 256u),
@@ -308,9 +310,9 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         // bias and activation of the layer entry, store ----
         // Lane (g, i) holds columns 2 g and 2 g + 1 of pixels 4 i .. 4 i + 3.  Swapping 16-lane rows between an even and
         // an odd pixel leaves it with four consecutive columns of one pixel: 16-byte stores, through a buffer descriptor
-        // that begins at the tile's first output row, so that a unit's address is one addition and what lies outside
-        // the layer (beyond the last pixel: the descriptor's end; beyond a row or the last column: an offset that no
-        // descriptor reaches) is not stored.
+        // that begins at the tile's first pixel, so that a unit's address is one addition and what lies outside the layer
+        // (beyond the last pixel: the descriptor's end; beyond a row or the last column: an offset that no descriptor
+        // reaches) is not stored.  A tile has at most 6 400 pixels of at most 2^18 bytes: offsets stay below 2^31.
         const int lane = mx_lane();
         const uint32_t g = (uint32_t)lane >> 4, i = (uint32_t)lane & 15u;
         const int col0 = ct * 8 + (int)(g >> 1) * 4;
@@ -318,7 +320,7 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         int unit_first = unit0;
         asm volatile("" : "+s"(unit_first));   // worked out again, not kept: the fill loop leaves few scalar registers
         const Pixels tile_px = tile_pixels_of(unit_first);
-        const uint32_t row_first = tile_px.row_first, tile_pixels = tile_px.count;
+        const uint32_t row_first = tile_px.row_first, before = tile_px.before, tile_pixels = tile_px.count;
         const int64_t m_first = tile_px.m_first;
         const uint32_t pixel_bytes = (uint32_t)p.Co * 4u;
         uint32_t *const out = (ints ? reinterpret_cast<uint32_t *>(p.out_i) + (int64_t)ksi * p.M * p.Co
@@ -328,7 +330,7 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         const rsrc_t out_rsrc = make_rsrc(out, out_bytes < 0x80000000u ? (uint32_t)out_bytes : 0x80000000u);
         constexpr uint32_t kNowhere = 0x80000000u;
         // This lane's pixels of the wavefront's unit u (in each pair of neighbours the even or the odd one), counted from
-        // the tile's first output row: px[jp]; kNowhere where there is none.  Where output rows are whole groups of four,
+        // the tile's first pixel: px[jp]; kNowhere where there is none.  Where output rows are whole groups of four,
         // pixels follow each other (those beyond the layer's last are left to the descriptors).
         const uint32_t j0 = g & 1u, px0 = ((uint32_t)wave * 16u + i) * 4u + j0;
         auto pixels_of = [&](const int u, uint32_t (&px)[2]) __attribute__((always_inline)) {
@@ -338,7 +340,7 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             } else {
                 const uint32_t grp = (uint32_t)(unit_first + wave + u * kMxWaves) * 16u + i;
                 const uint32_t row = mx_quotient(grp, p.div_groups), ow = (grp - row * (uint32_t)p.groups_per_row) * 4u + j0;
-                const uint32_t at = (row - row_first) * (uint32_t)p.ow + ow;
+                const uint32_t at = (row - row_first) * (uint32_t)p.ow + ow - before;
                 px[0] = ow < (uint32_t)p.ow && at < tile_pixels ? at : kNowhere;
                 px[1] = ow + 2u < (uint32_t)p.ow && at + 2u < tile_pixels ? at + 2u : kNowhere;
             }
