@@ -1,9 +1,10 @@
 """The generated fill loop of lutgemm_mx_kernel (tf-approximate_amd/csrc/gen_lookup_mx.py) waits for LDS and memory
 operations with derived counts.  This test runs the emitted text, three fills long, through a model of the hardware's
-two in-order queues and follows the data: no instruction may touch a register that an operation in flight has yet to
-write, at most 15 LDS operations may be outstanding, every sum must receive exactly the 16 looked-up quadruples of its
-pixels per fill, made from the activations of its own unit and fill, and every fill's rows must be loaded exactly once
-into the buffer that is not being read."""
+two in-order queues and follows the data of one wavefront: no instruction may touch a register that an operation in
+flight has yet to write, at most 15 LDS operations may be outstanding, every sum must start from its start value and
+receive exactly the 16 looked-up quadruples of its pixels per fill, made from the activations of its own unit and fill,
+and every fill's rows must be loaded exactly once while the fill before is looked up.  Which buffer they go to and how
+the wavefronts wait for each other is test_lookup_mx_workgroup.py's."""
 import importlib.util
 import os
 import re
@@ -52,6 +53,9 @@ def test_fill_loop(variant):
     units = variant[0]
     lines = [x for x in re.findall(r'"([^"]*)\\n\\t"', text)]
     m = Machine()
+    m.val["v%d" % gen.V_POLL] = "cinit"    # what the caller hands over in this register
+    starts = {}
+    vector_sums = {r for u in range(units) for j in range(4) for r in regs(gen.acc_reg(units, u, j)) if r[0] == "v"}
     base_of = {"v%d" % (gen.V_BASE + u): u for u in range(units)}
     loop, end = lines.index("Lfill_%=:"), lines.index("Lend_%=:")
     pc, fill, sums, loads, flips, steps, last_loads = 0, 0, {}, [], 0, 0, 0
@@ -123,14 +127,23 @@ def test_fill_loop(variant):
                 break
         elif op == "s_branch" and args[0].startswith("Lfill"):
             pc = loop
+        elif (op == "v_accvgpr_write_b32" or (op == "v_mov_b32" and regs(args[0])[0] in vector_sums)) and prologue:
+            m.touch([r for a in args for r in regs(a)], line)
+            assert args[0] not in starts
+            starts[args[0]] = m.val.get(args[1], args[1])
         else:
             m.touch([r for a in args for r in regs(a)], line)
+            assert not set(regs(args[0])) & set(starts), line
+            if regs(args[0]):
+                m.val[regs(args[0])[0]] = None
         assert len(m.lds) <= 15 and len(m.vm) <= 63
     assert end > loop and steps == FILLS
     # every sum: per fill 16 quadruples of its own unit and pixel, each step once, out of the fill's own buffer
-    assert len(sums) == 4 * units
+    # and started from the correction (low bytes) or zero (high bytes)
+    assert len(sums) == 4 * units and len(starts) == 16 * units
     for u in range(units):
         for j in range(4):
+            assert [starts[r] for r in regs(gen.acc_reg(units, u, j))] == ["cinit", "0"] * 2
             got = sums[tuple(regs(gen.acc_reg(units, u, j)))]
             assert sorted(got) == sorted(("look", f, u, j, c, f) for f in range(FILLS) for c in range(4)), (u, j)
     # the rows: 16 pieces of 1 KiB per fill, while the wavefront reads the other buffer (before the flip to it)
