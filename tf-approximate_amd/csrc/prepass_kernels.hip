@@ -524,6 +524,10 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
         batched_chain(std::integral_constant<int, 4>());
         return;
     }
+    // Scalar loads count down together with LDS reads, but in no order: while the compiler takes one to be in flight it waits
+    // for all reads of a batch before the first add (3x3/2 680->12 @49x59x38: 409 -> 440 us of pre-pass).
+    wait_lds_reads<0>();
+    chain_fence(s);
     for (int kh = 0; kh < g.KH; ++kh) {
         const int r = ohl * g.sh + kh * g.dh;        // LDS row of this tap; rows outside the image hold zeros,
         for (int kw = 0; kw < g.KW; ++kw) {          // and x + 0.0f == x, so they need no branch
