@@ -23,16 +23,17 @@ __device__ __forceinline__ void wait_lds_reads()
     __builtin_amdgcn_s_waitcnt(0xC07F | (PENDING << 8)); // vmcnt and expcnt left at their maxima
 }
 
-// Dword index of channel quad c4 of pixel (n, h, w) in xq, and of the first quad's row of image row nh = n * H + h.
+// Dword index of channel quad 0 of pixel (n, h, 0) in xq, and of the same where the image row is nh = n * H + h.  Padding
+// is written out for lutgemm_mx_kernel only, whose xq has fewer than 2^29 dwords.
 __device__ __forceinline__ int64_t xq_row(const XqLayout &lay, int64_t n, int h, int C4)
 {
     return (n * lay.Hp + h + lay.row0) * C4 * lay.Wp + lay.col0;
 }
 __device__ __forceinline__ int64_t xq_row_nh(const XqLayout &lay, int64_t nh, int H, int C4)
 {
-    if (lay.Hp != H) {
-        const int64_t n = nh / H;
-        return xq_row(lay, n, (int)(nh - n * H), C4);
+    if (lay.row0) {
+        const uint32_t n = (uint32_t)nh / (uint32_t)H;
+        return xq_row(lay, n, (int)((uint32_t)nh - n * (uint32_t)H), C4);
     }
     return nh * C4 * lay.Wp + lay.col0;
 }
@@ -43,24 +44,28 @@ __device__ __forceinline__ int64_t xq_row_nh(const XqLayout &lay, int64_t nh, in
 __device__ __forceinline__ void xq_fill_padding(uint32_t *__restrict__ xq, const XqLayout &lay, int N, int H, int C4,
                                                 uint32_t zp4, int64_t first, int64_t step)
 {
-    const int64_t row = (int64_t)C4 * lay.Wp;
-    const int64_t rows_total = ((int64_t)N * lay.row0 + lay.tail_rows()) * row;
-    for (int64_t i = first; i < rows_total; i += step) {
-        const int64_t k = i / row;
-        int64_t r = (int64_t)N * lay.Hp + (k - (int64_t)N * lay.row0);
-        if (k < (int64_t)N * lay.row0) {
-            const int64_t n = k / lay.row0;
-            r = n * lay.Hp + (k - n * lay.row0);
+    if ((lay.row0 | lay.col0) == 0) {   // one row behind the last image, a run of memory
+        const int64_t row = (int64_t)C4 * lay.Wp;
+        uint32_t *const tail = xq + (int64_t)N * H * row;
+        for (int64_t i = first; i < row; i += step)
+            tail[i] = zp4;
+        return;
+    }
+    const uint32_t row = (uint32_t)C4 * (uint32_t)lay.Wp, row0 = (uint32_t)lay.row0, col0 = (uint32_t)lay.col0;
+    const uint32_t Hp = (uint32_t)lay.Hp, front = (uint32_t)N * row0, rows = front + (uint32_t)lay.tail_rows();
+    for (int64_t at = first; at < (int64_t)rows * row; at += step) {
+        const uint32_t i = (uint32_t)at, k = i / row;
+        uint32_t r = (uint32_t)N * Hp + (k - front);
+        if (k < front) {
+            const uint32_t n = k / row0;
+            r = n * Hp + (k - n * row0);
         }
         xq[r * row + (i - k * row)] = zp4;
     }
-    if (lay.col0 == 0)
-        return;
-    const int64_t cols_total = (int64_t)N * H * C4 * lay.col0;
-    for (int64_t i = first; i < cols_total; i += step) {
-        const int64_t pl = i / lay.col0, nh = pl / C4, n = nh / H;   // plane, image row
-        const int c4 = (int)(pl - nh * C4), h = (int)(nh - n * H);
-        xq[((n * lay.Hp + h + lay.row0) * C4 + c4) * lay.Wp + (i - pl * lay.col0)] = zp4;
+    for (int64_t at = first; at < (int64_t)N * H * C4 * col0; at += step) {   // (none without column padding)
+        const uint32_t i = (uint32_t)at, pl = i / col0, nh = pl / (uint32_t)C4, n = nh / (uint32_t)H;   // plane, image row
+        const uint32_t c4 = pl - nh * (uint32_t)C4, h = nh - n * (uint32_t)H;
+        xq[((n * Hp + h + row0) * (uint32_t)C4 + c4) * (uint32_t)lay.Wp + (i - pl * col0)] = zp4;
     }
 }
 
@@ -72,7 +77,7 @@ __device__ __forceinline__ void xq_fill_padding(uint32_t *__restrict__ xq, const
 //   chsum[N][H][W]      sum over channels of the raw floats, c ascending
 // One thread per pixel: the channel loop is sequential so the sum has the reference's order within a pixel.
 __global__ void __launch_bounds__(256) quantize_relayout_kernel(const float *__restrict__ x, int64_t pixels,
-                                                                 int H, int W, int C, int C4, const XqLayout lay,
+                                                                 int N, int H, int W, int C, int C4, const XqLayout lay,
                                                                  const TensorQuant tq,
                                                                  const LayerQuant *__restrict__ lq_dev,
                                                                  uint32_t *__restrict__ xq,
@@ -80,7 +85,7 @@ __global__ void __launch_bounds__(256) quantize_relayout_kernel(const float *__r
 {
     const TensorQuant q = lq_dev ? lq_dev->in : tq;
     const int64_t pix = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    xq_fill_padding(xq, lay, (int)(pixels / ((int64_t)H * W)), H, C4, q.zp4, pix, (int64_t)gridDim.x * blockDim.x);
+    xq_fill_padding(xq, lay, N, H, C4, q.zp4, pix, (int64_t)gridDim.x * blockDim.x);
     if (pix >= pixels)
         return;
     const int w = (int)(pix % W);
@@ -108,15 +113,14 @@ __global__ void __launch_bounds__(256) quantize_relayout_kernel(const float *__r
 // Same result as quantize_relayout_kernel for C % 4 == 0, with fully coalesced reads: consecutive lanes
 // read consecutive float4 of the NHWC input (one float4 = the four channels of one xq dword).
 __global__ void __launch_bounds__(256) quantize_relayout_vec4_kernel(const float4 *__restrict__ x4, int64_t quads,
-                                                                      int H, int W, int C4, const XqLayout lay,
+                                                                      int N, int H, int W, int C4, const XqLayout lay,
                                                                       const TensorQuant tq,
                                                                       const LayerQuant *__restrict__ lq_dev,
                                                                       uint32_t *__restrict__ xq)
 {
     const TensorQuant q = lq_dev ? lq_dev->in : tq;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    xq_fill_padding(xq, lay, (int)(quads / ((int64_t)H * W * C4)), H, C4, q.zp4,
-                    (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride);
+    xq_fill_padding(xq, lay, N, H, C4, q.zp4, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += stride) {
         const float4 v = x4[i];
         const int64_t pix = i / C4;
@@ -269,33 +273,46 @@ __global__ void __launch_bounds__(kPsTile) patch_sums_tiled_kernel(const float *
         psum[m] = s;
 }
 
+// What a launch prepares a layer for.  lutgemm_mx_kernel reads xq with its padding written out and rows in a form of their
+// own; launches for the other kernels are instantiations without either, so that their code carries none of it (as run-time
+// values they cost the pre-pass of small layers 0.2 to 0.4 us: more arguments to fetch, more scalar registers to spill).
+struct PlainForm {
+    __device__ static XqLayout layout(const ConvGeom &g) { return {g.H, g.W, 0, 0}; }
+    __device__ static int mx_fills() { return 0; }
+};
+struct MxForm {
+    XqLayout lay;
+    int fills;        // of the rows, per column tile
+    __device__ const XqLayout &layout(const ConvGeom &) const { return lay; }
+    __device__ int mx_fills() const { return fills; }
+};
+
 // The filter pre-pass of a layer is independent of its input pre-pass: as two launches they would run one after
 // the other, so the launch below carries both: the filter work of filter_prep_kernel in workgroups of its own
 // (ordered as described at the members below), the patch sums in the others.
-struct FilterWork {
+struct FilterWork {   // members by size: every 64 bytes of arguments are a fetch that a small launch waits for
     const float *filter;
     const uint8_t *filter_codes;
-    int taps, C, C4, Co, nt, n_col_tiles;
-    TensorQuant tq;
     uint16_t *wq;
-    int sum_blocks;
     float *fsum;
+    const uint16_t *tableT;
+    uint16_t *px_rows;
+    // pack_total > 0: no pack blocks; the threads of the patch-sum blocks that run no chain pack the codes,
+    // each block its share of the pack_total elements
+    int64_t pack_total;
     // Order of the workgroups of a launch: the filter sums (long chains: first), rounded up to a multiple of 8 so
     // that workgroup index mod 8 stays the XCD for the others; the patch sums; the workgroups that pack filter codes
     // (many and short: they fill the tail).
     int sum8;         // sum_blocks rounded up to a multiple of 8
     int work_blocks;  // patch-sum workgroups
     int pack_blocks;  // 0: no pack workgroups
-    // pack_total > 0: no pack blocks; the threads of the patch-sum blocks that run no chain pack the codes,
-    // each block its share of the pack_total elements
-    int64_t pack_total;
+    int sum_blocks;
     // expand_blocks > 0: the last workgroups of the launch build the pre-expanded rows of lutgemm_px_kernel.hip
     // (px_expand.h), blockDim.x / 4 activation codes of one (column tile, pair of fills) each: the rows depend on the
     // filter and the table only, so they need not wait for the patch sums in a launch of their own
     int expand_blocks;
-    const uint16_t *tableT;
-    uint16_t *px_rows;
-    int mx_fills;     // > 0: rows in the form lutgemm_mx_kernel.hip reads, this many fills per column tile
+    int taps, C, C4, Co, nt, n_col_tiles;
+    TensorQuant tq;
 };
 
 __device__ __forceinline__ void filter_pack_element(const int64_t i, const float *__restrict__ filter,
@@ -337,6 +354,7 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
     const int segs = SEG ? (g.OW + wseg - 1) / wseg : 1;
     const int nb = SEG ? bid / segs : bid, seg = SEG ? bid - nb * segs : 0;   // nb: (image, band)
     const int n = nb / bands, band = nb - n * bands;
+    uint32_t *const xq_n = xq + xq_row(lay, n, 0, g.C4);
     const int oh0 = band * rb;
     const int ih_first = oh0 * g.sh - g.ph;  // input row held in LDS row 0 (may lie outside the image)
     const int own_lo = oh0 * g.sh;           // owned input rows: [own_lo, own_hi)
@@ -403,7 +421,7 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
                     *reinterpret_cast<float4 *>(&rows[(rr[u] * wc + ww[u]) * pitch + q * 4]) = f;
                     const int iw = iw_lo + ww[u];
                     if (xq && in_image && ih >= own_lo && ih < own_hi && (!SEG || (iw >= own_clo && iw < own_chi)))
-                        xq[xq_row(lay, n, ih, g.C4) + q * lay.Wp + iw] =
+                        xq_n[((uint32_t)ih * (uint32_t)g.C4 + (uint32_t)q) * (uint32_t)lay.Wp + (uint32_t)iw] =
                             phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
                             (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
                             (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
@@ -678,11 +696,11 @@ __global__ void __launch_bounds__(1024) patch_sums_smallc_kernel(const float *__
 
 // Same relayout for caller-supplied codes (uint8 NHWC).
 __global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__restrict__ codes, int64_t pixels,
-                                                              int H, int W, int C, int C4, const XqLayout lay,
+                                                              int N, int H, int W, int C, int C4, const XqLayout lay,
                                                               uint32_t zp4, uint32_t *__restrict__ xq)
 {
     const int64_t pix = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    xq_fill_padding(xq, lay, (int)(pixels / ((int64_t)H * W)), H, C4, zp4, pix, (int64_t)gridDim.x * blockDim.x);
+    xq_fill_padding(xq, lay, N, H, C4, zp4, pix, (int64_t)gridDim.x * blockDim.x);
     if (pix >= pixels)
         return;
     const int w = (int)(pix % W);
@@ -921,6 +939,7 @@ hipError_t launch_mx_expand_rows(const float *filter, const uint8_t *filter_code
 
 // One launch for the whole filter pre-pass: the first sum_blocks workgroups compute the column sums (skipped when
 // fsum is null), the next pack_blocks pack the codes, any further ones build pre-expanded rows.
+template <class Form>
 __global__ void __launch_bounds__(kFsThreads) filter_prep_kernel(const float *__restrict__ filter,
                                                                   const uint8_t *__restrict__ filter_codes, int taps,
                                                                   int C, int C4, int Co, int nt, int n_col_tiles,
@@ -929,7 +948,7 @@ __global__ void __launch_bounds__(kFsThreads) filter_prep_kernel(const float *__
                                                                   uint16_t *__restrict__ wq, int sum_blocks,
                                                                   float *__restrict__ fsum, int pack_blocks,
                                                                   const uint16_t *__restrict__ tableT,
-                                                                  uint16_t *__restrict__ px_rows, const int mx_fills)
+                                                                  uint16_t *__restrict__ px_rows, const Form form)
 {
     const TensorQuant q = lq_dev ? lq_dev->flt : tq;
     if ((int)blockIdx.x < sum_blocks) {
@@ -942,7 +961,8 @@ __global__ void __launch_bounds__(kFsThreads) filter_prep_kernel(const float *__
         filter_pack_element(i, filter, filter_codes, taps, C, C4, Co, nt, n_col_tiles, q, wq);
         return;
     }
-    px_expand_own_codes<kFsThreads / 4>(pb - pack_blocks, filter, filter_codes, taps, C, C4, Co, q, tableT, px_rows, mx_fills);
+    px_expand_own_codes<kFsThreads / 4>(pb - pack_blocks, filter, filter_codes, taps, C, C4, Co, q, tableT, px_rows,
+                                         form.mx_fills());
 }
 
 // Patch sums of a 1x1, stride-1, unpadded layer: the patch of an output pixel is the pixel itself, so the pixels
@@ -1187,7 +1207,8 @@ __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x
 
 // The filter work of a patch-sum launch: true if this workgroup is one of those that do it (and has done it), else
 // *bid is its index among the patch-sum workgroups.
-__device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const LayerQuant *__restrict__ lq_dev, int *bid)
+__device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const int mx_fills,
+                                                  const LayerQuant *__restrict__ lq_dev, int *bid)
 {
     const int b = (int)blockIdx.x;
     if (b < fw.sum8) {
@@ -1214,35 +1235,39 @@ __device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const La
     const int eb = pb - fw.pack_blocks;
     if (blockDim.x == 512)
         px_expand_own_codes<128>(eb, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, q, fw.tableT, fw.px_rows,
-                                 fw.mx_fills);
+                                 mx_fills);
     else
         px_expand_own_codes<256>(eb, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, q, fw.tableT, fw.px_rows,
-                                 fw.mx_fills);
+                                 mx_fills);
     return true;
 }
 
 // Bands cut into column segments: a kernel of its own, so that the common variants below stay as small as they were.
+template <class Form>
 __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *__restrict__ x, const ConvGeom g,
                                                                     int rb, int in_rows, int nthreads, int wseg,
                                                                     const TensorQuant tq,
                                                                     const LayerQuant *__restrict__ lq_dev,
                                                                     float *__restrict__ psum, uint32_t *__restrict__ xq,
-                                                                    const XqLayout lay, const FilterWork fw)
+                                                                    const FilterWork fw, const Form form)
 {
+    const XqLayout lay = form.layout(g);
     int bid;
-    if (filter_work_block(fw, lq_dev, &bid))
+    if (filter_work_block(fw, form.mx_fills(), lq_dev, &bid))
         return;
     patch_sums_rows_body<true>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw);
 }
 
+template <class Form>
 __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__restrict__ x, const ConvGeom g, int rb,
                                                                 int in_rows, int nthreads, const TensorQuant tq,
                                                                 const LayerQuant *__restrict__ lq_dev,
                                                                 float *__restrict__ psum, uint32_t *__restrict__ xq,
-                                                                const XqLayout lay, const FilterWork fw)
+                                                                const FilterWork fw, const Form form)
 {
+    const XqLayout lay = form.layout(g);
     int bid;
-    if (filter_work_block(fw, lq_dev, &bid))
+    if (filter_work_block(fw, form.mx_fills(), lq_dev, &bid))
         return;
     if (rb < 0) { // 1x1, stride 1, many channels, few pixels
         if (in_rows == 8)
@@ -1692,11 +1717,11 @@ hipError_t launch_quantize_relayout(const float *x, const ConvGeom &g, const Ten
         int64_t blocks = (quads + 256 * 4 - 1) / (256 * 4);
         if (blocks > 65536) blocks = 65536;
         hipLaunchKernelGGL(quantize_relayout_vec4_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
-                           reinterpret_cast<const float4 *>(x), quads, g.H, g.W, g.C4, lay, tq, lq_dev, xq);
+                           reinterpret_cast<const float4 *>(x), quads, g.N, g.H, g.W, g.C4, lay, tq, lq_dev, xq);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(quantize_relayout_kernel, dim3(blocks_for(pixels, 256)), dim3(256), 0, stream, x, pixels,
-                       g.H, g.W, g.C, g.C4, lay, tq, lq_dev, xq, chsum);
+                       g.N, g.H, g.W, g.C, g.C4, lay, tq, lq_dev, xq, chsum);
     return hipGetLastError();
 }
 
@@ -1940,7 +1965,6 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                         fw.expand_blocks = (int)eb;
                         fw.tableT = filter_job->tableT;
                         fw.px_rows = filter_job->px_rows;
-                        fw.mx_fills = mx ? mx->fills : 0;
                         lds = lds < need ? need : lds;
                         *px_done = true;
                     }
@@ -1948,21 +1972,24 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             }
             fw.work_blocks = (int)work_blocks;
             const unsigned grid = (unsigned)(fw.sum8 + work_blocks + fw.pack_blocks + fw.expand_blocks);
-            if (segmented) {
-                const hipError_t e =
-                    set_max_dynamic_lds_once(reinterpret_cast<const void *>(patch_sums_segments_kernel), device_lds_bytes());
+            auto launch = [&](const auto &form) {
+                using Form = std::decay_t<decltype(form)>;
+                const void *const kernel = segmented ? reinterpret_cast<const void *>(patch_sums_segments_kernel<Form>)
+                                                     : reinterpret_cast<const void *>(patch_sums_rows_kernel<Form>);
+                const hipError_t e = set_max_dynamic_lds_once(kernel, device_lds_bytes());
                 if (e != hipSuccess)
                     return e;
-                hipLaunchKernelGGL(patch_sums_segments_kernel, dim3(grid), dim3(block_threads), lds, stream, x, g, rb, in_rows, threads, wseg, tq, lq_dev, psum,
-                                   fuse ? xq_fused : nullptr, lay, fw);
+                uint32_t *const codes_out = fuse ? xq_fused : nullptr;
+                if (segmented)
+                    hipLaunchKernelGGL(patch_sums_segments_kernel<Form>, dim3(grid), dim3(block_threads), lds, stream, x, g, rb,
+                                       in_rows, threads, wseg, tq, lq_dev, psum, codes_out, fw, form);
+                else
+                    hipLaunchKernelGGL(patch_sums_rows_kernel<Form>, dim3(grid), dim3(block_threads), lds, stream, x, g, rb,
+                                       in_rows, threads, tq, lq_dev, psum, codes_out, fw, form);
                 return hipGetLastError();
-            }
-            const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(patch_sums_rows_kernel), device_lds_bytes());
-            if (e != hipSuccess)
-                return e;
-            hipLaunchKernelGGL(patch_sums_rows_kernel, dim3(grid), dim3(block_threads),
-                               lds, stream, x, g, rb, in_rows, threads, tq, lq_dev, psum, fuse ? xq_fused : nullptr, lay, fw);
-            return hipGetLastError();
+            };
+            const bool mx_form = (filter_job && filter_job->mx) || lay.row0 || lay.col0;
+            return mx_form ? launch(MxForm{lay, filter_job && filter_job->mx ? filter_job->mx->fills : 0}) : launch(PlainForm{});
         }
     }
     if (!vec && g.OW <= 1024 && g.C < 64) {
@@ -2048,7 +2075,7 @@ hipError_t launch_codes_relayout(const uint8_t *codes, const ConvGeom &g, const 
                                  hipStream_t stream)
 {
     const int64_t pixels = (int64_t)g.N * g.H * g.W;
-    hipLaunchKernelGGL(codes_relayout_kernel, dim3(blocks_for(pixels, 256)), dim3(256), 0, stream, codes, pixels, g.H,
+    hipLaunchKernelGGL(codes_relayout_kernel, dim3(blocks_for(pixels, 256)), dim3(256), 0, stream, codes, pixels, g.N, g.H,
                        g.W, g.C, g.C4, lay, zp4, xq);
     return hipGetLastError();
 }
@@ -2076,16 +2103,20 @@ hipError_t launch_filter_pack(const float *filter, const uint8_t *filter_codes, 
     }
     if (sum_blocks + pack_blocks + expand_blocks == 0)   // rows in a launch of their own, nothing else to do
         return hipSuccess;
-    if (lds) {
-        const hipError_t ea = set_max_dynamic_lds_once(reinterpret_cast<const void *>(filter_prep_kernel),
-                                                       (int)(lds > (size_t)kFsLdsBytes ? lds : (size_t)kFsLdsBytes));
-        if (ea != hipSuccess)
-            return ea;
-    }
-    hipLaunchKernelGGL(filter_prep_kernel, dim3((unsigned)(sum_blocks + pack_blocks + expand_blocks)), dim3(kFsThreads), lds,
-                       stream, filter, filter_codes, g.KH * g.KW, g.C, g.C4, g.Co, plan.nt, plan.n_col_tiles, tq, lq_dev,
-                       wq, sum_blocks, fsum, pack_blocks, tableT, px_rows, mx ? mx->fills : 0);
-    return hipGetLastError();
+    auto launch = [&](const auto &form) {
+        using Form = std::decay_t<decltype(form)>;
+        if (lds) {
+            const hipError_t ea = set_max_dynamic_lds_once(reinterpret_cast<const void *>(filter_prep_kernel<Form>),
+                                                           (int)(lds > (size_t)kFsLdsBytes ? lds : (size_t)kFsLdsBytes));
+            if (ea != hipSuccess)
+                return ea;
+        }
+        hipLaunchKernelGGL(filter_prep_kernel<Form>, dim3((unsigned)(sum_blocks + pack_blocks + expand_blocks)), dim3(kFsThreads),
+                           lds, stream, filter, filter_codes, g.KH * g.KW, g.C, g.C4, g.Co, plan.nt, plan.n_col_tiles, tq, lq_dev,
+                           wq, sum_blocks, fsum, pack_blocks, tableT, px_rows, form);
+        return hipGetLastError();
+    };
+    return mx ? launch(MxForm{XqLayout{}, mx->fills}) : launch(PlainForm{});
 }
 
 // Flat layout of the quantized input for channel counts that are no multiple of four: one thread per dword of xq.
@@ -2104,9 +2135,15 @@ __global__ void __launch_bounds__(256) quantize_flat_rows_kernel(const float *__
     const int dwords_per_row = row_bytes / 4;
     if (i >= ((int64_t)N * lay.Hp + lay.tail_rows()) * dwords_per_row)
         return;
-    const int64_t r = i / dwords_per_row, n = r / lay.Hp;
-    const int h = (int)(r - n * lay.Hp) - lay.row0;
-    const int b0 = (int)(i - r * dwords_per_row) * 4;
+    // (fewer than 2^29 dwords, see prepare_dense)
+    const uint32_t r = (uint32_t)i / (uint32_t)dwords_per_row;
+    uint32_t n = 0, h = r;   // without rows in front of the images they are one run of N * H rows
+    if (lay.row0) {
+        n = r / (uint32_t)lay.Hp;
+        h = r - n * (uint32_t)lay.Hp - (uint32_t)lay.row0;   // wraps for a row in front
+    }
+    const bool in_image = lay.row0 ? n < (uint32_t)N && h < (uint32_t)H : r < (uint32_t)N * (uint32_t)H;
+    const int b0 = (int)((uint32_t)i - r * (uint32_t)dwords_per_row) * 4;
     const uint32_t zp = qt.zp4 & 0xffu;
     uint32_t word = 0;
 #pragma unroll
@@ -2114,8 +2151,8 @@ __global__ void __launch_bounds__(256) quantize_flat_rows_kernel(const float *__
         const int b = b0 + k;
         const int px = b / C, c = b - px * C, w = px - pad_left;
         uint32_t code = zp;
-        if (n < N && h >= 0 && (unsigned)w < (unsigned)W) {
-            const int64_t src = ((n * H + h) * W + w) * C + c;
+        if (in_image && (unsigned)w < (unsigned)W) {
+            const int64_t src = (((int64_t)n * H + h) * W + w) * C + c;
             code = codes ? phys_row(codes[src])
                          : phys_row(quantize_code(fake_quant_value(x[src], qt), qt.offset, qt.inv_scale));
         }
