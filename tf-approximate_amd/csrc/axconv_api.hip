@@ -783,8 +783,8 @@ void prepare_mx(PreparedDense *pd)
 // A 1x1 filter with a stride only ever reads every stride-th pixel, and never needs padding: the op equals the 1x1
 // stride-1 op on the subsampled input.  Those pixels are gathered into the workspace first (element_bytes each:
 // floats, or bytes for the codes entry point), and every kernel then sees a dense, unpadded stride-1 layer with a
-// quarter (stride 2) of the pixels to quantize and sum.  allow_subsample = false keeps the layer as given (callers
-// with their own padding origin: `pads`, rows and columns).  allow_mx = false: the layer as the other kernels run it.
+// quarter (stride 2) of the pixels to quantize and sum.  Callers with a padding origin of their own (`pads`: rows and columns)
+// get the layer as given.  allow_mx = false: the layer as the other kernels run it.
 int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
                   int px_mode = kPxModeGlobal, bool allow_mx = true)
 {
@@ -1094,7 +1094,6 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         m.oh = g.OH;
         m.ow = g.OW;
         m.groups_per_row = (g.OW + 3) / 4;
-        m.groups = (int)((int64_t)g.N * g.OH * m.groups_per_row);
         m.linear = (g.OW & 3) == 0;
         m.div_groups = mx_div((uint32_t)m.groups_per_row);
         m.div_oh = mx_div((uint32_t)g.OH);
@@ -1474,14 +1473,11 @@ int axc_axconv2d_quint8(const axc_table *table, const axc_conv2d_desc *desc, con
     rc = validate_for_launch(desc, dims, false);
     if (rc != AXC_OK)
         return rc;
-    int pads[2];
-    axconv_tf1_pads(make_geom(dims), desc->padding, pads);
-    PreparedDense pd;
-    rc = prepare_dense_for(desc, workspace_bytes, pads, 1, &pd);   // the form run_dense gives it: where its sums may go
-    if (rc != AXC_OK)
-        return rc;
-    if (pd.empty)
+    const ConvGeom g = make_geom(dims);
+    if (g.M * g.Co == 0)   // no outputs
         return AXC_OK;
+    int pads[2];
+    axconv_tf1_pads(g, desc->padding, pads);
     if (!input || !filter || !output)
         return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
     return run_dense(table, desc, nullptr, nullptr, input, filter, offset_input, 0.0f, 0.0f, 0.0f, 0.0f, nullptr, output,

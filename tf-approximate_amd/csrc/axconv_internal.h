@@ -170,7 +170,7 @@ struct MxParams {
     int relu;
     int64_t M;
     int Co, oh, ow;
-    int groups, groups_per_row;    // groups of four neighbouring pixels of an output row: of the layer, per row
+    int groups_per_row;            // groups of four neighbouring pixels per output row
     int linear;                    // output rows are whole groups: pixel = 4 * group + position
     MxDiv div_groups, div_oh, div_c4, div_kw;
     // bytes in xq: of output pixel 0's tap (0, 0); between images, output rows, pixel groups, pixels of a group; between

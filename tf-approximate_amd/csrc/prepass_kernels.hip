@@ -1313,7 +1313,7 @@ __global__ void __launch_bounds__(256) depthwise_filter_kernel(const float *__re
 
 static inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
-// The extra [C4][W] row behind xq: every dword is the zero-point code x4.
+// Layers without taps or channels: every output is the same value.
 __global__ void __launch_bounds__(256) fill_u32_kernel(uint32_t *__restrict__ dst, int n, uint32_t value)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1955,7 +1955,7 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                     const size_t need = (size_t)(block_threads / 4) * kPxExpandPitch * 4 + 256;
                     // Every workgroup of a launch takes the same LDS.  Where the patch sums take so much that a CU
                     // holds fewer of these workgroups than its wavefront slots allow (2048 threads), the rows are
-                    // written more slowly; that still beats a launch of their own (north star -1.8 %, 3x3 128->128
+                    // written more slowly; that still beats a launch of their own (3x3 64->64 @56x56x64 -1.8 %, 3x3 128->128
                     // @28x28 -3.1 %) until the rows are many (1.2 GB: 0.26 -> 0.33 ms, +2.3 % on the layer).
                     const size_t lds_with = lds < need ? need : lds;
                     const bool slow = lds_with * (size_t)(2048 / block_threads) > (size_t)device_lds_bytes();
