@@ -41,9 +41,16 @@ CASES = [
     # odd numbers of channel quads, whose other kernel expands the rows inside its tiles
     ((8, 57, 55, 4), (5, 5, 40), 1, 1, "SAME", 2, False),        # one quad: four taps to a step of the filter position
     ((4, 40, 31, 12), (5, 5, 40), 1, 1, "SAME", 2, True),        # three
-    ((9, 40, 31, 9), (5, 3, 50), 1, 1, "SAME", 2, False),        # nine channels in three quads, fifty columns
     ((7, 61, 45, 20), (3, 3, 75), 2, 1, "VALID", 3, True),       # five
     ((5, 57, 29, 36), (3, 3, 40), 1, 1, "VALID", 4, True),       # nine
+    # flat layout: the codes under a filter row are one run of bytes
+    ((9, 40, 31, 9), (5, 3, 50), 1, 1, "SAME", 2, False),        # 27 bytes in seven quads, fifty columns
+    ((8, 57, 61, 3), (5, 5, 40), 1, 1, "SAME", 3, False),        # three bytes between pixels: a load per pixel
+    # ... and with four bytes between neighbouring outputs' pixels: one load for a group of four
+    ((16, 113, 111, 2), (3, 3, 40), 2, 1, "SAME", 4, False),     # two channels, stride 2
+    ((16, 112, 112, 2), (5, 5, 64), 2, 1, "VALID", 6, False),
+    ((8, 225, 223, 1), (5, 8, 33), 4, 1, "SAME", 2, False),      # one channel, stride 4, ragged
+    ((64, 31, 30, 1), (9, 9, 72), 4, 1, "VALID", 2, False),
 ]
 
 
@@ -74,12 +81,17 @@ def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, case):
     def run():
         return (op.accumulators(xd, fd, *MM), op(xd, fd, *MM), op(xd, fd, *MM, bias=bias, activation="relu"),
                 op(xd, fd, *MM, bias=bias), op(xd, fd, *MM, activation="relu"))
-    got = run()
+    ops.profile_enable(True)
+    ops.profile_reset()
     try:
+        got = run()
+        torch.cuda.synchronize()
+        assert {k for k in ops.profile_read() if k.startswith("lutgemm")} == {"lutgemm_px", "lutgemm_mx"}
         ops.set_preexpand(-1)
         want = run()
     finally:
         ops.set_preexpand(0)
+        ops.profile_enable(False)
     for g, w in zip(got, want):
         bad = g.view(torch.int32) != w.view(torch.int32)
         assert not bool(bad.any()), "%d of %d differ, first at %s" % (
@@ -142,3 +154,28 @@ def test_output_rows_beyond_2_gib(pkg, xs, fs):
         finally:
             ops.set_preexpand(0)
         assert torch.equal(got, want), "%d of %d differ" % (int((got != want).sum()), got.numel())
+
+
+def test_a_wait_that_runs_out_is_reported_by_the_next_call(pkg):
+    """With a wait limit of zero polls the first wavefront to look at a counter before its time gives up, the others
+    follow when they next wait, and every wavefront leaves the kernel.  The launch itself returns as usual; the next call
+    on the device reports it, once; with the limit restored the layer is right again."""
+    xs, fs = (16, 64, 64, 24), (3, 3, 24, 64)
+    ops = pkg.ops
+    assert ops.conv2d_matrix_plan(xs, fs) is not None
+    xd, fd = bench.device_tensors(pkg, xs, fs, "uniform", seed=1)
+    op = pkg.ApproxConv2DWithMinMaxVars([1, 1, 1, 1], 8, pkg.synth.table_random(2), "SAME")
+    good = op.accumulators(xd, fd, *MM).clone()
+    torch.cuda.synchronize()
+    ops.set_wait_limit(0)
+    try:
+        print("launch with a wait limit of 0 polls", flush=True)
+        op.accumulators(xd, fd, *MM)
+        torch.cuda.synchronize()
+    finally:
+        ops.set_wait_limit(1 << 20)
+    with pytest.raises(RuntimeError, match="gave up a wait"):
+        op.accumulators(xd, fd, *MM)
+    again = op.accumulators(xd, fd, *MM)      # reported once
+    torch.cuda.synchronize()
+    assert torch.equal(again, good)

@@ -98,28 +98,36 @@ def test_network_layer_at_full_batch_sampled_pixels(pkg, oracle, case):
     _sampled(pkg, oracle, case)
 
 
-def _plan_uses_preexpanded_rows(pkg, case, mode):
+def _dense_kernel(pkg, case, mode):
+    """The LUT-GEMM kernel that a layer runs under axc_set_preexpand(mode)."""
     _, xs, fs, stride, _ = case
     pkg.ops.set_preexpand(mode)
     try:
-        return bool(pkg.ops.conv2d_tile_plan(xs, fs, (1, stride, stride, 1))["preexpanded_rows"])
+        if pkg.ops.conv2d_matrix_plan(xs, fs, (1, stride, stride, 1)) is not None:
+            return "lutgemm_mx"
+        rows = pkg.ops.conv2d_tile_plan(xs, fs, (1, stride, stride, 1))["preexpanded_rows"]
+        return "lutgemm_px" if rows else "lutgemm_expand"
     finally:
         pkg.ops.set_preexpand(0)
 
 
+@pytest.mark.parametrize("mode", [1, -1])
 @pytest.mark.parametrize("case", [c for c in _layers() if not c[4]], ids=_id)
-def test_network_layer_sampled_pixels_in_the_kernel_the_planner_did_not_pick(pkg, oracle, case):
-    """Each dense layer once more with the other LUT-GEMM kernel: out of pre-expanded rows where the planner expands
-    inside the tiles, and the other way round.  Layers that can only run one way are skipped."""
-    own = _plan_uses_preexpanded_rows(pkg, case, 0)
-    other_mode = -1 if own else 1
-    if _plan_uses_preexpanded_rows(pkg, case, other_mode) == own:
-        pytest.skip("only one kernel can run this layer")
-    print("layer", _id(case), "preexpand", other_mode, flush=True)
-    pkg.ops.set_preexpand(other_mode)
+def test_network_layer_sampled_pixels_in_the_kernel_the_planner_did_not_pick(pkg, oracle, case, mode):
+    """Each dense layer once more in each LUT-GEMM kernel that is not the planner's choice: out of pre-expanded rows with
+    the sums on the vector ALUs (1), and expanding inside the tiles (-1)."""
+    kernel = _dense_kernel(pkg, case, mode)
+    if kernel == _dense_kernel(pkg, case, 0) or kernel == "lutgemm_expand" and mode == 1:
+        pytest.skip("the planner's own kernel, or one that cannot run this layer")
+    print("layer", _id(case), "preexpand", mode, flush=True)
+    pkg.ops.set_preexpand(mode)
+    pkg.ops.profile_enable(True)
+    pkg.ops.profile_reset()
     try:
         _sampled(pkg, oracle, case)
+        assert {k for k in pkg.ops.profile_read() if k.startswith("lutgemm")} == {kernel, kernel.replace("mx", "px")}
     finally:
+        pkg.ops.profile_enable(False)
         pkg.ops.set_preexpand(0)
 
 

@@ -1,8 +1,9 @@
 """The LUT-GEMM kernel that reads pre-expanded rows without a barrier between fills (lutgemm_pxf_kernel in
 tf-approximate_amd/csrc/lutgemm_px_kernel.hip): its wavefronts are held together by two LDS counters only.
 
-The planner picks it for tiles of 16 to 63 wavefront-rows with 16 fills or more (32 for a 1x1 filter), so the cases
-here are full-size layers, each asserted to get that kernel (tile plan code 2).  Every case is checked three ways:
+The planner gives it tiles of 16 to 63 wavefront-rows with 16 fills or more (32 for a 1x1 filter), where the layer does not
+run on the matrix cores.  So the cases here are full-size layers, with the matrix-core kernel switched off for all of
+them (axc_set_preexpand(1)), each asserted to get this kernel: tile plan code 2, and its launch timed.  Every case is checked three ways:
 the whole tensor of int32 sums and the whole float output bit for bit against the kernel that expands inside its tiles
 (itself pinned against the oracle by the per-layer tests), sampled pixels against the CPU oracle, and, where torch can
 restate the layer, the whole tensor of sums with the exact table against an fp64 convolution of the codes.  Shapes
@@ -23,6 +24,15 @@ from test_gpu_networks import exact_conv_of_codes
 pytestmark = pytest.mark.gpu
 
 MM = (-1.0, 1.0, -0.5, 0.5)
+
+
+@pytest.fixture(autouse=True)
+def out_of_preexpanded_rows(pkg):
+    """Which keeps the matrix-core kernel out; the cases' tile plans are what they are without it."""
+    pkg.ops.set_preexpand(1)
+    yield
+    pkg.ops.set_preexpand(0)
+
 
 CASES = [
     # input, filter, stride, dilation, padding
@@ -84,7 +94,7 @@ def test_barrier_free_kernel_whole_output_and_oracle(pkg, oracle, case):
         acc = op.accumulators(xd, fd, *MM)
         torch.cuda.synchronize()
         prof = ops.profile_read()
-        assert "lutgemm_px" in prof and "lutgemm_expand" not in prof, prof
+        assert "lutgemm_px" in prof and "lutgemm_mx" not in prof and "lutgemm_expand" not in prof, prof
         # rows beyond 512 MiB get a launch of their own, the others ride in a pre-pass launch
         assert ("px_expand_rows" in prof) == (fs[3] * fs[0] * fs[1] * xs[3] * 512 > 512 << 20), prof   # 512 bytes per filter element
         ops.set_preexpand(-1)
@@ -92,9 +102,9 @@ def test_barrier_free_kernel_whole_output_and_oracle(pkg, oracle, case):
         y0 = op(xd, fd, *MM)
         acc0 = op.accumulators(xd, fd, *MM)
         torch.cuda.synchronize()
-        assert "lutgemm_px" not in ops.profile_read()
+        assert not {"lutgemm_px", "lutgemm_mx"} & set(ops.profile_read())
     finally:
-        ops.set_preexpand(0)
+        ops.set_preexpand(1)
         ops.profile_enable(False)
     bad = acc != acc0
     assert not bool(bad.any()), "%d of %d sums differ from the other kernel's, first at %s" % (
@@ -118,7 +128,7 @@ def test_barrier_free_kernel_whole_output_and_oracle(pkg, oracle, case):
 
 
 def _random_layers(pkg, count, seed):
-    """Seeded random layers that the planner gives to the kernel (plan code 2)."""
+    """Seeded random layers that get the kernel (plan code 2)."""
     ops = pkg.ops
     rng = np.random.default_rng(seed)
     out = []
@@ -149,12 +159,17 @@ def test_random_full_size_layers_equal_the_expanding_kernel(pkg):
         table = pkg.synth.table_random(i)
         xd, fd = bench.device_tensors(pkg, xs, fs, "uniform", seed=i)
         op = pkg.ApproxConv2DWithMinMaxVars([1, stride, stride, 1], 8, table, padding)
+        ops.profile_enable(True)
+        ops.profile_reset()
         try:
             acc, y = op.accumulators(xd, fd, *MM), op(xd, fd, *MM)
+            torch.cuda.synchronize()
+            assert {k for k in ops.profile_read() if k.startswith("lutgemm")} == {"lutgemm_px"}, _id(case)
             ops.set_preexpand(-1)
             acc0, y0 = op.accumulators(xd, fd, *MM), op(xd, fd, *MM)
         finally:
-            ops.set_preexpand(0)
+            ops.set_preexpand(1)
+            ops.profile_enable(False)
         assert torch.equal(acc, acc0), _id(case)
         assert torch.equal(y.view(torch.int32), y0.view(torch.int32)), _id(case)
     assert len(heights) >= 24, heights

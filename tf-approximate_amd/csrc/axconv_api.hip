@@ -10,6 +10,7 @@
 #include <atomic>
 #include <cstdlib>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <tuple>
@@ -177,40 +178,49 @@ int wait_error_check(uint32_t **dev_word)
 }
 
 // ---- profiling: events around each kernel, on the launch stream ----
+struct ProfEvents {   // around one launch
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    ~ProfEvents()
+    {
+        if (e0)
+            (void)hipEventDestroy(e0);
+        if (e1)
+            (void)hipEventDestroy(e1);
+    }
+};
+
 struct ProfEntry {
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
+    std::vector<std::shared_ptr<ProfEvents>> pending;
     double total_ms = 0.0;
     int64_t launches = 0;
 };
 std::mutex g_prof_mutex;
 std::atomic<bool> g_prof_enabled{false};
-std::map<std::string, ProfEntry> g_prof;
+std::map<std::string, ProfEntry> &g_prof = *new std::map<std::string, ProfEntry>;   // (no HIP calls as the process ends)
 
-struct ProfScope {
-    const char *name;
+struct ProfScope {   // also: a second name that the time is entered under
+    const char *name, *also;
     hipStream_t stream;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    bool on;
-    ProfScope(const char *n, hipStream_t s) : name(n), stream(s), on(g_prof_enabled.load())
+    std::shared_ptr<ProfEvents> ev;
+    ProfScope(const char *n, hipStream_t s, const char *n2 = nullptr) : name(n), also(n2), stream(s)
     {
-        if (!on)
+        if (!g_prof_enabled.load())
             return;
-        if (hipEventCreate(&e0) != hipSuccess) {
-            on = false;
-        } else if (hipEventCreate(&e1) != hipSuccess) {
-            (void)hipEventDestroy(e0);
-            on = false;
-        } else {
-            (void)hipEventRecord(e0, stream);
-        }
+        ev = std::make_shared<ProfEvents>();
+        if (hipEventCreate(&ev->e0) != hipSuccess || hipEventCreate(&ev->e1) != hipSuccess)
+            ev.reset();
+        else
+            (void)hipEventRecord(ev->e0, stream);
     }
     ~ProfScope()
     {
-        if (!on)
+        if (!ev)
             return;
-        (void)hipEventRecord(e1, stream);
+        (void)hipEventRecord(ev->e1, stream);
         std::lock_guard<std::mutex> lock(g_prof_mutex);
-        g_prof[name].pending.emplace_back(e0, e1);
+        g_prof[name].pending.push_back(ev);
+        if (also)
+            g_prof[also].pending.push_back(ev);
     }
 };
 
@@ -218,12 +228,10 @@ void prof_drain_locked(ProfEntry &pe)
 {
     for (auto &ev : pe.pending) {
         float ms = 0.0f;
-        if (hipEventSynchronize(ev.second) == hipSuccess && hipEventElapsedTime(&ms, ev.first, ev.second) == hipSuccess) {
+        if (hipEventSynchronize(ev->e1) == hipSuccess && hipEventElapsedTime(&ms, ev->e0, ev->e1) == hipSuccess) {
             pe.total_ms += ms;
             pe.launches += 1;
         }
-        (void)hipEventDestroy(ev.first);
-        (void)hipEventDestroy(ev.second);
     }
     pe.pending.clear();
 }
@@ -1133,7 +1141,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             m.out_i = part;
         }
         {
-            ProfScope ps("lutgemm_px", stream);
+            ProfScope ps("lutgemm_px", stream, "lutgemm_mx");
             AXC_HIP(launch_dense_mx(m, stream));
         }
         if (mx->k_splits > 1) {
