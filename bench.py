@@ -13,11 +13,16 @@ fused epilogue) on seeded synthetic tensors that are already resident in HBM.  P
                the LDS read port (a lookup moves its 2-byte entry through it) and the issue rate of the kernel's
                accumulate instructions, each the larger of its nominal value (CUs x 256 B x clock, CUs x 64 lanes x
                clock) and what a probe kernel measures in this run.  `frac` is the larger of the two fractions,
-               `peak` the ceiling it belongs to; `frac_nominal_gather` is the same rate against the nominal
-               one-entry-per-bank-slot gather ceiling 256 CU x 32 lookups/clk x 2.4 GHz = 19.66 T/s.
+               `peak` the ceiling it belongs to; the *_measured fractions are against the probes alone
+               (frac_lookup_mix_measured: against one of the vector-ALU kernels' whole instruction mix per lookup);
+               `frac_nominal_gather` is the same rate against the nominal one-entry-per-bank-slot gather ceiling
+               256 CU x 32 lookups/clk x 2.4 GHz = 19.66 T/s, which a kernel reading eight entries per access can pass.
   layers       the same measurement for the layer shapes of the other benchmark configurations (fewer steps each),
-               every one with an oracle check of sampled output pixels; depthwise layers against HBM bandwidth
-  networks     images/s of the two synthetic ResNet-shaped networks, every convolution through the op
+               every one with an oracle check of sampled output pixels; depthwise layers against HBM bandwidth.  The
+               line holds [ms per call, kernel, its ms, fraction of its ceiling, sums bit-exact] of each; the whole
+               records go to stderr, one JSON line each
+  networks     ms per pass of the synthetic ResNet-shaped networks, every convolution through the op, eager and as
+               a replayed HIP graph (whole records on stderr)
   cpu_baseline the CPU oracle's reference-faithful single-thread path timed on this host on a bounded sample
 """
 import argparse
@@ -153,7 +158,9 @@ class Ceilings:
         valu_ceiling = max(self.valu_nominal, self.valu_lane_ops)
         port_ceiling = max(self.port_nominal, self.port_bytes)
         f_port = 2.0 * lookups_per_s / port_ceiling
-        ops_per_lookup = 0.0 if kernel == "lutgemm_mx" else self.ops_per_lookup   # the matrix cores make those sums
+        # with the sums on the matrix cores the vector ALUs make one address per eight entries
+        on_matrix_cores = kernel == "lutgemm_mx"
+        ops_per_lookup = 0.125 if on_matrix_cores else self.ops_per_lookup
         f_valu = lookups_per_s * ops_per_lookup / valu_ceiling
         bound = "lds" if f_port >= f_valu else "valu"
         peak = port_ceiling / 2.0 if bound == "lds" else valu_ceiling / ops_per_lookup
@@ -161,7 +168,8 @@ class Ceilings:
                 "frac_valu": round(f_valu, 4),
                 "frac_lds_port_measured": round(2.0 * lookups_per_s / self.port_bytes, 4),
                 "frac_valu_measured": round(lookups_per_s * ops_per_lookup / self.valu_lane_ops, 4),
-                "frac_lookup_mix_measured": round(lookups_per_s / self.mix, 4),
+                # (the probe's mix is that of the kernels whose sums the vector ALUs make)
+                "frac_lookup_mix_measured": None if on_matrix_cores else round(lookups_per_s / self.mix, 4),
                 "frac_nominal_gather": round(lookups_per_s / NOMINAL_LDS_LOOKUPS_PER_S, 4)}, peak
 
     def report(self):
@@ -300,15 +308,12 @@ def sampled_oracle_check(oracle, table, op, xd, fd, strides, depthwise, y, n_sam
     return bit_exact, linf
 
 
-def dense_kernel_name(ops, kernels_ms, xs, fs, strides):
-    """The LUT-GEMM kernel a dense layer ran: out of pre-expanded rows with the sums on the matrix cores or on the vector
-    ALUs, or expanding inside every tile.  The library times the first two under one name."""
-    if "lutgemm_px" not in kernels_ms:
-        return "lutgemm_expand"
-    if ops.conv2d_matrix_plan(tuple(xs), tuple(fs), (1, strides[0], strides[1], 1)) is None:
-        return "lutgemm_px"
-    kernels_ms["lutgemm_mx"] = kernels_ms.pop("lutgemm_px")
-    return "lutgemm_mx"
+def dense_kernel_name(kernels_ms):
+    """The LUT-GEMM kernel a dense layer ran, by the library's own timers: out of pre-expanded rows with the sums on the
+    matrix cores or on the vector ALUs, or expanding inside every tile."""
+    if "lutgemm_mx" in kernels_ms:
+        kernels_ms.pop("lutgemm_px")     # the same launch: the name of all that run out of pre-expanded rows
+    return next(k for k in ("lutgemm_mx", "lutgemm_px", "lutgemm_expand") if k in kernels_ms)
 
 
 def cpu_reference_sample(oracle, table, xd, fd, strides, depthwise, seconds=CPU_SAMPLE_S):
@@ -352,7 +357,7 @@ def measure_layer(pkg, ops, oracle, ceil, spec, steps=None, preroll_s=0.08):
     N, OH, OW, Cout = y.shape
     taps_c = fs[0] * fs[1] * (1 if depthwise else fs[2])
     lookups = N * OH * OW * Cout * taps_c
-    main = "depthwise_lut" if depthwise else dense_kernel_name(ops, kms, xs, fs, strides)
+    main = "depthwise_lut" if depthwise else dense_kernel_name(kms)
     kernel_ms = kms[main]
     rec = {"config": config, "layer": name, "input": list(xs), "filter": list(fs), "strides": list(strides),
            "codes": codes, "table": tkind, "M": N * OH * OW, "K": taps_c, "N": Cout, "lookups": lookups,
@@ -556,7 +561,7 @@ def main():
     lookups = n * oh * ow * co * taps_c
     gmacs = lookups / (ms_per_step * 1e-3) / 1e9
 
-    main_kernel = "depthwise_lut" if depthwise else dense_kernel_name(ops, kms, xs, fs, strides)
+    main_kernel = "depthwise_lut" if depthwise else dense_kernel_name(kms)
     main_ms = kms[main_kernel]
     achieved = lookups / (main_ms * 1e-3)
     ceil = Ceilings(ops)
@@ -600,15 +605,6 @@ def main():
             "kernel_ms": round(main_ms, 4),
             "lookups_per_launch": lookups,
             "ceilings": ceil.report(),
-            "note": "frac = the larger of frac_lds_port (2 bytes per lookup against the LDS read port) and frac_valu "
-                    "(accumulate instructions per lookup against the vector ALUs' issue rate), each against the larger "
-                    "of its nominal ceiling (CUs x 256 B x clock; CUs x 64 lanes x clock) and the rate a probe kernel "
-                    "measured in this run; the *_measured figures are against the probes alone; "
-                    "frac_lookup_mix_measured is against a probe made of the kernel's whole per-lookup instruction mix "
-                    "(address, 16-byte LDS read, accumulate) and nothing else, which neither of the two ceilings "
-                    "contains; frac_nominal_gather "
-                    "is against 256 CU x 32 lookups/clk x 2.4 GHz, a ceiling for one-entry gathers that a kernel "
-                    "reading 8 entries per access can pass",
             "hbm_algorithmic_bytes": hbm_bytes,
             "hbm_gbps_whole_op": round(hbm_bytes / (ms_per_step * 1e-3) / 1e9, 1),
             "hbm_frac_whole_op": round(hbm_bytes / (ms_per_step * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
@@ -673,14 +669,25 @@ def main():
     torch.cuda.empty_cache()
     if not args.no_layers:
         t_l = time.perf_counter()
-        result["layers"] = [measure_layer(pkg, ops, oracle, ceil, spec) for spec in LAYERS]
+        result["layers"] = {}
+        for spec in LAYERS:
+            r = measure_layer(pkg, ops, oracle, ceil, spec)
+            print(json.dumps(r), file=sys.stderr, flush=True)
+            result["layers"]["%s/%s/%s" % (r["config"].split("_")[0], r["layer"], r["table"])] = [
+                r["gpu_ms"], r["kernel"], r["kernel_ms"], r["frac"], r.get("acc_bit_exact")]
         result["layers_seconds"] = round(time.perf_counter() - t_l, 1)
     if not args.no_networks:
         t_n = time.perf_counter()
-        result["networks"] = [measure_network(pkg, "cifar_resnet_b128", 40, 10, graph=True),
-                              measure_network(pkg, "resnet50_b64", 12, 3, graph=True),
-                              measure_network(pkg, "cifar_resnet_b128", 40, 10, fused_layers=True),
-                              measure_network(pkg, "resnet50_b64", 12, 3, fused_layers=True)]
+        result["networks"] = {}
+        for name, n_steps, n_warmup, fused in (("cifar_resnet_b128", 40, 10, False), ("resnet50_b64", 12, 3, False),
+                                               ("cifar_resnet_b128", 40, 10, True), ("resnet50_b64", 12, 3, True)):
+            r = measure_network(pkg, name, n_steps, n_warmup, fused_layers=fused, graph=not fused)
+            print(json.dumps(r), file=sys.stderr, flush=True)
+            g = r.get("hip_graph", {})
+            result["networks"][name + ("_fused" if fused else "")] = dict(
+                {"ms_per_pass": r["ms_per_pass"], "images_per_s": r["images_per_s"]},
+                **({"graph_ms": g.get("ms_per_pass"), "graph_bitwise": g.get("replays_equal_eager_bitwise"),
+                    "graph_error": g.get("error")} if g else {}))
         result["networks_seconds"] = round(time.perf_counter() - t_n, 1)
     print(json.dumps(result))
 
