@@ -199,6 +199,21 @@ def test_strided_pixel_groups_stay_in_the_workspace(ops):
     assert seen > 10
 
 
+def test_matrix_core_kernel_where_it_was_measured_faster(ops):
+    """Layers with many weights for few pixels, timed both ways (whole op, us: on the matrix cores / expanding inside the
+    tiles), far enough from the line to tell: the rows cost pre-pass time, but not as much as turns all of them away."""
+    for xs, fs, stride, faster in [
+            ((28, 17, 17, 160), (3, 3, 160, 242), 1, True),       # 150 / 231
+            ((18, 15, 15, 832), (1, 1, 832, 131), 1, True),       # 60 / 93
+            ((15, 17, 17, 288), (1, 1, 288, 1495), 1, True),      # 128 / 170
+            ((64, 14, 14, 256), (3, 3, 256, 256), 1, True),       # 331 / 350
+            ((45, 13, 13, 64), (5, 5, 64, 776), 1, False),        # 648 / 581
+            ((22, 54, 13, 64), (1, 1, 64, 1712), 2, False),       # 57 / 49
+            ((64, 7, 7, 512), (3, 3, 512, 512), 1, False)]:       # 825 / 369
+        plan = ops.conv2d_matrix_plan(xs, fs, (1, stride, stride, 1))
+        assert (plan is not None) == faster, (xs, fs, plan)
+
+
 def test_workspace_sizes(ops, lib):
     desc = ops.make_desc((64, 56, 56, 64), (3, 3, 64, 64), (1, 1, 1, 1), "SAME")
     rc, n = _ws(lib, desc)
