@@ -147,7 +147,9 @@ int axc_conv2d_tile_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
 /* Whether the layer runs the kernel whose sums the matrix cores make instead (given a workspace of the size
  * axc_conv2d_workspace_bytes reports, and neither axc_set_preexpand nor axc_set_tile_columns pinning another), and how
  * that cuts it: plan = { 1 or 0 (then the rest is 0 too), units of 64 pixels per wavefront (the kernel's variant), units
- * per tile, row tiles, column tiles (8 columns), K splits, workgroups, fills of 16 filter elements per K split }. */
+ * per tile, row tiles, column tiles (8 columns), K splits, workgroups, fills of 16 filter elements per K split }.
+ * It runs out of rows of 512 bytes per filter element in the workspace, at most 2 GiB, which the workspace query counts; a
+ * launch whose workspace lacks room for them runs one of the other kernels, with the same results. */
 int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
 /* Pins the tile width the planner uses (16, 32 or 64 columns; 0 = its own choice, the default), process-wide, for
  * tests and timing of the wider-tile kernel variants.  The environment variable AXC_TILE_COLUMNS gives the initial
@@ -163,8 +165,8 @@ int axc_set_tile_columns(int columns);
  * plan of the kernel that expands inside its tiles when the workspace holds what that plan needs.  No counterpart
  * in the reference. */
 int axc_set_preexpand(int mode);
-/* The wavefronts of the kernel that plan code 2 stands for wait for each other by polling counters, every wait a bounded
- * number of polls (the default, 2^20 of ~150 cycles each, is far beyond any legitimate wait).  A wait that runs out ends
+/* The wavefronts of the kernels that plan code 2 and axc_conv2d_matrix_plan stand for wait for each other by polling counters,
+ * every wait a bounded number of polls (the default, 2^20 of ~150 cycles each, is far beyond any legitimate wait).  A wait that runs out ends
  * the launch early - every wavefront leaves the kernel, nothing hangs - and the NEXT launch call on that GPU returns
  * AXC_RUNTIME_ERROR once instead of launching: the earlier launch's output is incomplete.  This sets the number of
  * polls, process-wide; 0 makes every wait that is not satisfied at once give up (tests of the report).  No counterpart
@@ -246,7 +248,8 @@ int axc_conv2d_codes_acc_i32(const axc_table *table, const axc_conv2d_desc *desc
 
 /* Per-kernel timing with HIP events recorded on the launch stream.  While enabled, every kernel the
  * launch calls enqueue is bracketed by two events; axc_profile_read synchronizes them and returns the
- * accumulated milliseconds and launch count per kernel name since the last reset. */
+ * accumulated milliseconds and launch count per kernel name since the last reset.  A launch out of pre-expanded rows is
+ * entered as lutgemm_px, and as lutgemm_mx too where the matrix cores make its sums. */
 int axc_profile_enable(int enable);
 int axc_profile_reset(void);
 int axc_profile_read(int index, char *name, size_t name_bytes, double *total_ms, int64_t *launches);

@@ -1,4 +1,4 @@
-"""Independent numpy/torch statements of the op, used to pin the oracle (and, on the GPU box, to
+"""Independent numpy/torch statements of the op, used to pin the oracle (and, on the GPU, to
 cross-check the HIP path).  Written from the op's definition, not from the oracle's code:
 gathers with index arrays and library convolutions instead of the reference's loop nests."""
 import numpy as np
