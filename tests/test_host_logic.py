@@ -209,6 +209,7 @@ def test_matrix_core_kernel_where_it_was_measured_faster(ops):
             ((64, 14, 14, 256), (3, 3, 256, 256), 1, True),       # 331 / 350
             ((45, 13, 13, 64), (5, 5, 64, 776), 1, False),        # 648 / 581
             ((22, 54, 13, 64), (1, 1, 64, 1712), 2, False),       # 57 / 49
+            ((4, 14, 14, 797), (3, 3, 797, 38), 1, False),        # 1273 / 1019: patch sums pixel by pixel
             ((64, 7, 7, 512), (3, 3, 512, 512), 1, False)]:       # 825 / 369
         plan = ops.conv2d_matrix_plan(xs, fs, (1, stride, stride, 1))
         assert (plan is not None) == faster, (xs, fs, plan)

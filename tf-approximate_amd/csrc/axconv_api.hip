@@ -754,10 +754,10 @@ struct PreparedDense {
 // that it is the faster one.  ResNet-50's and the CIFAR network's layers, forced both ways (whole op, us): 3x3 64->64 @56x56
 // 289.8 -> 194.3, 1x1 64->256 @56x56 173.8 -> 153.9, 3x3 128->128 @28x28 309.1 -> 202.2, 3x3 16->16 @32x32x128 42.4 -> 32.4.
 // Where the models lie: 800 random layers whose predictions differ by less than a factor of two, timed both ways (whole op).
-// 337 run this kernel, 1.22 times as fast on average; eleven of those are more than 2 % slower for it (worst: 3x3/2 128->926
-// @31x31x107 1948 us against 1382, four loads a unit under 547 MB of rows; 3x3 797->38 @14x14x4 1273 against 1019; 3x3
-// 122->16 @214x53x5 416 against 344, loads 122 bytes apart; 1x1 32->240 @129x129x17 194 against 169, rows of no whole
-// groups), and 152 of the others would be faster by it, 12 % on average: both predictions miss by a tenth or two.
+// 334 run this kernel, 1.22 times as fast on average; ten of those are more than 2 % slower for it (worst: 3x3/2 128->926
+// @31x31x107 1948 us against 1382, four loads a unit under 547 MB of rows; 3x3 122->16 @214x53x5 416 against 344, loads
+// 122 bytes apart; 1x1 32->240 @129x129x17 194 against 169, rows of no whole groups), and 153 of the others would be faster by
+// it, 12 % on average: both predictions miss by a tenth or two.
 void prepare_mx(PreparedDense *pd)
 {
     const ConvGeom &g = pd->g;
@@ -783,10 +783,12 @@ void prepare_mx(PreparedDense *pd)
     // -> 330.7, 1x1 1024->512 @14x14x64 320.8 -> 280.9, 1x1 256->128 on one 56x56 image 35.7 -> 31.7.
     // Rows beyond some 20 MB for few pixels take 0.19 to 0.23 us a MB of pre-pass where the plan says 0.143 (pre-pass without
     // and with them, us: 5x5 448->48 @28x28x5, 275 MB, 65 / 129; 3x3 864->80 @14x14x41, 320 MB, 113 / 178; 5x5 64->776
-    // @13x13x45, 636 MB, 17 / 138).  Of the 800 layers above the term, with 0.07 us a MB, turns away nineteen, four of them
-    // slower (by up to 11 %); with 0.2, fitted to one layer, it turned away 25 more, 14 % faster on average.
+    // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Of the 800 layers above, 0.2 for all of them, fitted to one layer, turned away 22
+    // that are 16 % faster on average.  Channel counts that are no multiple of four keep the 0.2: their patch sums, which read
+    // memory pixel by pixel, slow down behind so many rows (3x3 797->38 @14x14x4, 147 MB: pre-pass 892 -> 1150 us, the op
+    // 1019 -> 1273).
     const double rows_bytes = (double)plan.n_col_tiles * plan.fills * 65536.0;
-    const double slow_rows = std::max(0.0, rows_bytes - 22e6) * 0.07e-12 * device_clock_hz();
+    const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) ? 0.2e-12 : 0.07e-12) * device_clock_hz();
     if (pd->plan.px ? plan.cost > pd->plan.cost : plan.cost + slow_rows > pd->plan.cost * 0.98)
         return;
     pd->mx = true;
