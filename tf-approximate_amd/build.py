@@ -2,12 +2,15 @@
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libaxconv_hip.so")
-SOURCES = ["axconv_api.hip", "lutgemm_kernel.hip", "lutgemm_px_kernel.hip", "lutgemm_mx_kernel.hip", "prepass_kernels.hip", "depthwise_kernel.hip"]
+SOURCES = ["axconv_api.hip", "lutgemm_kernel.hip", "lutgemm_px_kernel.hip", "lutgemm_mx_kernel.hip",
+           "lutgemm_mx_expand_kernel.hip", "prepass_kernels.hip", "depthwise_kernel.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -27,9 +30,7 @@ def generate():
             f.write(text)
 
 
-def build(verbose=False, extra=()):
-    generate()
-    cmd = ["hipcc"] + FLAGS + list(extra) + [os.path.join(CSRC, s) for s in SOURCES] + ["-o", LIB]
+def run(cmd, verbose):
     if verbose:
         print(" ".join(cmd))
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -39,6 +40,21 @@ def build(verbose=False, extra=()):
         raise RuntimeError("hipcc failed:\n" + out)
     if verbose and out.strip():
         print(out)
+
+
+def build(verbose=False, extra=()):
+    generate()
+    with tempfile.TemporaryDirectory() as tmp:
+        objects = [os.path.join(tmp, s + ".o") for s in SOURCES]
+
+        def compile_one(i):
+            return run(["hipcc"] + [f for f in FLAGS if f != "-shared"] + list(extra) +
+                       ["-c", os.path.join(CSRC, SOURCES[i]), "-o", objects[i]], verbose)
+        # largest first; hipcc itself uses one core
+        order = sorted(range(len(SOURCES)), key=lambda i: "mx" not in SOURCES[i])
+        with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
+            list(pool.map(compile_one, order))
+        run(["hipcc"] + FLAGS + objects + ["-o", LIB], verbose)
     build_harness(verbose)
     return LIB
 

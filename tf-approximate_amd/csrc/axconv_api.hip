@@ -20,6 +20,7 @@ using namespace axc;
 
 struct axc_table {
     uint16_t *dev_tableT; // [257 filter code][256 input code]; row 256 is zero
+    uint16_t *dev_tableF; // behind it in the same allocation: the same with the top bit of every byte flipped
     int device;
 };
 
@@ -441,6 +442,9 @@ std::atomic<int> g_px_mode{[] {
     const int v = env ? std::atoi(env) : 0;
     return (v == 1 || v == -1) ? v : 0;
 }()};
+// Rows of lutgemm_mx_kernel: 0 = the planner decides, 1 = only pre-expanded ones (layers that they do not suit run the other
+// kernels), 2 = its own wherever it can make them.  Set by axc_set_matrix_rows.
+std::atomic<int> g_mx_rows{0};
 constexpr size_t kPxMaxBytes = (size_t)2 << 30;     // most memory a layer's pre-expanded rows may take
 // Rows up to this size stay in the memory-side cache between the launch that writes them and the one that reads
 // them; larger sets are read from memory, and the cost model is less sure of them: they must promise a gain.
@@ -593,50 +597,65 @@ MxDiv mx_div(uint32_t d)
 }
 
 // Tiles of 64-pixel units x 8 columns: how many row tiles, which kernel variant, how many K splits.  Microseconds,
-// measured by running 3x3 layers of 9 and of 36 fills in every variant (U units per wavefront):
-//   a fill    0.30 + 0.138 U, at least 1.05 + 0.03 U (64 KiB of rows into LDS with every CU doing so: U = 2 takes 1.11, 8 1.45,
-//             13 2.1, 25 3.75); with four loads per unit instead of one (pixels that are no neighbouring dwords)
-//             0.35 + 0.243 U, at least 1.3
-//   a tile    1.3 + 0.70 U up to U = 6, then 0.42 a unit (18.8 at U = 25 while batches of six units waited for each other's
-//             stores, 13.5 without): geometry, the sums' start values, the outputs, stored in 32-byte pieces
+// measured by running 3x3 layers of 18 and of 72 fills at stride 1 and 2 in every variant (U units per wavefront; stride 1
+// loads a unit's activations at once, stride 2 - pixels that are no neighbouring dwords - by four loads):
+//   a fill    of pre-expanded rows 1.10 (U = 2), 1.32 (4), 1.51 (8), 2.10 (13), 2.53 (16), 3.05 (20), 3.75 (25); four loads
+//             1.30, 1.76, 2.42, 3.52, 4.25, 5.19, 6.39; of rows the kernel makes itself 1.43, 1.59, 2.03, 2.55, 2.95, 3.46;
+//             four loads 1.65, 1.88, 2.65, 3.85, 4.60, 5.70: the stores of the rows take the LDS 0.4 us of every fill
+//   a tile    1.3 + 0.70 U up to U = 6, then 0.42 a unit: geometry, the sums' start values, the outputs, stored in 32-byte
+//             pieces; rows of its own once a launch 1.0 + 0.33 U more (a first fill that waits for codes, then for entries)
 // K splits and the rows cost what they cost the other kernels (compute_plan).
-MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, bool one_load, int cus, double clock_hz)
+MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, bool one_load, bool expand, int cus,
+                       double clock_hz)
 {
     MxPlan best{};
     double best_cost = 1e300;
     const int n_col = (co + kMxCols - 1) / kMxCols;
     const int fills = (int)((quads + kMxFillQuads - 1) / kMxFillQuads);
-    const int max_units = kMxUnits[sizeof(kMxUnits) / sizeof(kMxUnits[0]) - 1];
+    const std::vector<int> heights = expand ? std::vector<int>(std::begin(kMxExpandUnits), std::end(kMxExpandUnits))
+                                            : std::vector<int>(std::begin(kMxUnits), std::end(kMxUnits));
+    const int max_units = heights.back();
     const int64_t total_units = (groups + 15) / 16;
     const int64_t cap = (int64_t)kMxWaves * max_units;
     const int64_t min_tiles = (total_units + cap - 1) / cap;
-    const double rows_bytes = (double)n_col * fills * 65536.0;
-    const double rows_us = rows_bytes <= 400e6 ? 1.5 + rows_bytes / 7e6 : 6.5 + rows_bytes / 4.5e6;
-    for (int ks : {1, 2, 3, 4, 6, 8, 12, 16}) {
+    const double rows_bytes = expand ? 0.0 : (double)n_col * fills * 65536.0;
+    const double rows_us = expand ? 0.0 : rows_bytes <= 400e6 ? 1.5 + rows_bytes / 7e6 : 6.5 + rows_bytes / 4.5e6;
+    for (int ks : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48}) {
         const int fps = (fills + ks - 1) / ks;
         if (ks > 1 && (fps < 4 || (int64_t)(ks - 1) * fps >= fills))
+            continue;
+        // expanding, a tile has two fills or more: filter codes are loaded two ahead
+        if (expand ? fills - (ks - 1) * fps < 2 : ks > 16)
             continue;
         std::vector<int64_t> cands{min_tiles};
         for (int64_t rounds = 1; rounds <= 64; ++rounds)
             for (int64_t n_row : {rounds * cus / ((int64_t)n_col * ks), rounds * cus / ((int64_t)n_col * ks) + 1})
                 if (n_row > min_tiles && n_row <= total_units)
                     cands.push_back(n_row);
+        if (expand)   // layers too small for whole rounds: whole tiles of every height
+            for (int u : heights)
+                cands.push_back((total_units + (int64_t)kMxWaves * u - 1) / ((int64_t)kMxWaves * u));
         for (int64_t n_row : cands) {
             const int64_t upt = (total_units + n_row - 1) / n_row;
             int units = 0;
-            for (int u : kMxUnits)
+            for (int u : heights)
                 if (!units && (int64_t)u * kMxWaves >= upt)
                     units = u;
             if (!units)
                 continue;
             const int64_t rows = (total_units + upt - 1) / upt;
             const int64_t tiles = rows * n_col * ks, rounds = (tiles + cus - 1) / cus;
-            const double fill = one_load ? std::max(1.05 + 0.03 * units, 0.30 + 0.138 * units)
-                                         : std::max(1.3, 0.35 + 0.243 * units);
+            const double u = units;
+            const double fill = expand ? (one_load ? std::max(1.28 + 0.09 * u, 0.87 + 0.131 * u)
+                                                   : std::max(1.38 + 0.135 * u, 0.83 + 0.236 * u))
+                                       : (one_load ? std::max(1.05 + 0.03 * u, 0.30 + 0.138 * u)
+                                                   : std::max(1.3, 0.35 + 0.243 * u));
             const double tile = 1.3 + 0.70 * std::min(units, 6) + 0.42 * std::max(units - 6, 0);
             double us = std::max((double)rounds * (fps * fill + tile), rows_bytes / 3e6);
+            if (expand)
+                us += 1.0 + 0.33 * u;
             if (ks > 1)
-                us += 7.1 + (double)(ks + 1) * (double)outputs * 4.0 * 1.46e-7;
+                us += (expand ? 4.5 : 7.1) + (double)(ks + 1) * (double)outputs * 4.0 * 1.46e-7;
             const double cost = (us + rows_us) * 1e-6 * clock_hz;
             if (cost < best_cost) {
                 best_cost = cost;
@@ -648,6 +667,7 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, b
                 best.k_splits = ks;
                 best.fills_per_split = fps;
                 best.grid = (int)(tiles < cus ? tiles : cus);
+                best.expand = expand ? 1 : 0;
                 best.cost = (float)cost;
             }
         }
@@ -655,20 +675,20 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, b
     return best;
 }
 
-MxPlan make_mx_plan(const ConvGeom &g, bool one_load, int cus)
+MxPlan make_mx_plan(const ConvGeom &g, bool one_load, bool expand, int cus)
 {
-    typedef std::tuple<int64_t, int, int64_t, int64_t, bool, int> Key;
+    typedef std::tuple<int64_t, int, int64_t, int64_t, bool, bool, int> Key;
     static std::mutex mu;
     static std::map<Key, MxPlan> cache;
     const int64_t quads = (int64_t)g.KH * g.KW * g.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
-    const Key key{quads, g.Co, groups, g.M * g.Co, one_load, cus};
+    const Key key{quads, g.Co, groups, g.M * g.Co, one_load, expand, cus};
     {
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end())
             return it->second;
     }
-    const MxPlan plan = compute_mx_plan(quads, g.Co, groups, g.M * g.Co, one_load, cus, device_clock_hz());
+    const MxPlan plan = compute_mx_plan(quads, g.Co, groups, g.M * g.Co, one_load, expand, cus, device_clock_hz());
     std::lock_guard<std::mutex> lock(mu);
     if (cache.size() >= 4096)
         cache.clear();
@@ -716,7 +736,9 @@ DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, const M
     w.sub_off = off; off += align_up(sub_bytes);
     w.xq_off = off; off += align_up(xq_bytes_of(g, lay, flat_row_bytes));   // + the zero-point row(s)
     w.psum_off = off; off += align_up((size_t)g.M * 4); // patch sums: one float per output pixel
-    w.wq_off = off; off += mx ? 0 : align_up((size_t)plan.n_col_tiles * plan.fills * 64 * 2);
+    w.wq_off = off;
+    off += align_up(!mx ? (size_t)plan.n_col_tiles * plan.fills * 64 * 2
+                        : mx->expand ? (size_t)mx->n_col_tiles * mx->fills * kMxCodeBytes : 0);
     w.fsum_off = off; off += align_up((size_t)g.Co * 4);
     w.layer_off = off;  // layer entry point: partial (min, max) pairs of both tensors, then the LayerQuant
     off += align_up((size_t)4 * kMinMaxBlocks * sizeof(float)) + align_up(sizeof(LayerQuant));
@@ -726,7 +748,7 @@ DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, const M
         off += align_up((size_t)k_splits * (size_t)g.M * g.Co * 4);
     w.total_no_px = off;
     w.px_off = off;
-    w.px_bytes = mx ? (size_t)mx->n_col_tiles * (size_t)mx->fills * 65536
+    w.px_bytes = mx ? (mx->expand ? 0 : (size_t)mx->n_col_tiles * (size_t)mx->fills * 65536)
                     : plan.px ? (size_t)plan.n_col_tiles * (size_t)(plan.fills / 2) * 65536 : 0;
     off += align_up(w.px_bytes);
     w.total = off;
@@ -750,15 +772,14 @@ struct PreparedDense {
     bool empty;
 };
 
-// Decides whether the layer runs lutgemm_mx_kernel: where the two cost models, fitted to the launch times of each, say
-// that it is the faster one.  ResNet-50's and the CIFAR network's layers, forced both ways (whole op, us): 3x3 64->64 @56x56
-// 289.8 -> 194.3, 1x1 64->256 @56x56 173.8 -> 153.9, 3x3 128->128 @28x28 309.1 -> 202.2, 3x3 16->16 @32x32x128 42.4 -> 32.4.
-// Where the models lie: 800 random layers whose predictions differ by less than a factor of two, timed both ways (whole op).
-// 334 run this kernel, 1.22 times as fast on average; ten of those are more than 2 % slower for it (worst: 3x3/2 128->926
-// @31x31x107 1948 us against 1382, four loads a unit under 547 MB of rows; 3x3 122->16 @214x53x5 416 against 344, loads
-// 122 bytes apart; 1x1 32->240 @129x129x17 194 against 169, rows of no whole groups), and 153 of the others would be faster by
-// it, 12 % on average: both predictions miss by a tenth or two.
-void prepare_mx(PreparedDense *pd)
+// Decides whether the layer runs lutgemm_mx_kernel, and whether out of pre-expanded rows or of rows that it makes itself:
+// what the cost models, fitted to the launch times of each, say is fastest.  Whole op, us, pre-expanded / own rows / other
+// kernels: 3x3 64->64 @56x56x64 201 / 260 / 302, 1x1 128->512 @28x28x64 111 / 135 / 160, 1x1 256->1024 @14x14x64 147 / 148 /
+// 168, 3x3 256->256 @14x14x64 346 / 275 / 378, 3x3 512->512 @7x7x64 820 / 275 / 376, 1x1 512->2048 @7x7x64 284 / 138 / 189, the
+// same on one image 235 / 61 / 68.  Own rows want few pixels for many weights, where writing 512 bytes per weight and reading
+// them back outweighs making them anew in every tile.  Over the layers of ResNet-50 at batch 64, 9 and 1 and of 240 random
+// layers, each timed in the three forms, the choice is 1.2, 1.2, 0.4 and 2 % above the fastest of the three.
+void prepare_mx(PreparedDense *pd, bool allow_rows)
 {
     const ConvGeom &g = pd->g;
     const XqLayout lay = padded_layout(g, pd->flat_row_bytes > 0);
@@ -768,29 +789,49 @@ void prepare_mx(PreparedDense *pd)
     if (g.M >= ((int64_t)1 << 31) - 4096 || g.Co > 65536)   // pixel numbers and a tile's output offsets in 31 bits
         return;
     // Pixels of a group that do not exist are read too, up to three pitches behind the input by a scalar offset, which a
-    // descriptor's bounds check need not cover: that must still be the workspace (a fill of rows, 64 KiB, lies behind).
+    // descriptor's bounds check need not cover: that must still be the workspace (a fill of rows, 64 KiB, lies behind, and
+    // without those the layer entry point's 4 * kMinMaxBlocks floats).
     const int64_t pitch = (int64_t)g.sw * (pd->flat_row_bytes ? g.C : 4);
     if (3 * pitch > 65536)
         return;
     ConvGeom gq = pd->gk;
     gq.OW = g.OW;
-    const MxPlan plan = make_mx_plan(gq, pitch == 4, device_cus());
-    if (plan.units == 0 || (size_t)plan.n_col_tiles * (size_t)plan.fills * 65536 > kPxMaxBytes)
-        return;
-    // Against the kernel that expands inside its tiles, which writes no rows, it must promise 2 %: predicted to be equal,
-    // 1x1 128->512 on one 28x28 image took 42 us against 28 (33 MB of rows for 784 pixels), 5x5 19->224 @12x28x52 95.4 / 94.4.
-    // Predicted 4 to 32 % faster, measured (whole op, us): 3x3/2 20->75 @61x45x7 45.2 -> 37.1, 3x3 256->256 @14x14x64 349.6
-    // -> 330.7, 1x1 1024->512 @14x14x64 320.8 -> 280.9, 1x1 256->128 on one 56x56 image 35.7 -> 31.7.
+    const MxPlan own = make_mx_plan(gq, pitch == 4, true, device_cus()), rows = make_mx_plan(gq, pitch == 4, false, device_cus());
+    const double us = 1e-6 * device_clock_hz();
     // Rows beyond some 20 MB for few pixels take 0.19 to 0.23 us a MB of pre-pass where the plan says 0.143 (pre-pass without
     // and with them, us: 5x5 448->48 @28x28x5, 275 MB, 65 / 129; 3x3 864->80 @14x14x41, 320 MB, 113 / 178; 5x5 64->776
-    // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Of the 800 layers above, 0.2 for all of them, fitted to one layer, turned away 22
-    // that are 16 % faster on average.  Channel counts that are no multiple of four keep the 0.2: their patch sums, which read
-    // memory pixel by pixel, slow down behind so many rows (3x3 797->38 @14x14x4, 147 MB: pre-pass 892 -> 1150 us, the op
-    // 1019 -> 1273).
-    const double rows_bytes = (double)plan.n_col_tiles * plan.fills * 65536.0;
-    const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) ? 0.2e-12 : 0.07e-12) * device_clock_hz();
-    if (pd->plan.px ? plan.cost > pd->plan.cost : plan.cost + slow_rows > pd->plan.cost * 0.98)
+    // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Channel counts that are no multiple of four keep 0.2: their patch sums, which
+    // read memory pixel by pixel, slow down behind so many rows (3x3 797->38 @14x14x4, 147 MB: pre-pass 892 -> 1150 us).
+    const double rows_bytes = (double)rows.n_col_tiles * rows.fills * 65536.0;
+    const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) ? 0.2e-6 : 0.07e-6) * us;
+    const bool rows_ok = allow_rows && rows.units && rows_bytes <= (double)kPxMaxBytes;
+    const bool own_ok = own.units && 3 * pitch <= (int64_t)(4 * kMinMaxBlocks * sizeof(float)) &&
+                        (int64_t)own.n_col_tiles * own.fills * kMxCodeBytes < ((int64_t)1 << 31);
+    const int mode = g_mx_rows.load(std::memory_order_relaxed);
+    bool expand = own_ok;
+    if (mode == 1) {
+        if (!rows_ok || (pd->plan.px ? rows.cost > pd->plan.cost : rows.cost + slow_rows > pd->plan.cost * 0.98))
+            return;
+        expand = false;
+    } else if (mode == 0) {
+        // What the plan of pre-expanded rows leaves out: a K split is a little cheaper, and under short chains of patch sums
+        // the first 10 MB of rows delay the launch that carries them (pre-pass without and with rows, us: 1x1 64->256
+        // @56x56x9, 8 MB, 9.0 / 14.9; 1x1 128->512 @28x28x9, 34 MB, 8.5 / 23.4; but 3x3 64->64 @8x8x128, 19 MB, 12.0 / 14.3).
+        const double rows_cost = rows.cost + slow_rows + (1.5 + (g.K <= 256 ? 0.35e-6 : 0.0) * std::min(rows_bytes, 10e6) -
+                                                          (rows.k_splits > 1 ? 2.6 : 0.0)) * us;
+        expand = own_ok && (!rows_ok || own.cost < rows_cost);
+        // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), and lower
+        // where outputs are many for few fills: their stores leave at 2.2 TB/s at best, 0.65 where columns do not come in
+        // fours (1x1 8->1808 @78x78x4, 176 MB: 151 us where the model says 39; 1x1 16->342 @38x38x38, 75 MB, 131, 16; 3x3
+        // 11->170 @220x220x25, 823 MB, 1924, 961).
+        const double other = std::max(pd->plan.cost * (pd->plan.px ? 1.12 : 1.06) + 5.0 * us,
+                                      (double)g.M * g.Co * 4.0 / ((g.Co & 3) ? 0.65e6 : 2.2e6) * us);
+        if ((expand ? own.cost : rows_cost) > other)
+            return;
+    }
+    if (!expand && !rows_ok)
         return;
+    const MxPlan &plan = expand ? own : rows;
     pd->mx = true;
     pd->mxp = plan;
     pd->lay = lay;
@@ -800,9 +841,10 @@ void prepare_mx(PreparedDense *pd)
 // stride-1 op on the subsampled input.  Those pixels are gathered into the workspace first (element_bytes each:
 // floats, or bytes for the codes entry point), and every kernel then sees a dense, unpadded stride-1 layer with a
 // quarter (stride 2) of the pixels to quantize and sum.  Callers with a padding origin of their own (`pads`: rows and columns)
-// get the layer as given.  allow_mx = false: the layer as the other kernels run it.
+// get the layer as given.  mx_mode: which forms of lutgemm_mx_kernel may run the layer.
+enum { kMxNone, kMxOwnRows, kMxAny };
 int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
-                  int px_mode = kPxModeGlobal, bool allow_mx = true)
+                  int px_mode = kPxModeGlobal, int mx_mode = kMxAny)
 {
     const bool allow_subsample = pads == nullptr;
     const bool allow_flat = allow_subsample;   // both are for callers that leave the padding origin to the library
@@ -875,9 +917,9 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     }
     pd->plan = make_plan(pd->gk, device_cus(), px_mode);
     pd->lay = plain_layout(pd->g);
-    if (allow_mx && px_mode == kPxModeGlobal && g_px_mode.load(std::memory_order_relaxed) == 0 &&
+    if (mx_mode != kMxNone && px_mode == kPxModeGlobal && g_px_mode.load(std::memory_order_relaxed) == 0 &&
         g_forced_nt.load(std::memory_order_relaxed) == 0)
-        prepare_mx(pd);
+        prepare_mx(pd, mx_mode == kMxAny);
     pd->ws = dense_workspace(pd->g, pd->plan, pd->mx ? &pd->mxp : nullptr, pd->lay, sub_bytes, pd->flat_row_bytes);
     return AXC_OK;
 }
@@ -900,11 +942,12 @@ int prepare_dense_for(const axc_conv2d_desc *desc, size_t workspace_bytes, const
     int rc = prepare_dense(desc, pd, pads, element_bytes);
     if (rc != AXC_OK || pd->empty)
         return rc;
-    if (pd->mx && workspace_bytes < pd->ws.total) {
-        rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, false);
-        if (rc != AXC_OK)
-            return rc;
-    }
+    for (int mx_mode : {kMxOwnRows, kMxNone})
+        if (pd->mx && workspace_bytes < pd->ws.total) {
+            rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, mx_mode);
+            if (rc != AXC_OK)
+                return rc;
+        }
     if (!pd->mx && pd->plan.px && workspace_bytes < pd->ws.total) {
         PreparedDense alt;
         rc = prepare_dense(desc, &alt, pads, element_bytes, -1);
@@ -960,7 +1003,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         return AXC_OK;
     }
     // a workspace without room for the pre-expanded rows still serves: the layer then runs without them
-    const bool use_px = (pd.mx || pd.plan.px) && workspace_bytes >= pd.ws.total;
+    const bool use_px = (pd.mx ? !pd.mxp.expand : pd.plan.px != 0) && workspace_bytes >= pd.ws.total;
     const MxPlan *const mx = pd.mx ? &pd.mxp : nullptr;
     if (workspace_bytes < pd.ws.total_no_px || (!workspace && pd.ws.total_no_px))
         return fail(AXC_INVALID_ARGUMENT, "workspace too small (see axc_conv2d_workspace_bytes)");
@@ -1092,6 +1135,9 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         m.xq_bytes = (uint32_t)xq_bytes_of(g, pd.lay, pd.flat_row_bytes);
         m.rows = px_rows;
         m.rows_bytes = (uint32_t)pd.ws.px_bytes;
+        m.wq = wq;
+        m.wq_bytes = (uint32_t)((size_t)mx->n_col_tiles * mx->fills * kMxCodeBytes);
+        m.tableF = table->dev_tableF;
         m.psum = psum;
         m.fsum = fsum;
         m.bias = bias;
@@ -1149,8 +1195,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             m.out_i = part;
         }
         {
-            ProfScope ps("lutgemm_px", stream, "lutgemm_mx");
-            AXC_HIP(launch_dense_mx(m, stream));
+            ProfScope ps(mx->expand ? "lutgemm_expand" : "lutgemm_px", stream, "lutgemm_mx");
+            AXC_HIP(mx->expand ? launch_dense_mx_expand(m, stream) : launch_dense_mx(m, stream));
         }
         if (mx->k_splits > 1) {
             p.plan.k_splits = mx->k_splits;
@@ -1345,17 +1391,21 @@ int axc_table_create(const uint16_t *host_table, axc_table **out)
     if (!host_table || !out)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
     // transpose to weight-code major: tableT[b][a] = T[(a << 8) | b]
-    std::vector<uint16_t> t((size_t)kTableRows * 256, 0); // row 256 stays zero: the null weight's row
+    const size_t entries = (size_t)kTableRows * 256;
+    std::vector<uint16_t> t(2 * entries, 0); // row 256 stays zero: the null weight's row
     for (int a = 0; a < 256; ++a)
         for (int b = 0; b < 256; ++b)
             t[(size_t)b * 256 + a] = host_table[(size_t)a * 256 + b];
+    for (size_t i = 0; i < entries; ++i)
+        t[entries + i] = t[i] ^ 0x8080u;
     axc_table *tab = new axc_table;
     tab->dev_tableT = nullptr;
     hipError_t e = hipGetDevice(&tab->device);
     if (e == hipSuccess)
-        e = hipMalloc(reinterpret_cast<void **>(&tab->dev_tableT), kTableAllocBytes);
+        e = hipMalloc(reinterpret_cast<void **>(&tab->dev_tableT), 2 * (size_t)kTableAllocBytes);
     if (e == hipSuccess)
-        e = hipMemcpy(tab->dev_tableT, t.data(), kTableAllocBytes, hipMemcpyHostToDevice);
+        e = hipMemcpy(tab->dev_tableT, t.data(), 2 * (size_t)kTableAllocBytes, hipMemcpyHostToDevice);
+    tab->dev_tableF = tab->dev_tableT + entries;
     if (e != hipSuccess) {
         if (tab->dev_tableT)
             (void)hipFree(tab->dev_tableT);
@@ -1601,7 +1651,7 @@ int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8])
     if (rc != AXC_OK)
         return rc;
     const MxPlan &m = pd.mxp;
-    const int32_t v[8] = {pd.mx ? 1 : 0, m.units, m.units_per_tile, m.n_row_tiles, m.n_col_tiles, m.k_splits, m.grid,
+    const int32_t v[8] = {pd.mx ? 1 + m.expand : 0, m.units, m.units_per_tile, m.n_row_tiles, m.n_col_tiles, m.k_splits, m.grid,
                           m.k_splits > 1 ? m.fills_per_split : m.fills};
     for (int i = 0; i < 8; ++i)
         plan[i] = pd.mx ? v[i] : 0;
@@ -1627,6 +1677,14 @@ int axc_set_preexpand(int mode)
     if (mode < -1 || mode > 1)
         return fail(AXC_INVALID_ARGUMENT, "preexpand mode must be 0 (planner's choice), 1 (whenever possible) or -1 (never)");
     g_px_mode.store(mode, std::memory_order_relaxed);
+    return AXC_OK;
+}
+
+int axc_set_matrix_rows(int mode)
+{
+    if (mode < 0 || mode > 2)
+        return fail(AXC_INVALID_ARGUMENT, "matrix rows mode must be 0 (planner's choice), 1 (pre-expanded only) or 2 (the kernel's own wherever possible)");
+    g_mx_rows.store(mode, std::memory_order_relaxed);
     return AXC_OK;
 }
 
@@ -1693,11 +1751,12 @@ int axc_conv2d_minmax_static(const axc_table *table, const axc_conv2d_desc *desc
     int rc = prepare_dense(desc, &pd);
     if (rc != AXC_OK)
         return rc;
-    if (pd.mx && pd.ws.total > kStaticScratchBytes) {   // without the room it would run as the other kernels do
-        rc = prepare_dense(desc, &pd, nullptr, 4, kPxModeGlobal, false);
-        if (rc != AXC_OK)
-            return rc;
-    }
+    for (int mx_mode : {kMxOwnRows, kMxNone})   // without the room it would run as run_dense re-plans it
+        if (pd.mx && pd.ws.total > kStaticScratchBytes) {
+            rc = prepare_dense(desc, &pd, nullptr, 4, kPxModeGlobal, mx_mode);
+            if (rc != AXC_OK)
+                return rc;
+        }
     size_t needed = (pd.mx || pd.plan.px) ? pd.ws.total : pd.ws.total_no_px;
     if (!pd.mx && pd.plan.px && needed > kStaticScratchBytes) {
         // without room for pre-expanded rows the layer runs as run_dense re-plans it, or as planned minus the rows

@@ -130,6 +130,8 @@ constexpr int kMxWaves = kMxThreads / 64;
 constexpr int kMxCols = 8;                     // columns per tile
 constexpr int kMxFillQuads = 4;                // channel quads (of any taps) per fill
 constexpr int kMxUnits[] = {2, 3, 4, 6, 8, 10, 13, 16, 20, 25};   // 64-pixel units per wavefront: the kernel's variants
+constexpr int kMxExpandUnits[] = {2, 3, 4, 6, 8, 10, 12, 13, 14, 16, 18, 20};   // the same where it makes its rows itself
+constexpr int kMxCodeBytes = 256;              // packed filter codes of a fill: 16 filter elements x 8 columns x uint16
 
 struct MxPlan {
     int units;             // units per wavefront, one of kMxUnits
@@ -138,6 +140,7 @@ struct MxPlan {
     int fills;             // fills of kMxFillQuads quads over the whole K
     int k_splits, fills_per_split;
     int grid;
+    int expand;            // 1: the kernel makes its rows itself, out of packed filter codes and the table
     float cost;            // cycles the planner's model expects
 };
 
@@ -159,8 +162,11 @@ struct MxParams {
     MxPlan plan;
     const void *xq;
     uint32_t xq_bytes;
-    const uint16_t *rows;
+    const uint16_t *rows;  // pre-expanded ones
     uint32_t rows_bytes;
+    const uint16_t *wq;    // plan.expand: filter codes [column tile][fill][filter element 0..15][column 0..7], and the table
+    uint32_t wq_bytes;     // with the top bit of every byte flipped, filter-code major
+    const uint16_t *tableF;
     const float *psum, *fsum, *bias;
     const int32_t *pixel_term, *column_term;   // not null (tf1 op): added to the integer outputs, by the first K split
     float *out_f;
@@ -309,7 +315,8 @@ bool px_free_running(const DensePlan &plan, int taps);   // the plan runs lutgem
 hipError_t launch_mx_expand_rows(const float *filter, const uint8_t *filter_codes, const ConvGeom &g, const MxPlan &plan,
                                  const TensorQuant &tq, const LayerQuant *lq_dev, const uint16_t *tableT, uint16_t *rows,
                                  hipStream_t stream);
-hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream);
+hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream);          // out of pre-expanded rows
+hipError_t launch_dense_mx_expand(const MxParams &p, hipStream_t stream);   // plan.expand
 hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials, float *out_f, int32_t *out_i,
                                   hipStream_t stream);
 // tf1 AxConv2D: what the zero points add to the sums of products, per output pixel and per output column; and the pass

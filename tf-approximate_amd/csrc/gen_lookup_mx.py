@@ -39,6 +39,9 @@ UNITS = (2, 3, 4, 6, 8, 10, 13, 16, 20, 25)   # tile heights: units of 64 pixels
 VARIANTS = [(u, vec) for u in UNITS for vec in (True, False)]
 W = 8                                         # lookups in flight (a unit is a whole number of rings)
 LOADS = 16                                    # 1 KiB loads per wavefront and fill
+XUNITS = (2, 3, 4, 6, 8, 10, 12, 13, 14, 16, 18, 20)   # tile heights of the expanding form (25 leaves it no registers)
+XVARIANTS = [(u, vec) for u in XUNITS for vec in (True, False)]
+CODE_BYTES = 256                              # packed filter codes of a fill: 128 x uint16
 
 # registers the assembly uses by number
 V_A, V_IDX, V_SEL, V_CH0, V_CH1, V_L16 = 0, 4, 5, 9, 10, 11
@@ -71,10 +74,11 @@ class Stream:
         self.lines.append(text)
 
     def lds(self, text):
+        if len(self.lds_q) == 15:          # all that the counter holds (the expanding form's bursts of stores)
+            self.wait_lds(self.lds_q[0])
         self.ins(text)
         self.count += 1
         self.lds_q.append(self.count)
-        assert len(self.lds_q) <= 15
         return self.count
 
     def vm(self, text):
@@ -110,6 +114,19 @@ def layout(units):
     return d, slots, ring, win, end, vacc
 
 
+def expand_layout(units):
+    """Registers of the expanding form behind those of layout(): a fill's filter codes, the addresses of their table rows,
+    the entries on their way in (two blocks of eight quadruples), the turned chunks on their way out, and the lane's
+    offsets into a table row and into the LDS buffer."""
+    end, vacc = layout(units)[4:]
+    codes = end + (end & 1)
+    row, land = codes + 4, codes + 12
+    out = land + 64
+    toff, ldst = out + 8, out + 9
+    assert ldst < vacc, (units, ldst, vacc)
+    return codes, row, land, out, toff, ldst
+
+
 def acc_reg(units, u, j):
     if u < AGPR_UNITS:
         r = 16 * u + 4 * j
@@ -118,7 +135,7 @@ def acc_reg(units, u, j):
     return "v[%d:%d]" % (r, r + 3)
 
 
-def emit(units, vec):
+def emit(units, vec, expand=False):
     d, slots, ring, win, end, vacc = layout(units)
     n_look, n_pair = 16 * units, 8 * units
     st = Stream()
@@ -211,6 +228,25 @@ def emit(units, vec):
         st.ins("s_mov_b64 exec, -1")
         return op
 
+    if expand:
+        codes, row, land, out, toff, ldst = expand_layout(units)
+
+    def row_addresses():     # of the table rows that the fill's eight filter codes of this lane name
+        for i in range(8):
+            st.ins("v_mad_u32_u16 v%d, v%d, %%[rowb], v%d%s"
+                   % (row + i, codes + i // 2, toff, " op_sel:[1,0,0,0]" if i & 1 else ""))
+
+    def row_load(i):         # entries of eight activation codes (block i / 8) of column i % 8
+        b, j = divmod(i, 8)
+        return st.vm("buffer_load_dwordx4 %s, v%d, %%[erc], 0 offen offset:%d" % (quad(land, i), row + j, 64 * b))
+
+    def chunk_store(i):      # activation code i % 8 of block i / 8: the square's column, as a row's 16 bytes
+        b, e = divmod(i, 8)
+        for k in range(4):
+            st.ins("v_perm_b32 v%d, v%d, v%d, %%[%s]" % (out + 4 * (i & 1) + k, land + 4 * (8 * b + 2 * k + 1) + e // 2,
+                                                        land + 4 * (8 * b + 2 * k) + e // 2, "hi" if e & 1 else "lo"))
+        st.lds("ds_write_b128 v%d, %s offset:%d" % (ldst, quad(out, i & 1), (e >> 2) * 256 + (e & 3) * 16384 + b * 2048))
+
     # ---- prologue: the sums' start values, the first activations, the first reads ----
     st.ins("s_nop 7")   # the caller's last vector instructions may have written the scalar operands of the loads below
     acts = {}
@@ -245,7 +281,15 @@ def emit(units, vec):
     arrive_at = cross - 3 if units > 3 else cross - 1
     look_whole_at = cross - 2 if units > 3 else cross
     look_free_at = 0
-    loaded = 0
+    if expand:               # loads as early as they go, the stores a memory round trip later, done before the arrival
+        per_pair = 4 if units == 2 else 2 if units <= 6 else 1
+        load_at = [1 + i // per_pair for i in range(LOADS)]
+        first_store = min(load_at[7] + max(2, 16 // per_pair if units <= 6 else 20), arrive_at - 6)
+        store_at = [first_store + (arrive_at - 1 - first_store) * i // 15 for i in range(LOADS)]
+        if units >= 8:       # one a pair, the second block's behind its own round trip
+            store_at = [first_store + i + (i // 8) * 4 for i in range(LOADS)]
+        assert store_at[-1] < arrive_at and load_at[-1] <= store_at[8], (units, load_at, store_at, arrive_at)
+    loaded = stored = 0
     load_ops = []
     ops = {}
     stepped = False
@@ -257,8 +301,8 @@ def emit(units, vec):
             ops["free"] = look("cboth")
         st.wait_lds(pending[n], pending[n + 1])
         m = n + W
-        if p == arrive_at:
-            assert loaded == LOADS
+        if p == arrive_at:   # (a wavefront's LDS operations happen in order: its stores before this)
+            assert loaded == LOADS and stored == (LOADS if expand else 0)
             st.wait_vm(*load_ops)
             ops["arrive"] = count("cboth")
         if p == look_whole_at:
@@ -282,6 +326,22 @@ def emit(units, vec):
                 koff_step()
                 stepped = True
             acts[nu % units] = act_load(nu % units)
+        if expand:
+            if p == 0:
+                row_addresses()
+            while loaded < LOADS and load_at[loaded] == p:
+                load_ops.append(row_load(loaded))
+                loaded += 1
+            if loaded == LOADS and p == load_at[-1]:
+                ops["codes"] = st.vm("buffer_load_dwordx4 %s, v%d, %%[wrc], %%[eoff] offen" % (quad(codes, 0), V_L16))
+            if p == store_at[0]:
+                need(ops["free"], "cboth", "%[free]", 3)
+            while stored < LOADS and store_at[stored] == p:
+                if stored % 8 == 0:
+                    st.wait_vm(*load_ops[stored:stored + 8])
+                chunk_store(stored)
+                stored += 1
+            continue
         if p == first_load:
             need(ops["free"], "cboth", "%[free]", 3)
         while loaded < LOADS and load_at[loaded] == p:
@@ -295,7 +355,11 @@ def emit(units, vec):
     count("cbcur")
     st.ins("s_xor_b32 %[cbcur], %[cbcur], 4")
     st.ins("s_xor_b32 %[cboth], %[cboth], 4")
-    st.ins("s_xor_b32 %[edst], %[edst], 0x10000")
+    if expand:
+        st.wait_vm(ops["codes"])
+        st.ins("v_xor_b32 v%d, 0x10000, v%d" % (ldst, ldst))
+    else:
+        st.ins("s_xor_b32 %[edst], %[edst], 0x10000")
     # counts: the buffer's next fill is two on (8 more events); whole and free alternate between the buffers
     st.ins("s_add_u32 %[gf], %[gf], 1")
     st.ins("s_sub_u32 %[left], %[left], 1")
@@ -316,8 +380,9 @@ def emit(units, vec):
     # the rows that follow: the tile's next fill, or the first one of the workgroup's next tile, or none: then ENEXT has bit
     # 31 set, which moves into the vector offset.  That one is what a descriptor's bounds check covers; the scalar offset
     # must stay inside the rows by itself.
-    st.ins("s_add_u32 %[eoff], %[eoff], 0x10000")
-    st.ins("s_cmp_eq_u32 %[left], 1")
+    # (expanding: the same for the filter codes, which are loaded one fill further ahead)
+    st.ins("s_add_u32 %%[eoff], %%[eoff], %d" % (CODE_BYTES if expand else 0x10000))
+    st.ins("s_cmp_eq_u32 %%[left], %d" % (2 if expand else 1))
     st.ins("s_cselect_b32 %[eoff], %[enext], %[eoff]")
     st.ins("s_and_b32 %[tmp], %[eoff], 0x80000000")
     st.ins("s_xor_b32 %[eoff], %[eoff], %[tmp]")
@@ -342,7 +407,9 @@ def emit(units, vec):
         outs.append('"={%s[%d:%d]}"(ACC[%d])' % (lo[0], b, b + 15, u))
     inouts = [("CH0", V_CH0), ("CH1", V_CH1), ("KOFF", V_KOFF), ("QL", V_Q), ("KWL", V_KW), ("CINIT", V_POLL), ("L16", V_L16)]
     outs += ['"+{v%d}"(%s)' % (r, name) for name, r in inouts]
-    scalars = [("cbcur", "CBCUR"), ("cboth", "CBOTH"), ("edst", "EDST"), ("gf", "GF"), ("left", "LEFT"), ("free", "FREE"),
+    if expand:
+        outs += ['"+{v[%d:%d]}"(CODES)' % (codes, codes + 3), '"+{v%d}"(LDST)' % ldst]
+    scalars = [("cbcur", "CBCUR"), ("cboth", "CBOTH")] + ([] if expand else [("edst", "EDST")]) + [("gf", "GF"), ("left", "LEFT"), ("free", "FREE"),
                ("whole", "WHOLE"), ("eoff", "EOFF")]
     outs += ['[%s] "+&s"(%s)' % s for s in scalars]
     outs += ['[fail] "=&s"(FAIL)', '[tmp] "=&s"(TMP)', '[ev] "=&s"(EV)']
@@ -355,16 +422,24 @@ def emit(units, vec):
     if not vec:
         ins += ['[p%d] "s"(KS.pitch[%d])' % (j, j - 1) for j in (1, 2, 3)]
     clob = ['"v%d"' % r for r in list(range(V_ADDR, V_ADDR + 4)) + [V_TMP, V_CB] + list(range(ring, end))]
+    if expand:
+        ins += ['"{v%d}"(TOFF)' % toff] + ['[%s] "s"(%s)' % x for x in [("wrc", "WRC"), ("rowb", "512u"), ("lo", "0x05040100u"),
+                                                                      ("hi", "0x07060302u")]]
+        clob += ['"v%d"' % r for r in range(row, toff)]
     clob += ['"m0"', '"scc"', '"vcc"', '"memory"']
     args = ("ACC, CH0, CH1, KOFF, QL, KWL, CINIT, L16, CBCUR, CBOTH, EDST, GF, LEFT, FREE, WHOLE, EOFF, FAIL, TMP, EV, AOP, "
             "IDX, SEL, BASE, XQ, ERC, ENEXT, CB0, SPIN, WHOLE0, KS")
+    if expand:
+        args = args.replace("EDST, ", "") + ", WRC, CODES, LDST, TOFF"
     text = " \\\n        ".join('"%s\\n\\t"' % line for line in st.lines)
-    return ("#define MX_FILLS_U%d_%s(%s) \\\n    asm volatile( \\\n        %s \\\n        : %s \\\n        : %s \\\n        : %s)\n"
-            % (units, "V" if vec else "S", args, text, ", ".join(outs), ", ".join(ins), ", ".join(clob)))
+    return ("#define MX_%sFILLS_U%d_%s(%s) \\\n    asm volatile( \\\n        %s \\\n        : %s \\\n        : %s \\\n        : %s)\n"
+            % ("X" if expand else "", units, "V" if vec else "S", args, text, ", ".join(outs), ", ".join(ins), ", ".join(clob)))
 
 
 if __name__ == "__main__":
     print("// Generated by gen_lookup_mx.py -- do not edit.")
     for variant in VARIANTS:
         print(emit(*variant))
+    for variant in XVARIANTS:
+        print(emit(*variant, expand=True))
     sys.exit(0)

@@ -277,14 +277,20 @@ __global__ void __launch_bounds__(kPsTile) patch_sums_tiled_kernel(const float *
 // own; launches for the other kernels are instantiations without either, so that their code carries none of it (as run-time
 // values they cost the pre-pass of small layers 0.2 to 0.4 us: more arguments to fetch, more scalar registers to spill).
 struct PlainForm {
+    static constexpr bool kMxCodes = false;
     __device__ static XqLayout layout(const ConvGeom &g) { return {g.H, g.W, 0, 0}; }
     __device__ static int mx_fills() { return 0; }
 };
 struct MxForm {
+    static constexpr bool kMxCodes = false;
     XqLayout lay;
     int fills;        // of the rows, per column tile
     __device__ const XqLayout &layout(const ConvGeom &) const { return lay; }
     __device__ int mx_fills() const { return fills; }
+};
+// ... and where that kernel makes its rows itself, filter codes packed for it (mx_pack_unit) instead of rows.
+struct MxCodesForm : MxForm {
+    static constexpr bool kMxCodes = true;
 };
 
 // The filter pre-pass of a layer is independent of its input pre-pass: as two launches they would run one after
@@ -319,6 +325,19 @@ __device__ __forceinline__ void filter_pack_element(const int64_t i, const float
                                                     const uint8_t *__restrict__ filter_codes, int taps, int C,
                                                     int C4, int Co, int nt, int n_col_tiles, const TensorQuant &qf,
                                                     uint16_t *__restrict__ wq);
+__device__ __forceinline__ void mx_pack_unit(const int64_t i, const int fills, const float *__restrict__ filter,
+                                             const uint8_t *__restrict__ filter_codes, int taps, int C, int C4, int Co,
+                                             const TensorQuant &qf, uint16_t *__restrict__ wq);
+
+// Element (or, for codes in lutgemm_mx_kernel's form, unit of eight elements) i of the filter's packing.
+template <class Form>
+__device__ __forceinline__ void pack_filter(const int64_t i, const Form &form, const FilterWork &fw, const TensorQuant &qf)
+{
+    if constexpr (Form::kMxCodes)
+        mx_pack_unit(i, form.mx_fills(), fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, qf, fw.wq);
+    else
+        filter_pack_element(i, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, fw.nt, fw.n_col_tiles, qf, fw.wq);
+}
 
 // Patch sums for C % 4 == 0 when the input rows under a band of output rows fit in LDS: same order and same
 // results as patch_sums_kernel.  A block owns `rb` consecutive output rows of one image (one thread per output
@@ -330,12 +349,12 @@ __device__ __forceinline__ void filter_pack_element(const int64_t i, const float
 // wseg: output columns per workgroup.  wseg == OW: whole rows.  Less (wide rows of many channels, which would not
 // fit LDS otherwise): a band is cut into column segments, each with the input columns under it in LDS (SEG; without
 // it the code is the one for whole rows, with no trace of the segments).
-template <bool SEG>
+template <bool SEG, class Form>
 __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x, const ConvGeom &g, const int rb,
                                                      const int in_rows, const int wseg, const TensorQuant &tq,
                                                      const LayerQuant *__restrict__ lq_dev, float *__restrict__ psum,
                                                      uint32_t *__restrict__ xq, const XqLayout &lay, const int bid_in, const int nblocks,
-                                                     const int nthreads, const FilterWork &fw)
+                                                     const int nthreads, const FilterWork &fw, const Form &form)
 {
     // xq != nullptr: the block also quantizes the input rows it owns among those it copies (the rows under its
     // own band of output rows; the launcher has checked that these lie inside every block's window and together
@@ -469,8 +488,7 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
             const int64_t last = first + share < fw.pack_total ? first + share : fw.pack_total;
             const TensorQuant qf = lq_dev ? lq_dev->flt : fw.tq;
             for (int64_t i = first + widx; i < last; i += workers)
-                filter_pack_element(i, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, fw.nt,
-                                    fw.n_col_tiles, qf, fw.wq);
+                pack_filter(i, form, fw, qf);
         }
         return;
     }
@@ -778,6 +796,47 @@ __device__ __forceinline__ void filter_pack_element(const int64_t i, const float
         wq[i] = filter_code_at(i, filter, filter_codes, taps, C, C4, Co, nt, qf);
 }
 
+// Filter codes as lutgemm_mx_kernel takes them where it makes its rows itself: [column tile of 8][fill][filter element
+// 0..15][column 0..7], the null weight where there is none.  Unit i (i < column tiles x fills x 16) is the 16 bytes of one
+// filter element and column tile, column tiles fastest: neighbouring threads read neighbouring columns.
+__device__ __forceinline__ void mx_pack_unit(const int64_t i, const int fills, const float *__restrict__ filter,
+                                             const uint8_t *__restrict__ filter_codes, int taps, int C, int C4, int Co,
+                                             const TensorQuant &qf, uint16_t *__restrict__ wq)
+{
+    const int n_col = (Co + kMxCols - 1) / kMxCols;
+    const int e = (int)(i / n_col), ct = (int)(i - (int64_t)e * n_col);
+    if (e >= fills * 16)
+        return;
+    const int tap = (e >> 2) / C4, c = ((e >> 2) - tap * C4) * 4 + (e & 3), col0 = ct * kMxCols;
+    uint32_t code[kMxCols];
+    if (tap >= taps || c >= C) {
+#pragma unroll
+        for (int j = 0; j < kMxCols; ++j)
+            code[j] = kNullWeight;
+    } else {
+        const int64_t at = ((int64_t)tap * C + c) * Co + col0;
+        auto quantized = [&](const float v) { return quantize_code(fake_quant_value(v, qf), qf.offset, qf.inv_scale); };
+        if (filter_codes) {
+#pragma unroll
+            for (int j = 0; j < kMxCols; ++j)
+                code[j] = filter_codes[at + (col0 + j < Co ? j : 0)];
+        } else if (col0 + kMxCols <= Co && ((reinterpret_cast<uintptr_t>(filter + at)) & 15) == 0) {
+            const float4 lo = *reinterpret_cast<const float4 *>(filter + at), hi = *reinterpret_cast<const float4 *>(filter + at + 4);
+            code[0] = quantized(lo.x); code[1] = quantized(lo.y); code[2] = quantized(lo.z); code[3] = quantized(lo.w);
+            code[4] = quantized(hi.x); code[5] = quantized(hi.y); code[6] = quantized(hi.z); code[7] = quantized(hi.w);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kMxCols; ++j)
+                code[j] = quantized(filter[at + (col0 + j < Co ? j : 0)]);
+        }
+#pragma unroll
+        for (int j = 0; j < kMxCols; ++j)
+            code[j] = col0 + j < Co ? code[j] : kNullWeight;
+    }
+    *reinterpret_cast<uint4 *>(wq + (((int64_t)ct * fills * 16 + e) * kMxCols)) =
+        make_uint4(code[0] | code[1] << 16, code[2] | code[3] << 16, code[4] | code[5] << 16, code[6] | code[7] << 16);
+}
+
 // Filter sums (tf2/src/approx_nn_conv_kernels.cpp:300-306): one sequential sum per output column, rows (h, w, c)
 // ascending.  The chain of K dependent adds sets the time, so everything else is kept off it, and memory latency
 // is covered by volume in flight: a block owns only kFsCols columns (64-byte pieces of filter rows), which leaves
@@ -958,7 +1017,10 @@ __global__ void __launch_bounds__(kFsThreads) filter_prep_kernel(const float *__
     const int pb = (int)blockIdx.x - sum_blocks;
     if (pb < pack_blocks) {
         const int64_t i = (int64_t)pb * blockDim.x + threadIdx.x;
-        filter_pack_element(i, filter, filter_codes, taps, C, C4, Co, nt, n_col_tiles, q, wq);
+        if constexpr (Form::kMxCodes)
+            mx_pack_unit(i, form.mx_fills(), filter, filter_codes, taps, C, C4, Co, q, wq);
+        else
+            filter_pack_element(i, filter, filter_codes, taps, C, C4, Co, nt, n_col_tiles, q, wq);
         return;
     }
     px_expand_own_codes<kFsThreads / 4>(pb - pack_blocks, filter, filter_codes, taps, C, C4, Co, q, tableT, px_rows,
@@ -1207,9 +1269,11 @@ __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x
 
 // The filter work of a patch-sum launch: true if this workgroup is one of those that do it (and has done it), else
 // *bid is its index among the patch-sum workgroups.
-__device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const int mx_fills,
+template <class Form>
+__device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const Form &form,
                                                   const LayerQuant *__restrict__ lq_dev, int *bid)
 {
+    const int mx_fills = form.mx_fills();
     const int b = (int)blockIdx.x;
     if (b < fw.sum8) {
         if (b < fw.sum_blocks) { // the launcher gives these workgroups 512 or 1024 threads
@@ -1228,7 +1292,7 @@ __device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const in
     const int pb = *bid - fw.work_blocks;
     if (pb < fw.pack_blocks || fw.expand_blocks == 0) {
         const int64_t i = (int64_t)pb * blockDim.x + threadIdx.x;
-        filter_pack_element(i, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, fw.nt, fw.n_col_tiles, q, fw.wq);
+        pack_filter(i, form, fw, q);
         return true;
     }
     // pre-expanded rows: blockDim.x / 4 activation codes of a pair of fills per workgroup
@@ -1253,9 +1317,9 @@ __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *
 {
     const XqLayout lay = form.layout(g);
     int bid;
-    if (filter_work_block(fw, form.mx_fills(), lq_dev, &bid))
+    if (filter_work_block(fw, form, lq_dev, &bid))
         return;
-    patch_sums_rows_body<true>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw);
+    patch_sums_rows_body<true>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw, form);
 }
 
 template <class Form>
@@ -1267,7 +1331,7 @@ __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__re
 {
     const XqLayout lay = form.layout(g);
     int bid;
-    if (filter_work_block(fw, form.mx_fills(), lq_dev, &bid))
+    if (filter_work_block(fw, form, lq_dev, &bid))
         return;
     if (rb < 0) { // 1x1, stride 1, many channels, few pixels
         if (in_rows == 8)
@@ -1280,7 +1344,7 @@ __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__re
         patch_sums_flat_body(x, g, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, in_rows);
         return;
     }
-    patch_sums_rows_body<false>(x, g, rb, in_rows, g.OW, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw);
+    patch_sums_rows_body<false>(x, g, rb, in_rows, g.OW, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw, form);
 }
 
 __global__ void __launch_bounds__(256) quantize_flat_kernel(const float *__restrict__ v, int64_t n, float offset,
@@ -1312,6 +1376,15 @@ __global__ void __launch_bounds__(256) depthwise_filter_kernel(const float *__re
 }
 
 static inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
+
+// What the packing of a layer's filter counts in: elements, or units of eight (mx_pack_unit); none where
+// lutgemm_mx_kernel reads pre-expanded rows only.
+static int64_t pack_items(const DensePlan &plan, const MxPlan *mx)
+{
+    if (!mx)
+        return (int64_t)plan.n_col_tiles * plan.fills * 64;
+    return mx->expand ? (int64_t)mx->n_col_tiles * mx->fills * 16 : 0;
+}
 
 // Layers without taps or channels: every output is the same value.
 __global__ void __launch_bounds__(256) fill_u32_kernel(uint32_t *__restrict__ dst, int n, uint32_t value)
@@ -1918,8 +1991,8 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             int block_threads = threads;
             if (filter_job && filter_done) {
                 const DensePlan &plan = *filter_job->plan;
-                const MxPlan *const mx = filter_job->mx;   // its kernel reads rows only: nothing to pack
-                const int64_t total = mx ? 0 : (int64_t)plan.n_col_tiles * plan.fills * 64;
+                const MxPlan *const mx = filter_job->mx;
+                const int64_t total = pack_items(plan, mx);
                 fw.filter = filter_job->filter;
                 fw.filter_codes = filter_job->filter_codes;
                 fw.taps = g.KH * g.KW;
@@ -1989,7 +2062,10 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                 return hipGetLastError();
             };
             const bool mx_form = (filter_job && filter_job->mx) || lay.row0 || lay.col0;
-            return mx_form ? launch(MxForm{lay, filter_job && filter_job->mx ? filter_job->mx->fills : 0}) : launch(PlainForm{});
+            const MxForm mxf = {lay, filter_job && filter_job->mx ? filter_job->mx->fills : 0};
+            if (filter_job && filter_job->mx && filter_job->mx->expand)
+                return launch(MxCodesForm{mxf});
+            return mx_form ? launch(mxf) : launch(PlainForm{});
         }
     }
     if (!vec && g.OW <= 1024 && g.C < 64) {
@@ -2086,7 +2162,7 @@ hipError_t launch_filter_pack(const float *filter, const uint8_t *filter_codes, 
 {
     if (px_done)
         *px_done = false;
-    const int64_t total = mx ? 0 : (int64_t)plan.n_col_tiles * plan.fills * 64;   // lutgemm_mx_kernel reads rows only
+    const int64_t total = pack_items(plan, mx);
     const int sum_blocks = (fsum && filter) ? (int)blocks_for(g.Co, kFsCols) : 0;
     const int pack_blocks = (int)blocks_for(total, kFsThreads);
     size_t lds = sum_blocks ? kFsLdsBytes : 0;
@@ -2116,6 +2192,8 @@ hipError_t launch_filter_pack(const float *filter, const uint8_t *filter_codes, 
                            wq, sum_blocks, fsum, pack_blocks, tableT, px_rows, form);
         return hipGetLastError();
     };
+    if (mx && mx->expand)
+        return launch(MxCodesForm{MxForm{XqLayout{}, mx->fills}});
     return mx ? launch(MxForm{XqLayout{}, mx->fills}) : launch(PlainForm{});
 }
 

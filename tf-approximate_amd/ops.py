@@ -339,9 +339,10 @@ def conv2d_matrix_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding=
     desc = make_desc(tuple(input_shape), tuple(filter_shape), list(strides), padding, (), "NHWC", list(dilations), 8)
     plan = (ctypes.c_int32 * 8)()
     _check(lib.axc_conv2d_matrix_plan(ctypes.byref(desc), plan))
-    keys = ("units_per_wavefront", "units_per_tile", "row_tiles", "column_tiles", "k_splits", "workgroups",
+    # own_rows: 0 = reads pre-expanded rows, 1 = makes them itself in every tile
+    keys = ("own_rows", "units_per_wavefront", "units_per_tile", "row_tiles", "column_tiles", "k_splits", "workgroups",
             "fills_per_split")
-    return dict(zip(keys, [int(v) for v in plan[1:]])) if plan[0] else None
+    return dict(zip(keys, [int(v) for v in [plan[0] - 1] + list(plan[1:])])) if plan[0] else None
 
 
 def set_tile_columns(columns):
@@ -352,6 +353,12 @@ def set_tile_columns(columns):
 def set_preexpand(mode):
     """Which dense layers run out of pre-expanded rows: 0 = the planner's choice, 1 = all that can, -1 = none."""
     _check(_lib.load().axc_set_preexpand(int(mode)))
+
+
+def set_matrix_rows(mode):
+    """Rows of the kernel whose sums the matrix cores make: 0 = the planner's choice, 1 = pre-expanded ones only, 2 = made
+    by the kernel itself wherever it can."""
+    _check(_lib.load().axc_set_matrix_rows(int(mode)))
 
 
 def set_wait_limit(polls):
