@@ -164,9 +164,6 @@ struct MxParams {
     uint32_t xq_bytes;
     const uint16_t *rows;  // pre-expanded ones
     uint32_t rows_bytes;
-    const uint16_t *wq;    // plan.expand: filter codes [column tile][fill][filter element 0..15][column 0..7], and the table
-    uint32_t wq_bytes;     // with the top bit of every byte flipped, filter-code major
-    const uint16_t *tableF;
     const float *psum, *fsum, *bias;
     const int32_t *pixel_term, *column_term;   // not null (tf1 op): added to the integer outputs, by the first K split
     float *out_f;
@@ -190,6 +187,9 @@ struct MxParams {
     uint32_t step_rows, step_groups, step_bytes, carry_row, carry_img;
     uint32_t spin_limit;
     uint32_t *wait_error;
+    const uint16_t *wq;    // plan.expand: filter codes [column tile][fill][filter element 0..15][column 0..7], and the table
+    const uint16_t *tableF;  // with the top bit of every byte flipped, filter-code major
+    uint32_t wq_bytes;
 };
 
 struct DepthwiseParams {

@@ -435,7 +435,10 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             }
         };
         const uint32_t at0 = SIMPLE && col0 >= p.Co ? kNowhere : px0 * pixel_bytes + (uint32_t)col0 * 4u;   // bytes of px0 (linear)
-        const bool quads = (p.Co & 3) == 0;
+        // Four columns leave as one 16-byte store, which needs no more than the alignment of a dword, and only those of an
+        // incomplete last group one by one (all of them, where columns do not come in fours: 1x1 16->342 @38x38x38 88.9 us).
+        const bool tail = !SIMPLE && (p.Co & 3) != 0 && ct * 8 + 8 > p.Co;
+        const bool whole = col0 + 4 <= p.Co;
         const float e_s1xs2 = p.lq_dev ? p.lq_dev->s1xs2 : p.s1xs2, e_m1 = p.lq_dev ? p.lq_dev->m1 : p.m1;
         const float e_m2 = p.lq_dev ? p.lq_dev->m2 : p.m2, e_km = p.lq_dev ? p.lq_dev->k_m1xm2 : p.k_m1xm2;
         float t3[4], bias[4];   // no bias: -0.0f, which changes no value
@@ -502,12 +505,13 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                         }
                         if (SIMPLE) {
                             __builtin_amdgcn_raw_buffer_store_b128(d, out_rsrc, (int)at[jp], 0, 0);
-                        } else if (quads) {
-                            __builtin_amdgcn_raw_buffer_store_b128(d, out_rsrc, (int)(col0 < p.Co ? at[jp] : kNowhere), 0, 0);
                         } else {
+                            __builtin_amdgcn_raw_buffer_store_b128(d, out_rsrc, (int)(whole ? at[jp] : kNowhere), 0, 0);
+                            if (tail) {
 #pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                __builtin_amdgcn_raw_buffer_store_b32(d[e], out_rsrc, (int)(col0 + e < p.Co ? at[jp] + 4u * e : kNowhere), 0, 0);
+                                for (int e = 0; e < 3; ++e)
+                                    __builtin_amdgcn_raw_buffer_store_b32(d[e], out_rsrc, (int)(!whole && col0 + e < p.Co ? at[jp] + 4u * e : kNowhere), 0, 0);
+                            }
                         }
                     }
                 }
