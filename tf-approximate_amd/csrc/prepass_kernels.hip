@@ -339,22 +339,49 @@ __device__ __forceinline__ void pack_filter(const int64_t i, const Form &form, c
         filter_pack_element(i, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, fw.nt, fw.n_col_tiles, qf, fw.wq);
 }
 
-// Patch sums for C % 4 == 0 when the input rows under a band of output rows fit in LDS: same order and same
+// How a chain of patch sums reads the channel quads of a pixel in LDS: quads | (quads per batch << 16).  Batches of 4 to 8
+// keep the reads a batch ahead of the adds; a pixel is padded with quads of zeros to whole batches of the size that wants the
+// fewest (9 quads to 10, 13 to 15, 23 to 24).  Without batches, every read waited for, a chain takes twice as long (3x3
+// 40->128 @17x73x3); below four quads the padding would cost more than that.
+__host__ __device__ inline int chain_form(const int C4)
+{
+    int best = C4;
+    if (C4 < 4)
+        return best;
+    int least = 1 << 30;
+    for (int b : {8, 6, 5, 4}) {
+        const int padded = (C4 + b - 1) / b * b;
+        if (padded < least) {
+            least = padded;
+            best = padded | (b << 16);
+        }
+    }
+    return best;
+}
+
+// Floats from pixel to pixel in LDS: an odd number of 16-byte units, so that the reads of neighbouring threads fall into
+// different banks (5x5 56->49 @104x104x43, 15 quads at a pitch of 16: 338 us of pre-pass).
+__host__ __device__ inline int band_pitch(const int quads) { return (quads | 1) * 4; }
+
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));   // global loads take four floats at any of them
+
+// Patch sums when the input rows under a band of output rows fit in LDS: same order and same
 // results as patch_sums_kernel.  A block owns `rb` consecutive output rows of one image (one thread per output
 // pixel) and first copies the input rows they touch into LDS, so every input float is fetched from memory
 // about once (plus the halo) instead of once per filter tap; the sequential chains then read LDS only.
-// Pixels are padded to C + 4 floats so that the 16-byte reads of neighbouring threads fall into different banks.
 // bid / nblocks: index of this workgroup among those that do this work (in dispatch order, so that bid & 7 is
 // the XCD); nthreads: the threads of the workgroup that take part (the others only meet the barrier).
 // wseg: output columns per workgroup.  wseg == OW: whole rows.  Less (wide rows of many channels, which would not
 // fit LDS otherwise): a band is cut into column segments, each with the input columns under it in LDS (SEG; without
 // it the code is the one for whole rows, with no trace of the segments).
-template <bool SEG, class Form>
+// copiers_in: those threads | quads per batch of a chain << 16 | quads of zeros behind a pixel << 20 (chain_form).  ANY: any channel count and alignment of x; without it
+// channels come in fours and x is 16-byte aligned.
+template <bool SEG, bool ANY, class Form>
 __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x, const ConvGeom &g, const int rb,
                                                      const int in_rows, const int wseg, const TensorQuant &tq,
                                                      const LayerQuant *__restrict__ lq_dev, float *__restrict__ psum,
                                                      uint32_t *__restrict__ xq, const XqLayout &lay, const int bid_in, const int nblocks,
-                                                     const int nthreads, const FilterWork &fw, const Form &form)
+                                                     const int copiers_in, const FilterWork &fw, const Form &form)
 {
     // xq != nullptr: the block also quantizes the input rows it owns among those it copies (the rows under its
     // own band of output rows; the launcher has checked that these lie inside every block's window and together
@@ -391,7 +418,24 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
         own_clo = ow0 * g.sw;
         own_chi = ow1 == g.OW ? g.W : ow1 * g.sw;
     }
-    const int pitch = g.C + 4;
+    const int zeros = copiers_in >> 20, quads = g.C4 + zeros;   // of a pixel in LDS: those behind C4 hold zeros
+    const int nthreads = copiers_in & 0xffff, pitch = band_pitch(quads);
+    // A pixel's last quad may be incomplete: it is loaded so that it ends with the pixel (C > 4), and shifted.
+    const int rest = ANY ? g.C & 3 : 0;
+    auto load_quad = [&](const float *px, const int q) __attribute__((always_inline)) {
+        if (!ANY)
+            return *reinterpret_cast<const float4 *>(px + q * 4);
+        const f4_any v = *reinterpret_cast<const f4_any *>(px + (rest && q == g.C4 - 1 ? g.C - 4 : q * 4));
+        return make_float4(v[0], v[1], v[2], v[3]);
+    };
+    auto settle_quad = [&](float4 v, const int q) __attribute__((always_inline)) {
+        if (!ANY || !rest || q != g.C4 - 1)
+            return fake_quant_value4(v, qt);
+        v = rest == 1 ? make_float4(v.w, 0.0f, 0.0f, 0.0f) : rest == 2 ? make_float4(v.z, v.w, 0.0f, 0.0f)
+                                                                      : make_float4(v.y, v.z, v.w, 0.0f);
+        v = fake_quant_value4(v, qt);
+        return make_float4(v.x, rest > 1 ? v.y : 0.0f, rest > 2 ? v.z : 0.0f, 0.0f);
+    };
     if (t >= nthreads) {
         // not taking part in the copy
     } else if (nthreads % g.C4 == 0) {
@@ -409,7 +453,7 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
         }
         const int wsteps = rpar > 1 ? 1 : (wc + wstep - 1) / wstep;
         const int iters = ((in_rows + rpar - 1) / rpar) * wsteps;
-        const float *const xn = x + (int64_t)n * g.H * g.W * g.C + q * 4;
+        const float *const xn = x + (int64_t)n * g.H * g.W * g.C;
         int r_next = r0, ws_next = 0; // (row, column step) of the next item
         for (int it0 = 0; it0 < iters; it0 += kInFlight) {
             float4 v[kInFlight];
@@ -427,13 +471,13 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
                 const int wcl = iw_lo + (ww[u] < wc ? ww[u] : wc - 1);
                 v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 if (it0 + u < iters)   // the same for the whole workgroup: no load for items nobody has
-                    v[u] = *reinterpret_cast<const float4 *>(xn + ((int64_t)ih * g.W + wcl) * g.C);
+                    v[u] = load_quad(xn + ((int64_t)ih * g.W + wcl) * g.C, q);
             }
 #pragma unroll
             for (int u = 0; u < kInFlight; ++u) {
                 const int ih = ih_first + rr[u];
                 const bool in_image = (unsigned)ih < (unsigned)g.H;
-                float4 f = fake_quant_value4(v[u], qt);
+                float4 f = settle_quad(v[u], q);
                 if (!in_image)
                     f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // rows outside the image are zeros
                 if (it0 + u < iters && rr[u] < in_rows && ww[u] < wc) {
@@ -457,14 +501,16 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
             const int ih = ih_first + r;
             float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if ((unsigned)ih < (unsigned)g.H)
-                v = fake_quant_value4(
-                    *reinterpret_cast<const float4 *>(x + (((int64_t)n * g.H + ih) * g.W + iw_lo + w) * g.C + q * 4), qt);
+                v = settle_quad(load_quad(x + (((int64_t)n * g.H + ih) * g.W + iw_lo + w) * g.C, q), q);
             *reinterpret_cast<float4 *>(&rows[(r * wc + w) * pitch + q * 4]) = v;
         }
     }
     float *const zero_px = rows + (size_t)in_rows * wc * pitch; // one pixel of zeros behind the rows (see below)
-    if (t < g.C4)
-        *reinterpret_cast<float4 *>(zero_px + t * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i = t; i < quads; i += (int)blockDim.x)
+        *reinterpret_cast<float4 *>(zero_px + i * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (zeros > 0)
+        for (int i = t; i < in_rows * wc * zeros; i += (int)blockDim.x)
+            *reinterpret_cast<float4 *>(&rows[i / zeros * pitch + (g.C4 + i % zeros) * 4]) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     __syncthreads();
     // Chains go to the wavefronts of the block starting from a different one in blocks that are likely to share a
     // CU (wavefronts of a block are spread over the SIMDs in order), so that their chains do not share a SIMD.
@@ -499,11 +545,11 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
     __builtin_amdgcn_s_setprio(3);   // the chain is the critical path: its wavefront issues ahead of the others on its SIMD
     const auto batched_chain = [&](auto batch_tag) {
         // The chain of K dependent adds is what takes the time here, so nothing else may wait on it: the taps and
-        // their channels form one flat list of batches of 32 floats (16 where the channel quads are no multiple of 8), the LDS reads of a batch are issued a batch
+        // their channels form one flat list of batches of 16 to 32 floats, the LDS reads of a batch are issued a batch
         // ahead of its adds, and every lane takes every tap - a tap outside the image reads the pixel of zeros
         // (x + 0 == x; the sum starts at +0 and so is never -0) instead of branching around it.
-        constexpr int kBatch = decltype(batch_tag)::value; // 16-byte reads per batch: 8, or 4 for 16 channels and the like
-        const int bpt = g.C4 / kBatch, nb = g.KH * g.KW * bpt;
+        constexpr int kBatch = decltype(batch_tag)::value; // 16-byte reads per batch: 4 to 8 (chain_form)
+        const int bpt = quads / kBatch, nb = g.KH * g.KW * bpt;
         int kh = 0, kw = 0, bi = 0;
         auto tap_src = [&]() -> const float4 * {
             const int iw = iw0 + kw * g.dw;
@@ -552,13 +598,11 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
         }
         psum[((int64_t)n * g.OH + oh) * g.OW + ow] = s;
     };
-    if ((g.C4 & 7) == 0) {
-        batched_chain(std::integral_constant<int, 8>());
-        return;
-    }
-    if ((g.C4 & 3) == 0) {
-        batched_chain(std::integral_constant<int, 4>());
-        return;
+    switch ((copiers_in >> 16) & 15) {
+    case 8: batched_chain(std::integral_constant<int, 8>()); return;
+    case 6: batched_chain(std::integral_constant<int, 6>()); return;
+    case 5: batched_chain(std::integral_constant<int, 5>()); return;
+    case 4: batched_chain(std::integral_constant<int, 4>()); return;
     }
     // Scalar loads count down together with LDS reads, but in no order: while the compiler takes one to be in flight it waits
     // for all reads of a batch before the first add (3x3/2 680->12 @49x59x38: 409 -> 440 us of pre-pass).
@@ -1307,7 +1351,7 @@ __device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const Fo
 }
 
 // Bands cut into column segments: a kernel of its own, so that the common variants below stay as small as they were.
-template <class Form>
+template <bool ANY, class Form>
 __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *__restrict__ x, const ConvGeom g,
                                                                     int rb, int in_rows, int nthreads, int wseg,
                                                                     const TensorQuant tq,
@@ -1319,10 +1363,10 @@ __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *
     int bid;
     if (filter_work_block(fw, form, lq_dev, &bid))
         return;
-    patch_sums_rows_body<true>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw, form);
+    patch_sums_rows_body<true, ANY>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw, form);
 }
 
-template <class Form>
+template <bool ANY, class Form>
 __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__restrict__ x, const ConvGeom g, int rb,
                                                                 int in_rows, int nthreads, const TensorQuant tq,
                                                                 const LayerQuant *__restrict__ lq_dev,
@@ -1333,18 +1377,18 @@ __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__re
     int bid;
     if (filter_work_block(fw, form, lq_dev, &bid))
         return;
-    if (rb < 0) { // 1x1, stride 1, many channels, few pixels
+    if (!ANY && rb < 0) { // 1x1, stride 1, many channels, few pixels
         if (in_rows == 8)
             patch_sums_deep_body<8>(x, g, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks);
         else
             patch_sums_deep_body<16>(x, g, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks);
         return;
     }
-    if (rb == 0) { // 1x1, stride 1: flat pixel list
+    if (!ANY && rb == 0) { // 1x1, stride 1: flat pixel list
         patch_sums_flat_body(x, g, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, in_rows);
         return;
     }
-    patch_sums_rows_body<false>(x, g, rb, in_rows, g.OW, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw, form);
+    patch_sums_rows_body<false, ANY>(x, g, rb, in_rows, g.OW, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw, form);
 }
 
 __global__ void __launch_bounds__(256) quantize_flat_kernel(const float *__restrict__ v, int64_t n, float offset,
@@ -1825,11 +1869,11 @@ static bool best_band(const ConvGeom &g, int wseg, int sum_blocks, int64_t lds_l
     const double K = (double)g.KH * g.KW * g.C;
     const int64_t lds_max = device_lds_bytes();
     const int nsegs = (g.OW + wseg - 1) / wseg;
-    const int64_t row_bytes = (int64_t)input_columns_under(g, wseg) * (g.C + 4) * 4;
+    const int64_t row_bytes = (int64_t)input_columns_under(g, wseg) * band_pitch(chain_form(g.C4) & 0xffff) * 4;
     bool found = false;
     for (int cand = 1; cand <= g.OH && cand * wseg <= 1024; ++cand) {
         const int rows_needed = (cand - 1) * g.sh + (g.KH - 1) * g.dh + 1;
-        const int64_t lds = rows_needed * row_bytes + (int64_t)(g.C + 4) * 4;
+        const int64_t lds = rows_needed * row_bytes + (int64_t)band_pitch(chain_form(g.C4) & 0xffff) * 4;
         if (lds > lds_limit)
             break;
         const int chains = cand * wseg;
@@ -1880,10 +1924,10 @@ static void choose_band(const ConvGeom &g, int sum_blocks, int *rb_out, int *in_
         if (wseg == last_wseg || wseg < 4)
             continue;
         last_wseg = wseg;
-        const int64_t row_bytes = (int64_t)input_columns_under(g, wseg) * (g.C + 4) * 4;
+        const int64_t row_bytes = (int64_t)input_columns_under(g, wseg) * band_pitch(chain_form(g.C4) & 0xffff) * 4;
         for (int cand = 1; cand <= g.OH && cand * wseg <= 1024; ++cand) {
             const int rows_needed = (cand - 1) * g.sh + (g.KH - 1) * g.dh + 1;
-            if (rows_needed * row_bytes + (int64_t)(g.C + 4) * 4 > lds_two)
+            if (rows_needed * row_bytes + (int64_t)band_pitch(chain_form(g.C4) & 0xffff) * 4 > lds_two)
                 break;
             if (cand * wseg > best_chains && (best_chains == 7 || cand * wseg * 100 > best_chains * 115 ||
                                               wseg == *wseg_out)) {
@@ -1929,10 +1973,13 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
     const bool vec = (g.C & 3) == 0 && ((uintptr_t)x & 15) == 0;
     if (flat_row_bytes && vec)   // the flat layout belongs to channel counts that are no multiple of four
         return hipErrorInvalidValue;
-    if (vec && g.OW <= 1024) {
+    // Channel counts that are no multiple of four, from 64 on: the same bands, loaded at any alignment (3x3 521->64
+    // @17x17x79 1337 us pixel by pixel out of memory).  Below that patch_sums_smallc_kernel has them.
+    const bool any = !vec && g.C >= 64;
+    if ((vec || any) && g.OW <= 1024) {
         // largest band of output rows whose input rows fit in 96 KiB of LDS and whose pixels fit in one block,
         // but no larger than what still leaves every CU a few blocks
-        const int64_t row_bytes = (int64_t)g.W * (g.C + 4) * 4;
+        const int64_t row_bytes = (int64_t)g.W * band_pitch(chain_form(g.C4) & 0xffff) * 4;
         int rb = 0, in_rows = 0;
         for (int cand = 1; cand <= g.OH && cand * g.OW <= 1024; ++cand) {
             const int rows_needed = (cand - 1) * g.sh + (g.KH - 1) * g.dh + 1;
@@ -1944,7 +1991,7 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             in_rows = rows_needed;
         }
         // 1x1, stride 1, no padding, and a band would hold few pixels (many channels): the flat-list variant
-        const bool flat = g.KH == 1 && g.KW == 1 && g.sh == 1 && g.sw == 1 && g.ph == 0 && g.pw == 0 &&
+        const bool flat = vec && g.KH == 1 && g.KW == 1 && g.sh == 1 && g.sw == 1 && g.ph == 0 && g.pw == 0 &&
                           rb * g.OW < 192;
         int wseg = g.OW;   // output columns per workgroup: whole rows unless choose_band cuts them
         if (!flat)
@@ -1971,17 +2018,21 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             // same along the row where a band is cut into column segments (segment s owns input columns
             // [s*wseg*sw, (s+1)*wseg*sw), the last one up to W).
             const bool segmented = !flat && wseg < g.OW;
-            const bool fuse = xq_fused && fused &&
+            // (of the threads a whole number per channel quad takes part in the copy: each keeps its quad)
+            const int form_of_chain = chain_form(g.C4);
+            const int copiers = (g.C4 <= threads ? threads / g.C4 * g.C4 : threads) | (form_of_chain >> 16) << 16 |
+                                ((form_of_chain & 0xffff) - g.C4) << 20;
+            const bool fuse = xq_fused && fused && !flat_row_bytes &&
                               (flat || (g.sh - 1 + g.ph <= (g.KH - 1) * g.dh &&
-                                        (g.OH - 1) * g.sh - g.ph + (g.KH - 1) * g.dh >= g.H - 1 && threads % g.C4 == 0 &&
+                                        (g.OH - 1) * g.sh - g.ph + (g.KH - 1) * g.dh >= g.H - 1 && g.C4 <= threads &&
                                         (!segmented || (g.sw - 1 + g.pw <= (g.KW - 1) * g.dw &&
                                                         (g.OW - 1) * g.sw - g.pw + (g.KW - 1) * g.dw >= g.W - 1))));
             if (fuse)
                 *fused = true;
-            const size_t band_row_bytes = (size_t)input_columns_under(g, wseg) * (g.C + 4) * 4;
+            const size_t band_row_bytes = (size_t)input_columns_under(g, wseg) * band_pitch(chain_form(g.C4) & 0xffff) * 4;
             size_t lds = deep ? (size_t)deep_lds_bytes(in_rows)
                               : flat ? (size_t)in_rows * kFlatPitch * 4
-                                     : (size_t)in_rows * band_row_bytes + (size_t)(g.C + 4) * 4; // + the pixel of zeros
+                                     : (size_t)in_rows * band_row_bytes + (size_t)band_pitch(chain_form(g.C4) & 0xffff) * 4; // + the pixel of zeros
             const int bands = flat ? 0 : (g.OH + rb - 1) / rb;
             const int64_t work_blocks =
                 flat ? (g.M + in_rows - 1) / in_rows : (int64_t)g.N * bands * ((g.OW + wseg - 1) / wseg);
@@ -2045,21 +2096,25 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             }
             fw.work_blocks = (int)work_blocks;
             const unsigned grid = (unsigned)(fw.sum8 + work_blocks + fw.pack_blocks + fw.expand_blocks);
-            auto launch = [&](const auto &form) {
+            auto launch_as = [&](const auto &form, auto any_tag) {
                 using Form = std::decay_t<decltype(form)>;
-                const void *const kernel = segmented ? reinterpret_cast<const void *>(patch_sums_segments_kernel<Form>)
-                                                     : reinterpret_cast<const void *>(patch_sums_rows_kernel<Form>);
+                constexpr bool kAny = decltype(any_tag)::value;
+                const void *const kernel = segmented ? reinterpret_cast<const void *>(patch_sums_segments_kernel<kAny, Form>)
+                                                     : reinterpret_cast<const void *>(patch_sums_rows_kernel<kAny, Form>);
                 const hipError_t e = set_max_dynamic_lds_once(kernel, device_lds_bytes());
                 if (e != hipSuccess)
                     return e;
                 uint32_t *const codes_out = fuse ? xq_fused : nullptr;
                 if (segmented)
-                    hipLaunchKernelGGL(patch_sums_segments_kernel<Form>, dim3(grid), dim3(block_threads), lds, stream, x, g, rb,
-                                       in_rows, threads, wseg, tq, lq_dev, psum, codes_out, fw, form);
+                    hipLaunchKernelGGL((patch_sums_segments_kernel<kAny, Form>), dim3(grid), dim3(block_threads), lds, stream, x, g,
+                                       rb, in_rows, copiers, wseg, tq, lq_dev, psum, codes_out, fw, form);
                 else
-                    hipLaunchKernelGGL(patch_sums_rows_kernel<Form>, dim3(grid), dim3(block_threads), lds, stream, x, g, rb,
-                                       in_rows, threads, tq, lq_dev, psum, codes_out, fw, form);
+                    hipLaunchKernelGGL((patch_sums_rows_kernel<kAny, Form>), dim3(grid), dim3(block_threads), lds, stream, x, g,
+                                       rb, in_rows, flat ? threads : copiers, tq, lq_dev, psum, codes_out, fw, form);
                 return hipGetLastError();
+            };
+            auto launch = [&](const auto &form) {
+                return any ? launch_as(form, std::true_type()) : launch_as(form, std::false_type());
             };
             const bool mx_form = (filter_job && filter_job->mx) || lay.row0 || lay.col0;
             const MxForm mxf = {lay, filter_job && filter_job->mx ? filter_job->mx->fills : 0};
