@@ -149,7 +149,7 @@ int axc_conv2d_tile_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
  * that cuts it: plan = { 1 or 2, or 0 (then the rest is 0 too), units of 64 pixels per wavefront (the kernel's variant),
  * units per tile, row tiles, column tiles (8 columns), K splits, workgroups, fills of 16 filter elements per K split }.
  * 1: it runs out of rows of 512 bytes per filter element in the workspace, at most 2 GiB, which the workspace query counts;
- * 2: it makes the rows itself in every tile.  A launch whose workspace lacks room runs in the other form or one of the other
+ * 2: it makes the rows itself in every tile; 3: the same with the operands exchanged, output pixels for columns.  A launch whose workspace lacks room runs in the other form or one of the other
  * kernels, with the same results. */
 int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
 /* Pins the tile width the planner uses (16, 32 or 64 columns; 0 = its own choice, the default), process-wide, for
@@ -167,8 +167,8 @@ int axc_set_tile_columns(int columns);
  * in the reference. */
 int axc_set_preexpand(int mode);
 /* Which rows the kernel of axc_conv2d_matrix_plan reads: 0 = the planner decides (the default), 1 = pre-expanded ones only
- * (layers that those do not suit run the other kernels), 2 = made by the kernel itself wherever it can; process-wide, for
- * tests and timing; a workspace query and the launch it is for must see the same value.  Results do not depend on it.  No
+ * (layers that those do not suit run the other kernels), 2 = made by the kernel itself wherever it can, 3 = the same with
+ * the operands exchanged; process-wide, for tests and timing; a workspace query and the launch it is for must see the same value.  Results do not depend on it.  No
  * counterpart in the reference. */
 int axc_set_matrix_rows(int mode);
 /* The wavefronts of the kernels that plan code 2 and axc_conv2d_matrix_plan stand for wait for each other by polling counters,

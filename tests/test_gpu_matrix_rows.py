@@ -38,6 +38,24 @@ CASES = [
 ]
 
 
+# ... and with the operands exchanged: few pixels, none of them or of the columns in eights or fours, channel counts that are
+# no multiple of four, filters whose patches leave the image, a strided 1x1 layer (gathered first), wide and tall tiles
+SWAPPED = [
+    ((1, 7, 7, 512), (3, 3, 512), 1, 1, "SAME"),
+    ((1, 7, 7, 64), (1, 1, 1030), 1, 1, "SAME"),
+    ((1, 1, 1, 300), (1, 1, 77), 1, 1, "SAME"),          # one pixel
+    ((2, 5, 3, 7), (3, 3, 9), 1, 1, "SAME"),             # 63 filter elements, few columns
+    ((1, 9, 5, 17), (5, 4, 260), 1, 1, "SAME"),
+    ((2, 9, 11, 65), (3, 3, 50), 2, 1, "VALID"),
+    ((1, 14, 14, 256), (1, 1, 1024), 1, 1, "SAME"),
+    ((1, 14, 14, 128), (1, 1, 512), 2, 1, "SAME"),
+    ((3, 6, 7, 20), (3, 3, 2050), 1, 2, "SAME"),
+    ((1, 12, 12, 96), (3, 3, 5000), 1, 1, "SAME"),       # several tiles per workgroup
+    ((1, 40, 1, 32), (7, 1, 333), 1, 1, "SAME"),
+    ((1, 1, 1100, 36), (1, 3, 40), 1, 1, "SAME"),        # rows too wide for bands: patch sums of another kernel
+]
+
+
 def _id(case):
     xs, fs, stride, dil, padding = case
     return "%dx%dx%dx%d-%dx%d-to%d-s%d-d%d-%s" % (xs + fs + (stride, dil, padding))
@@ -52,17 +70,23 @@ def own_rows(pkg):
         pkg.ops.set_matrix_rows(0)
 
 
+@pytest.fixture()
+def swapped(pkg):
+    pkg.ops.set_matrix_rows(3)
+    try:
+        yield pkg.ops
+    finally:
+        pkg.ops.set_matrix_rows(0)
+
+
 def _plan(ops, case):
     xs, fs, stride, dil, padding = case
     return ops.conv2d_matrix_plan(xs, (fs[0], fs[1], xs[3], fs[2]), (1, stride, stride, 1), padding, (1, dil, dil, 1))
 
 
-@pytest.mark.parametrize("case", CASES, ids=_id)
-def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, own_rows, case):
+def _compare(pkg, oracle, ops, case):
     print("case", _id(case), flush=True)
     xs, fs, stride, dil, padding = case
-    plan = _plan(own_rows, case)
-    assert plan is not None and plan["own_rows"] == 1, plan
     table = pkg.synth.table_random(sum(xs) + fs[2])
     xd, fd = bench.device_tensors(pkg, xs, (fs[0], fs[1], xs[3], fs[2]), "uniform", seed=sum(xs) + 3 * sum(fs))
     bias = torch.linspace(-1.0, 1.0, fs[2], device=xd.device)
@@ -71,11 +95,11 @@ def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, own_rows, case
     def run():
         return op.accumulators(xd, fd, *MM), op(xd, fd, *MM), op(xd, fd, *MM, bias=bias, activation="relu")
     got = run()
-    own_rows.set_preexpand(-1)
+    ops.set_preexpand(-1)
     try:
         want = run()
     finally:
-        own_rows.set_preexpand(0)
+        ops.set_preexpand(0)
     for g, w in zip(got, want):
         bad = g.view(torch.int32) != w.view(torch.int32)
         assert not bool(bad.any()), "%d of %d differ, first at %s" % (
@@ -88,11 +112,46 @@ def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, own_rows, case
         assert refimpl.linf_rel(got[1].cpu().numpy(), y_ref) <= 1e-5
 
 
+@pytest.mark.parametrize("case", CASES, ids=_id)
+def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, own_rows, case):
+    plan = _plan(own_rows, case)
+    assert plan is not None and plan["own_rows"] == 1, plan
+    _compare(pkg, oracle, own_rows, case)
+
+
+@pytest.mark.parametrize("case", SWAPPED, ids=_id)
+def test_operands_exchanged(pkg, oracle, swapped, case):
+    plan = _plan(swapped, case)
+    assert plan is not None and plan["own_rows"] == 2, plan
+    _compare(pkg, oracle, swapped, case)
+
+
+@pytest.mark.parametrize("case", [SWAPPED[0], SWAPPED[3], SWAPPED[5], SWAPPED[7]], ids=_id)
+def test_layer_call_with_operands_exchanged(pkg, swapped, case):
+    xs, fs, stride, _, padding = case
+    table = pkg.ops.TruthTable(pkg.synth.table_noisy(5))
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(11)
+    x = torch.randn(xs, device="cuda:0", generator=gen)
+    f = torch.randn((fs[0], fs[1], xs[3], fs[2]), device="cuda:0", generator=gen)
+    bias = torch.linspace(-1.0, 1.0, fs[2], device="cuda:0")
+    layer = pkg.ops.FakeApproxConv2D((stride, stride), table, padding, activation="relu")
+    got = layer(x, f, bias)
+    swapped.set_preexpand(-1)
+    try:
+        want = layer(x, f, bias)
+    finally:
+        swapped.set_preexpand(0)
+    assert torch.equal(got, want)
+
+
 def test_every_tile_height_is_covered(own_rows):
     assert {_plan(own_rows, c)["units_per_wavefront"] for c in CASES} >= {2, 3, 4, 6, 8, 10, 12, 13, 14, 16, 18, 20}
 
 
-def test_codes_entry_point_and_integer_op(pkg, oracle, own_rows):
+@pytest.mark.parametrize("mode", [2, 3])
+def test_codes_entry_point_and_integer_op(pkg, own_rows, mode):
+    own_rows.set_matrix_rows(mode)
     xs, fs = (3, 14, 14, 48), (3, 3, 48, 40)
     rng = np.random.RandomState(5)
     x, f = rng.randint(0, 256, xs).astype(np.uint8), rng.randint(0, 256, fs).astype(np.uint8)

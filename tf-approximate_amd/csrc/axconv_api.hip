@@ -20,7 +20,8 @@ using namespace axc;
 
 struct axc_table {
     uint16_t *dev_tableT; // [257 filter code][256 input code]; row 256 is zero
-    uint16_t *dev_tableF; // behind it in the same allocation: the same with the top bit of every byte flipped
+    uint16_t *dev_tableF; // behind it in the same allocation: the same with the top bit of every byte flipped,
+    uint16_t *dev_tableS; // and [257 input code][256 filter code], flipped too
     int device;
 };
 
@@ -443,7 +444,8 @@ std::atomic<int> g_px_mode{[] {
     return (v == 1 || v == -1) ? v : 0;
 }()};
 // Rows of lutgemm_mx_kernel: 0 = the planner decides, 1 = only pre-expanded ones (layers that they do not suit run the other
-// kernels), 2 = its own wherever it can make them.  Set by axc_set_matrix_rows.
+// kernels), 2 = its own wherever it can make them, 3 = with its operands exchanged wherever it can.  Set by
+// axc_set_matrix_rows.
 std::atomic<int> g_mx_rows{0};
 constexpr size_t kPxMaxBytes = (size_t)2 << 30;     // most memory a layer's pre-expanded rows may take
 // Rows up to this size stay in the memory-side cache between the launch that writes them and the one that reads
@@ -605,8 +607,12 @@ MxDiv mx_div(uint32_t d)
 //   a tile    1.3 + 0.70 U up to U = 6, then 0.42 a unit: geometry, the sums' start values, the outputs, stored in 32-byte
 //             pieces; rows of its own once a launch 1.0 + 0.33 U more (a first fill that waits for codes, then for entries)
 // K splits and the rows cost what they cost the other kernels (compute_plan).
-MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, bool one_load, bool expand, int cus,
-                       double clock_hz)
+// Four loads a few bytes apart (the flat layout's) are cheaper than four of a quad plane's: 1.3 + 0.155 U (7x7/2 3->64
+// @224x224x64, U = 20: 4.1).
+enum class MxLoads { kOne, kFour, kFourClose };
+// own_pass: sums go through memory and a pass of their own without a K split too.
+MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, MxLoads loads, bool expand, bool own_pass,
+                       int cus, double clock_hz)
 {
     MxPlan best{};
     double best_cost = 1e300;
@@ -646,7 +652,9 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, b
             const int64_t rows = (total_units + upt - 1) / upt;
             const int64_t tiles = rows * n_col * ks, rounds = (tiles + cus - 1) / cus;
             const double u = units;
+            const bool one_load = loads == MxLoads::kOne;
             const double fill = expand ? (one_load ? std::max(1.28 + 0.09 * u, 0.87 + 0.131 * u)
+                                          : loads == MxLoads::kFourClose ? 1.3 + 0.155 * u
                                                    : std::max(1.38 + 0.135 * u, 0.83 + 0.236 * u))
                                        : (one_load ? std::max(1.05 + 0.03 * u, 0.30 + 0.138 * u)
                                                    : std::max(1.3, 0.35 + 0.243 * u));
@@ -654,7 +662,7 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, b
             double us = std::max((double)rounds * (fps * fill + tile), rows_bytes / 3e6);
             if (expand)
                 us += 1.0 + 0.33 * u;
-            if (ks > 1)
+            if (ks > 1 || own_pass)
                 us += (expand ? 4.5 : 7.1) + (double)(ks + 1) * (double)outputs * 4.0 * 1.46e-7;
             const double cost = (us + rows_us) * 1e-6 * clock_hz;
             if (cost < best_cost) {
@@ -675,20 +683,19 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, b
     return best;
 }
 
-MxPlan make_mx_plan(const ConvGeom &g, bool one_load, bool expand, int cus)
+MxPlan make_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, MxLoads loads, bool expand, bool own_pass, int cus)
 {
-    typedef std::tuple<int64_t, int, int64_t, int64_t, bool, bool, int> Key;
+    typedef std::tuple<int64_t, int, int64_t, int64_t, MxLoads, bool, bool, int> Key;
     static std::mutex mu;
     static std::map<Key, MxPlan> cache;
-    const int64_t quads = (int64_t)g.KH * g.KW * g.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
-    const Key key{quads, g.Co, groups, g.M * g.Co, one_load, expand, cus};
+    const Key key{quads, co, groups, outputs, loads, expand, own_pass, cus};
     {
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end())
             return it->second;
     }
-    const MxPlan plan = compute_mx_plan(quads, g.Co, groups, g.M * g.Co, one_load, expand, cus, device_clock_hz());
+    const MxPlan plan = compute_mx_plan(quads, co, groups, outputs, loads, expand, own_pass, cus, device_clock_hz());
     std::lock_guard<std::mutex> lock(mu);
     if (cache.size() >= 4096)
         cache.clear();
@@ -731,10 +738,13 @@ struct DenseWorkspace {
 DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, const MxPlan *mx, const XqLayout &lay,
                                size_t sub_bytes, int flat_row_bytes)
 {
+    const bool swap = mx && mx->swap;
+    const SwapPack sp = swap_pack_of(g);
     DenseWorkspace w;
     size_t off = 0;
     w.sub_off = off; off += align_up(sub_bytes);
-    w.xq_off = off; off += align_up(xq_bytes_of(g, lay, flat_row_bytes));   // + the zero-point row(s)
+    w.xq_off = off;
+    off += align_up(swap ? (size_t)sp.quads * sp.pitch * 4 + 16 : xq_bytes_of(g, lay, flat_row_bytes));   // + the zero-point row(s)
     w.psum_off = off; off += align_up((size_t)g.M * 4); // patch sums: one float per output pixel
     w.wq_off = off;
     off += align_up(!mx ? (size_t)plan.n_col_tiles * plan.fills * 64 * 2
@@ -744,7 +754,9 @@ DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, const M
     off += align_up((size_t)4 * kMinMaxBlocks * sizeof(float)) + align_up(sizeof(LayerQuant));
     w.part_off = off;   // int32 partial sums of the K splits
     const int k_splits = mx ? mx->k_splits : plan.k_splits;
-    if (k_splits > 1)
+    if (swap)           // always: they are turned on their way to the output
+        off += align_up((size_t)k_splits * (size_t)g.Co * (size_t)((g.M + 3) & ~(int64_t)3) * 4);
+    else if (k_splits > 1)
         off += align_up((size_t)k_splits * (size_t)g.M * g.Co * 4);
     w.total_no_px = off;
     w.px_off = off;
@@ -779,6 +791,21 @@ struct PreparedDense {
 // same on one image 235 / 61 / 68.  Own rows want few pixels for many weights, where writing 512 bytes per weight and reading
 // them back outweighs making them anew in every tile.  Over the layers of ResNet-50 at batch 64, 9 and 1 and of 240 random
 // layers, each timed in the three forms, the choice is 1.2, 1.2, 0.4 and 2 % above the fastest of the three.
+// The same kernel with its operands exchanged (SwapPack), for layers with fewer output pixels than columns; units = 0: not
+// for this layer.
+MxPlan prepare_swap(const ConvGeom &g)
+{
+    const SwapPack sp = swap_pack_of(g);
+    const int64_t xq_bytes = (int64_t)sp.quads * sp.pitch * 4, wq_bytes = (int64_t)sp.tiles * sp.fills * kMxCodeBytes;
+    if (g.M > 65536 || xq_bytes >= (int64_t)1 << 30 || wq_bytes >= (int64_t)1 << 30)   // offsets in 31 bits
+        return MxPlan{};
+    MxPlan plan = make_mx_plan(sp.quads, (int)((g.M + 3) & ~(int64_t)3), sp.pitch / 4, g.M * g.Co, MxLoads::kOne, true, true, device_cus());
+    plan.swap = 1;
+    // both operands packed: two bytes per filter element of every pixel, a byte per weight
+    plan.cost += (float)(((double)wq_bytes / 2.0e6 + (double)xq_bytes / 4.0e6) * 1e-6 * device_clock_hz());
+    return plan;
+}
+
 void prepare_mx(PreparedDense *pd, bool allow_rows)
 {
     const ConvGeom &g = pd->g;
@@ -794,9 +821,11 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
     const int64_t pitch = (int64_t)g.sw * (pd->flat_row_bytes ? g.C : 4);
     if (3 * pitch > 65536)
         return;
-    ConvGeom gq = pd->gk;
-    gq.OW = g.OW;
-    const MxPlan own = make_mx_plan(gq, pitch == 4, true, device_cus()), rows = make_mx_plan(gq, pitch == 4, false, device_cus());
+    const int64_t quads = (int64_t)pd->gk.KH * pd->gk.KW * pd->gk.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
+    const MxLoads loads = pitch == 4 ? MxLoads::kOne : pd->flat_row_bytes && pitch <= 16 ? MxLoads::kFourClose : MxLoads::kFour;
+    const MxPlan own = make_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, true, false, device_cus());
+    const MxPlan rows = make_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, false, false, device_cus());
+    MxPlan swap = prepare_swap(g);
     const double us = 1e-6 * device_clock_hz();
     // Rows beyond some 20 MB for few pixels take 0.19 to 0.23 us a MB of pre-pass where the plan says 0.143 (pre-pass without
     // and with them, us: 5x5 448->48 @28x28x5, 275 MB, 65 / 129; 3x3 864->80 @14x14x41, 320 MB, 113 / 178; 5x5 64->776
@@ -809,6 +838,11 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
                         (int64_t)own.n_col_tiles * own.fills * kMxCodeBytes < ((int64_t)1 << 31);
     const int mode = g_mx_rows.load(std::memory_order_relaxed);
     bool expand = own_ok;
+    if (mode == 3 && swap.units) {
+        pd->mx = true;
+        pd->mxp = swap;
+        return;
+    }
     if (mode == 1) {
         if (!rows_ok || (pd->plan.px ? rows.cost > pd->plan.cost : rows.cost + slow_rows > pd->plan.cost * 0.98))
             return;
@@ -817,7 +851,8 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
         // What the plan of pre-expanded rows leaves out: a K split is a little cheaper, and under short chains of patch sums
         // the first 10 MB of rows delay the launch that carries them (pre-pass without and with rows, us: 1x1 64->256
         // @56x56x9, 8 MB, 9.0 / 14.9; 1x1 128->512 @28x28x9, 34 MB, 8.5 / 23.4; but 3x3 64->64 @8x8x128, 19 MB, 12.0 / 14.3).
-        const double rows_cost = rows.cost + slow_rows + (1.5 + (g.K <= 256 ? 0.35e-6 : 0.0) * std::min(rows_bytes, 10e6) -
+        // (and loads a few bytes apart are cheaper than planned)
+        const double rows_cost = rows.cost * (loads == MxLoads::kFourClose ? 0.85 : 1.0) + slow_rows + (1.5 + (g.K <= 256 ? 0.35e-6 : 0.0) * std::min(rows_bytes, 10e6) -
                                                           (rows.k_splits > 1 ? 2.6 : 0.0)) * us;
         expand = own_ok && (!rows_ok || own.cost < rows_cost);
         // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), and lower
@@ -826,6 +861,12 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
         // 11->170 @220x220x25, 823 MB, 1924, 961).
         const double other = std::max(pd->plan.cost * (pd->plan.px ? 1.12 : 1.06) + 5.0 * us,
                                       (double)g.M * g.Co * 4.0 / ((g.Co & 3) ? 0.65e6 : 2.2e6) * us);
+        const double best = std::min(expand ? (double)own.cost : rows_ok ? rows_cost : 1e30, other);
+        if (swap.units && swap.cost < best) {
+            pd->mx = true;
+            pd->mxp = swap;
+            return;
+        }
         if ((expand ? own.cost : rows_cost) > other)
             return;
     }
@@ -1042,20 +1083,34 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     }
     const bool flat = pd.flat_row_bytes > 0;
     const ConvGeom &gk = pd.gk;   // the layer as the LUT-GEMM kernels and the filter packing see it
+    const bool swap = mx && mx->swap;
     bool quantized_by_patch_sums = false, filter_done = false, px_done = false;
     uint16_t *const px_rows = use_px ? reinterpret_cast<uint16_t *>(ws + pd.ws.px_off) : nullptr;
     if (out_f && !codes_mode) {
         // carries the filter pre-pass, and with it the pre-expanded rows, along when it can
         ProfScope ps(flat ? "patch_sums_flat" : "patch_sums", stream);
-        const FilterJob job = {filter, filter_codes, &pd.plan, tq_f, wq, fsum, table->dev_tableT, px_rows, mx};
-        if (flat)   // the patch sums write the flat layout where they hold the rows anyway, else the pass below does
+        const FilterJob job = {filter, filter_codes, &pd.plan, tq_f, wq, fsum, table->dev_tableT, px_rows, mx, xq};
+        if (swap)   // the launch packs both operands, unless it is one that takes no filter work along
+            AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, plain_layout(g), nullptr, nullptr, &job, &filter_done));
+        else if (flat)   // the patch sums write the flat layout where they hold the rows anyway, else the pass below does
             AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, pd.lay, xq, &quantized_by_patch_sums, nullptr,
                                       nullptr, pd.flat_row_bytes));
         else
             AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, pd.lay, xq, &quantized_by_patch_sums, &job,
                                       &filter_done, 0, &px_done));
     }
-    if (flat && !quantized_by_patch_sums) {
+    if (swap) {
+        if (!filter_done && out_f && !codes_mode) {
+            ProfScope ps("filter_pack", stream);   // the filter's sums
+            AXC_HIP(launch_filter_pack(filter, filter_codes, g, pd.plan, mx, tq_f, lq_dev, wq, fsum, stream));
+        }
+        if (!filter_done) {
+            ProfScope ps("swap_pack", stream);
+            AXC_HIP(launch_swap_pack(input, codes_mode ? input_codes : nullptr, codes_mode ? nullptr : filter, filter_codes, g,
+                                     tq_in, tq_f, lq_dev, xq, wq, stream));
+        }
+        filter_done = true;
+    } else if (flat && !quantized_by_patch_sums) {
         ProfScope ps("quantize_flat_rows", stream);
         AXC_HIP(launch_quantize_flat_rows(input, codes_mode ? input_codes : nullptr, g, pd.lay, g.pw, pd.flat_row_bytes, tq_in,
                                           lq_dev, reinterpret_cast<uint8_t *>(xq), stream));
@@ -1127,6 +1182,59 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         }
         p.px_rows = px_rows;
         p.px_bytes = (uint32_t)pd.ws.px_bytes;
+    }
+    if (swap) {
+        const SwapPack sp = swap_pack_of(g);
+        MxParams m = {};
+        m.plan = *mx;
+        m.xq = xq;
+        m.xq_bytes = (uint32_t)((size_t)sp.quads * sp.pitch * 4 + 16);
+        m.wq = wq;
+        m.wq_bytes = (uint32_t)((size_t)sp.tiles * sp.fills * kMxCodeBytes);
+        m.tableF = table->dev_tableS;
+        const int m_pitch = (int)((g.M + 3) & ~(int64_t)3);
+        int32_t *const part = reinterpret_cast<int32_t *>(ws + pd.ws.part_off);
+        m.out_i = part;
+        m.M = g.Co;
+        m.Co = m_pitch;
+        m.oh = 1;
+        m.ow = g.Co;
+        m.groups_per_row = sp.pitch / 4;
+        m.linear = (g.Co & 3) == 0;
+        m.div_groups = mx_div((uint32_t)m.groups_per_row);
+        m.div_oh = mx_div(1u);
+        m.div_c4 = mx_div((uint32_t)sp.quads);
+        m.div_kw = mx_div(1u);
+        m.pitch = 4;
+        m.group_step = 16;
+        m.quad_step = (uint32_t)sp.pitch * 4u;
+        // one tap, one row, one image: what lies behind them lies behind the input
+        m.img_step = m.orow_step = m.kh_step = m.kw_step = (uint32_t)sp.quads * m.quad_step;
+        m.c4 = sp.quads;
+        m.kw = 1;
+        m.dq = kMxFillQuads;
+        m.doff = (uint32_t)kMxFillQuads * m.quad_step;
+        const uint32_t step = kMxWaves * 16u;
+        m.step_groups = step % (uint32_t)m.groups_per_row;
+        m.step_rows = 0;   // (of one row: whole rows are images)
+        m.step_bytes = step / (uint32_t)m.groups_per_row * m.img_step + m.step_groups * m.group_step;
+        m.carry_row = m.orow_step - (uint32_t)m.groups_per_row * m.group_step;
+        m.spin_limit = p.spin_limit;
+        m.wait_error = p.wait_error;
+        {
+            ProfScope ps("lutgemm_expand", stream, "lutgemm_mx");
+            AXC_HIP(launch_dense_mx_expand(m, stream));
+        }
+        {
+            ProfScope ps("splitk_epilogue", stream);
+            p.g = g;
+            AXC_HIP(launch_swap_epilogue(p, part, mx->k_splits, m_pitch, out_f, out_i, stream));
+        }
+        if (tf1_offset_filter) {
+            ProfScope ps("axconv_correction", stream);
+            AXC_HIP(launch_axconv_correction(g, pixel_term, column_term, out_i, stream));
+        }
+        return AXC_OK;
     }
     if (mx) {
         MxParams m = {};
@@ -1392,20 +1500,23 @@ int axc_table_create(const uint16_t *host_table, axc_table **out)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
     // transpose to weight-code major: tableT[b][a] = T[(a << 8) | b]
     const size_t entries = (size_t)kTableRows * 256;
-    std::vector<uint16_t> t(2 * entries, 0); // row 256 stays zero: the null weight's row
+    std::vector<uint16_t> t(3 * entries, 0); // row 256 stays zero: the null weight's row
     for (int a = 0; a < 256; ++a)
         for (int b = 0; b < 256; ++b)
             t[(size_t)b * 256 + a] = host_table[(size_t)a * 256 + b];
-    for (size_t i = 0; i < entries; ++i)
+    for (size_t i = 0; i < entries; ++i) {
         t[entries + i] = t[i] ^ 0x8080u;
+        t[2 * entries + i] = (i < 65536 ? host_table[i] : 0u) ^ 0x8080u;
+    }
     axc_table *tab = new axc_table;
     tab->dev_tableT = nullptr;
     hipError_t e = hipGetDevice(&tab->device);
     if (e == hipSuccess)
-        e = hipMalloc(reinterpret_cast<void **>(&tab->dev_tableT), 2 * (size_t)kTableAllocBytes);
+        e = hipMalloc(reinterpret_cast<void **>(&tab->dev_tableT), 3 * (size_t)kTableAllocBytes);
     if (e == hipSuccess)
-        e = hipMemcpy(tab->dev_tableT, t.data(), 2 * (size_t)kTableAllocBytes, hipMemcpyHostToDevice);
+        e = hipMemcpy(tab->dev_tableT, t.data(), 3 * (size_t)kTableAllocBytes, hipMemcpyHostToDevice);
     tab->dev_tableF = tab->dev_tableT + entries;
+    tab->dev_tableS = tab->dev_tableF + entries;
     if (e != hipSuccess) {
         if (tab->dev_tableT)
             (void)hipFree(tab->dev_tableT);
@@ -1651,7 +1762,7 @@ int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8])
     if (rc != AXC_OK)
         return rc;
     const MxPlan &m = pd.mxp;
-    const int32_t v[8] = {pd.mx ? 1 + m.expand : 0, m.units, m.units_per_tile, m.n_row_tiles, m.n_col_tiles, m.k_splits, m.grid,
+    const int32_t v[8] = {pd.mx ? 1 + m.expand + m.swap : 0, m.units, m.units_per_tile, m.n_row_tiles, m.n_col_tiles, m.k_splits, m.grid,
                           m.k_splits > 1 ? m.fills_per_split : m.fills};
     for (int i = 0; i < 8; ++i)
         plan[i] = pd.mx ? v[i] : 0;
@@ -1682,8 +1793,8 @@ int axc_set_preexpand(int mode)
 
 int axc_set_matrix_rows(int mode)
 {
-    if (mode < 0 || mode > 2)
-        return fail(AXC_INVALID_ARGUMENT, "matrix rows mode must be 0 (planner's choice), 1 (pre-expanded only) or 2 (the kernel's own wherever possible)");
+    if (mode < 0 || mode > 3)
+        return fail(AXC_INVALID_ARGUMENT, "matrix rows mode must be 0 (planner's choice), 1 (pre-expanded only), 2 (the kernel's own wherever possible) or 3 (the same with operands exchanged)");
     g_mx_rows.store(mode, std::memory_order_relaxed);
     return AXC_OK;
 }

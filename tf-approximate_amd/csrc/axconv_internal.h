@@ -141,6 +141,7 @@ struct MxPlan {
     int k_splits, fills_per_split;
     int grid;
     int expand;            // 1: the kernel makes its rows itself, out of packed filter codes and the table
+    int swap;              // 1 (with expand): operands exchanged, see SwapPack
     float cost;            // cycles the planner's model expects
 };
 
@@ -153,6 +154,23 @@ struct XqLayout {
     int Hp, Wp, row0, col0;
     __host__ __device__ int tail_rows() const { return row0 == 0 ? 1 : row0 + (col0 > 0 ? 1 : 0); }
 };
+
+// Few output pixels under many weights: lutgemm_mx_kernel with its operands exchanged.  A fill costs what it costs
+// however few pixels look it up, so the operand with the fewer rows makes the fills: output pixels stand where columns
+// stood (8 to a tile, the codes of their patches packed as filter codes are), and the filter's columns where pixels stood,
+// an image of one row, Co pixels and K channels.  The table is taken the other way round, sums come out as [Co][M].
+struct SwapPack {
+    int K, quads, fills;   // filter elements, ceil(K / 4), ceil(quads / 4)
+    int cols, pitch;       // Co, and Co rounded up to fours
+    int tiles;             // ceil(M / 8)
+    __host__ __device__ int64_t filter_units() const { return (int64_t)quads * (pitch / 4); }
+    __host__ __device__ int64_t units() const { return filter_units() + (int64_t)tiles * fills * 16; }
+};
+inline SwapPack swap_pack_of(const ConvGeom &g)
+{
+    const int quads = (g.K + 3) / 4;
+    return {g.K, quads, (quads + 3) / 4, g.Co, (g.Co + 3) & ~3, (int)((g.M + 7) / 8)};
+}
 
 struct MxDiv {             // division by a constant for 31-bit numbers: mulhi(n, mul) >> shift; mul = 0: n itself
     uint32_t mul, shift;
@@ -275,7 +293,8 @@ struct FilterJob {
     float *fsum;
     const uint16_t *tableT;   // with px_rows: the transposed table the pre-expanded rows are built from
     uint16_t *px_rows;        // nullptr: the layer does not run out of pre-expanded rows
-    const MxPlan *mx;         // not null: the layer runs lutgemm_mx_kernel, whose rows those are; no packed filter
+    const MxPlan *mx;         // not null: the layer runs lutgemm_mx_kernel, whose rows those are
+    uint32_t *swap_xq;        // mx->swap: the filter's codes as that kernel's input (wq: those of the patches)
 };
 // xq_fused / fused: the launch may also quantize the input into xq (then *fused is set);
 // filter_job / filter_done: it may also do the filter pre-pass (then *filter_done is set), and with it build the
@@ -315,6 +334,13 @@ bool px_free_running(const DensePlan &plan, int taps);   // the plan runs lutgem
 hipError_t launch_mx_expand_rows(const float *filter, const uint8_t *filter_codes, const ConvGeom &g, const MxPlan &plan,
                                  const TensorQuant &tq, const LayerQuant *lq_dev, const uint16_t *tableT, uint16_t *rows,
                                  hipStream_t stream);
+// mx->swap, where no other launch has done it: both operands packed, from floats or codes; and the pass behind the LUT-GEMM,
+// which adds the K splits' [Co][M] sums (rows of m_pitch), turns them and applies the op's epilogue
+hipError_t launch_swap_pack(const float *x, const uint8_t *codes, const float *filter, const uint8_t *filter_codes,
+                            const ConvGeom &g, const TensorQuant &tq_in, const TensorQuant &tq_f, const LayerQuant *lq_dev,
+                            uint32_t *xq, uint16_t *wq, hipStream_t stream);
+hipError_t launch_swap_epilogue(const DenseParams &p, const int32_t *partials, int k_splits, int m_pitch, float *out_f,
+                                int32_t *out_i, hipStream_t stream);
 hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream);          // out of pre-expanded rows
 hipError_t launch_dense_mx_expand(const MxParams &p, hipStream_t stream);   // plan.expand
 hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials, float *out_f, int32_t *out_i,

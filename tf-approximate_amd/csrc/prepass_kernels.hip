@@ -292,6 +292,11 @@ struct MxForm {
 struct MxCodesForm : MxForm {
     static constexpr bool kMxCodes = true;
 };
+// ... and with the operands exchanged, both packed in that launch (swap_pack_unit).
+struct SwapForm : MxForm {
+    SwapPack pack;
+    uint32_t *xq;
+};
 
 // The filter pre-pass of a layer is independent of its input pre-pass: as two launches they would run one after
 // the other, so the launch below carries both: the filter work of filter_prep_kernel in workgroups of its own
@@ -329,11 +334,20 @@ __device__ __forceinline__ void mx_pack_unit(const int64_t i, const int fills, c
                                              const uint8_t *__restrict__ filter_codes, int taps, int C, int C4, int Co,
                                              const TensorQuant &qf, uint16_t *__restrict__ wq);
 
-// Element (or, for codes in lutgemm_mx_kernel's form, unit of eight elements) i of the filter's packing.
+__device__ __forceinline__ void swap_pack_unit(const int64_t i, const SwapPack &sp, const float *__restrict__ x,
+                                               const uint8_t *__restrict__ codes, const float *__restrict__ filter,
+                                               const uint8_t *__restrict__ filter_codes, const ConvGeom &g,
+                                               const TensorQuant &qi, const TensorQuant &qf, uint32_t *__restrict__ xq,
+                                               uint16_t *__restrict__ wq);
+
+// Element (or, for codes in lutgemm_mx_kernel's form, unit of eight elements or so) i of the filter's packing.
 template <class Form>
-__device__ __forceinline__ void pack_filter(const int64_t i, const Form &form, const FilterWork &fw, const TensorQuant &qf)
+__device__ __forceinline__ void pack_filter(const int64_t i, const Form &form, const FilterWork &fw, const float *x,
+                                            const ConvGeom &g, const TensorQuant &qi, const TensorQuant &qf)
 {
-    if constexpr (Form::kMxCodes)
+    if constexpr (std::is_same<Form, SwapForm>::value)
+        swap_pack_unit(i, form.pack, x, nullptr, fw.filter, nullptr, g, qi, qf, form.xq, fw.wq);
+    else if constexpr (Form::kMxCodes)
         mx_pack_unit(i, form.mx_fills(), fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, qf, fw.wq);
     else
         filter_pack_element(i, fw.filter, fw.filter_codes, fw.taps, fw.C, fw.C4, fw.Co, fw.nt, fw.n_col_tiles, qf, fw.wq);
@@ -534,7 +548,7 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
             const int64_t last = first + share < fw.pack_total ? first + share : fw.pack_total;
             const TensorQuant qf = lq_dev ? lq_dev->flt : fw.tq;
             for (int64_t i = first + widx; i < last; i += workers)
-                pack_filter(i, form, fw, qf);
+                pack_filter(i, form, fw, x, g, qt, qf);
         }
         return;
     }
@@ -879,6 +893,92 @@ __device__ __forceinline__ void mx_pack_unit(const int64_t i, const int fills, c
     }
     *reinterpret_cast<uint4 *>(wq + (((int64_t)ct * fills * 16 + e) * kMxCols)) =
         make_uint4(code[0] | code[1] << 16, code[2] | code[3] << 16, code[4] | code[5] << 16, code[6] | code[7] << 16);
+}
+
+// Both operands of a layer that runs with them exchanged (SwapPack).  The first units are the filter's: four columns of a
+// quad of the K order, as the kernel's quantized input, [quad][column] dwords of four row-permuted codes.  The others are the
+// patches': a filter element of eight output pixels, the input's code under it - the zero point's outside the image, the
+// null weight beyond K or M -, [tile of 8 pixels][filter element][pixel]; neighbouring threads read neighbouring channels.
+__device__ __forceinline__ void swap_pack_unit(const int64_t i, const SwapPack &sp, const float *__restrict__ x,
+                                               const uint8_t *__restrict__ codes, const float *__restrict__ filter,
+                                               const uint8_t *__restrict__ filter_codes, const ConvGeom &g,
+                                               const TensorQuant &qi, const TensorQuant &qf, uint32_t *__restrict__ xq,
+                                               uint16_t *__restrict__ wq)
+{
+    const int64_t nf = sp.filter_units();
+    if (i < nf) {
+        const int per_quad = sp.pitch >> 2;
+        const int quad = (int)(i / per_quad), n0 = (int)(i - (int64_t)quad * per_quad) * 4;
+        uint32_t d[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int k = quad * 4 + r < sp.K ? quad * 4 + r : sp.K - 1;
+            const int64_t at = (int64_t)k * sp.cols + n0;
+            uint32_t c[4];
+            if (filter_codes) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    c[j] = filter_codes[at + (n0 + j < sp.cols ? j : 0)];
+            } else {
+                float4 v;
+                if (n0 + 4 <= sp.cols) {
+                    const f4_any f = *reinterpret_cast<const f4_any *>(filter + at);
+                    v = make_float4(f[0], f[1], f[2], f[3]);
+                } else {
+                    v = make_float4(filter[at], filter[at + (n0 + 1 < sp.cols ? 1 : 0)], filter[at + (n0 + 2 < sp.cols ? 2 : 0)], 0.0f);
+                }
+                v = fake_quant_value4(v, qf);
+                c[0] = quantize_code(v.x, qf.offset, qf.inv_scale);
+                c[1] = quantize_code(v.y, qf.offset, qf.inv_scale);
+                c[2] = quantize_code(v.z, qf.offset, qf.inv_scale);
+                c[3] = quantize_code(v.w, qf.offset, qf.inv_scale);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                d[j] |= phys_row(c[j]) << (8 * r);
+        }
+        *reinterpret_cast<uint4 *>(xq + (int64_t)quad * sp.pitch + n0) = make_uint4(d[0], d[1], d[2], d[3]);
+        return;
+    }
+    const int64_t u = i - nf;
+    const int per_tile = sp.fills * 16, tile = (int)(u / per_tile), k = (int)(u - (int64_t)tile * per_tile);
+    if (tile >= sp.tiles)
+        return;
+    uint32_t c[8];
+    const int tap = k / g.C, ch = k - tap * g.C, kh = tap / g.KW, kw = tap - kh * g.KW;
+    const uint32_t zp = qi.zp4 & 255u, zero = ((zp & 63u) << 2) | (zp >> 6);   // phys_row's inverse
+    const int64_t m0 = (int64_t)tile * 8, row = m0 / g.OW;
+    int ow = (int)(m0 - row * g.OW), n = (int)(row / g.OH), oh = (int)(row - (int64_t)n * g.OH);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int ih = oh * g.sh - g.ph + kh * g.dh, iw = ow * g.sw - g.pw + kw * g.dw;
+        const bool there = m0 + j < g.M && k < sp.K, inside = there && (unsigned)ih < (unsigned)g.H && (unsigned)iw < (unsigned)g.W;
+        const int64_t at = inside ? (((int64_t)n * g.H + ih) * g.W + iw) * g.C + ch : 0;
+        if (codes)
+            c[j] = codes[at];
+        else
+            c[j] = quantize_code(fake_quant_value(x[at], qi), qi.offset, qi.inv_scale);
+        c[j] = inside ? c[j] : there ? zero : (uint32_t)kNullWeight;
+        if (++ow == g.OW) {
+            ow = 0;
+            if (++oh == g.OH) {
+                oh = 0;
+                ++n;
+            }
+        }
+    }
+    *reinterpret_cast<uint4 *>(wq + u * 8) = make_uint4(c[0] | c[1] << 16, c[2] | c[3] << 16, c[4] | c[5] << 16, c[6] | c[7] << 16);
+}
+
+__global__ void __launch_bounds__(256) swap_pack_kernel(const float *__restrict__ x, const uint8_t *__restrict__ codes,
+                                                        const float *__restrict__ filter,
+                                                        const uint8_t *__restrict__ filter_codes, const ConvGeom g,
+                                                        const SwapPack sp, const TensorQuant tq_in, const TensorQuant tq_f,
+                                                        const LayerQuant *__restrict__ lq_dev, uint32_t *__restrict__ xq,
+                                                        uint16_t *__restrict__ wq)
+{
+    swap_pack_unit((int64_t)blockIdx.x * 256 + threadIdx.x, sp, x, codes, filter, filter_codes, g, lq_dev ? lq_dev->in : tq_in,
+                   lq_dev ? lq_dev->flt : tq_f, xq, wq);
 }
 
 // Filter sums (tf2/src/approx_nn_conv_kernels.cpp:300-306): one sequential sum per output column, rows (h, w, c)
@@ -1314,8 +1414,8 @@ __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x
 // The filter work of a patch-sum launch: true if this workgroup is one of those that do it (and has done it), else
 // *bid is its index among the patch-sum workgroups.
 template <class Form>
-__device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const Form &form,
-                                                  const LayerQuant *__restrict__ lq_dev, int *bid)
+__device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const Form &form, const float *x, const ConvGeom &g,
+                                                  const TensorQuant &tq, const LayerQuant *__restrict__ lq_dev, int *bid)
 {
     const int mx_fills = form.mx_fills();
     const int b = (int)blockIdx.x;
@@ -1336,7 +1436,7 @@ __device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const Fo
     const int pb = *bid - fw.work_blocks;
     if (pb < fw.pack_blocks || fw.expand_blocks == 0) {
         const int64_t i = (int64_t)pb * blockDim.x + threadIdx.x;
-        pack_filter(i, form, fw, q);
+        pack_filter(i, form, fw, x, g, lq_dev ? lq_dev->in : tq, q);
         return true;
     }
     // pre-expanded rows: blockDim.x / 4 activation codes of a pair of fills per workgroup
@@ -1361,7 +1461,7 @@ __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *
 {
     const XqLayout lay = form.layout(g);
     int bid;
-    if (filter_work_block(fw, form, lq_dev, &bid))
+    if (filter_work_block(fw, form, x, g, tq, lq_dev, &bid))
         return;
     patch_sums_rows_body<true, ANY>(x, g, rb, in_rows, wseg, tq, lq_dev, psum, xq, lay, bid, fw.work_blocks, nthreads, fw, form);
 }
@@ -1375,7 +1475,7 @@ __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__re
 {
     const XqLayout lay = form.layout(g);
     int bid;
-    if (filter_work_block(fw, form, lq_dev, &bid))
+    if (filter_work_block(fw, form, x, g, tq, lq_dev, &bid))
         return;
     if (!ANY && rb < 0) { // 1x1, stride 1, many channels, few pixels
         if (in_rows == 8)
@@ -1427,6 +1527,8 @@ static int64_t pack_items(const DensePlan &plan, const MxPlan *mx)
 {
     if (!mx)
         return (int64_t)plan.n_col_tiles * plan.fills * 64;
+    if (mx->swap)
+        return 0;   // (its own: SwapPack)
     return mx->expand ? (int64_t)mx->n_col_tiles * mx->fills * 16 : 0;
 }
 
@@ -1749,6 +1851,83 @@ hipError_t launch_fill_u32(uint32_t *dst, int64_t n, uint32_t value, hipStream_t
     return hipGetLastError();
 }
 
+hipError_t launch_swap_pack(const float *x, const uint8_t *codes, const float *filter, const uint8_t *filter_codes,
+                            const ConvGeom &g, const TensorQuant &tq_in, const TensorQuant &tq_f, const LayerQuant *lq_dev,
+                            uint32_t *xq, uint16_t *wq, hipStream_t stream)
+{
+    const SwapPack sp = swap_pack_of(g);
+    hipLaunchKernelGGL(swap_pack_kernel, dim3(blocks_for(sp.units(), 256)), dim3(256), 0, stream, x, codes, filter, filter_codes,
+                       g, sp, tq_in, tq_f, lq_dev, xq, wq);
+    return hipGetLastError();
+}
+
+// The op's epilogue for sums that lutgemm_mx_kernel made with its operands exchanged: [split][column][pixel], rows of
+// m_pitch (a multiple of four).  A workgroup turns 16 columns x 16 pixels; its four wavefronts add a quarter of the splits
+// each, four pixels of a column per lane, eight loads in flight (one wavefront for all 32 splits of 3x3 512->512 on one 7x7
+// image, a load at a time: 14.9 us).
+__global__ void __launch_bounds__(256) swap_epilogue_kernel(const int32_t *__restrict__ part, int ks, int64_t M, int Co,
+                                                            int m_pitch, const float *__restrict__ psum,
+                                                            const float *__restrict__ fsum, float s1xs2, float m1, float m2,
+                                                            float k_m1xm2, const LayerQuant *__restrict__ lq_dev,
+                                                            const float *__restrict__ bias, int relu,
+                                                            float *__restrict__ out_f, int32_t *__restrict__ out_i)
+{
+    __shared__ int32_t turned[4][16][17];
+    const int t = threadIdx.x, wave = t >> 6;
+    const int n0 = (int)blockIdx.y * 16;
+    const int64_t m0 = (int64_t)blockIdx.x * 16;
+    {
+        const int nl = (t >> 2) & 15, ml = (t & 3) * 4;
+        int4 a = make_int4(0, 0, 0, 0);
+        if (n0 + nl < Co && m0 + ml < m_pitch) {
+            const int64_t step = (int64_t)Co * m_pitch;
+            const int32_t *src = part + (int64_t)(n0 + nl) * m_pitch + m0 + ml + wave * step;
+#pragma unroll 8
+            for (int k = wave; k < ks; k += 4, src += 4 * step) {
+                const int4 v = *reinterpret_cast<const int4 *>(src);
+                a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
+            }
+        }
+        int32_t *const to = &turned[wave][ml][nl];
+        to[0] = a.x; to[17] = a.y; to[34] = a.z; to[51] = a.w;
+    }
+    const int ml = t >> 4, nl = t & 15, col = n0 + nl;
+    const int64_t m = m0 + ml;
+    const bool there = m < M && col < Co;
+    float ps = 0.0f, fs = 0.0f, bs = -0.0f;   // (adding -0 changes nothing)
+    if (there && out_f) {
+        ps = psum[m];
+        fs = fsum[col];
+        bs = bias ? bias[col] : -0.0f;
+    }
+    if (lq_dev) {
+        s1xs2 = lq_dev->s1xs2;
+        m1 = lq_dev->m1;
+        m2 = lq_dev->m2;
+        k_m1xm2 = lq_dev->k_m1xm2;
+    }
+    __syncthreads();
+    if (!there)
+        return;
+    const int32_t a = turned[0][ml][nl] + turned[1][ml][nl] + turned[2][ml][nl] + turned[3][ml][nl];
+    if (out_i) {
+        out_i[m * Co + col] = a;
+        return;
+    }
+    float r = __fadd_rn(__fmul_rn((float)a, s1xs2), __fmul_rn(m2, ps));
+    r = __fadd_rn(__fsub_rn(__fadd_rn(r, __fmul_rn(m1, fs)), k_m1xm2), bs);
+    out_f[m * Co + col] = relu ? fmaxf(r, 0.0f) : r;
+}
+
+hipError_t launch_swap_epilogue(const DenseParams &p, const int32_t *partials, int k_splits, int m_pitch, float *out_f,
+                                int32_t *out_i, hipStream_t stream)
+{
+    const dim3 grid((unsigned)((p.g.M + 15) / 16), (unsigned)((p.g.Co + 15) / 16));
+    hipLaunchKernelGGL(swap_epilogue_kernel, grid, dim3(256), 0, stream, partials, k_splits, p.g.M, p.g.Co, m_pitch, p.psum,
+                       p.fsum, p.s1xs2, p.m1, p.m2, p.k_m1xm2, p.lq_dev, p.bias, p.relu, out_f, out_i);
+    return hipGetLastError();
+}
+
 // Reduction of the K splits' int32 partial sums (exact, so the order does not matter) followed by the op's
 // epilogue (approx_nn_conv_kernels.cpp:250-253), four consecutive columns per thread when Co % 4 == 0.
 template <int V>
@@ -2043,7 +2222,7 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             if (filter_job && filter_done) {
                 const DensePlan &plan = *filter_job->plan;
                 const MxPlan *const mx = filter_job->mx;
-                const int64_t total = pack_items(plan, mx);
+                const int64_t total = mx && mx->swap ? swap_pack_of(g).units() : pack_items(plan, mx);
                 fw.filter = filter_job->filter;
                 fw.filter_codes = filter_job->filter_codes;
                 fw.taps = g.KH * g.KW;
@@ -2063,7 +2242,9 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                 // Only while each of them has a few elements to pack: under few patch-sum blocks the packing would outlast
                 // everything else (3x3 512->512 on one 7x7 image: 880 elements a thread, 505 us of a launch of 41).
                 const int64_t packers = work_blocks * (block_threads / 4) * (4 - (rb * wseg + 63) / 64);
-                if (!flat && rb * wseg <= 3 * 64 && total <= 16 * packers)
+                // (An item of lutgemm_mx_kernel's is eight elements: 3x3 256->256 on one 14x14 image 21.1 -> 18.4 us.  Where both
+                // operands are packed it is more than that: never.)
+                if (!flat && !(mx && mx->swap) && rb * wseg <= 3 * 64 && total * (mx ? 8 : 1) <= 16 * packers)
                     fw.pack_total = total;
                 fw.sum8 = (fw.sum_blocks + 7) & ~7;
                 fw.pack_blocks = fw.pack_total > 0 ? 0 : (int)blocks_for(total, block_threads);
@@ -2118,6 +2299,8 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
             };
             const bool mx_form = (filter_job && filter_job->mx) || lay.row0 || lay.col0;
             const MxForm mxf = {lay, filter_job && filter_job->mx ? filter_job->mx->fills : 0};
+            if (filter_job && filter_job->mx && filter_job->mx->swap)
+                return launch(SwapForm{mxf, swap_pack_of(g), filter_job->swap_xq});
             if (filter_job && filter_job->mx && filter_job->mx->expand)
                 return launch(MxCodesForm{mxf});
             return mx_form ? launch(mxf) : launch(PlainForm{});

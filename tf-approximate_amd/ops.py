@@ -339,7 +339,7 @@ def conv2d_matrix_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding=
     desc = make_desc(tuple(input_shape), tuple(filter_shape), list(strides), padding, (), "NHWC", list(dilations), 8)
     plan = (ctypes.c_int32 * 8)()
     _check(lib.axc_conv2d_matrix_plan(ctypes.byref(desc), plan))
-    # own_rows: 0 = reads pre-expanded rows, 1 = makes them itself in every tile
+    # own_rows: 0 = reads pre-expanded rows, 1 = makes them itself in every tile, 2 = the same with the operands exchanged
     keys = ("own_rows", "units_per_wavefront", "units_per_tile", "row_tiles", "column_tiles", "k_splits", "workgroups",
             "fills_per_split")
     return dict(zip(keys, [int(v) for v in [plan[0] - 1] + list(plan[1:])])) if plan[0] else None
@@ -357,7 +357,7 @@ def set_preexpand(mode):
 
 def set_matrix_rows(mode):
     """Rows of the kernel whose sums the matrix cores make: 0 = the planner's choice, 1 = pre-expanded ones only, 2 = made
-    by the kernel itself wherever it can."""
+    by the kernel itself wherever it can, 3 = the same with the operands exchanged."""
     _check(_lib.load().axc_set_matrix_rows(int(mode)))
 
 
