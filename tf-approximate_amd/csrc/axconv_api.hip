@@ -602,13 +602,14 @@ MxDiv mx_div(uint32_t d)
 // measured by running 3x3 layers of 18 and of 72 fills at stride 1 and 2 in every variant (U units per wavefront; stride 1
 // loads a unit's activations at once, stride 2 - pixels that are no neighbouring dwords - by four loads):
 //   a fill    of pre-expanded rows 1.10 (U = 2), 1.32 (4), 1.51 (8), 2.10 (13), 2.53 (16), 3.05 (20), 3.75 (25); four loads
-//             1.30, 1.76, 2.42, 3.52, 4.25, 5.19, 6.39; of rows the kernel makes itself 1.43, 1.59, 2.03, 2.55, 2.95, 3.46;
-//             four loads 1.65, 1.88, 2.65, 3.85, 4.60, 5.70: the stores of the rows take the LDS 0.4 us of every fill
+//             1.30, 1.76, 2.42, 3.52, 4.25, 5.19, 6.39; of rows the kernel makes itself 0.95 (U = 2), 1.98 (10), 2.29 (12),
+//             2.55 (14), 2.83 (16), 3.09 (18), four loads 2.63 (8), 3.10, 3.49, 3.96, 4.49, 4.95: the stores of the rows
+//             take the LDS 0.35 us of every fill
 //   a tile    1.3 + 0.70 U up to U = 6, then 0.42 a unit: geometry, the sums' start values, the outputs, stored in 32-byte
-//             pieces; rows of its own once a launch 1.0 + 0.33 U more (a first fill that waits for codes, then for entries)
+//             pieces; rows of its own 2.0 more once a launch (a first fill that waits for codes, then for entries)
 // K splits and the rows cost what they cost the other kernels (compute_plan).
-// Four loads a few bytes apart (the flat layout's) are cheaper than four of a quad plane's: 1.3 + 0.155 U (7x7/2 3->64
-// @224x224x64, U = 20: 4.1).
+// Four loads a few bytes apart (the flat layout's) are cheaper than four of a quad plane's: 1.0 + 0.14 U (7x7/2 3->64
+// @224x224x64, U = 20: 3.8).
 enum class MxLoads { kOne, kFour, kFourClose };
 // own_pass: sums go through memory and a pass of their own without a K split too.
 MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, MxLoads loads, bool expand, bool own_pass,
@@ -630,8 +631,7 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, M
         const int fps = (fills + ks - 1) / ks;
         if (ks > 1 && (fps < 4 || (int64_t)(ks - 1) * fps >= fills))
             continue;
-        // expanding, a tile has two fills or more: filter codes are loaded two ahead
-        if (expand ? fills - (ks - 1) * fps < 2 : ks > 16)
+        if (expand ? fills - (ks - 1) * fps < kMxMinExpandFills : ks > 16)
             continue;
         std::vector<int64_t> cands{min_tiles};
         for (int64_t rounds = 1; rounds <= 64; ++rounds)
@@ -653,15 +653,14 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, M
             const int64_t tiles = rows * n_col * ks, rounds = (tiles + cus - 1) / cus;
             const double u = units;
             const bool one_load = loads == MxLoads::kOne;
-            const double fill = expand ? (one_load ? std::max(1.28 + 0.09 * u, 0.87 + 0.131 * u)
-                                          : loads == MxLoads::kFourClose ? 1.3 + 0.155 * u
-                                                   : std::max(1.38 + 0.135 * u, 0.83 + 0.236 * u))
+            const double fill = expand ? (one_load ? std::max(0.93, 0.62 + 0.138 * u)
+                                                   : loads == MxLoads::kFourClose ? 1.0 + 0.14 * u : 0.83 + 0.229 * u)
                                        : (one_load ? std::max(1.05 + 0.03 * u, 0.30 + 0.138 * u)
                                                    : std::max(1.3, 0.35 + 0.243 * u));
             const double tile = 1.3 + 0.70 * std::min(units, 6) + 0.42 * std::max(units - 6, 0);
             double us = std::max((double)rounds * (fps * fill + tile), rows_bytes / 3e6);
             if (expand)
-                us += 1.0 + 0.33 * u;
+                us += 2.0;
             if (ks > 1 || own_pass)
                 us += (expand ? 4.5 : 7.1) + (double)(ks + 1) * (double)outputs * 4.0 * 1.46e-7;
             const double cost = (us + rows_us) * 1e-6 * clock_hz;

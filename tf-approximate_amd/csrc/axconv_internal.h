@@ -130,7 +130,8 @@ constexpr int kMxWaves = kMxThreads / 64;
 constexpr int kMxCols = 8;                     // columns per tile
 constexpr int kMxFillQuads = 4;                // channel quads (of any taps) per fill
 constexpr int kMxUnits[] = {2, 3, 4, 6, 8, 10, 13, 16, 20, 25};   // 64-pixel units per wavefront: the kernel's variants
-constexpr int kMxExpandUnits[] = {2, 3, 4, 6, 8, 10, 12, 13, 14, 16, 18, 20};   // the same where it makes its rows itself
+constexpr int kMxExpandUnits[] = {2, 3, 4, 6, 8, 10, 12, 13, 14, 16, 18};   // the same where it makes its rows itself
+constexpr int kMxMinExpandFills = 3;           // ... and the fewest fills of its tiles (it loads that far ahead)
 constexpr int kMxCodeBytes = 256;              // packed filter codes of a fill: 16 filter elements x 8 columns x uint16
 
 struct MxPlan {

@@ -32,6 +32,19 @@ when its share of a fill has arrived and 1 when it has finished reading it.  A f
 are there (whole), and its buffer refilled once all four have read it (free).  Both are looked at ahead of the point
 that needs them; a look that finds too small a count goes into a bounded loop of further looks (SPIN of them) out of
 line, and a loop that runs out leaves the assembly with FAIL set.
+
+The expanding form (emit(..., expand=True), macros MX_XFILLS_*) makes a fill's rows itself, out of the truth table:
+nothing is written to memory and read back.  A wavefront makes the rows of 64 activation codes, in two blocks of 32.
+Lane (s, c), s = bits 1-4 of the lane and c = bits 5 and 0, has the fill's filter element s: per block it loads 16
+bytes - the entries of eight activation codes - of the table rows of the element's eight filter codes, turns that
+8 x 8 square of 16-bit entries with 32 v_perm_b32 and stores eight 16-byte chunks, one per activation code.  Two
+neighbouring lanes read 32 consecutive bytes, and 16 lanes that the LDS serves together store into 16 or 8 different
+chunks.  (Lane order measured on the load, turn and store alone, 256 workgroups, us a fill: s in the low bits 1.76, its
+loads alone 1.76; c in the low bits 0.90, its stores alone 0.85; this one 0.92, stores 0.51, which leaves the LDS to the
+lookups.)  While fill f is looked up the entries of fill f + 1 are turned and stored, those of fill f + 2 loaded into the
+registers that this leaves free, and the filter codes of fill f + 3 loaded; both stay loaded from tile to tile, which makes
+three fills the shortest tile.  (With entries loaded and stored within one fill, us a fill for U = 2, 4, 8, 14: 1.43, 1.59,
+2.03, 2.69; like this 1.08, 1.25, 1.55, 2.3.)
 """
 import sys
 
@@ -39,7 +52,7 @@ UNITS = (2, 3, 4, 6, 8, 10, 13, 16, 20, 25)   # tile heights: units of 64 pixels
 VARIANTS = [(u, vec) for u in UNITS for vec in (True, False)]
 W = 8                                         # lookups in flight (a unit is a whole number of rings)
 LOADS = 16                                    # 1 KiB loads per wavefront and fill
-XUNITS = (2, 3, 4, 6, 8, 10, 12, 13, 14, 16, 18, 20)   # tile heights of the expanding form (25 leaves it no registers)
+XUNITS = (2, 3, 4, 6, 8, 10, 12, 13, 14, 16, 18)   # tile heights of the expanding form (20 and 25 leave it too few registers)
 XVARIANTS = [(u, vec) for u in XUNITS for vec in (True, False)]
 CODE_BYTES = 256                              # packed filter codes of a fill: 128 x uint16
 
@@ -69,6 +82,7 @@ class Stream:
 
     def __init__(self):
         self.lines, self.slow, self.lds_q, self.vm_q, self.count = [], [], [], [], 0
+        self.tags = {}                     # vector-memory operations that a loop carries: what they are
 
     def ins(self, text):
         self.lines.append(text)
@@ -81,12 +95,21 @@ class Stream:
         self.lds_q.append(self.count)
         return self.count
 
-    def vm(self, text):
+    def vm(self, text, tag=None):
         self.ins(text)
         self.count += 1
         self.vm_q.append(self.count)
+        self.tags[self.count] = tag
         assert len(self.vm_q) <= 63
         return self.count
+
+    def carry(self, tags):                 # the operations in flight where a loop begins, as its end leaves them
+        self.vm_q = []
+        for tag in tags:
+            self.count += 1
+            self.vm_q.append(self.count)
+            self.tags[self.count] = tag
+        return {self.tags[op]: op for op in self.vm_q}
 
     def wait_lds(self, *ops):
         ops = [op for op in ops if op in self.lds_q]
@@ -136,6 +159,18 @@ def acc_reg(units, u, j):
 
 
 def emit(units, vec, expand=False):
+    if not expand:
+        return emit_form(units, vec, expand)[0]
+    tags = []
+    for _ in range(4):                     # until the loop's end leaves in flight what its beginning assumed
+        text, end = emit_form(units, vec, expand, tags)
+        if end == tags:
+            return text
+        tags = end
+    raise ValueError(units)
+
+
+def emit_form(units, vec, expand, carried=None):
     d, slots, ring, win, end, vacc = layout(units)
     n_look, n_pair = 16 * units, 8 * units
     st = Stream()
@@ -155,9 +190,9 @@ def emit(units, vec, expand=False):
         st.ins("v_add_u32 v%d, v%d, v%d" % (V_TMP, V_BASE + u, V_KOFF))
         r = ring + 4 * slots[u]
         if vec:
-            return [st.vm("buffer_load_dwordx4 v[%d:%d], v%d, %%[xq], 0 offen" % (r, r + 3, V_TMP))]
-        return [st.vm("buffer_load_dword v%d, v%d, %%[xq], %s offen" % (r + j, V_TMP, "0" if j == 0 else "%%[p%d]" % j))
-                for j in range(4)]
+            return [st.vm("buffer_load_dwordx4 v[%d:%d], v%d, %%[xq], 0 offen" % (r, r + 3, V_TMP), ("act", u, 0))]
+        return [st.vm("buffer_load_dword v%d, v%d, %%[xq], %s offen" % (r + j, V_TMP, "0" if j == 0 else "%%[p%d]" % j),
+                      ("act", u, j)) for j in range(4)]
 
     def koff_step():         # every lane's filter position moves on by four quads: (tap column, quad) with carries
         st.ins("v_add_u32 v%d, %%[dq], v%d" % (V_Q, V_Q))
@@ -238,7 +273,7 @@ def emit(units, vec, expand=False):
 
     def row_load(i):         # entries of eight activation codes (block i / 8) of column i % 8
         b, j = divmod(i, 8)
-        return st.vm("buffer_load_dwordx4 %s, v%d, %%[erc], 0 offen offset:%d" % (quad(land, i), row + j, 64 * b))
+        return st.vm("buffer_load_dwordx4 %s, v%d, %%[erc], 0 offen offset:%d" % (quad(land, i), row + j, 64 * b), ("row", i))
 
     def chunk_store(i):      # activation code i % 8 of block i / 8: the square's column, as a row's 16 bytes
         b, e = divmod(i, 8)
@@ -263,6 +298,8 @@ def emit(units, vec, expand=False):
                     st.ins("v_mov_b32 v%d, %s" % (base, "0" if r & 1 else "v%d" % V_POLL))
     st.ins("s_mov_b32 %[fail], 0")
     need(None, "cbcur", "%[whole0]", 1)
+    if expand:               # nothing is in flight but what the loop counts itself
+        st.wait_vm(*st.vm_q)
     st.wait_vm(*acts[0])
     pending = {}
     for n in range(W):
@@ -273,6 +310,10 @@ def emit(units, vec, expand=False):
     # cbcur / cboth: LDS addresses of the counters of this fill's buffer and of the other one; whole: what the other
     # counter must reach for the next fill to be readable (0 behind the tile's last fill); free: ... for the other
     # buffer to be refilled
+    entering = {}
+    if expand:
+        entering = st.carry(carried)
+        acts = {u: [op for tag, op in entering.items() if tag[:2] == ("act", u)] for u in range(d)}
     entry_vm, entry_lds = list(st.vm_q), list(st.lds_q)
     first_load = 4 if units > 2 else 2                      # pair in which the first load is issued
     last_load = n_pair * 3 // 4 if units > 3 else n_pair // 2
@@ -281,14 +322,12 @@ def emit(units, vec, expand=False):
     arrive_at = cross - 3 if units > 3 else cross - 1
     look_whole_at = cross - 2 if units > 3 else cross
     look_free_at = 0
-    if expand:               # loads as early as they go, the stores a memory round trip later, done before the arrival
-        per_pair = 4 if units == 2 else 2 if units <= 6 else 1
-        load_at = [1 + i // per_pair for i in range(LOADS)]
-        first_store = min(load_at[7] + max(2, 16 // per_pair if units <= 6 else 20), arrive_at - 6)
+    if expand:               # stores from when the buffer may be free to the arrival, a block's loads behind its stores
+        first_store = 1 if units == 2 else 2
         store_at = [first_store + (arrive_at - 1 - first_store) * i // 15 for i in range(LOADS)]
-        if units >= 8:       # one a pair, the second block's behind its own round trip
-            store_at = [first_store + i + (i // 8) * 4 for i in range(LOADS)]
-        assert store_at[-1] < arrive_at and load_at[-1] <= store_at[8], (units, load_at, store_at, arrive_at)
+        per_pair = 2 if units <= 3 else 1
+        load_at = [store_at[i // 8 * 8 + 7] + i % 8 // per_pair for i in range(LOADS)]
+        assert load_at[-1] < n_pair and load_at[7] <= store_at[15]
     loaded = stored = 0
     load_ops = []
     ops = {}
@@ -302,8 +341,9 @@ def emit(units, vec, expand=False):
         st.wait_lds(pending[n], pending[n + 1])
         m = n + W
         if p == arrive_at:   # (a wavefront's LDS operations happen in order: its stores before this)
-            assert loaded == LOADS and stored == (LOADS if expand else 0)
-            st.wait_vm(*load_ops)
+            assert stored == LOADS if expand else loaded == LOADS
+            if not expand:
+                st.wait_vm(*load_ops)
             ops["arrive"] = count("cboth")
         if p == look_whole_at:
             ops["whole"] = look("cboth")
@@ -329,18 +369,17 @@ def emit(units, vec, expand=False):
         if expand:
             if p == 0:
                 row_addresses()
-            while loaded < LOADS and load_at[loaded] == p:
-                load_ops.append(row_load(loaded))
-                loaded += 1
-            if loaded == LOADS and p == load_at[-1]:
                 ops["codes"] = st.vm("buffer_load_dwordx4 %s, v%d, %%[wrc], %%[eoff] offen" % (quad(codes, 0), V_L16))
             if p == store_at[0]:
                 need(ops["free"], "cboth", "%[free]", 3)
             while stored < LOADS and store_at[stored] == p:
                 if stored % 8 == 0:
-                    st.wait_vm(*load_ops[stored:stored + 8])
+                    st.wait_vm(*[entering.get(("row", i)) for i in range(stored, stored + 8)])
                 chunk_store(stored)
                 stored += 1
+            while loaded < LOADS and load_at[loaded] == p:
+                load_ops.append(row_load(loaded))
+                loaded += 1
             continue
         if p == first_load:
             need(ops["free"], "cboth", "%[free]", 3)
@@ -380,17 +419,20 @@ def emit(units, vec, expand=False):
     # the rows that follow: the tile's next fill, or the first one of the workgroup's next tile, or none: then ENEXT has bit
     # 31 set, which moves into the vector offset.  That one is what a descriptor's bounds check covers; the scalar offset
     # must stay inside the rows by itself.
-    # (expanding: the same for the filter codes, which are loaded one fill further ahead)
+    # (expanding: the same for the filter codes, which are loaded two fills further ahead)
     st.ins("s_add_u32 %%[eoff], %%[eoff], %d" % (CODE_BYTES if expand else 0x10000))
-    st.ins("s_cmp_eq_u32 %%[left], %d" % (2 if expand else 1))
+    st.ins("s_cmp_eq_u32 %%[left], %d" % (3 if expand else 1))
     st.ins("s_cselect_b32 %[eoff], %[enext], %[eoff]")
     st.ins("s_and_b32 %[tmp], %[eoff], 0x80000000")
     st.ins("s_xor_b32 %[eoff], %[eoff], %[tmp]")
     st.ins("v_or_b32 v%d, %%[tmp], v%d" % (V_L16, V_L16))
     # the state the loop was entered with: W reads and D units of activations in flight, nothing else that counts
     # (operations older than those only make a wait stricter)
-    assert st.vm_q == [op for x in range(1, d) for op in acts[x]][-len(st.vm_q):] or not st.vm_q
-    assert len(st.vm_q) <= len(entry_vm)
+    if not expand:
+        assert st.vm_q == [op for x in range(1, d) for op in acts[x]][-len(st.vm_q):] or not st.vm_q
+        assert len(st.vm_q) <= len(entry_vm)
+    leaving = [st.tags[op] for op in st.vm_q]
+    assert None not in leaving
     assert [op for op in st.lds_q if op in pending.values()] == [pending[n_look + i] for i in range(W)]
     assert len(entry_lds) == W
     st.ins("s_branch Lfill_%=")
@@ -409,6 +451,8 @@ def emit(units, vec, expand=False):
     outs += ['"+{v%d}"(%s)' % (r, name) for name, r in inouts]
     if expand:
         outs += ['"+{v[%d:%d]}"(CODES)' % (codes, codes + 3), '"+{v%d}"(LDST)' % ldst]
+    if expand:
+        outs += ['"+{v[%d:%d]}"(LAND[%d])' % (land + 16 * i, land + 16 * i + 15, i) for i in range(4)]
     scalars = [("cbcur", "CBCUR"), ("cboth", "CBOTH")] + ([] if expand else [("edst", "EDST")]) + [("gf", "GF"), ("left", "LEFT"), ("free", "FREE"),
                ("whole", "WHOLE"), ("eoff", "EOFF")]
     outs += ['[%s] "+&s"(%s)' % s for s in scalars]
@@ -425,15 +469,16 @@ def emit(units, vec, expand=False):
     if expand:
         ins += ['"{v%d}"(TOFF)' % toff] + ['[%s] "s"(%s)' % x for x in [("wrc", "WRC"), ("rowb", "512u"), ("lo", "0x05040100u"),
                                                                       ("hi", "0x07060302u")]]
-        clob += ['"v%d"' % r for r in range(row, toff)]
+        clob += ['"v%d"' % r for r in range(row, toff) if not land <= r < land + 64]
     clob += ['"m0"', '"scc"', '"vcc"', '"memory"']
     args = ("ACC, CH0, CH1, KOFF, QL, KWL, CINIT, L16, CBCUR, CBOTH, EDST, GF, LEFT, FREE, WHOLE, EOFF, FAIL, TMP, EV, AOP, "
             "IDX, SEL, BASE, XQ, ERC, ENEXT, CB0, SPIN, WHOLE0, KS")
     if expand:
-        args = args.replace("EDST, ", "") + ", WRC, CODES, LDST, TOFF"
+        args = args.replace("EDST, ", "") + ", WRC, CODES, LDST, TOFF, LAND"
     text = " \\\n        ".join('"%s\\n\\t"' % line for line in st.lines)
-    return ("#define MX_%sFILLS_U%d_%s(%s) \\\n    asm volatile( \\\n        %s \\\n        : %s \\\n        : %s \\\n        : %s)\n"
+    text = ("#define MX_%sFILLS_U%d_%s(%s) \\\n    asm volatile( \\\n        %s \\\n        : %s \\\n        : %s \\\n        : %s)\n"
             % ("X" if expand else "", units, "V" if vec else "S", args, text, ", ".join(outs), ", ".join(ins), ", ".join(clob)))
+    return text, leaving
 
 
 if __name__ == "__main__":

@@ -17,7 +17,6 @@ hipError_t launch_dense_mx_expand(const MxParams &p, hipStream_t stream)
     case 14: return launch_mx_units<14, true>(p, stream);
     case 16: return launch_mx_units<16, true>(p, stream);
     case 18: return launch_mx_units<18, true>(p, stream);
-    case 20: return launch_mx_units<20, true>(p, stream);
     }
     return hipErrorInvalidValue;
 }

@@ -101,7 +101,7 @@ __device__ __forceinline__ void mx_fills(i32x16 (&acc)[U], uint32_t &ch0, uint32
 }
 
 // The same for the expanding form: codes of the fill that is expanded next, where the lane's chunks go in the other buffer,
-// the lane's offset into a table row.
+// the lane's offset into a table row, and the entries of the fill stored next.
 template <int U, bool VEC>
 __device__ __forceinline__ void mx_xfills(i32x16 (&acc)[U], uint32_t &ch0, uint32_t &ch1, uint32_t &koff, uint32_t &ql,
                                           uint32_t &kwl, uint32_t &cinit, uint32_t &l16, uint32_t &cbcur, uint32_t &cboth,
@@ -110,16 +110,16 @@ __device__ __forceinline__ void mx_xfills(i32x16 (&acc)[U], uint32_t &ch0, uint3
                                           const uint32_t (&sel)[4], const uint32_t (&base)[U], const rsrc_t xq,
                                           const rsrc_t erc, const uint32_t enext, const uint32_t spin, const uint32_t whole0,
                                           const MxKStep &ks, const rsrc_t wrc, mx_u32x4 &codes, uint32_t &ldst,
-                                          const uint32_t toff)
+                                          const uint32_t toff, i32x16 (&land)[4])
 {
     uint32_t tmp, ev;
 #define AXC_MX_CASE(N)                                                                                                  \
     if constexpr (U == N && VEC)                                                                                        \
         MX_XFILLS_U##N##_V(acc, ch0, ch1, koff, ql, kwl, cinit, l16, cbcur, cboth, gf, left, free_at, whole, eoff, fail, \
-                           tmp, ev, aop, idx, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks, wrc, codes, ldst, toff); \
+                           tmp, ev, aop, idx, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks, wrc, codes, ldst, toff, land); \
     if constexpr (U == N && !VEC)                                                                                       \
         MX_XFILLS_U##N##_S(acc, ch0, ch1, koff, ql, kwl, cinit, l16, cbcur, cboth, gf, left, free_at, whole, eoff, fail, \
-                           tmp, ev, aop, idx, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks, wrc, codes, ldst, toff);
+                           tmp, ev, aop, idx, sel, base, xq, erc, enext, kMxCb, spin, whole0, ks, wrc, codes, ldst, toff, land);
     AXC_MX_CASE(2)
     AXC_MX_CASE(3)
     AXC_MX_CASE(4)
@@ -131,7 +131,6 @@ __device__ __forceinline__ void mx_xfills(i32x16 (&acc)[U], uint32_t &ch0, uint3
     AXC_MX_CASE(14)
     AXC_MX_CASE(16)
     AXC_MX_CASE(18)
-    AXC_MX_CASE(20)
 #undef AXC_MX_CASE
     (void)tmp;
     (void)ev;
@@ -141,23 +140,35 @@ __device__ __forceinline__ void mx_xfills(i32x16 (&acc)[U], uint32_t &ch0, uint3
 __device__ __forceinline__ uint32_t mx_x_element(const uint32_t lane) { return (lane >> 1) & 15u; }
 __device__ __forceinline__ uint32_t mx_x_codes(const uint32_t lane) { return (lane & 1u) | ((lane >> 5) << 1); }
 
-// The expanding form's very first fill of a workgroup: this wavefront's share of its rows, into buffer 0.
-__device__ __forceinline__ void mx_x_first_fill(const rsrc_t trc, const mx_u32x4 codes, const uint32_t toff, const uint32_t ldst)
+// The entries of a fill that this lane turns: quadruple 8 b + j for block b and column j.
+__device__ __forceinline__ void mx_x_entries(const rsrc_t trc, const mx_u32x4 codes, const uint32_t toff, i32x16 (&land)[4])
+{
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int j = i & 7;
+        const uint32_t code = (j & 1) ? codes[j >> 1] >> 16 : codes[j >> 1] & 0xffffu;
+        const mx_u32x4 row = __builtin_bit_cast(
+            mx_u32x4, __builtin_amdgcn_raw_buffer_load_b128(trc, (int)(code * 512u + toff + 64u * (i >> 3)), 0, 0));
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            land[i >> 2][(i & 3) * 4 + k] = (int32_t)row[k];
+    }
+}
+
+// ... turned and stored as chunks of rows: the very first fill of a workgroup.
+__device__ __forceinline__ void mx_x_store(const i32x16 (&land)[4], const uint32_t ldst)
 {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-        mx_u32x4 row[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t code = (j & 1) ? codes[j >> 1] >> 16 : codes[j >> 1] & 0xffffu;
-            row[j] = __builtin_bit_cast(mx_u32x4, __builtin_amdgcn_raw_buffer_load_b128(trc, (int)(code * 512u + toff + 64u * b), 0, 0));
-        }
+        auto row = [&](const int j, const int k) __attribute__((always_inline)) {
+            return (uint32_t)land[2 * b + (j >> 2)][(j & 3) * 4 + k];
+        };
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             mx_u32x4 d;
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                d[k] = __builtin_amdgcn_perm(row[2 * k + 1][e >> 1], row[2 * k][e >> 1], (e & 1) ? 0x07060302u : 0x05040100u);
+                d[k] = __builtin_amdgcn_perm(row(2 * k + 1, e >> 1), row(2 * k, e >> 1), (e & 1) ? 0x07060302u : 0x05040100u);
             *(__attribute__((address_space(3))) mx_u32x4 *)(uintptr_t)(ldst + (e >> 2) * 256u + (e & 3) * 16384u + b * 2048u) = d;
         }
     }
@@ -214,7 +225,10 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
     if (tile_first >= tile_end)
         return;
     const uint32_t wofs = EXPAND ? 0u : (uint32_t)wave * kMxWaveBytes;
-    mx_u32x4 codes = {0u, 0u, 0u, 0u};   // expanding: this lane's filter codes of the fill expanded next
+    // expanding: this lane's filter codes of the fill whose entries are loaded next; and those of the fill stored next
+    constexpr uint32_t kCodesAhead = 3;   // fills by which the loop loads filter codes ahead
+    mx_u32x4 codes = {0u, 0u, 0u, 0u};
+    i32x16 land[4];
     auto first_fill_of = [&](const int ctv) __attribute__((always_inline)) {
         const int ksi = ctv / p.plan.n_col_tiles;
         return (uint32_t)((ctv - ksi * p.plan.n_col_tiles) * F + ksi * Fs);
@@ -232,8 +246,12 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                 return __builtin_bit_cast(mx_u32x4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (int)s16, (int)at, 0));
             };
             const mx_u32x4 first = load(eoff);
-            codes = load(eoff + kStep);   // (a tile has two fills or more)
-            mx_x_first_fill(e_rsrc, first, ((uint32_t)wave * 64u + c * 8u) * 2u, ((uint32_t)wave * 16u + c * 2u) * 256u + s16);
+            codes = load(eoff + kStep);   // (a tile has kCodesAhead fills or more)
+            const uint32_t toff = ((uint32_t)wave * 64u + c * 8u) * 2u;
+            mx_x_entries(e_rsrc, first, toff, land);
+            mx_x_store(land, ((uint32_t)wave * 16u + c * 2u) * 256u + s16);
+            mx_x_entries(e_rsrc, codes, toff, land);
+            codes = load(eoff + 2u * kStep);
         } else {
 #pragma unroll
             for (int j = 0; j < (int)kMxWaveBytes / 1024; ++j)
@@ -371,14 +389,14 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             // the other buffer is free once fill gf - 1 is read (fill 1 goes into a buffer never used)
             uint32_t free_at = gf == 0u ? 0u : mx_free(gf - 1u), whole = Ft > 1 ? mx_whole(gf + 1u) : 0u;
             const uint32_t whole0 = mx_whole(gf);
-            if constexpr (EXPAND) {   // filter codes are loaded two fills ahead
-                const uint32_t after = Ft > 2 ? ((uint32_t)(ct * F + f0) + 2u) * kStep : enext;
+            if constexpr (EXPAND) {   // filter codes are loaded three fills ahead
+                const uint32_t after = Ft > (int)kCodesAhead ? ((uint32_t)(ct * F + f0) + kCodesAhead) * kStep : enext;
                 const uint32_t s16 = mx_x_element((uint32_t)lane) * 16u, c = mx_x_codes((uint32_t)lane);
                 uint32_t eoff = after & 0x7fffffffu, l16 = s16 | (after & 0x80000000u);
                 uint32_t ldst = ((uint32_t)wave * 16u + c * 2u) * 256u + s16 + other * (uint32_t)kPxFillBytes;
                 mx_xfills<U, VEC>(acc, ch0, ch1, koff, ql, kwl, cinit, l16, cbcur, cboth, gf, left, free_at, whole, eoff, fail,
                                   aop, idx, sel, base, xq_rsrc, e_rsrc, enext, p.spin_limit, whole0, ks, w_rsrc, codes, ldst,
-                                  ((uint32_t)wave * 64u + c * 8u) * 2u);
+                                  ((uint32_t)wave * 64u + c * 8u) * 2u, land);
             } else {
                 const uint32_t after = Ft > 1 ? ((uint32_t)(ct * F + f0) + 1u) * kStep + wofs : enext;
                 uint32_t eoff = after & 0x7fffffffu, l16 = (uint32_t)lane * 16u | (after & 0x80000000u);
