@@ -181,6 +181,7 @@ __device__ __forceinline__ void mx_x_store(const i32x16 (&land)[4], const uint32
 template <int U, bool VEC, bool SIMPLE, bool EXPAND>
 __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParams p)
 {
+    fetch_arguments<sizeof(MxParams)>();
     const bool linear = SIMPLE || p.linear;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 

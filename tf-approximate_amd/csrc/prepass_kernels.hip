@@ -1450,6 +1450,10 @@ __device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const Fo
     return true;
 }
 
+// Arguments of the two kernels below, but for a few bytes.
+template <class Form>
+constexpr int kPatchArgumentBytes = 8 + sizeof(ConvGeom) + 12 + sizeof(TensorQuant) + 24 + sizeof(FilterWork) + sizeof(Form);
+
 // Bands cut into column segments: a kernel of its own, so that the common variants below stay as small as they were.
 template <bool ANY, class Form>
 __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *__restrict__ x, const ConvGeom g,
@@ -1459,6 +1463,7 @@ __global__ void __launch_bounds__(1024) patch_sums_segments_kernel(const float *
                                                                     float *__restrict__ psum, uint32_t *__restrict__ xq,
                                                                     const FilterWork fw, const Form form)
 {
+    fetch_arguments<kPatchArgumentBytes<Form>>();
     const XqLayout lay = form.layout(g);
     int bid;
     if (filter_work_block(fw, form, x, g, tq, lq_dev, &bid))
@@ -1473,6 +1478,7 @@ __global__ void __launch_bounds__(1024) patch_sums_rows_kernel(const float *__re
                                                                 float *__restrict__ psum, uint32_t *__restrict__ xq,
                                                                 const FilterWork fw, const Form form)
 {
+    fetch_arguments<kPatchArgumentBytes<Form>>();
     const XqLayout lay = form.layout(g);
     int bid;
     if (filter_work_block(fw, form, x, g, tq, lq_dev, &bid))
