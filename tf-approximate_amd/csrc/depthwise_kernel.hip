@@ -24,6 +24,7 @@ __device__ __forceinline__ DwEpilogue dw_epilogue_consts(const DepthwiseParams &
     return {p.s1xs2, p.m1, p.m2, p.k_m1xm2};
 }
 
+// The filters, strides and dilations that no window kernel below is made for.
 // Every output (pixel, channel) is its own dot product over the KH*KW taps, so there is no weight
 // reuse across lanes to expand: lanes look single entries up in the LDS-resident table,
 // T[b][a] at byte b*512 + a*2.  Lanes walk consecutive channels (NHWC: coalesced loads and stores).
@@ -299,6 +300,161 @@ __global__ void __launch_bounds__(kBlockThreads) depthwise_lut3x3_kernel(const D
     }
 }
 
+// Filters other than 3x3, at the same strides and without dilation: the same window of converted input columns, sized by
+// the filter.  What bounds the kernel is the LDS: a lookup is one ds_read_u16, and with CH channels side by side the 64 / CH
+// lanes of the same channel hit random rows, CH banks wide.  The table rows of KH * KW taps x CH channels have to fit the
+// LDS, two taps to a dword as in the 3x3 kernel, so CH is 32 for up to five taps and 8 for 5x5 (104 KiB).  Lanes of
+// another channel group of the wavefront take another task - image, band of R output rows, column segment - each, so that
+// small images fill a wavefront too.  us, by gathers of single entries from the whole table with an input value fetched once
+// per tap / here: 5x5 on 64x56x56x192 1643 / 210, at stride 2 446 / 119, on 69x10x10x544 165 / 35; 5x1 on 64x56x56x192 533 / 74;
+// 3x1 on 35x77x77x18 42.7 / 17.9.  (R: what 128 registers hold; four output rows of 5x5 spilled twelve.)
+template <int KH, int KW, int S, int R, int CH, bool OUT_I32>
+__global__ void __launch_bounds__(kBlockThreads) depthwise_lut_window_kernel(const DepthwiseParams p, const int seg_len,
+                                                                              const int nseg, const int wgs_per_group,
+                                                                              const int group_slots)
+{
+    constexpr int TAPS = KH * KW, PLANES = (TAPS + 1) / 2, STRIDE = PLANES * CH * 4;   // bytes per activation code
+    constexpr int SUBS = 64 / CH;                      // tasks side by side in a wavefront
+    constexpr int RIN = (R - 1) * S + KH;              // input rows under R output rows
+    constexpr int NEW = S < KW ? S : KW;               // input columns that enter the window with an output column
+    constexpr int SLOTS = KW + NEW;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cl = lane & (CH - 1), sub = lane / CH;
+    const int slot = (int)blockIdx.x / wgs_per_group, member = (int)blockIdx.x - slot * wgs_per_group;
+    if (slot >= group_slots)
+        return;
+    const TensorQuant q = dw_input_quant(p);
+    const DwEpilogue ep = dw_epilogue_consts(p);
+    const dw_rsrc_t x_rsrc = dw_make_rsrc(p.x, (uint32_t)((int64_t)p.N * p.H * p.W * p.C * 4));
+    const dw_rsrc_t o_rsrc = dw_make_rsrc(OUT_I32 ? static_cast<const void *>(p.out_i) : static_cast<const void *>(p.out_f),
+                                          (uint32_t)(p.M * p.C * 4));
+    const dw_rsrc_t t_rsrc = dw_make_rsrc(p.tableT, (uint32_t)kTableAllocBytes);
+    const uint32_t col_bytes = (uint32_t)p.C * 4u;
+    const int bands = (p.OH + R - 1) / R;
+    const int tasks = p.N * bands * nseg;              // (image, band, column segment), segment fastest
+    const int ngroups = (p.C + CH - 1) / CH;
+    const int run_first = (int)((int64_t)tasks * member / wgs_per_group);
+    const int run_end = (int)((int64_t)tasks * (member + 1) / wgs_per_group);
+
+    for (int group = slot; group < ngroups; group += group_slots) {
+        const int chan = group * CH + cl;
+        const bool live = chan < p.C;
+        __syncthreads();                                // every wavefront is done with the previous group's rows
+        for (int item = tid; item < PLANES * CH * 32; item += kBlockThreads) {
+            const int c = item & (CH - 1), piece = (item / CH) & 31, tp = item / (CH * 32);
+            const int ch = group * CH + c;
+            const uint32_t code0 = ch < p.C ? p.wcodes[(2 * tp) * p.C + ch] : kNullWeight;
+            const uint32_t code1 = (ch < p.C && 2 * tp + 1 < TAPS) ? p.wcodes[(2 * tp + 1) * p.C + ch] : kNullWeight;
+            const u32x4 v0 = __builtin_amdgcn_raw_buffer_load_b128(t_rsrc, (int)(code0 * 512u + (uint32_t)piece * 16u), 0, 0);
+            const u32x4 v1 = __builtin_amdgcn_raw_buffer_load_b128(t_rsrc, (int)(code1 * 512u + (uint32_t)piece * 16u), 0, 0);
+            unsigned char *dst = lds_dw + (8 * piece) * STRIDE + tp * (CH * 4) + c * 4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                *reinterpret_cast<uint32_t *>(dst + (2 * e) * STRIDE) = (v0[e] & 0xffffu) | (v1[e] << 16);
+                *reinterpret_cast<uint32_t *>(dst + (2 * e + 1) * STRIDE) = (v0[e] >> 16) | (v1[e] & 0xffff0000u);
+            }
+        }
+        __syncthreads();
+
+        const float t3 = (!OUT_I32 && live) ? __fmul_rn(ep.m1, p.fsum[chan]) : 0.0f;
+        const float bias = (!OUT_I32 && p.bias && live) ? p.bias[chan] : -0.0f;   // none: changes no value
+        const uint32_t lane_base = (uint32_t)reinterpret_cast<uintptr_t>(lds_dw) + (uint32_t)cl * 4u;
+        typedef const __attribute__((address_space(3))) uint16_t *lds_entry_ptr;
+
+        for (int first = run_first + wave * SUBS; first < run_end; first += kWaves * SUBS) {
+            const int task = first + sub;
+            const bool mine = live && task < run_end;
+            const int seg = task % nseg, nb = task / nseg;
+            const int band = nb % bands, n = nb / bands;
+            const int oh0 = band * R, ow0 = seg * seg_len;
+            const int len = mine ? (ow0 + seg_len < p.OW ? ow0 + seg_len : p.OW) - ow0 : 0;
+            const int ih0 = oh0 * S - p.ph, iw0 = ow0 * S - p.pw;
+            uint32_t rowoff[RIN];                       // 2^31: outside, and whatever is added to it is too
+#pragma unroll
+            for (int r = 0; r < RIN; ++r) {
+                const int ih = ih0 + r;
+                rowoff[r] = (mine && (unsigned)ih < (unsigned)p.H) ? (uint32_t)((((int64_t)n * p.H + ih) * p.W * p.C + chan) * 4)
+                                                                   : 0x80000000u;
+            }
+            uint32_t ooff[R];
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr)
+                ooff[rr] = (mine && oh0 + rr < p.OH)
+                               ? (uint32_t)((((int64_t)(n * p.OH + oh0 + rr) * p.OW + ow0) * p.C + chan) * 4)
+                               : 0x80000000u;
+
+            // Window column i of output column k is input column iw0 + k * S + i, the (k * NEW + i)-th that enters the
+            // window, and lives in that number's slot.
+            float val[RIN][SLOTS];
+            uint32_t off[RIN][SLOTS];
+            auto load_col = [&](const int iw, auto slot_tag, const bool wanted) {
+                constexpr int SL = decltype(slot_tag)::value;
+                const bool inside = wanted && (unsigned)iw < (unsigned)p.W;
+                const uint32_t coff = inside ? (uint32_t)iw * col_bytes : 0x80000000u;
+#pragma unroll
+                for (int r = 0; r < RIN; ++r) {
+                    const uint32_t at = (rowoff[r] | coff) & 0x80000000u ? 0x80000000u : rowoff[r] + coff;
+                    val[r][SL] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(x_rsrc, (int)at, 0, 0));
+                }
+            };
+            auto convert_col = [&](auto slot_tag) {
+                constexpr int SL = decltype(slot_tag)::value;
+#pragma unroll
+                for (int r = 0; r < RIN; ++r) {
+                    val[r][SL] = fake_quant_value(val[r][SL], q);
+                    off[r][SL] = __umul24(quantize_code(val[r][SL], q.offset, q.inv_scale), (uint32_t)STRIDE) + lane_base;
+                }
+            };
+            static_for<0, KW>([&](auto j) { load_col(iw0 + decltype(j)::value, j, true); });
+            static_for<0, KW>([&](auto j) { convert_col(j); });
+
+            auto step = [&](const int k, auto phase_tag) {
+                constexpr int PH = decltype(phase_tag)::value;   // k % SLOTS
+                static_for<0, NEW>([&](auto j) {   // the columns that enter with the next output column
+                    constexpr int J = decltype(j)::value;
+                    load_col(iw0 + (k + 1) * S + KW - NEW + J, std::integral_constant<int, ((PH + 1) * NEW + KW - NEW + J) % SLOTS>(),
+                             k + 1 < len);
+                });
+                const uint32_t ocol = k < len ? (uint32_t)k * col_bytes : 0x80000000u;
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) {
+                    uint32_t acc = 0;
+                    float psum = 0.0f;
+#pragma unroll
+                    for (int kh = 0; kh < KH; ++kh)
+#pragma unroll
+                        for (int kw = 0; kw < KW; ++kw) {
+                            const int ps = (NEW * PH + kw) % SLOTS, tap = kh * KW + kw;
+                            psum = __fadd_rn(psum, val[rr * S + kh][ps]);
+                            acc += reinterpret_cast<lds_entry_ptr>(off[rr * S + kh][ps])[(tap >> 1) * (CH * 2) + (tap & 1)];
+                        }
+                    uint32_t outw;
+                    if (OUT_I32) {
+                        outw = acc;
+                    } else {
+                        const float t2 = __fadd_rn(__fmul_rn((float)(int32_t)acc, ep.s1xs2), __fmul_rn(ep.m2, psum));
+                        float v = __fsub_rn(__fadd_rn(t2, t3), ep.k_m1xm2);
+                        v = __fadd_rn(v, bias);
+                        outw = __float_as_uint(p.relu ? fmaxf(v, 0.0f) : v);
+                    }
+                    const uint32_t at = (ooff[rr] | ocol) & 0x80000000u ? 0x80000000u : ooff[rr] + ocol;
+                    __builtin_amdgcn_raw_buffer_store_b32(outw, o_rsrc, (int)at, 0, 0);
+                }
+                static_for<0, NEW>([&](auto j) {
+                    convert_col(std::integral_constant<int, ((PH + 1) * NEW + KW - NEW + decltype(j)::value) % SLOTS>());
+                });
+            };
+            for (int k = 0; k < seg_len; k += SLOTS)
+                static_for<0, SLOTS>([&](auto ph) {
+                    if (k + decltype(ph)::value < seg_len)
+                        step(k + decltype(ph)::value, ph);
+                });
+        }
+    }
+}
+
 template <typename Kernel, typename... Args>
 static hipError_t launch_with_lds(Kernel kernel, int grid, int lds_bytes, hipStream_t stream, Args... args)
 {
@@ -309,11 +465,52 @@ static hipError_t launch_with_lds(Kernel kernel, int grid, int lds_bytes, hipStr
     return hipGetLastError();
 }
 
+// Workgroups per channel group and channel groups at a time as in launch_depthwise; segments so that a workgroup's rounds
+// of tasks times the columns a task loads (its segment and the window's restart) are fewest.
+template <int KH, int KW, int S, int R, int CH>
+static hipError_t launch_window(const DepthwiseParams &p, bool out_i32, hipStream_t stream)
+{
+    const int cus = device_cus();
+    const int ngroups = (p.C + CH - 1) / CH;
+    const int wgs_per_group = cus / ngroups < 1 ? 1 : cus / ngroups, group_slots = cus / ngroups < 1 ? cus : ngroups;
+    const int bands = (p.OH + R - 1) / R;
+    int nseg = 1, seg_len = p.OW;
+    int64_t best = -1;
+    for (int ns = 1; ns <= p.OW; ++ns) {
+        const int sl = (p.OW + ns - 1) / ns;
+        if (ns > 1 && sl < 8)
+            break;
+        const int ns_eff = (p.OW + sl - 1) / sl;
+        const int64_t tasks = (int64_t)p.N * bands * ns_eff, per_wg = (tasks + wgs_per_group - 1) / wgs_per_group;
+        if (tasks >= (int64_t)1 << 31)
+            continue;
+        const int64_t cost = ((per_wg + kWaves * (64 / CH) - 1) / (kWaves * (64 / CH))) * (sl + KW);
+        if (best < 0 || cost < best) {
+            best = cost;
+            nseg = ns_eff;
+            seg_len = sl;
+        }
+    }
+    constexpr int kLds = (KH * KW + 1) / 2 * CH * 4 * 256;
+    const int grid = wgs_per_group * group_slots;
+    return out_i32 ? launch_with_lds(depthwise_lut_window_kernel<KH, KW, S, R, CH, true>, grid, kLds, stream, p, seg_len, nseg,
+                                     wgs_per_group, group_slots)
+                   : launch_with_lds(depthwise_lut_window_kernel<KH, KW, S, R, CH, false>, grid, kLds, stream, p, seg_len, nseg,
+                                     wgs_per_group, group_slots);
+}
+
 hipError_t launch_depthwise(const DepthwiseParams &p, bool out_i32, int grid, hipStream_t stream)
 {
-    // the 3x3 kernel addresses input and output with 32-bit byte offsets and keeps the top of that range free
-    const bool banked = p.KH == 3 && p.KW == 3 && p.dh == 1 && p.dw == 1 && p.sh == p.sw && (p.sw == 1 || p.sw == 2) &&
-                        (int64_t)p.N * p.H * p.W * p.C * 4 < 0x7fffffffll && p.M * p.C * 4 < 0x7fffffffll;
+    // the window kernels address input and output with 32-bit byte offsets and keep the top of that range free
+    const bool windowed = p.dh == 1 && p.dw == 1 && p.sh == p.sw && (p.sw == 1 || p.sw == 2) &&
+                          (int64_t)p.N * p.H * p.W * p.C * 4 < 0x7fffffffll && p.M * p.C * 4 < 0x7fffffffll;
+    const bool banked = windowed && p.KH == 3 && p.KW == 3;
+    if (windowed && p.KH == 5 && p.KW == 5)
+        return p.sw == 1 ? launch_window<5, 5, 1, 3, 8>(p, out_i32, stream) : launch_window<5, 5, 2, 2, 8>(p, out_i32, stream);
+    if (windowed && p.KH == 5 && p.KW == 1)
+        return p.sw == 1 ? launch_window<5, 1, 1, 4, 32>(p, out_i32, stream) : launch_window<5, 1, 2, 4, 32>(p, out_i32, stream);
+    if (windowed && p.KH == 3 && p.KW == 1)
+        return p.sw == 1 ? launch_window<3, 1, 1, 4, 32>(p, out_i32, stream) : launch_window<3, 1, 2, 4, 32>(p, out_i32, stream);
     if (banked) {
         const int cus = device_cus();
         const int R = p.sw == 1 ? 4 : 2;
