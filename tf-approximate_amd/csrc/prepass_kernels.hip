@@ -771,27 +771,47 @@ __global__ void __launch_bounds__(1024) patch_sums_smallc_kernel(const float *__
 }
 
 // Same relayout for caller-supplied codes (uint8 NHWC).
+// A workgroup turns 1024 dwords, Q channel quads of 1024 / Q pixels: read along the channels of a pixel, written along the
+// pixels of a quad (a thread for all quads of a pixel wrote and read 4 bytes per line: 1x82x82x350 70 us).
+template <int Q>
 __global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__restrict__ codes, int64_t pixels,
                                                               int N, int H, int W, int C, int C4, const XqLayout lay,
                                                               uint32_t zp4, uint32_t *__restrict__ xq)
 {
-    const int64_t pix = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    xq_fill_padding(xq, lay, N, H, C4, zp4, pix, (int64_t)gridDim.x * blockDim.x);
-    if (pix >= pixels)
-        return;
-    const int w = (int)(pix % W);
-    const int64_t nh = pix / W;
-    const uint8_t *src = codes + pix * C;
-    uint32_t *const dst = xq + xq_row_nh(lay, nh, H, C4) + w;
-    for (int c4 = 0; c4 < C4; ++c4) {
-        uint32_t packed = 0;
+    constexpr int P = 1024 / Q;
+    __shared__ uint32_t tile[Q][P + 1];
+    const int t = threadIdx.x;
+    xq_fill_padding(xq, lay, N, H, C4, zp4, ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + t,
+                    (int64_t)gridDim.x * gridDim.y * 256);
+    const int64_t pix0 = (int64_t)blockIdx.x * P;
+    const int q0 = (int)blockIdx.y * Q;
+    const bool dwords = (C & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3) == 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = c4 * 4 + i;
-            if (c < C)
-                packed |= phys_row(src[c]) << (8 * i);
+    for (int i = 0; i < 4; ++i) {
+        const int at = i * 256 + t, p = at / Q, q = at % Q, c = (q0 + q) * 4;
+        const int64_t pix = pix0 + p;
+        uint32_t v = 0;
+        if (pix < pixels && q0 + q < C4) {
+            const uint8_t *const src = codes + pix * C + c;
+            if (dwords) {
+                v = *reinterpret_cast<const uint32_t *>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v |= (c + e < C ? (uint32_t)src[e] : 0u) << (8 * e);
+            }
         }
-        dst[(int64_t)c4 * lay.Wp] = packed;
+        tile[q][p] = ((v >> 2) & 0x3f3f3f3fu) | ((v & 0x03030303u) << 6);   // phys_row of every byte
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int at = i * 256 + t, q = at / P, p = at % P;
+        const int64_t pix = pix0 + p;
+        if (pix < pixels && q0 + q < C4) {
+            const int64_t nh = pix / W;
+            xq[xq_row_nh(lay, nh, H, C4) + (int64_t)(q0 + q) * lay.Wp + (pix - nh * W)] = tile[q][p];
+        }
     }
 }
 
@@ -1705,10 +1725,8 @@ __device__ __forceinline__ uint32_t sum_of_bytes(const uint8_t *__restrict__ src
         s = __builtin_amdgcn_sad_u8(v.y, 0u, s);
         s = __builtin_amdgcn_sad_u8(v.z, 0u, s);
         s = __builtin_amdgcn_sad_u8(v.w, 0u, s);
-    } else if constexpr (V == 4) {
-        s = __builtin_amdgcn_sad_u8(*reinterpret_cast<const uint32_t *>(src), 0u, 0u);
     } else {
-        s = *src;
+        s = __builtin_amdgcn_sad_u8(*reinterpret_cast<const uint32_t *>(src), 0u, 0u);
     }
     return s;
 }
@@ -1729,6 +1747,7 @@ __global__ void __launch_bounds__(kAxSumThreads) axconv_terms_kernel(const uint8
         const int cl = t % kAxSumCols, slice = t / kAxSumCols, col = (int)blockIdx.x * kAxSumCols + cl;
         uint32_t s = 0;
         if (col < g.Co)
+#pragma unroll 8
             for (int k = slice; k < g.K; k += kAxSumSlices)
                 s += fcodes[(int64_t)k * g.Co + col];
         ax_lds[t] = s;
@@ -1753,11 +1772,23 @@ __global__ void __launch_bounds__(kAxSumThreads) axconv_terms_kernel(const uint8
     __syncthreads();
     // the rows inside the image are one run of memory
     const int first = ih0 < 0 ? -ih0 : 0, last = g.H - ih0 < rows_in ? g.H - ih0 : rows_in;   // [first, last) of rows_in
-    const int chunks = g.C / V;   // of a pixel
+    const int chunks = V == 1 ? (g.C + 15) / 16 : g.C / V;   // of a pixel; byte by byte: 16 bytes and a remainder
     const uint8_t *const src = codes + ((int64_t)n * g.H + ih0 + first) * g.W * g.C;
     const int total = last > first ? (last - first) * g.W * chunks : 0;
-    for (int i = t; i < total; i += kAxSumThreads)
-        atomicAdd(&ax_lds[first * g.W + i / chunks], sum_of_bytes<V>(src + (int64_t)i * V));
+    for (int i = t; i < total; i += kAxSumThreads) {
+        const int px = i / chunks;
+        uint32_t s = 0;
+        if constexpr (V == 1) {
+            const int at = (i - px * chunks) * 16;
+            const uint8_t *const from = src + (int64_t)px * g.C + at;
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                s += at + e < g.C ? (uint32_t)from[at + e < g.C ? e : 0] : 0u;
+        } else {
+            s = sum_of_bytes<V>(src + (int64_t)i * V);
+        }
+        atomicAdd(&ax_lds[first * g.W + px], s);
+    }
     __syncthreads();
     for (int i = t; i < rows * g.OW; i += kAxSumThreads) {
         const int r = i / g.OW, ow = i - r * g.OW;
@@ -2395,8 +2426,10 @@ hipError_t launch_codes_relayout(const uint8_t *codes, const ConvGeom &g, const 
                                  hipStream_t stream)
 {
     const int64_t pixels = (int64_t)g.N * g.H * g.W;
-    hipLaunchKernelGGL(codes_relayout_kernel, dim3(blocks_for(pixels, 256)), dim3(256), 0, stream, codes, pixels, g.N, g.H,
-                       g.W, g.C, g.C4, lay, zp4, xq);
+    const int Q = g.C4 <= 4 ? 4 : g.C4 <= 8 ? 8 : 16;
+    auto kernel = Q == 4 ? codes_relayout_kernel<4> : Q == 8 ? codes_relayout_kernel<8> : codes_relayout_kernel<16>;
+    hipLaunchKernelGGL(kernel, dim3(blocks_for(pixels, 1024 / Q), (unsigned)((g.C4 + Q - 1) / Q)), dim3(256), 0, stream, codes,
+                       pixels, g.N, g.H, g.W, g.C, g.C4, lay, zp4, xq);
     return hipGetLastError();
 }
 
