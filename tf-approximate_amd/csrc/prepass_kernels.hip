@@ -1006,7 +1006,8 @@ __global__ void __launch_bounds__(256) swap_pack_kernel(const float *__restrict_
 // is covered by volume in flight: a block owns only kFsCols columns (64-byte pieces of filter rows), which leaves
 // each of its loads a whole row of lead.  It walks the filter rows in passes of kFsRows: all its threads (512 or
 // 1024) load a pass kFsAhead passes ahead of its use and store it into one half of an LDS stage; meanwhile the
-// first kFsCols lanes extend the sums from the other half.  A lone wavefront issues about one instruction every
+// first kFsCols lanes extend the sums from the other half.  The wavefront of those lanes does nothing else: loading and
+// storing its share of a pass it waited for memory in every pass (12.6 cycles an add).  A lone wavefront issues about one instruction every
 // four cycles whatever its kind, so the stage is column-major and a lane fetches four rows per LDS read, one batch
 // of 16 rows ahead of the adds: 21 instructions per 16 adds.  One barrier per pass.  Rows beyond K are staged as zeros and summed like the others: the sums start at +0 and
 // so are never -0, and x + 0 == x.
@@ -1019,11 +1020,12 @@ template <int THREADS>
 __device__ __forceinline__ void filter_sums_block(const int block, const float *__restrict__ filter, int K, int Co,
                                                   const TensorQuant &q, float *__restrict__ fsum)
 {
-    constexpr int kBatch = 16, kStep = THREADS / kFsCols, kPer = kFsRows / kStep; // loads per thread per pass
+    constexpr int kBatch = 16, kStep = (THREADS - 64) / kFsCols, kPer = (kFsRows + kStep - 1) / kStep; // loads per thread per pass
     float *const stage = reinterpret_cast<float *>(fs_lds);
     const int col0 = block * kFsCols;
     const int t = threadIdx.x;
-    const int cl = t % kFsCols, rsub = t / kFsCols;
+    const bool copies = t >= 64;
+    const int cl = t % kFsCols, rsub = (t - 64) / kFsCols;
     const bool col_ok = col0 + cl < Co;
     const float *const src = filter + (col_ok ? col0 + cl : Co - 1);
     const int npass = (K + kFsRows - 1) / kFsRows;
@@ -1046,22 +1048,35 @@ __device__ __forceinline__ void filter_sums_block(const int block, const float *
             float f = from[i];
             if (q.fq)
                 f = fake_quant_value(f, q);
-            half[cl * kFsPitch + r] = (pass * kFsRows + r < K) ? f : 0.0f;
+            if (r < kFsRows)
+                half[cl * kFsPitch + r] = (pass * kFsRows + r < K) ? f : 0.0f;
         }
     };
+    if (copies) {
 #pragma unroll
-    for (int u = 0; u < kFsAhead; ++u)
-        issue(v[u], u);
-    store(v[0], 0);
-    issue(v[0], kFsAhead);
+        for (int u = 0; u < kFsAhead; ++u)
+            issue(v[u], u);
+        store(v[0], 0);
+        issue(v[0], kFsAhead);
+        __syncthreads();
+        // one pass: `next` holds pass p + 1 (stored now, then refilled with the loads of pass p + 1 + kFsAhead)
+        auto copy_step = [&](const int p, float(&next)[kPer]) {
+            store(next, p + 1);
+            issue(next, p + 1 + kFsAhead);
+            __syncthreads();
+        };
+        static_assert(kFsAhead == 3, "the pass loop below rotates three register sets");
+        for (int p0 = 0; p0 < npass; p0 += kFsAhead) {
+            copy_step(p0, v[1]);
+            copy_step(p0 + 1, v[2]);
+            copy_step(p0 + 2, v[0]);
+        }
+        return;
+    }
     __syncthreads();
     float s = 0.0f;
     __builtin_amdgcn_s_setprio(3);   // the chain is the critical path: its wavefront issues ahead of the others on its SIMD
-    // one pass: `next` holds pass p + 1 (stored now, then refilled with the loads of pass p + 1 + kFsAhead);
-    // pass p lies in its half of the stage
-    auto pass_step = [&](const int p, float(&next)[kPer]) {
-        store(next, p + 1);
-        issue(next, p + 1 + kFsAhead);
+    for (int p = 0; p < (npass + kFsAhead - 1) / kFsAhead * kFsAhead; ++p) {   // pass p lies in its half of the stage
         if (t < kFsCols && p < npass) {
             const float4 *const half = reinterpret_cast<const float4 *>(stage + (p & 1) * (kFsCols * kFsPitch) + t * kFsPitch);
             const int left = K - p * kFsRows;
@@ -1097,12 +1112,6 @@ __device__ __forceinline__ void filter_sums_block(const int block, const float *
             }
         }
         __syncthreads();
-    };
-    static_assert(kFsAhead == 3, "the pass loop below rotates three register sets");
-    for (int p0 = 0; p0 < npass; p0 += kFsAhead) {
-        pass_step(p0, v[1]);
-        pass_step(p0 + 1, v[2]);
-        pass_step(p0 + 2, v[0]);
     }
     if (t < kFsCols && col_ok)
         fsum[col0 + t] = s;
