@@ -13,6 +13,9 @@ MM = (-0.9, 1.3, -0.5, 0.5)
 CASES = [(xs, k, s, padding) for k in ((5, 5), (5, 1), (3, 1)) for xs, s, padding in [
     ((2, 7, 9, 13), 1, "SAME"), ((1, 5, 5, 8), 1, "VALID"), ((3, 17, 30, 40), 1, "SAME"), ((1, 12, 70, 33), 2, "SAME"),
     ((2, 13, 11, 9), 2, "VALID"), ((1, 3, 2, 70), 1, "SAME"), ((9, 6, 50, 24), 2, "SAME")] if padding == "SAME" or xs[1] >= k[0]]
+# the column filters, and 5x5 at stride 2, take the window kernel from 2^18 (2^17) outputs on: the same images, more of them
+CASES += [((-(-(1 << 18) // (-(-xs[1] // s) * -(-xs[2] // s) * xs[3])) * 2,) + xs[1:], k, s, padding)
+          for xs, k, s, padding in CASES if k[1] == 1 or s == 2]
 
 
 def _id(c):
@@ -37,7 +40,7 @@ def test_against_the_oracle(pkg, oracle, case):
     assert np.array_equal(acc, acc_ref) and np.array_equal(y, y_ref)
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[3], CASES[9], CASES[17]], ids=_id)
+@pytest.mark.parametrize("case", [CASES[0], CASES[3], CASES[9], CASES[17], CASES[-1], CASES[-8]], ids=_id)
 def test_layer_call_and_tail(pkg, oracle, case):
     x, f = _tensors(case)
     strides = (case[2], case[2])

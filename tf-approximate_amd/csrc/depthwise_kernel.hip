@@ -466,7 +466,8 @@ static hipError_t launch_with_lds(Kernel kernel, int grid, int lds_bytes, hipStr
 }
 
 // Workgroups per channel group and channel groups at a time as in launch_depthwise; segments so that a workgroup's rounds
-// of tasks times the columns a task loads (its segment and the window's restart) are fewest.
+// of tasks times the columns a task loads (its segment and the window's restart) are fewest, however short they get: with
+// segments of 8 columns and more only, 5x5 on 4x20x20x64 took 24.5 us against 12.5, on 64x56x56x192 no less (both unsegmented).
 template <int KH, int KW, int S, int R, int CH>
 static hipError_t launch_window(const DepthwiseParams &p, bool out_i32, hipStream_t stream)
 {
@@ -478,8 +479,6 @@ static hipError_t launch_window(const DepthwiseParams &p, bool out_i32, hipStrea
     int64_t best = -1;
     for (int ns = 1; ns <= p.OW; ++ns) {
         const int sl = (p.OW + ns - 1) / ns;
-        if (ns > 1 && sl < 8)
-            break;
         const int ns_eff = (p.OW + sl - 1) / sl;
         const int64_t tasks = (int64_t)p.N * bands * ns_eff, per_wg = (tasks + wgs_per_group - 1) / wgs_per_group;
         if (tasks >= (int64_t)1 << 31)
@@ -505,11 +504,17 @@ hipError_t launch_depthwise(const DepthwiseParams &p, bool out_i32, int grid, hi
     const bool windowed = p.dh == 1 && p.dw == 1 && p.sh == p.sw && (p.sw == 1 || p.sw == 2) &&
                           (int64_t)p.N * p.H * p.W * p.C * 4 < 0x7fffffffll && p.M * p.C * 4 < 0x7fffffffll;
     const bool banked = windowed && p.KH == 3 && p.KW == 3;
-    if (windowed && p.KH == 5 && p.KW == 5)
-        return p.sw == 1 ? launch_window<5, 5, 1, 3, 8>(p, out_i32, stream) : launch_window<5, 5, 2, 2, 8>(p, out_i32, stream);
-    if (windowed && p.KH == 5 && p.KW == 1)
+    // Below these outputs a workgroup spends longer on turning the table into its filter's rows than it saves afterwards, us
+    // here / with the general kernel: 3x1 102 k outputs 8.4 / 7.5, 410 k 8.8 / 9.5; 5x1 102 k 10.0 / 8.3, 410 k 10.3 / 11.1; 5x5
+    // stride 2 102 k 14.4 / 14.6, 41 k and less 14.8 / 14.0; 5x5 stride 1 from the smallest on 12.0 / 13.2.
+    const int64_t outputs = p.M * p.C;
+    if (windowed && p.KH == 5 && p.KW == 5 && p.sw == 1)
+        return launch_window<5, 5, 1, 3, 8>(p, out_i32, stream);
+    if (windowed && p.KH == 5 && p.KW == 5 && outputs >= 1 << 17)
+        return launch_window<5, 5, 2, 2, 8>(p, out_i32, stream);
+    if (windowed && p.KH == 5 && p.KW == 1 && outputs >= 1 << 18)
         return p.sw == 1 ? launch_window<5, 1, 1, 4, 32>(p, out_i32, stream) : launch_window<5, 1, 2, 4, 32>(p, out_i32, stream);
-    if (windowed && p.KH == 3 && p.KW == 1)
+    if (windowed && p.KH == 3 && p.KW == 1 && outputs >= 1 << 18)
         return p.sw == 1 ? launch_window<3, 1, 1, 4, 32>(p, out_i32, stream) : launch_window<3, 1, 2, 4, 32>(p, out_i32, stream);
     if (banked) {
         const int cus = device_cus();
