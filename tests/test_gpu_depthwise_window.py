@@ -1,6 +1,7 @@
-"""depthwise_lut_window_kernel (tf-approximate_amd/csrc/depthwise_kernel.hip): 5x5, 5x1 and 3x1 filters at strides 1 and 2,
-against the depthwise oracle, int32 sums and floats bit for bit: images smaller than a band or a window, last bands, segments
-and channel groups that are incomplete, both paddings, inputs off the quantization grid, bias and ReLU, the layer call."""
+"""depthwise_lut_window_kernel (tf-approximate_amd/csrc/depthwise_kernel.hip): 5x5, 5x1 and 3x1 filters at strides 1 and 2
+(and the 3x3 kernel's column segments), against the depthwise oracle, int32 sums and floats bit for bit: images smaller than
+a band or a window, last bands, segments and channel groups that are incomplete, both paddings, inputs off the quantization
+grid, bias and ReLU, the layer call."""
 import numpy as np
 import pytest
 import torch
@@ -16,6 +17,9 @@ CASES = [(xs, k, s, padding) for k in ((5, 5), (5, 1), (3, 1)) for xs, s, paddin
 # the column filters, and 5x5 at stride 2, take the window kernel from 2^18 (2^17) outputs on: the same images, more of them
 CASES += [((-(-(1 << 18) // (-(-xs[1] // s) * -(-xs[2] // s) * xs[3])) * 2,) + xs[1:], k, s, padding)
           for xs, k, s, padding in CASES if k[1] == 1 or s == 2]
+# 3x3: column segments down to one pixel while every task has a wavefront, of 8 to 24 pixels beyond
+CASES += [((1, 9, 30, 40), (3, 3), 1, "SAME"), ((2, 9, 30, 2080), (3, 3), 1, "VALID"), ((11, 9, 30, 2080), (3, 3), 1, "SAME"),
+          ((1, 13, 59, 40), (3, 3), 2, "SAME"), ((2, 13, 59, 2080), (3, 3), 2, "SAME"), ((11, 13, 59, 2080), (3, 3), 2, "VALID")]
 
 
 def _id(c):
@@ -40,7 +44,7 @@ def test_against_the_oracle(pkg, oracle, case):
     assert np.array_equal(acc, acc_ref) and np.array_equal(y, y_ref)
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[3], CASES[9], CASES[17], CASES[-1], CASES[-8]], ids=_id)
+@pytest.mark.parametrize("case", [CASES[0], CASES[3], CASES[9], CASES[17], CASES[-7], CASES[-14], CASES[-6], CASES[-1]], ids=_id)
 def test_layer_call_and_tail(pkg, oracle, case):
     x, f = _tensors(case)
     strides = (case[2], case[2])
