@@ -127,6 +127,27 @@ def test_operands_exchanged(pkg, oracle, swapped, case):
     _compare(pkg, oracle, swapped, case)
 
 
+# 1x1 layers whose images count as one row of pixels (in fours, in twos, each for itself), and those just outside that rule
+FOLDED = [
+    ((4, 7, 7, 128), (1, 1, 40), 1, 1, "SAME"),
+    ((8, 15, 17, 132), (1, 1, 30), 1, 1, "VALID"),       # 1020 pixels a row
+    ((6, 10, 21, 256), (1, 1, 64), 1, 1, "SAME"),        # two images
+    ((3, 14, 14, 600), (1, 1, 36), 1, 1, "SAME"),        # one
+    ((12, 14, 13, 256), (1, 1, 64), 2, 1, "SAME"),       # gathered 7x7 first
+    ((6, 7, 7, 128), (1, 1, 40), 1, 1, "SAME"),          # six images of 7x7 are no fours
+    ((4, 16, 17, 128), (1, 1, 40), 1, 1, "SAME"),        # 272 pixels in rows of 17
+    ((4, 15, 19, 128), (1, 1, 40), 1, 1, "SAME"),        # 1140 pixels: too many
+]
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("case", FOLDED, ids=_id)
+def test_rows_of_whole_images(pkg, oracle, own_rows, case, mode):
+    assert np.prod(case[0]) * case[1][2] < 3e8   # so that the oracle has them
+    own_rows.set_matrix_rows(mode)
+    _compare(pkg, oracle, own_rows, case)
+
+
 @pytest.mark.parametrize("case", [SWAPPED[0], SWAPPED[3], SWAPPED[5], SWAPPED[7]], ids=_id)
 def test_layer_call_with_operands_exchanged(pkg, swapped, case):
     xs, fs, stride, _, padding = case

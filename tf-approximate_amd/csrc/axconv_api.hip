@@ -783,13 +783,6 @@ struct PreparedDense {
     bool empty;
 };
 
-// Decides whether the layer runs lutgemm_mx_kernel, and whether out of pre-expanded rows or of rows that it makes itself:
-// what the cost models, fitted to the launch times of each, say is fastest.  Whole op, us, pre-expanded / own rows / other
-// kernels: 3x3 64->64 @56x56x64 201 / 260 / 302, 1x1 128->512 @28x28x64 111 / 135 / 160, 1x1 256->1024 @14x14x64 147 / 148 /
-// 168, 3x3 256->256 @14x14x64 346 / 275 / 378, 3x3 512->512 @7x7x64 820 / 275 / 376, 1x1 512->2048 @7x7x64 284 / 138 / 189, the
-// same on one image 235 / 61 / 68.  Own rows want few pixels for many weights, where writing 512 bytes per weight and reading
-// them back outweighs making them anew in every tile.  Over the layers of ResNet-50 at batch 64, 9 and 1 and of 240 random
-// layers, each timed in the three forms, the choice is 1.2, 1.2, 0.4 and 2 % above the fastest of the three.
 // The same kernel with its operands exchanged (SwapPack), for layers with fewer output pixels than columns; units = 0: not
 // for this layer.
 MxPlan prepare_swap(const ConvGeom &g)
@@ -805,6 +798,13 @@ MxPlan prepare_swap(const ConvGeom &g)
     return plan;
 }
 
+// Decides whether the layer runs lutgemm_mx_kernel, and whether out of pre-expanded rows or of rows that it makes itself:
+// what the cost models, fitted to the launch times of each, say is fastest.  Whole op, us, pre-expanded / own rows / other
+// kernels: 3x3 64->64 @56x56x64 201 / 260 / 302, 1x1 128->512 @28x28x64 111 / 135 / 160, 1x1 256->1024 @14x14x64 147 / 148 /
+// 168, 3x3 256->256 @14x14x64 346 / 275 / 378, 3x3 512->512 @7x7x64 820 / 275 / 376, 1x1 512->2048 @7x7x64 284 / 138 / 189, the
+// same on one image 235 / 61 / 68.  Own rows want few pixels for many weights, where writing 512 bytes per weight and reading
+// them back outweighs making them anew in every tile.  Over the layers of ResNet-50 at batch 64, 9 and 1 and of 240 random
+// layers, each timed in the three forms, the choice is 1.2, 1.2, 0.4 and 2 % above the fastest of the three.
 void prepare_mx(PreparedDense *pd, bool allow_rows)
 {
     const ConvGeom &g = pd->g;
@@ -828,8 +828,9 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
     const double us = 1e-6 * device_clock_hz();
     // Rows beyond some 20 MB for few pixels take 0.19 to 0.23 us a MB of pre-pass where the plan says 0.143 (pre-pass without
     // and with them, us: 5x5 448->48 @28x28x5, 275 MB, 65 / 129; 3x3 864->80 @14x14x41, 320 MB, 113 / 178; 5x5 64->776
-    // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Channel counts that are no multiple of four keep 0.2: their patch sums, which
-    // read memory pixel by pixel, slow down behind so many rows (3x3 797->38 @14x14x4, 147 MB: pre-pass 892 -> 1150 us).
+    // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Channel counts that are no multiple of four keep 0.2,
+    // fitted while their patch sums read memory pixel by pixel, as below 64 channels they still do (3x3 797->38 @14x14x4, 147 MB:
+    // pre-pass 892 -> 1150 us then).
     const double rows_bytes = (double)rows.n_col_tiles * rows.fills * 65536.0;
     const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) ? 0.2e-6 : 0.07e-6) * us;
     const bool rows_ok = allow_rows && rows.units && rows_bytes <= (double)kPxMaxBytes;
@@ -917,6 +918,21 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
         pd->g.W = pd->g.OW;
         pd->g.sh = pd->g.sw = 1;
         sub_bytes = (size_t)pd->g.M * pd->g.C * element_bytes;
+    }
+    // A 1x1 filter at stride 1 sees a list of pixels.  Rows that are no whole groups of four pixels (7x7, 14x14) leave lanes of
+    // lutgemm_mx_kernel without a pixel - 56 units of 64 where 49 have pixels - and store by the pixel: one image, or the two
+    // or four that make whole groups, count as one row (ResNet-50 at batch 64 9782 -> 9632 us, its 1x1 layers 5 to 8 %).  From 128 channels and 192 pixels on, where the patch sums go by the
+    // list of pixels in any case (launch_patch_sums), up to the 1024 pixels a row may have there.
+    if (allow_subsample && pd->g.KH == 1 && pd->g.KW == 1 && pd->g.sh == 1 && pd->g.sw == 1 && pd->g.ph == 0 && pd->g.pw == 0 &&
+        (pd->g.W & 3) != 0 && (pd->g.C & 3) == 0 && pd->g.C >= 128) {
+        const int64_t pixels = (int64_t)pd->g.H * pd->g.W;
+        const int images = pixels & 1 ? 4 : pixels & 2 ? 2 : 1;
+        if (images * pixels >= 192 && images * pixels <= 1024 && pd->g.N % images == 0 &&
+            (pd->g.N + images) * pixels * pd->g.C < (int64_t)1 << 31) {   // (offsets into the codes and the row behind them)
+            pd->g.N /= images;
+            pd->g.H = pd->g.OH = 1;
+            pd->g.W = pd->g.OW = (int)(images * pixels);
+        }
     }
     // Channel counts that are no multiple of four (3-channel stems) would pad every pixel to whole quads: a quarter
     // of a 3-channel layer's lookups would hit the null weight.  With a filter dilation of 1 along the row, the KW * C
@@ -1074,7 +1090,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         const ConvGeom &gf = pd.g_full;
         void *sub = ws + pd.ws.sub_off;
         AXC_HIP(launch_subsample(codes_mode ? static_cast<const void *>(input_codes) : static_cast<const void *>(input),
-                                 codes_mode ? 1 : 4, gf.N, gf.H, gf.W, gf.C, gf.sh, gf.sw, g.H, g.W, sub, stream));
+                                 codes_mode ? 1 : 4, gf.N, gf.H, gf.W, gf.C, gf.sh, gf.sw, gf.OH, gf.OW, sub, stream));
         if (codes_mode)
             input_codes = static_cast<const uint8_t *>(sub);
         else
