@@ -66,8 +66,8 @@ LAYERS = [
     ("cfg3_inverted_residual", "expand_1x1_32_192", (64, 112, 112, 32), (1, 1, 32, 192), (1, 1), False, "uniform", "trunc2"),
     ("cfg3_inverted_residual", "dw3x3_192_s1", (64, 112, 112, 192), (3, 3, 192, 1), (1, 1), True, "uniform", "trunc4"),
     ("cfg3_inverted_residual", "dw3x3_192_s2", (64, 112, 112, 192), (3, 3, 192, 1), (2, 2), True, "uniform", "trunc2"),
-    # a depthwise filter that is not 3x3 runs the generic kernel (whole table in LDS, one-entry gathers)
-    ("cfg3_inverted_residual", "dw5x5_192_s1_generic", (64, 56, 56, 192), (5, 5, 192, 1), (1, 1), True, "uniform", "trunc4"),
+    # a depthwise filter that is not 3x3
+    ("cfg3_inverted_residual", "dw5x5_192_s1", (64, 56, 56, 192), (5, 5, 192, 1), (1, 1), True, "uniform", "trunc4"),
     ("cfg3_inverted_residual", "project_1x1_192_32", (64, 112, 112, 192), (1, 1, 192, 32), (1, 1), False, "uniform", "trunc4"),
     ("cfg4_resnet50", "stem_7x7s2_3_64", (64, 224, 224, 3), (7, 7, 3, 64), (2, 2), False, "uniform", "uniform_error"),
     ("cfg4_resnet50", "stage1_1x1_64_256", (64, 56, 56, 64), (1, 1, 64, 256), (1, 1), False, "uniform", "uniform_error"),
@@ -111,6 +111,8 @@ PROFILED_TRAFFIC = {
                                                       "profiles/lutgemm_px_conv1x1_b64_112x112x192_to_32.md"),
     ("conv3x3_b64_28x28x128_to_128", "lutgemm_px"): (2.000 * 130204.7 * 1024 + 1.000 * 54284.1 * 1024,
                                                      "profiles/lutgemm_px_conv3x3_b64_28x28x128_to_128.md"),
+    ("conv3x3_b64_7x7x512_to_512", "lutgemm_mx"): (2.000 * 10646.9 * 1024 + 1.000 * 25088.0 * 1024,
+                                                   "profiles/lutgemm_mx_expand_conv3x3_b64_7x7x512_to_512.md"),
     ("conv3x3_b64_7x7x512_to_512", "lutgemm_expand"): (2.000 * 8874.8 * 1024 + 1.000 * 55210.4 * 1024,
                                                        "profiles/lutgemm_expand_conv3x3_b64_7x7x512_to_512.md"),
     ("dw3x3_b64_112x112x192_s1", "depthwise_lut"): (2.000 * 360914 * 1024 + 1.000 * 602112 * 1024,
