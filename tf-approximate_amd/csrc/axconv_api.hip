@@ -921,7 +921,7 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     }
     // A 1x1 filter at stride 1 sees a list of pixels.  Rows that are no whole groups of four pixels (7x7, 14x14) leave lanes of
     // lutgemm_mx_kernel without a pixel - 56 units of 64 where 49 have pixels - and store by the pixel: one image, or the two
-    // or four that make whole groups, count as one row (ResNet-50 at batch 64 9782 -> 9632 us, its 1x1 layers 5 to 8 %).  From 128 channels and 192 pixels on, where the patch sums go by the
+    // or four that make whole groups, count as one row (ResNet-50 at batch 64 9782 -> 9632 us, its 1x1 layers 3 to 7 %).  From 128 channels and 192 pixels on, where the patch sums go by the
     // list of pixels in any case (launch_patch_sums), up to the 1024 pixels a row may have there.
     if (allow_subsample && pd->g.KH == 1 && pd->g.KW == 1 && pd->g.sh == 1 && pd->g.sw == 1 && pd->g.ph == 0 && pd->g.pw == 0 &&
         (pd->g.W & 3) != 0 && (pd->g.C & 3) == 0 && pd->g.C >= 128) {

@@ -277,12 +277,12 @@ __global__ void __launch_bounds__(kPsTile) patch_sums_tiled_kernel(const float *
 // own; launches for the other kernels are instantiations without either, so that their code carries none of it (as run-time
 // values they cost the pre-pass of small layers 0.2 to 0.4 us: more arguments to fetch, more scalar registers to spill).
 struct PlainForm {
-    static constexpr bool kMxCodes = false;
+    static constexpr bool kMxCodes = false, kChainAlone = false;
     __device__ static XqLayout layout(const ConvGeom &g) { return {g.H, g.W, 0, 0}; }
     __device__ static int mx_fills() { return 0; }
 };
 struct MxForm {
-    static constexpr bool kMxCodes = false;
+    static constexpr bool kMxCodes = false, kChainAlone = false;
     XqLayout lay;
     int fills;        // of the rows, per column tile
     __device__ const XqLayout &layout(const ConvGeom &) const { return lay; }
@@ -290,10 +290,11 @@ struct MxForm {
 };
 // ... and where that kernel makes its rows itself, filter codes packed for it (mx_pack_unit) instead of rows.
 struct MxCodesForm : MxForm {
-    static constexpr bool kMxCodes = true;
+    static constexpr bool kMxCodes = true, kChainAlone = true;
 };
 // ... and with the operands exchanged, both packed in that launch (swap_pack_unit).
 struct SwapForm : MxForm {
+    static constexpr bool kChainAlone = true;
     SwapPack pack;
     uint32_t *xq;
 };
@@ -1006,26 +1007,30 @@ __global__ void __launch_bounds__(256) swap_pack_kernel(const float *__restrict_
 // is covered by volume in flight: a block owns only kFsCols columns (64-byte pieces of filter rows), which leaves
 // each of its loads a whole row of lead.  It walks the filter rows in passes of kFsRows: all its threads (512 or
 // 1024) load a pass kFsAhead passes ahead of its use and store it into one half of an LDS stage; meanwhile the
-// first kFsCols lanes extend the sums from the other half.  The wavefront of those lanes does nothing else: loading and
-// storing its share of a pass it waited for memory in every pass (12.6 cycles an add).  A lone wavefront issues about one instruction every
+// first kFsCols lanes extend the sums from the other half.  A lone wavefront issues about one instruction every
 // four cycles whatever its kind, so the stage is column-major and a lane fetches four rows per LDS read, one batch
-// of 16 rows ahead of the adds: 21 instructions per 16 adds.  One barrier per pass.  Rows beyond K are staged as zeros and summed like the others: the sums start at +0 and
-// so are never -0, and x + 0 == x.
+// of 16 rows ahead of the adds: 21 instructions per 16 adds.  One barrier per pass.  Rows beyond K are staged as zeros and
+// summed like the others: the sums start at +0 and so are never -0, and x + 0 == x.
+// CHAIN_ALONE: the wavefront of those lanes does nothing else; with its share of the loads and stores it waits for memory in
+// every pass (12.6 cycles an add).  Launches of lutgemm_mx_kernel's own rows and exchanged operands have it - few patches under
+// many weights, where the filter sums are the launch's critical path: 3x3 512->512 @7x7 on 1 / 9 / 64 images 31.3 / 31.0 / 31.7 us,
+// 26.6 / 26.2 / 28.2 with it.  The others take longer with it (3x3 64->64 @56x56x64 31.4 -> 32.9, 3x3 512->512 @28x28x64
+// 180 -> 185).
 constexpr int kFsCols = 16, kFsRows = 256, kFsPitch = kFsRows + 4, kFsAhead = 3, kFsThreads = 1024;
 constexpr int kFsLdsBytes = 2 * kFsCols * kFsPitch * 4; // 32.5 KiB: two halves of [column][row], rows padded by 4
 
 extern __shared__ __align__(16) unsigned char fs_lds[];
 
-template <int THREADS>
+template <int THREADS, bool CHAIN_ALONE>
 __device__ __forceinline__ void filter_sums_block(const int block, const float *__restrict__ filter, int K, int Co,
                                                   const TensorQuant &q, float *__restrict__ fsum)
 {
-    constexpr int kBatch = 16, kStep = (THREADS - 64) / kFsCols, kPer = (kFsRows + kStep - 1) / kStep; // loads per thread per pass
+    constexpr int kFirst = CHAIN_ALONE ? 64 : 0;   // first thread that copies
+    constexpr int kBatch = 16, kStep = (THREADS - kFirst) / kFsCols, kPer = (kFsRows + kStep - 1) / kStep; // loads per thread per pass
     float *const stage = reinterpret_cast<float *>(fs_lds);
     const int col0 = block * kFsCols;
     const int t = threadIdx.x;
-    const bool copies = t >= 64;
-    const int cl = t % kFsCols, rsub = (t - 64) / kFsCols;
+    const int cl = t % kFsCols, rsub = (t - kFirst) / kFsCols;
     const bool col_ok = col0 + cl < Co;
     const float *const src = filter + (col_ok ? col0 + cl : Co - 1);
     const int npass = (K + kFsRows - 1) / kFsRows;
@@ -1048,35 +1053,40 @@ __device__ __forceinline__ void filter_sums_block(const int block, const float *
             float f = from[i];
             if (q.fq)
                 f = fake_quant_value(f, q);
-            if (r < kFsRows)
+            if (!CHAIN_ALONE || r < kFsRows)
                 half[cl * kFsPitch + r] = (pass * kFsRows + r < K) ? f : 0.0f;
         }
     };
-    if (copies) {
+    if (!CHAIN_ALONE || t >= kFirst) {
 #pragma unroll
         for (int u = 0; u < kFsAhead; ++u)
             issue(v[u], u);
         store(v[0], 0);
         issue(v[0], kFsAhead);
-        __syncthreads();
-        // one pass: `next` holds pass p + 1 (stored now, then refilled with the loads of pass p + 1 + kFsAhead)
-        auto copy_step = [&](const int p, float(&next)[kPer]) {
-            store(next, p + 1);
-            issue(next, p + 1 + kFsAhead);
-            __syncthreads();
-        };
-        static_assert(kFsAhead == 3, "the pass loop below rotates three register sets");
+    }
+    __syncthreads();
+    // one pass: `next` holds pass p + 1 (stored now, then refilled with the loads of pass p + 1 + kFsAhead)
+    auto copy_step = [&](const int p, float(&next)[kPer]) {
+        store(next, p + 1);
+        issue(next, p + 1 + kFsAhead);
+    };
+    static_assert(kFsAhead == 3, "the pass loops below rotate three register sets");
+    if (CHAIN_ALONE && t >= kFirst) {
         for (int p0 = 0; p0 < npass; p0 += kFsAhead) {
             copy_step(p0, v[1]);
+            __syncthreads();
             copy_step(p0 + 1, v[2]);
+            __syncthreads();
             copy_step(p0 + 2, v[0]);
+            __syncthreads();
         }
         return;
     }
-    __syncthreads();
     float s = 0.0f;
     __builtin_amdgcn_s_setprio(3);   // the chain is the critical path: its wavefront issues ahead of the others on its SIMD
-    for (int p = 0; p < (npass + kFsAhead - 1) / kFsAhead * kFsAhead; ++p) {   // pass p lies in its half of the stage
+    auto pass_step = [&](const int p, float(&next)[kPer]) {   // pass p lies in its half of the stage
+        if (!CHAIN_ALONE)
+            copy_step(p, next);
         if (t < kFsCols && p < npass) {
             const float4 *const half = reinterpret_cast<const float4 *>(stage + (p & 1) * (kFsCols * kFsPitch) + t * kFsPitch);
             const int left = K - p * kFsRows;
@@ -1112,6 +1122,11 @@ __device__ __forceinline__ void filter_sums_block(const int block, const float *
             }
         }
         __syncthreads();
+    };
+    for (int p0 = 0; p0 < npass; p0 += kFsAhead) {
+        pass_step(p0, v[1]);
+        pass_step(p0 + 1, v[2]);
+        pass_step(p0 + 2, v[0]);
     }
     if (t < kFsCols && col_ok)
         fsum[col0 + t] = s;
@@ -1184,7 +1199,7 @@ __global__ void __launch_bounds__(kFsThreads) filter_prep_kernel(const float *__
 {
     const TensorQuant q = lq_dev ? lq_dev->flt : tq;
     if ((int)blockIdx.x < sum_blocks) {
-        filter_sums_block<kFsThreads>((int)blockIdx.x, filter, taps * C, Co, q, fsum);
+        filter_sums_block<kFsThreads, false>((int)blockIdx.x, filter, taps * C, Co, q, fsum);
         return;
     }
     const int pb = (int)blockIdx.x - sum_blocks;
@@ -1452,9 +1467,9 @@ __device__ __forceinline__ bool filter_work_block(const FilterWork &fw, const Fo
         if (b < fw.sum_blocks) { // the launcher gives these workgroups 512 or 1024 threads
             const TensorQuant q = lq_dev ? lq_dev->flt : fw.tq;
             if (blockDim.x == 512)
-                filter_sums_block<512>(b, fw.filter, fw.taps * fw.C, fw.Co, q, fw.fsum);
+                filter_sums_block<512, Form::kChainAlone>(b, fw.filter, fw.taps * fw.C, fw.Co, q, fw.fsum);
             else
-                filter_sums_block<1024>(b, fw.filter, fw.taps * fw.C, fw.Co, q, fw.fsum);
+                filter_sums_block<1024, Form::kChainAlone>(b, fw.filter, fw.taps * fw.C, fw.Co, q, fw.fsum);
         }
         return true;
     }
