@@ -9,6 +9,7 @@ import torch
 
 import bench
 import refimpl
+import test_gpu_matrix_sums
 
 pytestmark = pytest.mark.gpu
 
@@ -118,6 +119,25 @@ def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, own_rows, case
     plan = _plan(own_rows, case)
     assert plan is not None and plan["own_rows"] == 1, plan
     _compare(pkg, oracle, own_rows, case)
+
+
+@pytest.mark.parametrize("case", [c[:5] for c in test_gpu_matrix_sums.CASES], ids=_id)
+def test_the_cases_of_pre_expanded_rows_as_planned(pkg, oracle, case):
+    """The cases chosen for the heights of the kernel that reads pre-expanded rows, in the form that the planner picks."""
+    plan = _plan(pkg.ops, case)
+    assert plan is not None
+    pkg.ops.profile_enable(True)
+    pkg.ops.profile_reset()
+    try:
+        xs, fs, stride, dil, padding = case
+        xd, fd = bench.device_tensors(pkg, xs, (fs[0], fs[1], xs[3], fs[2]), "uniform", seed=1)
+        pkg.ApproxConv2DWithMinMaxVars([1, stride, stride, 1], 8, pkg.synth.table_exact(), padding,
+                                       dilations=[1, dil, dil, 1])(xd, fd, *MM)
+        names = set(pkg.ops.profile_read())
+    finally:
+        pkg.ops.profile_enable(False)
+    assert "lutgemm_mx" in names and ("lutgemm_px" in names) == (plan["own_rows"] == 0), (plan, names)
+    _compare(pkg, oracle, pkg.ops, case)
 
 
 @pytest.mark.parametrize("case", SWAPPED, ids=_id)

@@ -64,6 +64,18 @@ def _plan(pkg, case):
     return pkg.ops.conv2d_matrix_plan(xs, (fs[0], fs[1], xs[3], fs[2]), (1, stride, stride, 1), padding, (1, dil, dil, 1))
 
 
+@pytest.fixture()
+def pre_expanded_rows(pkg):
+    """The heights and K splits of CASES are those of the kernel that reads pre-expanded rows; where the planner would have
+    it make its rows itself instead, test_gpu_matrix_rows.py runs the same cases as planned."""
+    pkg.ops.set_matrix_rows(1)
+    try:
+        yield
+    finally:
+        pkg.ops.set_matrix_rows(0)
+
+
+@pytest.mark.usefixtures("pre_expanded_rows")
 @pytest.mark.parametrize("case", CASES, ids=_id)
 def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, case):
     print("case", _id(case), flush=True)
@@ -104,6 +116,7 @@ def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, case):
         assert refimpl.linf_rel(got[1].cpu().numpy(), y_ref) <= 1e-5
 
 
+@pytest.mark.usefixtures("pre_expanded_rows")
 def test_every_tile_height_is_covered(pkg):
     assert {_plan(pkg, c)["units_per_wavefront"] for c in CASES} >= {2, 3, 4, 6, 8, 10, 13, 16, 20, 25}
 

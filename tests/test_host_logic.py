@@ -199,6 +199,16 @@ def test_strided_pixel_groups_stay_in_the_workspace(ops):
     assert seen > 10
 
 
+@pytest.fixture()
+def pre_expanded_rows(ops):
+    ops.set_matrix_rows(1)
+    try:
+        yield
+    finally:
+        ops.set_matrix_rows(0)
+
+
+@pytest.mark.usefixtures("pre_expanded_rows")   # the figures are that form's; the next test has the planner's own choice
 def test_matrix_core_kernel_where_it_was_measured_faster(ops):
     """Layers with many weights for few pixels, timed both ways (whole op, us: on the matrix cores / expanding inside the
     tiles), far enough from the line to tell: the rows cost pre-pass time, but not as much as turns all of them away."""
