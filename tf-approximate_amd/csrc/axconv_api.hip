@@ -775,6 +775,7 @@ struct PreparedDense {
     ConvGeom gk;         // what the planner and the LUT-GEMM kernels see (differs from g in the flat layout)
     int flat_row_bytes;  // > 0: xq in the flat layout, rows of this many bytes
     bool subsample;
+    bool folded;         // whole images of a 1x1 layer count as one row (g, not g_full)
     DensePlan plan;
     bool mx;             // the layer runs lutgemm_mx_kernel, cut as mxp says (plan then only describes the other kernels)
     MxPlan mxp;
@@ -882,10 +883,11 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
 // stride-1 op on the subsampled input.  Those pixels are gathered into the workspace first (element_bytes each:
 // floats, or bytes for the codes entry point), and every kernel then sees a dense, unpadded stride-1 layer with a
 // quarter (stride 2) of the pixels to quantize and sum.  Callers with a padding origin of their own (`pads`: rows and columns)
-// get the layer as given.  mx_mode: which forms of lutgemm_mx_kernel may run the layer.
+// get the layer as given.  mx_mode: which forms of lutgemm_mx_kernel may run the layer.  allow_fold: images of a 1x1 layer may
+// count as one row.
 enum { kMxNone, kMxOwnRows, kMxAny };
 int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
-                  int px_mode = kPxModeGlobal, int mx_mode = kMxAny)
+                  int px_mode = kPxModeGlobal, int mx_mode = kMxAny, bool allow_fold = true)
 {
     const bool allow_subsample = pads == nullptr;
     const bool allow_flat = allow_subsample;   // both are for callers that leave the padding origin to the library
@@ -903,7 +905,7 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
         pd->g.ph = pd->g_full.ph = pads[0];
         pd->g.pw = pd->g_full.pw = pads[1];
     }
-    pd->subsample = false;
+    pd->subsample = pd->folded = false;
     pd->empty = pd->g.M * pd->g.Co == 0; // approx_nn_conv_ops.cpp:449
     if (pd->empty || pd->g.K == 0) {
         pd->plan = DensePlan{};
@@ -923,12 +925,13 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     // lutgemm_mx_kernel without a pixel - 56 units of 64 where 49 have pixels - and store by the pixel: one image, or the two
     // or four that make whole groups, count as one row (ResNet-50 at batch 64 9782 -> 9632 us, its 1x1 layers 3 to 7 %).  From 128 channels and 192 pixels on, where the patch sums go by the
     // list of pixels in any case (launch_patch_sums), up to the 1024 pixels a row may have there.
-    if (allow_subsample && pd->g.KH == 1 && pd->g.KW == 1 && pd->g.sh == 1 && pd->g.sw == 1 && pd->g.ph == 0 && pd->g.pw == 0 &&
-        (pd->g.W & 3) != 0 && (pd->g.C & 3) == 0 && pd->g.C >= 128) {
+    if (allow_subsample && allow_fold && pd->g.KH == 1 && pd->g.KW == 1 && pd->g.sh == 1 && pd->g.sw == 1 && pd->g.ph == 0 &&
+        pd->g.pw == 0 && (pd->g.W & 3) != 0 && (pd->g.C & 3) == 0 && pd->g.C >= 128) {
         const int64_t pixels = (int64_t)pd->g.H * pd->g.W;
         const int images = pixels & 1 ? 4 : pixels & 2 ? 2 : 1;
         if (images * pixels >= 192 && images * pixels <= 1024 && pd->g.N % images == 0 &&
             (pd->g.N + images) * pixels * pd->g.C < (int64_t)1 << 31) {   // (offsets into the codes and the row behind them)
+            pd->folded = true;
             pd->g.N /= images;
             pd->g.H = pd->g.OH = 1;
             pd->g.W = pd->g.OW = (int)(images * pixels);
@@ -991,25 +994,35 @@ void axconv_tf1_pads(const ConvGeom &g, int padding, int pads[2])
 // The layer as it runs with this much workspace: in the form the planner prefers if that fits, else in the next one.
 // Without room for the pre-expanded rows it runs the kernel that expands inside its tiles, with the tile shape and K
 // split the planner prices for THAT kernel, if the workspace holds what that plan needs (its K split may ask for partial
-// sums the other plan has none of); otherwise with the plan at hand.
+// sums the other plan has none of); otherwise with the plan at hand.  Images that count as one row have a longer row of zero
+// points behind them (1x1 4500->8 @30x34x6: 32.1 MB of codes instead of 27.7): where nothing fits with it, they do not.
+// *needed: the least that any of these forms asks for.
 int prepare_dense_for(const axc_conv2d_desc *desc, size_t workspace_bytes, const int *pads, int element_bytes,
-                      PreparedDense *pd)
+                      PreparedDense *pd, size_t *needed = nullptr)
 {
-    int rc = prepare_dense(desc, pd, pads, element_bytes);
-    if (rc != AXC_OK || pd->empty)
-        return rc;
-    for (int mx_mode : {kMxOwnRows, kMxNone})
-        if (pd->mx && workspace_bytes < pd->ws.total) {
-            rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, mx_mode);
+    size_t least = SIZE_MAX;
+    for (bool fold : {true, false}) {
+        for (int mx_mode : {kMxAny, kMxOwnRows, kMxNone}) {
+            const int rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, mx_mode, fold);
             if (rc != AXC_OK)
                 return rc;
+            least = std::min(least, pd->ws.total_no_px);
+            if (!pd->mx || workspace_bytes >= pd->ws.total)
+                break;
         }
-    if (!pd->mx && pd->plan.px && workspace_bytes < pd->ws.total) {
-        PreparedDense alt;
-        rc = prepare_dense(desc, &alt, pads, element_bytes, -1);
-        if (rc == AXC_OK && workspace_bytes >= alt.ws.total)
-            *pd = alt;
+        if (!pd->mx && pd->plan.px && workspace_bytes < pd->ws.total) {
+            PreparedDense alt;
+            if (prepare_dense(desc, &alt, pads, element_bytes, -1, kMxNone, fold) == AXC_OK) {
+                least = std::min(least, alt.ws.total);
+                if (workspace_bytes >= alt.ws.total)
+                    *pd = alt;
+            }
+        }
+        if (!pd->folded || workspace_bytes >= pd->ws.total_no_px)
+            break;
     }
+    if (needed)
+        *needed = least;
     return AXC_OK;
 }
 
@@ -1874,24 +1887,10 @@ int axc_conv2d_minmax_static(const axc_table *table, const axc_conv2d_desc *desc
     if (!table || !desc)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
     PreparedDense pd;
-    int rc = prepare_dense(desc, &pd);
+    size_t needed;
+    int rc = prepare_dense_for(desc, kStaticScratchBytes, nullptr, 4, &pd, &needed);
     if (rc != AXC_OK)
         return rc;
-    for (int mx_mode : {kMxOwnRows, kMxNone})   // without the room it would run as run_dense re-plans it
-        if (pd.mx && pd.ws.total > kStaticScratchBytes) {
-            rc = prepare_dense(desc, &pd, nullptr, 4, kPxModeGlobal, mx_mode);
-            if (rc != AXC_OK)
-                return rc;
-        }
-    size_t needed = (pd.mx || pd.plan.px) ? pd.ws.total : pd.ws.total_no_px;
-    if (!pd.mx && pd.plan.px && needed > kStaticScratchBytes) {
-        // without room for pre-expanded rows the layer runs as run_dense re-plans it, or as planned minus the rows
-        PreparedDense alt;
-        rc = prepare_dense(desc, &alt, nullptr, 4, -1);
-        if (rc != AXC_OK)
-            return rc;
-        needed = std::min(alt.ws.total, pd.ws.total_no_px);
-    }
     if (needed > kStaticScratchBytes) {
         char msg[200];
         snprintf(msg, sizeof(msg), "layer needs %zu bytes of workspace, the static workspace holds %zu: use "
