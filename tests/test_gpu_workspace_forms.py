@@ -57,3 +57,35 @@ def test_images_that_count_as_one_row_in_the_static_workspace(pkg):
     assert torch.equal(got, want)
     rc, got = layer.in_workspace(32 << 20)
     assert rc == 0 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("xs,fs,static_form", [
+    ((32, 56, 56, 64), (3, 3, 64, 128), {"lutgemm_mx"}),                  # planned with rows (38 MB): makes them itself
+    ((256, 5, 44, 128), (3, 3, 128, 16), {"lutgemm_px", "lutgemm_mx"}),   # planned with K splits (sums of 22 MB): rows, no split
+], ids=["own_rows", "rows"])
+def test_another_form_of_the_matrix_core_kernel(pkg, xs, fs, static_form):
+    """The static workspace lacks the room for what the planner prefers, but not for another form of the same kernel."""
+    layer = _Layer(pkg, xs, fs, 5)
+    assert layer.ws_bytes > 32 << 20
+    plan = pkg.ops.conv2d_matrix_plan(xs, fs)
+    assert plan is not None and (plan["own_rows"] == 0) == ("lutgemm_px" not in static_form), plan
+    rc, want = layer.in_workspace(layer.ws_bytes)
+    assert rc == 0 and not bool(want.isnan().any())
+    planned = layer.kernels
+    assert ("lutgemm_px" in planned) == (plan["own_rows"] == 0)
+    rc, got = layer.static()
+    assert rc == 0, layer.lib.axc_last_error()
+    assert layer.kernels - {"lutgemm_expand"} == static_form
+    assert torch.equal(got, want)
+    # down to where none of its forms fits any more
+    pkg.ops.set_preexpand(-1)
+    try:
+        n = ctypes.c_size_t()
+        assert layer.lib.axc_conv2d_workspace_bytes(ctypes.byref(layer.desc), ctypes.byref(n)) == 0
+    finally:
+        pkg.ops.set_preexpand(0)
+    rc, got = layer.in_workspace(n.value)
+    assert rc == 0, layer.lib.axc_last_error()
+    assert torch.equal(got, want)
+    rc, _ = layer.in_workspace(1 << 20)
+    assert rc != 0 and b"workspace too small" in layer.lib.axc_last_error()

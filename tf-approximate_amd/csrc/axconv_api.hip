@@ -806,7 +806,8 @@ MxPlan prepare_swap(const ConvGeom &g)
 // same on one image 235 / 61 / 68.  Own rows want few pixels for many weights, where writing 512 bytes per weight and reading
 // them back outweighs making them anew in every tile.  Over the layers of ResNet-50 at batch 64, 9 and 1 and of 240 random
 // layers, each timed in the three forms, the choice is 1.2, 1.2, 0.4 and 2 % above the fastest of the three.
-void prepare_mx(PreparedDense *pd, bool allow_rows)
+enum { kMxNone, kMxOwnRows, kMxRows, kMxAny };   // which forms may run the layer (own rows: operands exchanged too)
+void prepare_mx(PreparedDense *pd, int forms)
 {
     const ConvGeom &g = pd->g;
     const XqLayout lay = padded_layout(g, pd->flat_row_bytes > 0);
@@ -834,10 +835,10 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
     // pre-pass 892 -> 1150 us then).
     const double rows_bytes = (double)rows.n_col_tiles * rows.fills * 65536.0;
     const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) ? 0.2e-6 : 0.07e-6) * us;
-    const bool rows_ok = allow_rows && rows.units && rows_bytes <= (double)kPxMaxBytes;
+    const bool rows_ok = forms != kMxOwnRows && rows.units && rows_bytes <= (double)kPxMaxBytes;
     const bool own_ok = own.units && 3 * pitch <= (int64_t)(4 * kMinMaxBlocks * sizeof(float)) &&
                         (int64_t)own.n_col_tiles * own.fills * kMxCodeBytes < ((int64_t)1 << 31);
-    const int mode = g_mx_rows.load(std::memory_order_relaxed);
+    const int mode = forms == kMxRows ? 1 : g_mx_rows.load(std::memory_order_relaxed);
     bool expand = own_ok;
     if (mode == 3 && swap.units) {
         pd->mx = true;
@@ -885,7 +886,6 @@ void prepare_mx(PreparedDense *pd, bool allow_rows)
 // quarter (stride 2) of the pixels to quantize and sum.  Callers with a padding origin of their own (`pads`: rows and columns)
 // get the layer as given.  mx_mode: which forms of lutgemm_mx_kernel may run the layer.  allow_fold: images of a 1x1 layer may
 // count as one row.
-enum { kMxNone, kMxOwnRows, kMxAny };
 int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
                   int px_mode = kPxModeGlobal, int mx_mode = kMxAny, bool allow_fold = true)
 {
@@ -978,7 +978,7 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     pd->lay = plain_layout(pd->g);
     if (mx_mode != kMxNone && px_mode == kPxModeGlobal && g_px_mode.load(std::memory_order_relaxed) == 0 &&
         g_forced_nt.load(std::memory_order_relaxed) == 0)
-        prepare_mx(pd, mx_mode == kMxAny);
+        prepare_mx(pd, mx_mode);
     pd->ws = dense_workspace(pd->g, pd->plan, pd->mx ? &pd->mxp : nullptr, pd->lay, sub_bytes, pd->flat_row_bytes);
     return AXC_OK;
 }
@@ -1002,7 +1002,7 @@ int prepare_dense_for(const axc_conv2d_desc *desc, size_t workspace_bytes, const
 {
     size_t least = SIZE_MAX;
     for (bool fold : {true, false}) {
-        for (int mx_mode : {kMxAny, kMxOwnRows, kMxNone}) {
+        for (int mx_mode : {kMxAny, kMxOwnRows, kMxRows, kMxNone}) {   // (rows: no K split where the others' sums do not fit)
             const int rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, mx_mode, fold);
             if (rc != AXC_OK)
                 return rc;
