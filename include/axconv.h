@@ -146,12 +146,14 @@ int axc_qint32_range_for_multiplication(float min_a, float max_a, float min_b, f
 int axc_conv2d_tile_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
 /* Whether the layer runs the kernel whose sums the matrix cores make instead (given a workspace of the size
  * axc_conv2d_workspace_bytes reports, and neither axc_set_preexpand nor axc_set_tile_columns pinning another), and how
- * that cuts it: plan = { 1 or 2, or 0 (then the rest is 0 too), units of 64 pixels per wavefront (the kernel's variant),
- * units per tile, row tiles, column tiles (8 columns), K splits, workgroups, fills of 16 filter elements per K split }.
- * 1: it runs out of rows of 512 bytes per filter element in the workspace, at most 2 GiB, which the workspace query counts;
- * 2: it makes the rows itself in every tile; 3: the same with the operands exchanged, output pixels for columns.  A launch whose workspace lacks room runs in the other form or one of the other
- * kernels, with the same results. */
+ * that cuts it: plan = { 1 or 0 (then the rest is 0 too), units of 64 pixels per wavefront (the kernel's variant), units
+ * per tile, row tiles, column tiles (8 columns), K splits, workgroups, fills of 16 filter elements per K split }. */
 int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
+/* Which rows that kernel reads: 0 = the layer does not run it; 1 = pre-expanded ones, 512 bytes per filter element in the
+ * workspace, at most 2 GiB, which the workspace query counts; 2 = its own, made in every tile; 3 = the same with the operands
+ * exchanged: the plan's pixels are then the layer's output columns, and its columns the output pixels.  A launch whose
+ * workspace lacks room runs in another form or one of the other kernels, with the same results. */
+int axc_conv2d_matrix_rows(const axc_conv2d_desc *desc, int32_t *rows);
 /* Pins the tile width the planner uses (16, 32 or 64 columns; 0 = its own choice, the default), process-wide, for
  * tests and timing of the wider-tile kernel variants.  The environment variable AXC_TILE_COLUMNS gives the initial
  * value and is read once, when the library is loaded.  Like axc_set_preexpand it is process-wide; a workspace query and
@@ -166,10 +168,10 @@ int axc_set_tile_columns(int columns);
  * plan of the kernel that expands inside its tiles when the workspace holds what that plan needs.  No counterpart
  * in the reference. */
 int axc_set_preexpand(int mode);
-/* Which rows the kernel of axc_conv2d_matrix_plan reads: 0 = the planner decides (the default), 1 = pre-expanded ones only
- * (layers that those do not suit run the other kernels), 2 = made by the kernel itself wherever it can, 3 = the same with
- * the operands exchanged; process-wide, for tests and timing; a workspace query and the launch it is for must see the same value.  Results do not depend on it.  No
- * counterpart in the reference. */
+/* Pins what axc_conv2d_matrix_rows reports: 0 = the planner decides (the default), 1 = pre-expanded rows only (layers that
+ * those do not suit run the other kernels), 2 = rows made by the kernel itself wherever it can, 3 = the same with the operands
+ * exchanged; process-wide, for tests and timing; a workspace query and the launch it is for must see the same value.
+ * Results do not depend on it.  No counterpart in the reference. */
 int axc_set_matrix_rows(int mode);
 /* The wavefronts of the kernels that plan code 2 and axc_conv2d_matrix_plan stand for wait for each other by polling counters,
  * every wait a bounded number of polls (the default, 2^20 of ~150 cycles each, is far beyond any legitimate wait).  A wait that runs out ends

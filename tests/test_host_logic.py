@@ -225,6 +225,26 @@ def test_matrix_core_kernel_where_it_was_measured_faster(ops):
         assert (plan is not None) == faster, (xs, fs, plan)
 
 
+def test_matrix_plan_says_yes_or_no_in_every_form(ops, lib):
+    """plan[0] of axc_conv2d_matrix_plan is 1 whichever rows the kernel reads; axc_conv2d_matrix_rows says which."""
+    desc = ops.make_desc((3, 14, 14, 64), (1, 1, 64, 8), (1, 1, 1, 1), "SAME")
+    plan, rows = (ctypes.c_int32 * 8)(), ctypes.c_int32(-1)
+    try:
+        for mode, want in ((1, 1), (2, 2), (3, 3)):
+            ops.set_matrix_rows(mode)
+            assert lib.axc_conv2d_matrix_rows(ctypes.byref(desc), ctypes.byref(rows)) == 0 and rows.value == want
+            assert lib.axc_conv2d_matrix_plan(ctypes.byref(desc), plan) == 0 and plan[0] == 1 and plan[1] > 0
+    finally:
+        ops.set_matrix_rows(0)
+    ops.set_preexpand(-1)
+    try:
+        assert lib.axc_conv2d_matrix_rows(ctypes.byref(desc), ctypes.byref(rows)) == 0 and rows.value == 0
+        assert lib.axc_conv2d_matrix_plan(ctypes.byref(desc), plan) == 0 and list(plan) == [0] * 8
+    finally:
+        ops.set_preexpand(0)
+    assert lib.axc_conv2d_matrix_rows(ctypes.byref(desc), None) == 1
+
+
 def test_workspace_sizes(ops, lib):
     desc = ops.make_desc((64, 56, 56, 64), (3, 3, 64, 64), (1, 1, 1, 1), "SAME")
     rc, n = _ws(lib, desc)

@@ -1790,10 +1790,22 @@ int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8])
     if (rc != AXC_OK)
         return rc;
     const MxPlan &m = pd.mxp;
-    const int32_t v[8] = {pd.mx ? 1 + m.expand + m.swap : 0, m.units, m.units_per_tile, m.n_row_tiles, m.n_col_tiles, m.k_splits, m.grid,
+    const int32_t v[8] = {1, m.units, m.units_per_tile, m.n_row_tiles, m.n_col_tiles, m.k_splits, m.grid,
                           m.k_splits > 1 ? m.fills_per_split : m.fills};
     for (int i = 0; i < 8; ++i)
         plan[i] = pd.mx ? v[i] : 0;
+    return AXC_OK;
+}
+
+int axc_conv2d_matrix_rows(const axc_conv2d_desc *desc, int32_t *rows)
+{
+    if (!rows)
+        return fail(AXC_INVALID_ARGUMENT, "null argument");
+    PreparedDense pd;
+    int rc = prepare_dense(desc, &pd);
+    if (rc != AXC_OK)
+        return rc;
+    *rows = pd.mx ? 1 + pd.mxp.expand + pd.mxp.swap : 0;
     return AXC_OK;
 }
 

@@ -339,10 +339,14 @@ def conv2d_matrix_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding=
     desc = make_desc(tuple(input_shape), tuple(filter_shape), list(strides), padding, (), "NHWC", list(dilations), 8)
     plan = (ctypes.c_int32 * 8)()
     _check(lib.axc_conv2d_matrix_plan(ctypes.byref(desc), plan))
+    rows = ctypes.c_int32()
+    _check(lib.axc_conv2d_matrix_rows(ctypes.byref(desc), ctypes.byref(rows)))
+    if not plan[0]:
+        return None
     # own_rows: 0 = reads pre-expanded rows, 1 = makes them itself in every tile, 2 = the same with the operands exchanged
-    keys = ("own_rows", "units_per_wavefront", "units_per_tile", "row_tiles", "column_tiles", "k_splits", "workgroups",
+    keys = ("units_per_wavefront", "units_per_tile", "row_tiles", "column_tiles", "k_splits", "workgroups",
             "fills_per_split")
-    return dict(zip(keys, [int(v) for v in [plan[0] - 1] + list(plan[1:])])) if plan[0] else None
+    return dict(zip(keys, [int(v) for v in plan[1:]]), own_rows=rows.value - 1)
 
 
 def set_tile_columns(columns):
