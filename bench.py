@@ -313,9 +313,8 @@ def sampled_oracle_check(oracle, table, op, xd, fd, strides, depthwise, y, n_sam
 def dense_kernel_name(kernels_ms):
     """The LUT-GEMM kernel a dense layer ran, by the library's own timers: out of pre-expanded rows with the sums on the
     matrix cores or on the vector ALUs, or expanding inside every tile."""
-    if "lutgemm_mx" in kernels_ms:       # the same launch: the name of all that run out of pre-expanded rows, or that
-        kernels_ms.pop("lutgemm_px", None)   # expand table rows themselves
-        kernels_ms.pop("lutgemm_expand", None)
+    if "lutgemm_mx" in kernels_ms:           # where it reads pre-expanded rows, the same launch: the name of all that do
+        kernels_ms.pop("lutgemm_px", None)
     return next(k for k in ("lutgemm_mx", "lutgemm_px", "lutgemm_expand") if k in kernels_ms)
 
 

@@ -1250,7 +1250,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         m.spin_limit = p.spin_limit;
         m.wait_error = p.wait_error;
         {
-            ProfScope ps("lutgemm_expand", stream, "lutgemm_mx");
+            ProfScope ps("lutgemm_mx", stream);
             AXC_HIP(launch_dense_mx_expand(m, stream));
         }
         {
@@ -1331,7 +1331,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             m.out_i = part;
         }
         {
-            ProfScope ps(mx->expand ? "lutgemm_expand" : "lutgemm_px", stream, "lutgemm_mx");
+            ProfScope ps("lutgemm_mx", stream, mx->expand ? nullptr : "lutgemm_px");
             AXC_HIP(mx->expand ? launch_dense_mx_expand(m, stream) : launch_dense_mx(m, stream));
         }
         if (mx->k_splits > 1) {
