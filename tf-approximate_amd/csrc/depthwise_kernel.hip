@@ -1,5 +1,6 @@
 // Depthwise LUT convolution (channel multiplier 1) and the LDS / VALU rate probes.
 #include "axconv_internal.h"
+#include "depthwise_segments.h"
 
 #include <type_traits>
 
@@ -475,26 +476,15 @@ static hipError_t launch_window(const DepthwiseParams &p, bool out_i32, hipStrea
     const int ngroups = (p.C + CH - 1) / CH;
     const int wgs_per_group = cus / ngroups < 1 ? 1 : cus / ngroups, group_slots = cus / ngroups < 1 ? cus : ngroups;
     const int bands = (p.OH + R - 1) / R;
-    int nseg = 1, seg_len = p.OW;
-    int64_t best = -1;
-    for (int ns = 1; ns <= p.OW; ++ns) {
-        const int sl = (p.OW + ns - 1) / ns;
-        const int ns_eff = (p.OW + sl - 1) / sl;
-        const int64_t tasks = (int64_t)p.N * bands * ns_eff, per_wg = (tasks + wgs_per_group - 1) / wgs_per_group;
-        if (tasks >= (int64_t)1 << 31)
-            continue;
-        const int64_t cost = ((per_wg + kWaves * (64 / CH) - 1) / (kWaves * (64 / CH))) * (sl + KW);
-        if (best < 0 || cost < best) {
-            best = cost;
-            nseg = ns_eff;
-            seg_len = sl;
-        }
-    }
+    const Segments seg = best_segments(p.OW, [&](const int count, const int length) {
+        const int64_t tasks = (int64_t)p.N * bands * count, per_wg = (tasks + wgs_per_group - 1) / wgs_per_group;
+        return tasks < (int64_t)1 << 31 ? (per_wg + kWaves * (64 / CH) - 1) / (kWaves * (64 / CH)) * (length + KW) : (int64_t)-1;
+    });
     constexpr int kLds = (KH * KW + 1) / 2 * CH * 4 * 256;
     const int grid = wgs_per_group * group_slots;
-    return out_i32 ? launch_with_lds(depthwise_lut_window_kernel<KH, KW, S, R, CH, true>, grid, kLds, stream, p, seg_len, nseg,
+    return out_i32 ? launch_with_lds(depthwise_lut_window_kernel<KH, KW, S, R, CH, true>, grid, kLds, stream, p, seg.length, seg.count,
                                      wgs_per_group, group_slots)
-                   : launch_with_lds(depthwise_lut_window_kernel<KH, KW, S, R, CH, false>, grid, kLds, stream, p, seg_len, nseg,
+                   : launch_with_lds(depthwise_lut_window_kernel<KH, KW, S, R, CH, false>, grid, kLds, stream, p, seg.length, seg.count,
                                      wgs_per_group, group_slots);
 }
 
