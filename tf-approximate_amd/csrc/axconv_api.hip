@@ -1526,16 +1526,22 @@ int axc_table_create(const uint16_t *host_table, axc_table **out)
 {
     if (!host_table || !out)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
-    // transpose to weight-code major: tableT[b][a] = T[(a << 8) | b]
-    const size_t entries = (size_t)kTableRows * 256;
-    std::vector<uint16_t> t(3 * entries, 0); // row 256 stays zero: the null weight's row
-    for (int a = 0; a < 256; ++a)
-        for (int b = 0; b < 256; ++b)
-            t[(size_t)b * 256 + a] = host_table[(size_t)a * 256 + b];
-    for (size_t i = 0; i < entries; ++i) {
-        t[entries + i] = t[i] ^ 0x8080u;
-        t[2 * entries + i] = (i < 65536 ? host_table[i] : 0u) ^ 0x8080u;
-    }
+    // weight-code major: tableT[b][a] = T[(a << 8) | b], in squares that the first-level cache holds by row and by column, and
+    // the two flipped copies by whole vectors (us a table with its upload, same machine: entry by entry 143 for the first alone, 181 for three; 42)
+    const size_t entries = (size_t)kTableRows * 256, used = 65536;   // row 256: the null weight's, zeros
+    std::vector<uint16_t> t(3 * entries);
+    uint16_t *const T = t.data(), *const F = T + entries, *const S = F + entries;
+    for (int a0 = 0; a0 < 256; a0 += 16)
+        for (int b0 = 0; b0 < 256; b0 += 16)
+            for (int b = b0; b < b0 + 16; ++b)
+                for (int a = a0; a < a0 + 16; ++a)
+                    T[b * 256 + a] = host_table[a * 256 + b];
+    for (size_t i = 0; i < entries; ++i)
+        F[i] = T[i] ^ 0x8080u;
+    for (size_t i = 0; i < used; ++i)
+        S[i] = host_table[i] ^ 0x8080u;
+    for (size_t i = used; i < entries; ++i)
+        S[i] = 0x8080u;
     axc_table *tab = new axc_table;
     tab->dev_tableT = nullptr;
     hipError_t e = hipGetDevice(&tab->device);
