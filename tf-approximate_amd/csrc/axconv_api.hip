@@ -619,9 +619,9 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, M
     double best_cost = 1e300;
     const int n_col = (co + kMxCols - 1) / kMxCols;
     const int fills = (int)((quads + kMxFillQuads - 1) / kMxFillQuads);
-    const std::vector<int> heights = expand ? std::vector<int>(std::begin(kMxExpandUnits), std::end(kMxExpandUnits))
-                                            : std::vector<int>(std::begin(kMxUnits), std::end(kMxUnits));
-    const int max_units = heights.back();
+    const int *const first_height = expand ? std::begin(kMxExpandUnits) : std::begin(kMxUnits);
+    const int *const last_height = (expand ? std::end(kMxExpandUnits) : std::end(kMxUnits)) - 1;
+    const int max_units = *last_height;
     const int64_t total_units = (groups + 15) / 16;
     const int64_t cap = (int64_t)kMxWaves * max_units;
     const int64_t min_tiles = (total_units + cap - 1) / cap;
@@ -633,22 +633,16 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, M
             continue;
         if (expand ? fills - (ks - 1) * fps < kMxMinExpandFills : ks > 16)
             continue;
-        std::vector<int64_t> cands{min_tiles};
-        for (int64_t rounds = 1; rounds <= 64; ++rounds)
-            for (int64_t n_row : {rounds * cus / ((int64_t)n_col * ks), rounds * cus / ((int64_t)n_col * ks) + 1})
-                if (n_row > min_tiles && n_row <= total_units)
-                    cands.push_back(n_row);
-        if (expand)   // layers too small for whole rounds: whole tiles of every height
-            for (int u : heights)
-                cands.push_back((total_units + (int64_t)kMxWaves * u - 1) / ((int64_t)kMxWaves * u));
-        for (int64_t n_row : cands) {
+        uint64_t seen[2] = {0u, 0u};   // units per tile (at most 100) that have been looked at
+        auto consider = [&](const int64_t n_row) {
             const int64_t upt = (total_units + n_row - 1) / n_row;
-            int units = 0;
-            for (int u : heights)
-                if (!units && (int64_t)u * kMxWaves >= upt)
-                    units = u;
-            if (!units)
-                continue;
+            if (upt > kMxWaves * max_units || (seen[upt >> 6] >> (upt & 63) & 1u))
+                return;
+            seen[upt >> 6] |= (uint64_t)1 << (upt & 63);
+            const int *height = first_height;
+            while ((int64_t)*height * kMxWaves < upt)
+                ++height;
+            const int units = *height;
             const int64_t rows = (total_units + upt - 1) / upt;
             const int64_t tiles = rows * n_col * ks, rounds = (tiles + cus - 1) / cus;
             const double u = units;
@@ -677,29 +671,68 @@ MxPlan compute_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, M
                 best.expand = expand ? 1 : 0;
                 best.cost = (float)cost;
             }
-        }
+        };
+        consider(min_tiles);
+        for (int64_t rounds = 1; rounds <= 64; ++rounds)
+            for (int64_t n_row : {rounds * cus / ((int64_t)n_col * ks), rounds * cus / ((int64_t)n_col * ks) + 1})
+                if (n_row > min_tiles && n_row <= total_units)
+                    consider(n_row);
+        if (expand)   // layers too small for whole rounds: whole tiles of every height
+            for (const int *height = first_height; height <= last_height; ++height)
+                consider((total_units + (int64_t)kMxWaves * *height - 1) / ((int64_t)kMxWaves * *height));
     }
     return best;
 }
 
-MxPlan make_mx_plan(int64_t quads, int co, int64_t groups, int64_t outputs, MxLoads loads, bool expand, bool own_pass, int cus)
+// The same kernel with its operands exchanged (SwapPack), for layers with fewer output pixels than columns; units = 0: not
+// for this layer.
+MxPlan compute_swap_plan(const ConvGeom &g, int cus, double clock_hz)
 {
-    typedef std::tuple<int64_t, int, int64_t, int64_t, MxLoads, bool, bool, int> Key;
+    const SwapPack sp = swap_pack_of(g);
+    const int64_t xq_bytes = (int64_t)sp.quads * sp.pitch * 4, wq_bytes = (int64_t)sp.tiles * sp.fills * kMxCodeBytes;
+    if (g.M > 65536 || xq_bytes >= (int64_t)1 << 30 || wq_bytes >= (int64_t)1 << 30)   // offsets in 31 bits
+        return MxPlan{};
+    MxPlan plan = compute_mx_plan(sp.quads, (int)((g.M + 3) & ~(int64_t)3), sp.pitch / 4, g.M * g.Co, MxLoads::kOne, true, true, cus,
+                                  clock_hz);
+    plan.swap = 1;
+    // both operands packed: two bytes per filter element of every pixel, a byte per weight
+    plan.cost += (float)(((double)wq_bytes / 2.0e6 + (double)xq_bytes / 4.0e6) * 1e-6 * clock_hz);
+    return plan;
+}
+
+struct MxPlans {
+    MxPlan rows, own, swap;   // out of pre-expanded rows, of rows made in the kernel, with its operands exchanged
+};
+
+// All of a layer's plans in one entry: every call looks them up, and three entries cost it a microsecond.
+MxPlans make_mx_plans(const ConvGeom &g, int64_t quads, int64_t groups, MxLoads loads, int cus)
+{
+    struct Key {
+        int64_t quads, groups, m;
+        int k, co, loads, cus;
+        bool operator<(const Key &o) const
+        {
+            return std::tie(quads, groups, m, k, co, loads, cus) < std::tie(o.quads, o.groups, o.m, o.k, o.co, o.loads, o.cus);
+        }
+    };
     static std::mutex mu;
-    static std::map<Key, MxPlan> cache;
-    const Key key{quads, co, groups, outputs, loads, expand, own_pass, cus};
+    static std::map<Key, MxPlans> cache;
+    const Key key{quads, groups, g.M, g.K, g.Co, (int)loads, cus};
     {
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end())
             return it->second;
     }
-    const MxPlan plan = compute_mx_plan(quads, co, groups, outputs, loads, expand, own_pass, cus, device_clock_hz());
+    const double clock_hz = device_clock_hz();
+    const MxPlans plans = {compute_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, false, false, cus, clock_hz),
+                           compute_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, true, false, cus, clock_hz),
+                           compute_swap_plan(g, cus, clock_hz)};
     std::lock_guard<std::mutex> lock(mu);
     if (cache.size() >= 4096)
         cache.clear();
-    cache[key] = plan;
-    return plan;
+    cache[key] = plans;
+    return plans;
 }
 
 XqLayout plain_layout(const ConvGeom &g) { return {g.H, g.W, 0, 0}; }
@@ -784,21 +817,6 @@ struct PreparedDense {
     bool empty;
 };
 
-// The same kernel with its operands exchanged (SwapPack), for layers with fewer output pixels than columns; units = 0: not
-// for this layer.
-MxPlan prepare_swap(const ConvGeom &g)
-{
-    const SwapPack sp = swap_pack_of(g);
-    const int64_t xq_bytes = (int64_t)sp.quads * sp.pitch * 4, wq_bytes = (int64_t)sp.tiles * sp.fills * kMxCodeBytes;
-    if (g.M > 65536 || xq_bytes >= (int64_t)1 << 30 || wq_bytes >= (int64_t)1 << 30)   // offsets in 31 bits
-        return MxPlan{};
-    MxPlan plan = make_mx_plan(sp.quads, (int)((g.M + 3) & ~(int64_t)3), sp.pitch / 4, g.M * g.Co, MxLoads::kOne, true, true, device_cus());
-    plan.swap = 1;
-    // both operands packed: two bytes per filter element of every pixel, a byte per weight
-    plan.cost += (float)(((double)wq_bytes / 2.0e6 + (double)xq_bytes / 4.0e6) * 1e-6 * device_clock_hz());
-    return plan;
-}
-
 // Decides whether the layer runs lutgemm_mx_kernel, and whether out of pre-expanded rows or of rows that it makes itself:
 // what the cost models, fitted to the launch times of each, say is fastest.  Whole op, us, pre-expanded / own rows / other
 // kernels: 3x3 64->64 @56x56x64 201 / 260 / 302, 1x1 128->512 @28x28x64 111 / 135 / 160, 1x1 256->1024 @14x14x64 147 / 148 /
@@ -824,9 +842,8 @@ void prepare_mx(PreparedDense *pd, int forms)
         return;
     const int64_t quads = (int64_t)pd->gk.KH * pd->gk.KW * pd->gk.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
     const MxLoads loads = pitch == 4 ? MxLoads::kOne : pd->flat_row_bytes && pitch <= 16 ? MxLoads::kFourClose : MxLoads::kFour;
-    const MxPlan own = make_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, true, false, device_cus());
-    const MxPlan rows = make_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, false, false, device_cus());
-    MxPlan swap = prepare_swap(g);
+    const MxPlans plans = make_mx_plans(g, quads, groups, loads, device_cus());
+    const MxPlan &own = plans.own, &rows = plans.rows, &swap = plans.swap;
     const double us = 1e-6 * device_clock_hz();
     // Rows beyond some 20 MB for few pixels take 0.19 to 0.23 us a MB of pre-pass where the plan says 0.143 (pre-pass without
     // and with them, us: 5x5 448->48 @28x28x5, 275 MB, 65 / 129; 3x3 864->80 @14x14x41, 320 MB, 113 / 178; 5x5 64->776
