@@ -1,5 +1,5 @@
-"""best_segments (tf-approximate_amd/csrc/depthwise_segments.h) on the host: the choice of a search over every segment count,
-for the cost that the depthwise window kernels have, without looking at every count."""
+"""best_segments (tf-approximate_amd/csrc/depthwise_segments.h) on the host: the choices of searches over every segment
+count, for the costs that the depthwise window kernels have, without looking at every count."""
 import os
 import subprocess
 
@@ -49,6 +49,36 @@ int main()
                             return 1;
                         }
                     }
+    // the 3x3 kernel's rule: 8 to 24 columns, fewer while every task has a wavefront
+    for (long nb : {1L, 3L, 64L, 1217L, 400000L})
+        for (int wgs : {1, 8, 85, 256})
+            for (int ow = 1; ow < 260; ++ow) {
+                auto per_wg = [&](const int count) { return ((int64_t)nb * count + wgs - 1) / wgs; };
+                const Segments got = best_segments(ow, [&](const int count, const int length) {
+                    if (length > 24 || (count > 1 && length < 8 && per_wg(count) > 16))
+                        return (int64_t)-1;
+                    return (per_wg(count) + 15) / 16 * (length + 3);
+                });
+                int count = 1, length = ow;
+                int64_t best = -1;
+                for (int ns = 1; ns <= ow; ++ns) {
+                    const int sl = (ow + ns - 1) / ns, ne = (ow + sl - 1) / sl;
+                    if (ns > 1 && sl < 8 && per_wg(ne) > 16)
+                        break;
+                    if (sl > 24 && (ow + ns) / (ns + 1) >= 8)
+                        continue;
+                    const int64_t c = (per_wg(ne) + 15) / 16 * (sl + 3);
+                    if (best < 0 || c < best) {
+                        best = c;
+                        count = ne;
+                        length = sl;
+                    }
+                }
+                if (got.count != count || got.length != length) {
+                    printf("3x3 nb %ld wgs %d ow %d: %d x %d, not %d x %d\n", nb, wgs, ow, got.count, got.length, count, length);
+                    return 1;
+                }
+            }
     const Segments none = best_segments(9, [](int, int) { return (int64_t)-1; });
     return none.count == 1 && none.length == 9 ? 0 : 1;
 }

@@ -525,27 +525,16 @@ hipError_t launch_depthwise(const DepthwiseParams &p, bool out_i32, int grid, hi
         // product among segments of 8 to 24 columns - shorter ones restart the window too often -, but of any length while
         // every task has a wavefront: there a task's columns are a serial chain, us with 8 columns and more / with any:
         // 8x13x14x224 18.9 / 12.6, 1x20x20x64 16.3 / 11.8, 16x28x28x192 19.1 / 16.1, 64x14x14x384 21.7 / 19.7.
-        int nseg = 1, seg_len = p.OW;
-        int64_t best = -1;
-        for (int ns = 1; ns <= p.OW; ++ns) {
-            const int sl = (p.OW + ns - 1) / ns;
-            const int ns_eff = (p.OW + sl - 1) / sl;
-            const int64_t tasks = (int64_t)p.N * band_pairs * ns_eff;
-            const int64_t per_wg = (tasks + wgs_per_group - 1) / wgs_per_group;
-            if (ns > 1 && sl < 8 && per_wg > kWaves)
-                break;
-            if (sl > 24 && (p.OW + ns) / (ns + 1) >= 8)
-                continue;       // long segments let the wavefronts that share halo rows drift apart (measured: 1 % slower)
-            const int64_t cost = ((per_wg + kWaves - 1) / kWaves) * (sl + 3);
-            if (best < 0 || cost < best) {
-                best = cost;
-                nseg = ns_eff;
-                seg_len = sl;
-            }
-        }
+        // Beyond 24, the wavefronts that share halo rows drift apart (measured: 1 % slower).
+        const Segments seg = best_segments(p.OW, [&](const int count, const int length) {
+            const int64_t tasks = (int64_t)p.N * band_pairs * count, per_wg = (tasks + wgs_per_group - 1) / wgs_per_group;
+            if (length > 24 || (count > 1 && length < 8 && per_wg > kWaves))
+                return (int64_t)-1;
+            return (per_wg + kWaves - 1) / kWaves * (length + 3);
+        });
         const int g3 = wgs_per_group * group_slots;
 #define AXC_DW_LAUNCH_AS(S_, R_, I32_, FQ_, EPI_)                                                                     \
-    launch_with_lds(depthwise_lut3x3_kernel<S_, R_, I32_, FQ_, EPI_>, g3, kDwLdsBytes, stream, p, seg_len, nseg,         \
+    launch_with_lds(depthwise_lut3x3_kernel<S_, R_, I32_, FQ_, EPI_>, g3, kDwLdsBytes, stream, p, seg.length, seg.count, \
                     wgs_per_group, group_slots)
 #define AXC_DW_LAUNCH(S_, R_)                                                                                        \
     (out_i32    ? AXC_DW_LAUNCH_AS(S_, R_, true, false, false)                                                           \
