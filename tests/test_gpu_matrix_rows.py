@@ -219,3 +219,117 @@ def test_two_layers_in_turn(pkg, own_rows):
     for _ in range(3):
         for op, xd, fd, want in layers:
             assert torch.equal(op(xd, fd, *MM), want)
+
+
+# sizes that the planner would not give this form to: many pixels, up to the bounds of compute_swap_plan (65536 pixels, packed
+# codes of 1 GiB on either side)
+SWAPPED_FAR = [
+    ((3, 57, 61, 24), (3, 3, 44), 1, 1, "SAME"),         # 10431 pixels
+    ((16, 64, 64, 4), (3, 3, 12), 1, 1, "SAME"),         # 65536
+    ((16, 64, 64, 908), (3, 3, 8), 1, 1, "SAME"),        # ... of 8172 elements: 1.07 GB of packed codes
+    ((1, 2, 2, 1820), (3, 3, 65536), 1, 1, "SAME"),      # and as much on the filter's side
+]
+
+
+@pytest.mark.parametrize("case", SWAPPED_FAR, ids=_id)
+def test_operands_exchanged_up_to_the_bounds(pkg, oracle, swapped, case):
+    plan = _plan(swapped, case)
+    assert plan is not None and plan["own_rows"] == 2, plan
+    _compare(pkg, oracle, swapped, case)
+
+
+# input, filter, stride, the launch behind the lookups in the exchanged form
+CODES = [
+    ((3, 14, 14, 48), (3, 3, 48, 40), 1, "SAME"),
+    ((2, 15, 13, 64), (3, 3, 64, 24), 2, "VALID"),
+    ((2, 14, 14, 130), (1, 1, 130, 36), 2, "SAME"),      # strided 1x1: codes gathered first
+    ((4, 7, 7, 256), (1, 1, 256, 64), 1, "SAME"),        # images that count as one row
+]
+
+
+@pytest.mark.parametrize("mode", [2, 3])
+@pytest.mark.parametrize("xs,fs,stride,padding", CODES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_codes_as_given(pkg, oracle, own_rows, xs, fs, stride, padding, mode):
+    """conv2d_codes_acc_i32 in both forms: the same sums as the kernel that expands inside its tiles, and as the oracle's."""
+    print("case", xs, fs, stride, padding, mode, flush=True)
+    ops = own_rows
+    ops.set_matrix_rows(mode)
+    plan = ops.conv2d_matrix_plan(xs, fs, (1, stride, stride, 1), padding)
+    assert plan is not None and plan["own_rows"] == mode - 1, plan
+    rng = np.random.RandomState(sum(xs))
+    x, f = rng.randint(0, 256, xs).astype(np.uint8), rng.randint(0, 256, fs).astype(np.uint8)
+    host_table = pkg.synth.table_random(9)
+    table = ops.TruthTable(host_table)
+    xd, fd = torch.from_numpy(x).to("cuda:0"), torch.from_numpy(f).to("cuda:0")
+
+    def run():
+        return ops.conv2d_codes_acc_i32(table, xd, fd, 77, (1, stride, stride, 1), padding)
+    ops.profile_enable(True)
+    ops.profile_reset()
+    try:
+        got = run()
+        names = set(ops.profile_read())
+    finally:
+        ops.profile_enable(False)
+    assert {k for k in names if k.startswith("lutgemm")} == {"lutgemm_mx"} and ("swap_pack" in names) == (mode == 3), names
+    ops.set_preexpand(-1)
+    try:
+        want = run()
+    finally:
+        ops.set_preexpand(0)
+    assert torch.equal(got, want)
+    patches = refimpl.gather_patches(x, 77, fs[0], fs[1], (stride, stride), padding, (1, 1))
+    assert np.array_equal(got.cpu().numpy().reshape(-1, fs[3]),
+                          oracle.lut_gemm_codes(host_table, patches.reshape(-1, fs[0] * fs[1] * fs[2]), f.reshape(-1, fs[3])))
+
+
+@pytest.mark.parametrize("mode", [2, 3])
+@pytest.mark.parametrize("xs,fs,stride", [((2, 14, 14, 64), (1, 1, 64, 8), 5), ((1, 13, 11, 40), (3, 3, 40, 12), 4)],
+                         ids=["1x1", "3x3"])
+def test_integer_op_with_a_padding_origin_of_its_own(pkg, oracle, own_rows, xs, fs, stride, mode):
+    """The tf1 op in both forms; its windows begin behind the image's first pixel (1x1: a padding of -1)."""
+    print("case", xs, fs, stride, mode, flush=True)
+    ops = own_rows
+    ops.set_matrix_rows(mode)
+    rng = np.random.RandomState(sum(xs) + mode)
+    x, f = rng.randint(0, 256, xs).astype(np.uint8), rng.randint(0, 256, fs).astype(np.uint8)
+    table = pkg.synth.table_random(4)
+    ops.profile_enable(True)
+    ops.profile_reset()
+    try:
+        out, _, _ = ops.ax_conv2d(torch.from_numpy(x).to("cuda:0"), torch.from_numpy(f).to("cuda:0"), *MM,
+                                  [1, stride, stride, 1], "SAME", ops.TruthTable(table))
+        names = set(ops.profile_read())
+    finally:
+        ops.profile_enable(False)
+    assert {k for k in names if k.startswith("lutgemm")} == {"lutgemm_mx"}, names
+    off_in = ops.float_to_quantized_unclamped_quint8(0.0, MM[0], MM[1])
+    off_f = ops.float_to_quantized_unclamped_quint8(0.0, MM[2], MM[3])
+    assert np.array_equal(out.cpu().numpy(), oracle.axconv2d_tf1(table, x, f, off_in, off_f, stride, "SAME"))
+
+
+@pytest.mark.parametrize("mode", [2, 3])
+def test_a_wait_that_runs_out_is_reported_by_the_next_call(pkg, own_rows, mode):
+    """With a wait limit of zero polls every wavefront leaves the kernel (tests/test_lookup_mx_expand.py follows them), the
+    launch returns as usual, the next call on the device reports it, once, and with the limit restored the layer is right."""
+    ops = own_rows
+    ops.set_matrix_rows(mode)
+    xs, fs = (8, 32, 32, 64), (3, 3, 64, 64)
+    plan = ops.conv2d_matrix_plan(xs, fs)
+    assert plan is not None and plan["own_rows"] == mode - 1, plan
+    xd, fd = bench.device_tensors(pkg, xs, fs, "uniform", seed=1)
+    op = pkg.ApproxConv2DWithMinMaxVars([1, 1, 1, 1], 8, pkg.synth.table_random(2), "SAME")
+    good = op.accumulators(xd, fd, *MM).clone()
+    torch.cuda.synchronize()
+    ops.set_wait_limit(0)
+    try:
+        print("launch with a wait limit of 0 polls", flush=True)
+        op.accumulators(xd, fd, *MM)
+        torch.cuda.synchronize()
+    finally:
+        ops.set_wait_limit(1 << 20)
+    with pytest.raises(RuntimeError, match="gave up a wait"):
+        op.accumulators(xd, fd, *MM)
+    again = op.accumulators(xd, fd, *MM)
+    torch.cuda.synchronize()
+    assert torch.equal(again, good)

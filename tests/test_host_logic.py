@@ -199,6 +199,50 @@ def test_strided_pixel_groups_stay_in_the_workspace(ops):
     assert seen > 10
 
 
+def test_strided_pixel_groups_of_own_rows_stay_in_the_workspace(ops):
+    """The same where the kernel makes its rows itself: no rows lie behind the quantized input then, but the layer entry
+    point's minima and maxima (32 KiB) do."""
+    ops.set_matrix_rows(2)
+    try:
+        for xs, fs, pitch_of_one in [((1, 3, 9000, 32), (1, 2, 32, 8), 4), ((1, 2, 20000, 64), (1, 2, 64, 24), 4),
+                                     ((2, 40, 32000, 2), (7, 9, 2, 16), 2)]:
+            for stride, inside in ((32768 // (3 * pitch_of_one), True), (32768 // (3 * pitch_of_one) + 1, False)):
+                plan = ops.conv2d_matrix_plan(xs, fs, (1, 1, stride, 1))
+                assert (plan is not None and plan["own_rows"] == 1) == inside, (xs, fs, stride, plan)
+    finally:
+        ops.set_matrix_rows(0)
+
+
+@pytest.mark.parametrize("xs,co,padding,rows", [
+    ((64, 7, 7, 512), 2048, "SAME", 4),        # rows of four images, of two, of one
+    ((64, 15, 17, 132), 128, "VALID", 4),
+    ((66, 10, 21, 256), 256, "SAME", 2),
+    ((64, 14, 14, 1024), 256, "SAME", 1),
+    ((66, 7, 7, 512), 2048, "SAME", 0),        # 66 images of 7x7 are no fours
+    ((64, 14, 14, 124), 256, "SAME", 0),       # too few channels
+    ((64, 16, 18, 126), 256, "SAME", 0),       # not in fours
+    ((64, 12, 14, 128), 256, "SAME", 0),       # 168 pixels: too few
+    ((64, 15, 19, 128), 256, "SAME", 0),       # 1140 of four images: too many
+])
+@pytest.mark.parametrize("stride", [1, 2])
+def test_images_that_count_as_one_row(ops, xs, co, padding, rows, stride):
+    """1x1 layers whose images have no whole groups of four pixels a row: 64-pixel units of whole images where `rows` of them
+    count as one row, of single rows with their last groups incomplete elsewhere.  (Stride 2: the same pixels, gathered.)"""
+    n, h, w, c = xs
+    groups = n * h * w // 4 if rows else n * h * ((w + 3) // 4)
+    units = -(-groups // 16)
+    ops.set_matrix_rows(2)
+    try:
+        plan = ops.conv2d_matrix_plan((n, h * stride, w * stride, c), (1, 1, c, co), (1, stride, stride, 1), padding)
+    finally:
+        ops.set_matrix_rows(0)
+    assert plan is not None
+    upt = plan["units_per_tile"]
+    assert plan["row_tiles"] == -(-units // upt), (plan, units)
+    other = -(-(n * h * ((w + 3) // 4) if rows else n * h * w // 4) // 16)
+    assert plan["row_tiles"] != -(-other // upt) or upt != -(-other // plan["row_tiles"]), (plan, units, other)
+
+
 @pytest.fixture()
 def pre_expanded_rows(ops):
     ops.set_matrix_rows(1)

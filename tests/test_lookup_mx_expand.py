@@ -143,7 +143,7 @@ class Wave:
         whole = lambda f: 4 * (2 * (f >> 1) + 1)
         self.s = {"gf": gf, "cbcur": CB + 4 * (gf & 1), "cboth": CB + 4 * other, "left": count, "enext": enext,
                   "free": 0 if gf == 0 else 4 * (2 * ((gf - 1) >> 1) + 2), "whole": whole(gf + 1) if count > 1 else 0,
-                  "whole0": whole(gf), "eoff": after & 0x7fffffff, "cb0": CB, "spin": 1 << 20, "rowb": 512,
+                  "whole0": whole(gf), "eoff": after & 0x7fffffff, "cb0": CB, "spin": g.spin, "rowb": 512,
                   "lo": 0x05040100, "hi": 0x07060302, "c4": p.c4, "kwn": p.kw, "p1": p.pitch, "p2": 2 * p.pitch, "p3": 3 * p.pitch}
         taps = 4 // p.c4
         dq, dkw = 4 % p.c4, taps % p.kw
@@ -287,8 +287,13 @@ class Wave:
 
     def end_tile(self):
         g, p = self.g, self.g.p
-        check(self.s["fail"] == 0, "a wait has run out")
         check(not self.vm and not self.lds, "operations in flight at the end")
+        if self.s["fail"] and g.spin == 0:       # as the kernel does: tell the others, and leave
+            g.counter[2] = 1
+            g.gave_up += 1
+            self.done = True
+            return
+        check(self.s["fail"] == 0, "a wait has run out")
         ct, f0, count = g.tiles[self.tile]
         for u in range(p.units):
             lo, hi = p.sums(self.index, u, ct, f0, count)
@@ -308,8 +313,8 @@ class Wave:
 
 
 class Group:
-    def __init__(self, problem, tiles, rng, mutate=None):
-        self.p, self.tiles = problem, tiles
+    def __init__(self, problem, tiles, rng, mutate=None, spin=1 << 20):
+        self.p, self.tiles, self.spin, self.gave_up = problem, tiles, spin, 0
         lines = re.findall(r'"([^"]*)\\n\\t"', gen.emit(problem.units, problem.vec, expand=True))
         self.lines = mutate(lines) if mutate else lines
         self.at = {x[:-1]: i for i, x in enumerate(self.lines) if x.endswith(":")}
@@ -366,6 +371,21 @@ def test_sums_of_four_wavefronts(variant, tiles):
 @pytest.mark.parametrize("variant", [v for v in gen.XVARIANTS if v[1] == (v[0] % 4 == 0) or v[0] in (2, 3)], ids=str)
 def test_sums_of_four_wavefronts_in_every_height(variant):
     run(variant, TILES["two tiles"], seed=variant[0], fills=3)
+
+
+@pytest.mark.parametrize("variant", [(2, True), (3, False), (6, True)], ids=str)
+def test_waits_of_no_further_polls_end_in_every_wavefront(variant):
+    """With a limit of zero polls a wavefront that looks too early gives up, and whoever waits for it does too: all of them
+    leave, with nothing in flight."""
+    gave_up = 0
+    for seed in range(6):
+        rng = random.Random(seed)
+        with np.errstate(over="ignore"):
+            group = Group(Problem(rng, variant[0], variant[1], 4, 2), [(1, 0, 4), (0, 0, 3)], rng, spin=0)
+            group.run(rng)
+        assert all(w.done for w in group.waves)
+        gave_up += group.gave_up
+    assert gave_up > 0
 
 
 def without(pattern):
