@@ -26,6 +26,10 @@ CASES = [
     ((2, 7, 9, 16), 3, 3, 8, 1, "VALID", 0),
     ((2, 7, 9, 12), 3, 3, 8, 1, "VALID", 0),           # below four quads: no batches
     ((1, 5, 6, 1100), 3, 3, 8, 1, "SAME", 0),          # 275 quads: 275 of 512 threads copy
+    ((128, 47, 47, 28), 1, 1, 8, 1, "SAME", 0),        # bands of one row: one item a thread
+    ((1200, 1, 30, 67), 1, 1, 8, 1, "SAME", 0),
+    ((20, 30, 214, 12), 1, 1, 8, 1, "SAME", 0),        # three
+    ((30, 30, 94, 12), 3, 3, 8, 1, "SAME", 0),         # six
 ]
 
 

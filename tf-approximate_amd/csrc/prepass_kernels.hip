@@ -458,7 +458,10 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
         // 16-byte loads in flight at a time.  The loads are unconditional (coordinates clamped into the image, the
         // result replaced by zeros afterwards) so that each store waits for its own load only.
         // A narrow image leaves most threads without a column: they then take further rows (rpar rows side by side).
-        constexpr int kInFlight = 16;
+        // (Fewer in flight where a thread has fewer items: index arithmetic, selects and quantization of sixteen were most of
+        // what the workgroups of one-row bands did, pre-pass in us with sixteen / as here: 1x1 28->8 @47x47x128 74 / 44, 12->8
+        // @153x153x68 122 / 74, 32->16 @94x94x86 57 / 43.  Leaving the loops of sixteen early instead makes the first store
+        // wait for every load: 3x3 64->64 @56x56x64 32 / 62.)
         const int q = t % g.C4, wstep = nthreads / g.C4;
         const int rpar = wstep >= 2 * wc ? wstep / wc : 1;
         int w0 = t / g.C4, r0 = 0;
@@ -469,44 +472,53 @@ __device__ __forceinline__ void patch_sums_rows_body(const float *__restrict__ x
         const int wsteps = rpar > 1 ? 1 : (wc + wstep - 1) / wstep;
         const int iters = ((in_rows + rpar - 1) / rpar) * wsteps;
         const float *const xn = x + (int64_t)n * g.H * g.W * g.C;
-        int r_next = r0, ws_next = 0; // (row, column step) of the next item
-        for (int it0 = 0; it0 < iters; it0 += kInFlight) {
-            float4 v[kInFlight];
-            int rr[kInFlight], ww[kInFlight];
+        auto copy_items = [&](auto in_flight) __attribute__((always_inline)) {
+            constexpr int kInFlight = decltype(in_flight)::value;
+            int r_next = r0, ws_next = 0; // (row, column step) of the next item
+            for (int it0 = 0; it0 < iters; it0 += kInFlight) {
+                float4 v[kInFlight];
+                int rr[kInFlight], ww[kInFlight];
 #pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
-                rr[u] = r_next;
-                ww[u] = w0 + ws_next * wstep;
-                if (++ws_next == wsteps) {
-                    ws_next = 0;
-                    r_next += rpar;
+                for (int u = 0; u < kInFlight; ++u) {
+                    rr[u] = r_next;
+                    ww[u] = w0 + ws_next * wstep;
+                    if (++ws_next == wsteps) {
+                        ws_next = 0;
+                        r_next += rpar;
+                    }
+                    int ih = ih_first + rr[u];
+                    ih = ih < 0 ? 0 : (ih >= g.H ? g.H - 1 : ih);
+                    const int wcl = iw_lo + (ww[u] < wc ? ww[u] : wc - 1);
+                    v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    if (it0 + u < iters)   // the same for the whole workgroup: no load for items nobody has
+                        v[u] = load_quad(xn + ((int64_t)ih * g.W + wcl) * g.C, q);
                 }
-                int ih = ih_first + rr[u];
-                ih = ih < 0 ? 0 : (ih >= g.H ? g.H - 1 : ih);
-                const int wcl = iw_lo + (ww[u] < wc ? ww[u] : wc - 1);
-                v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (it0 + u < iters)   // the same for the whole workgroup: no load for items nobody has
-                    v[u] = load_quad(xn + ((int64_t)ih * g.W + wcl) * g.C, q);
-            }
 #pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
-                const int ih = ih_first + rr[u];
-                const bool in_image = (unsigned)ih < (unsigned)g.H;
-                float4 f = settle_quad(v[u], q);
-                if (!in_image)
-                    f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // rows outside the image are zeros
-                if (it0 + u < iters && rr[u] < in_rows && ww[u] < wc) {
-                    *reinterpret_cast<float4 *>(&rows[(rr[u] * wc + ww[u]) * pitch + q * 4]) = f;
-                    const int iw = iw_lo + ww[u];
-                    if (xq && in_image && ih >= own_lo && ih < own_hi && (!SEG || (iw >= own_clo && iw < own_chi)))
-                        xq_n[((uint32_t)ih * (uint32_t)g.C4 + (uint32_t)q) * (uint32_t)lay.Wp + (uint32_t)iw] =
-                            phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
-                            (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
-                            (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
-                            (phys_row(quantize_code(f.w, qt.offset, qt.inv_scale)) << 24);
+                for (int u = 0; u < kInFlight; ++u) {
+                    const int ih = ih_first + rr[u];
+                    const bool in_image = (unsigned)ih < (unsigned)g.H;
+                    float4 f = settle_quad(v[u], q);
+                    if (!in_image)
+                        f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // rows outside the image are zeros
+                    if (it0 + u < iters && rr[u] < in_rows && ww[u] < wc) {
+                        *reinterpret_cast<float4 *>(&rows[(rr[u] * wc + ww[u]) * pitch + q * 4]) = f;
+                        const int iw = iw_lo + ww[u];
+                        if (xq && in_image && ih >= own_lo && ih < own_hi && (!SEG || (iw >= own_clo && iw < own_chi)))
+                            xq_n[((uint32_t)ih * (uint32_t)g.C4 + (uint32_t)q) * (uint32_t)lay.Wp + (uint32_t)iw] =
+                                phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
+                                (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
+                                (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
+                                (phys_row(quantize_code(f.w, qt.offset, qt.inv_scale)) << 24);
+                    }
                 }
             }
-        }
+        };
+        if (iters == 1)
+            copy_items(std::integral_constant<int, 1>());
+        else if (iters <= 4)
+            copy_items(std::integral_constant<int, 4>());
+        else
+            copy_items(std::integral_constant<int, 16>());
     } else {
         const int quads_per_row = wc * g.C4;
         const int total = in_rows * quads_per_row;
