@@ -269,6 +269,33 @@ def test_matrix_core_kernel_where_it_was_measured_faster(ops):
         assert (plan is not None) == faster, (xs, fs, plan)
 
 
+@pytest.mark.parametrize("xs,fs,rows", [
+    ((64, 56, 56, 64), (3, 3, 64, 64), 1),            # 184 / 229 / 336
+    ((64, 28, 28, 128), (1, 1, 128, 512), 1),         # 103 / 117 / 170
+    ((85, 31, 31, 228), (1, 1, 228, 656), 1),         # 420 / 451 / 589
+    ((64, 7, 7, 512), (3, 3, 512, 512), 2),           # 368 / 241 / 368
+    ((64, 14, 14, 256), (3, 3, 256, 256), 2),         # 333 / 236 / 349
+    ((4, 14, 14, 797), (3, 3, 797, 38), 2),           # 160 / 128 / 190
+    ((1, 18, 18, 216), (5, 5, 216, 160), 2),          # - / 75 / 123
+    ((1, 7, 7, 512), (3, 3, 512, 512), 3),            # 151 / 110 / 151, exchanged 45
+    ((1, 7, 7, 512), (1, 1, 512, 2048), 3),           # 69 / 47 / 69, exchanged 27
+    ((20, 16, 8, 130), (3, 3, 130, 1248), 3),         # - / 235 / 344, exchanged 196
+    # one or two fills: where outputs are stored faster
+    ((10, 139, 139, 10), (1, 1, 10, 976), 0),         # 466 / - / 246
+    ((72, 61, 61, 11), (1, 1, 11, 720), 0),           # 445 / - / 245
+    ((8, 80, 80, 18), (1, 1, 18, 144), 0),            # 40 / - / 31
+    ((9, 125, 125, 11), (1, 1, 11, 431), 1),          # 136 / - / 355
+    ((1, 176, 176, 8), (1, 1, 8, 1524), 1),           # 97 / - / 198
+    ((1, 222, 222, 16), (1, 1, 16, 660), 1),          # 93 / - / 149
+])
+def test_the_planners_choice_where_it_is_far_from_the_line(ops, lib, xs, fs, rows):
+    """Layers timed in every form (whole op, us: pre-expanded rows / own rows / sums on the vector ALUs), a fifth or more
+    apart."""
+    desc, got = ops.make_desc(xs, fs, (1, 1, 1, 1), "SAME"), ctypes.c_int32(-1)
+    assert lib.axc_conv2d_matrix_rows(ctypes.byref(desc), ctypes.byref(got)) == 0
+    assert got.value == rows
+
+
 def test_matrix_plan_says_yes_or_no_in_every_form(ops, lib):
     """plan[0] of axc_conv2d_matrix_plan is 1 whichever rows the kernel reads; axc_conv2d_matrix_rows says which."""
     desc = ops.make_desc((3, 14, 14, 64), (1, 1, 64, 8), (1, 1, 1, 1), "SAME")

@@ -841,21 +841,23 @@ void prepare_mx(PreparedDense *pd, int forms)
     if (3 * pitch > 65536)
         return;
     const int64_t quads = (int64_t)pd->gk.KH * pd->gk.KW * pd->gk.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
+    const int64_t fills = (quads + kMxFillQuads - 1) / kMxFillQuads;
     const MxLoads loads = pitch == 4 ? MxLoads::kOne : pd->flat_row_bytes && pitch <= 16 ? MxLoads::kFourClose : MxLoads::kFour;
     const MxPlans plans = make_mx_plans(g, quads, groups, loads, device_cus());
     const MxPlan &own = plans.own, &rows = plans.rows, &swap = plans.swap;
     const double us = 1e-6 * device_clock_hz();
     // Rows beyond some 20 MB for few pixels take 0.19 to 0.23 us a MB of pre-pass where the plan says 0.143 (pre-pass without
     // and with them, us: 5x5 448->48 @28x28x5, 275 MB, 65 / 129; 3x3 864->80 @14x14x41, 320 MB, 113 / 178; 5x5 64->776
-    // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Channel counts that are no multiple of four keep 0.2,
-    // fitted while their patch sums read memory pixel by pixel, as below 64 channels they still do (3x3 797->38 @14x14x4, 147 MB:
-    // pre-pass 892 -> 1150 us then).
+    // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Channel counts below 64 that are no multiple of four have a patch-sum kernel of
+    // their own, which they delay by more: 0.2 (whole op without and with them, us: 3x3/2 14->704 @53x168x52, 540 / 563; but 1x1
+    // 226->656 @31x31x85 1124 / 612, which 0.2 from 64 channels on kept off them).
+    // (Mode 1 keeps the rule it was fitted with, 0.2 for all of them.)
+    const int mode = forms == kMxRows ? 1 : g_mx_rows.load(std::memory_order_relaxed);
     const double rows_bytes = (double)rows.n_col_tiles * rows.fills * 65536.0;
-    const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) ? 0.2e-6 : 0.07e-6) * us;
+    const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) && (g.C < 64 || mode == 1) ? 0.2e-6 : 0.07e-6) * us;
     const bool rows_ok = forms != kMxOwnRows && rows.units && rows_bytes <= (double)kPxMaxBytes;
     const bool own_ok = own.units && 3 * pitch <= (int64_t)(4 * kMinMaxBlocks * sizeof(float)) &&
                         (int64_t)own.n_col_tiles * own.fills * kMxCodeBytes < ((int64_t)1 << 31);
-    const int mode = forms == kMxRows ? 1 : g_mx_rows.load(std::memory_order_relaxed);
     bool expand = own_ok;
     if (mode == 3 && swap.units) {
         pd->mx = true;
@@ -867,26 +869,32 @@ void prepare_mx(PreparedDense *pd, int forms)
             return;
         expand = false;
     } else if (mode == 0) {
+        // Outputs that are many for few fills are bound by their stores, which leave this kernel, 32 bytes of eight columns at a
+        // time, at 2.0 TB/s at best, the vector-ALU kernels at 3.0 where their pieces of 16 columns are whole lines of 64
+        // bytes, 1.4 where they only come in fours, 0.65 else (TB/s, here / there: 1x1 10->976 @139x139x10 1.62 / 3.04, 11->720
+        // @61x61x72 1.73 / 3.15, 16->660 of 49 284 pixels 1.40 / 0.87, 8->1524 of 30 976 1.94 / 0.95, 11->431 @125x125x9 1.79 /
+        // 0.68).  Before this one had a bound too, the first of these took 466 us instead of 250, the second 447 instead of 245.
+        const double bytes = (double)g.M * g.Co * 4.0, store = bytes / 2.0e6 * us;
+        const double store_other = bytes / ((g.Co & 3) ? 0.65e6 : (g.Co & 15) ? 1.4e6 : 3.0e6) * us;
+        const double own_cost = std::max((double)own.cost, store);
         // What the plan of pre-expanded rows leaves out: a K split is a little cheaper, and under short chains of patch sums
         // the first 10 MB of rows delay the launch that carries them (pre-pass without and with rows, us: 1x1 64->256
         // @56x56x9, 8 MB, 9.0 / 14.9; 1x1 128->512 @28x28x9, 34 MB, 8.5 / 23.4; but 3x3 64->64 @8x8x128, 19 MB, 12.0 / 14.3).
         // (and loads a few bytes apart are cheaper than planned)
-        const double rows_cost = rows.cost * (loads == MxLoads::kFourClose ? 0.85 : 1.0) + slow_rows + (1.5 + (g.K <= 256 ? 0.35e-6 : 0.0) * std::min(rows_bytes, 10e6) -
-                                                          (rows.k_splits > 1 ? 2.6 : 0.0)) * us;
-        expand = own_ok && (!rows_ok || own.cost < rows_cost);
-        // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), and lower
-        // where outputs are many for few fills: their stores leave at 2.2 TB/s at best, 0.65 where columns do not come in
-        // fours (1x1 8->1808 @78x78x4, 176 MB: 151 us where the model says 39; 1x1 16->342 @38x38x38, 75 MB, 131, 16; 3x3
-        // 11->170 @220x220x25, 823 MB, 1924, 961).
-        const double other = std::max(pd->plan.cost * (pd->plan.px ? 1.12 : 1.06) + 5.0 * us,
-                                      (double)g.M * g.Co * 4.0 / ((g.Co & 3) ? 0.65e6 : 2.2e6) * us);
-        const double best = std::min(expand ? (double)own.cost : rows_ok ? rows_cost : 1e30, other);
-        if (swap.units && swap.cost < best) {
+        const double rows_cost = std::max(rows.cost * (loads == MxLoads::kFourClose ? 0.85 : 1.0) + slow_rows, store) +
+                                 (1.5 + (g.K <= 256 ? 0.35e-6 : 0.0) * std::min(rows_bytes, 10e6) - (rows.k_splits > 1 ? 2.6 : 0.0)) * us;
+        expand = own_ok && (!rows_ok || own_cost < rows_cost);
+        const double mine = expand ? own_cost : rows_ok ? rows_cost : 1e30;
+        // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), but hardly for
+        // one or two fills stored in whole lines (1x1 18->144 @80x80x8 30.5 us there, 33.2 here, predicted 14.7 and 16.6).
+        const double left_out = fills <= 2 && (g.Co & 15) == 0 ? 1.0 : 5.0;
+        const double other = std::max(pd->plan.cost * (pd->plan.px ? 1.12 : 1.06) + left_out * us, store_other);
+        if (swap.units && swap.cost < std::min(mine, other)) {
             pd->mx = true;
             pd->mxp = swap;
             return;
         }
-        if ((expand ? own.cost : rows_cost) > other)
+        if (mine > other)
             return;
     }
     if (!expand && !rows_ok)
