@@ -287,6 +287,10 @@ def test_matrix_core_kernel_where_it_was_measured_faster(ops):
     ((9, 125, 125, 11), (1, 1, 11, 431), 1),          # 136 / - / 355
     ((1, 176, 176, 8), (1, 1, 8, 1524), 1),           # 97 / - / 198
     ((1, 222, 222, 16), (1, 1, 16, 660), 1),          # 93 / - / 149
+    ((32, 28, 28, 16), (1, 1, 16, 1192), 1),          # 52 / - / 83
+    ((64, 56, 56, 32), (1, 1, 32, 512), 1),           # 171 / - / 207
+    ((32, 56, 56, 14), (1, 1, 14, 512), 1),           # 73 / - / 93
+    ((64, 112, 112, 12), (1, 1, 12, 256), 0),         # as 12->384 of 460800 pixels: 324 / - / 221
 ])
 def test_the_planners_choice_where_it_is_far_from_the_line(ops, lib, xs, fs, rows):
     """Layers timed in every form (whole op, us: pre-expanded rows / own rows / sums on the vector ALUs), a fifth or more

@@ -869,13 +869,14 @@ void prepare_mx(PreparedDense *pd, int forms)
             return;
         expand = false;
     } else if (mode == 0) {
-        // Outputs that are many for few fills are bound by their stores, which leave this kernel, 32 bytes of eight columns at a
-        // time, at 2.0 TB/s at best, the vector-ALU kernels at 3.0 where their pieces of 16 columns are whole lines of 64
-        // bytes, 1.4 where they only come in fours, 0.65 else (TB/s, here / there: 1x1 10->976 @139x139x10 1.62 / 3.04, 11->720
-        // @61x61x72 1.73 / 3.15, 16->660 of 49 284 pixels 1.40 / 0.87, 8->1524 of 30 976 1.94 / 0.95, 11->431 @125x125x9 1.79 /
-        // 0.68).  Before this one had a bound too, the first of these took 466 us instead of 250, the second 447 instead of 245.
-        const double bytes = (double)g.M * g.Co * 4.0, store = bytes / 2.0e6 * us;
-        const double store_other = bytes / ((g.Co & 3) ? 0.65e6 : (g.Co & 15) ? 1.4e6 : 3.0e6) * us;
+        // Outputs that are many for few fills are bound by their stores.  The vector-ALU kernels' leave at 3.0 TB/s at best where
+        // their pieces of 16 columns are whole lines of 64 bytes, 1.3 where they only come in fours, 0.65 else, whatever their
+        // number; this kernel's, 32 bytes of eight columns at a time, as fast as its tiles are done while the memory-side cache
+        // (256 MB) takes them in, at 2.0 beyond.  us here / there: 16->1192 @28x28x32, 120 MB, 52 / 83; 8->1524 of 30 976 pixels,
+        // 189 MB, 97 / 198; 14->512 @56x56x32, 206 MB, 73 / 93; 11->431 @125x125x9, 242 MB, 136 / 355; but 12->384 of 460 800, 708
+        // MB, 324 / 221, and 10->976 @139x139x10, 754 MB, 466 / 246, which came here while this kernel had no bound.
+        const double bytes = (double)g.M * g.Co * 4.0, store = bytes > 256e6 ? bytes / 2.0e6 * us : 0.0;
+        const double store_other = bytes / ((g.Co & 3) ? 0.65e6 : (g.Co & 15) ? 1.3e6 : 3.0e6) * us;
         const double own_cost = std::max((double)own.cost, store);
         // What the plan of pre-expanded rows leaves out: a K split is a little cheaper, and under short chains of patch sums
         // the first 10 MB of rows delay the launch that carries them (pre-pass without and with rows, us: 1x1 64->256
@@ -885,9 +886,9 @@ void prepare_mx(PreparedDense *pd, int forms)
                                  (1.5 + (g.K <= 256 ? 0.35e-6 : 0.0) * std::min(rows_bytes, 10e6) - (rows.k_splits > 1 ? 2.6 : 0.0)) * us;
         expand = own_ok && (!rows_ok || own_cost < rows_cost);
         const double mine = expand ? own_cost : rows_ok ? rows_cost : 1e30;
-        // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), but hardly for
-        // one or two fills stored in whole lines (1x1 18->144 @80x80x8 30.5 us there, 33.2 here, predicted 14.7 and 16.6).
-        const double left_out = fills <= 2 && (g.Co & 15) == 0 ? 1.0 : 5.0;
+        // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), less so for one or
+        // two fills and few outputs in whole lines (1x1 18->144 @80x80x8 40 us here, 31 there, predicted 16.6 and 14.7).
+        const double left_out = fills <= 2 && (g.Co & 15) == 0 && bytes < 60e6 ? 2.0 : 5.0;
         const double other = std::max(pd->plan.cost * (pd->plan.px ? 1.12 : 1.06) + left_out * us, store_other);
         if (swap.units && swap.cost < std::min(mine, other)) {
             pd->mx = true;
