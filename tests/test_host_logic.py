@@ -280,6 +280,7 @@ def test_matrix_core_kernel_where_it_was_measured_faster(ops):
     ((1, 7, 7, 512), (3, 3, 512, 512), 3),            # 151 / 110 / 151, exchanged 45
     ((1, 7, 7, 512), (1, 1, 512, 2048), 3),           # 69 / 47 / 69, exchanged 27
     ((20, 16, 8, 130), (3, 3, 130, 1248), 3),         # - / 235 / 344, exchanged 196
+    ((1, 12, 12, 3), (7, 7, 3, 560), 2),              # - / 32 / -, exchanged 35: a launch more
     # one or two fills: where outputs are stored faster
     ((10, 139, 139, 10), (1, 1, 10, 976), 0),         # 466 / - / 246
     ((72, 61, 61, 11), (1, 1, 11, 720), 0),           # 445 / - / 245

@@ -890,7 +890,10 @@ void prepare_mx(PreparedDense *pd, int forms)
         // two fills and few outputs in whole lines (1x1 18->144 @80x80x8 40 us here, 31 there, predicted 16.6 and 14.7).
         const double left_out = fills <= 2 && (g.Co & 15) == 0 && bytes < 60e6 ? 2.0 : 5.0;
         const double other = std::max(pd->plan.cost * (pd->plan.px ? 1.12 : 1.06) + left_out * us, store_other);
-        if (swap.units && swap.cost < std::min(mine, other)) {
+        // Exchanged operands are packed by the launch of the patch sums, or by one more where that takes no work along (3x1/2
+        // 21->1056 @39x193x2 72 us, the vector ALUs 57; 7x7 3->560 on one 12x12 image 35, rows of its own 32).
+        const double swap_cost = swap.cost + ((g.C & 3) && g.C < 64 ? 8.0 : 0.0) * us;
+        if (swap.units && swap_cost < std::min(mine, other)) {
             pd->mx = true;
             pd->mxp = swap;
             return;
