@@ -221,6 +221,27 @@ def test_two_layers_in_turn(pkg, own_rows):
             assert torch.equal(op(xd, fd, *MM), want)
 
 
+# strided layers whose rows of codes, with their padding, would be a multiple of 128 bytes: one column more in front
+WIDER = [
+    ((4, 31, 31, 16), (3, 3, 24), 2, 1, "SAME"),         # 32 -> 33
+    ((3, 9, 32, 20), (3, 3, 12), 2, 1, "VALID"),         # no padding of its own
+    ((2, 10, 95, 24), (3, 3, 30), 3, 1, "SAME"),         # 96
+    ((2, 63, 63, 12), (5, 5, 16), 4, 1, "SAME"),
+    ((1, 40, 124, 8), (3, 3, 20), 2, 2, "SAME"),         # dilation
+    ((3, 31, 31, 48), (3, 3, 70), 2, 1, "SAME"),
+]
+
+
+@pytest.mark.parametrize("mode,case", [(2, c) for c in WIDER] + [(1, ((64, 63, 63, 64), (3, 3, 64), 2, 1, "SAME")),
+                                                                 (1, ((32, 32, 32, 64), (3, 3, 128), 2, 1, "VALID"))],
+                         ids=lambda v: _id(v) if isinstance(v, tuple) else str(v))
+def test_strided_rows_of_128_bytes(pkg, oracle, own_rows, mode, case):
+    own_rows.set_matrix_rows(mode)
+    plan = _plan(own_rows, case)
+    assert plan is not None and plan["own_rows"] == mode - 1, plan
+    _compare(pkg, oracle, own_rows, case)
+
+
 # sizes that the planner would not give this form to: many pixels, up to the bounds of compute_swap_plan (65536 pixels, packed
 # codes of 1 GiB on either side)
 SWAPPED_FAR = [
@@ -244,6 +265,7 @@ CODES = [
     ((2, 15, 13, 64), (3, 3, 64, 24), 2, "VALID"),
     ((2, 14, 14, 130), (1, 1, 130, 36), 2, "SAME"),      # strided 1x1: codes gathered first
     ((4, 7, 7, 256), (1, 1, 256, 64), 1, "SAME"),        # images that count as one row
+    ((2, 31, 31, 24), (3, 3, 24, 16), 2, "SAME"),        # one column more in front of rows of 128 bytes
 ]
 
 

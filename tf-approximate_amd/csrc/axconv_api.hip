@@ -737,7 +737,8 @@ MxPlans make_mx_plans(const ConvGeom &g, int64_t quads, int64_t groups, MxLoads 
 
 XqLayout plain_layout(const ConvGeom &g) { return {g.H, g.W, 0, 0}; }
 
-// The layout with the padding written out: as many rows / columns in front as the larger of the two paddings.
+// The layout with the padding written out: as many rows / columns in front as the larger of the two paddings, or one column
+// more.
 XqLayout padded_layout(const ConvGeom &g, bool flat)
 {
     const int below = (g.OH - 1) * g.sh - g.ph + (g.KH - 1) * g.dh + 1 - g.H;
@@ -747,6 +748,14 @@ XqLayout padded_layout(const ConvGeom &g, bool flat)
     l.col0 = flat ? 0 : std::max(0, std::max(g.pw, right));
     l.Hp = g.H + l.row0;
     l.Wp = g.W + l.col0;
+    // At a stride a load takes one dword of every pixel, on four quad planes at a time.  With planes a multiple of 128 bytes
+    // apart its 64 dwords meet on few of the cache's lines and banks: one more column in front (us with and without, in tiles of
+    // rows made in the kernel / pre-expanded: 3x3/2 64->64 @63x63x64 140 / 196, 129 / 180; 64->1840 on one 159x159 image 305 /
+    // 496; 32->64 @31x31x64 42 / 49, 40 / 46).  At stride 1, 16 bytes a lane, it makes no difference.
+    if (!flat && g.sw > 1 && (l.Wp & 31) == 0) {
+        ++l.col0;
+        ++l.Wp;
+    }
     return l;
 }
 
