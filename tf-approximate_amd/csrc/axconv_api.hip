@@ -897,7 +897,7 @@ void prepare_mx(PreparedDense *pd, int forms)
         const double mine = expand ? own_cost : rows_ok ? rows_cost : 1e30;
         // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), less so for one or
         // two fills and few outputs in whole lines (1x1 18->144 @80x80x8 40 us here, 31 there, predicted 16.6 and 14.7).
-        const double left_out = fills <= 2 && (g.Co & 15) == 0 && bytes < 60e6 ? 2.0 : 5.0;
+        const double left_out = fills <= 2 && (g.Co & 15) == 0 && bytes < 60e6 ? 2.5 : 5.0;
         const double other = std::max(pd->plan.cost * (pd->plan.px ? 1.12 : 1.06) + left_out * us, store_other);
         // Exchanged operands are packed by the launch of the patch sums, or by one more where that takes no work along (3x1/2
         // 21->1056 @39x193x2 72 us, the vector ALUs 57; 7x7 3->560 on one 12x12 image 35, rows of its own 32).
