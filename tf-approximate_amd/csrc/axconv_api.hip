@@ -604,7 +604,8 @@ MxDiv mx_div(uint32_t d)
 //   a fill    of pre-expanded rows 1.10 (U = 2), 1.32 (4), 1.51 (8), 2.10 (13), 2.53 (16), 3.05 (20), 3.75 (25); four loads
 //             1.30, 1.76, 2.42, 3.52, 4.25, 5.19, 6.39; of rows the kernel makes itself 0.95 (U = 2), 1.98 (10), 2.29 (12),
 //             2.55 (14), 2.83 (16), 3.09 (18), four loads 2.63 (8), 3.10, 3.49, 3.96, 4.49, 4.95: the stores of the rows
-//             take the LDS 0.35 us of every fill
+//             take the LDS 0.35 us of every fill (1x1 layers of 18 and 72 fills, a tile per workgroup: 1.10 (2), 1.11 (3),
+//             1.28 (4), 1.50 (6), 1.78 (8), 2.06 (10), 2.35 (12), 2.65 (14), 2.92 (16), 3.22 (18))
 //   a tile    1.3 + 0.70 U up to U = 6, then 0.42 a unit: geometry, the sums' start values, the outputs, stored in 32-byte
 //             pieces; rows of its own 2.0 more once a launch (a first fill that waits for codes, then for entries)
 // K splits and the rows cost what they cost the other kernels (compute_plan).
@@ -828,11 +829,12 @@ struct PreparedDense {
 
 // Decides whether the layer runs lutgemm_mx_kernel, and whether out of pre-expanded rows or of rows that it makes itself:
 // what the cost models, fitted to the launch times of each, say is fastest.  Whole op, us, pre-expanded / own rows / other
-// kernels: 3x3 64->64 @56x56x64 201 / 260 / 302, 1x1 128->512 @28x28x64 111 / 135 / 160, 1x1 256->1024 @14x14x64 147 / 148 /
-// 168, 3x3 256->256 @14x14x64 346 / 275 / 378, 3x3 512->512 @7x7x64 820 / 275 / 376, 1x1 512->2048 @7x7x64 284 / 138 / 189, the
-// same on one image 235 / 61 / 68.  Own rows want few pixels for many weights, where writing 512 bytes per weight and reading
-// them back outweighs making them anew in every tile.  Over the layers of ResNet-50 at batch 64, 9 and 1 and of 240 random
-// layers, each timed in the three forms, the choice is 1.2, 1.2, 0.4 and 2 % above the fastest of the three.
+// kernels (- : mode 1 leaves the layer to the other kernels too): 3x3 64->64 @56x56x64 184 / 229 / 336, 1x1 128->512 @28x28x64
+// 103 / 117 / 170, 1x1 256->1024 @14x14x64 108 / 113 / 159, 3x3 256->256 @14x14x64 333 / 236 / 349, 3x3 512->512 @7x7x64 - /
+// 240 / 369, 1x1 512->2048 @7x7x64 - / 103 / 175, the same on one image - / 47 / 69 and with its operands exchanged 27, 3x3
+// 512->512 on one 7x7 image - / 111 / 151, exchanged 44.  Own rows want few pixels for many weights, where writing 512 bytes per weight
+// and reading them back outweighs making them anew in every tile.  Over 240 random layers, each timed in every form, the choice
+// is 1.7 % above the fastest.
 enum { kMxNone, kMxOwnRows, kMxRows, kMxAny };   // which forms may run the layer (own rows: operands exchanged too)
 void prepare_mx(PreparedDense *pd, int forms)
 {

@@ -1,4 +1,5 @@
-// Dense LUT-GEMM whose sums are made by the matrix cores (gfx950), out of pre-expanded rows.
+// Dense LUT-GEMM whose sums are made by the matrix cores (gfx950), out of pre-expanded rows or
+// of rows that it makes itself (EXPAND).
 //
 // Every product is a lookup in the truth table, as in the other kernels: per activation code a 256-byte row of LDS
 // holds the table entries of 128 slots (16 filter elements x 8 columns), and a lane fetches eight of them with one

@@ -1936,8 +1936,8 @@ hipError_t launch_swap_pack(const float *x, const uint8_t *codes, const float *f
 
 // The op's epilogue for sums that lutgemm_mx_kernel made with its operands exchanged: [split][column][pixel], rows of
 // m_pitch (a multiple of four).  A workgroup turns 16 columns x 16 pixels; its four wavefronts add a quarter of the splits
-// each, four pixels of a column per lane, eight loads in flight (one wavefront for all 32 splits of 3x3 512->512 on one 7x7
-// image, a load at a time: 14.9 us).
+// each, four pixels of a column per lane, eight loads in flight (3x3 512->512 on one 7x7 image, 32 splits: 7 us; one wavefront
+// for all splits, a load at a time, 14.9).
 __global__ void __launch_bounds__(256) swap_epilogue_kernel(const int32_t *__restrict__ part, int ks, int64_t M, int Co,
                                                             int m_pitch, const float *__restrict__ psum,
                                                             const float *__restrict__ fsum, float s1xs2, float m1, float m2,
