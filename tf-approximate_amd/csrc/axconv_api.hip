@@ -832,9 +832,9 @@ struct PreparedDense {
 // kernels (- : mode 1 leaves the layer to the other kernels too): 3x3 64->64 @56x56x64 184 / 229 / 336, 1x1 128->512 @28x28x64
 // 103 / 117 / 170, 1x1 256->1024 @14x14x64 108 / 113 / 159, 3x3 256->256 @14x14x64 333 / 236 / 349, 3x3 512->512 @7x7x64 - /
 // 240 / 369, 1x1 512->2048 @7x7x64 - / 103 / 175, the same on one image - / 47 / 69 and with its operands exchanged 27, 3x3
-// 512->512 on one 7x7 image - / 111 / 151, exchanged 44.  Own rows want few pixels for many weights, where writing 512 bytes per weight
-// and reading them back outweighs making them anew in every tile.  Over 240 random layers, each timed in every form, the choice
-// is 1.7 % above the fastest.
+// 512->512 on one 7x7 image - / 111 / 151, exchanged 44.  Own rows want few pixels for many weights, where writing 512 bytes
+// per weight and reading them back outweighs making them anew in every tile.  Over 240 random layers, each timed in every
+// form, the choice is 1.7 % above the fastest.
 enum { kMxNone, kMxOwnRows, kMxRows, kMxAny };   // which forms may run the layer (own rows: operands exchanged too)
 void prepare_mx(PreparedDense *pd, int forms)
 {
@@ -963,8 +963,9 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     }
     // A 1x1 filter at stride 1 sees a list of pixels.  Rows that are no whole groups of four pixels (7x7, 14x14) leave lanes of
     // lutgemm_mx_kernel without a pixel - 56 units of 64 where 49 have pixels - and store by the pixel: one image, or the two
-    // or four that make whole groups, count as one row (ResNet-50 at batch 64 9782 -> 9632 us, its 1x1 layers 3 to 7 %).  From 128 channels and 192 pixels on, where the patch sums go by the
-    // list of pixels in any case (launch_patch_sums), up to the 1024 pixels a row may have there.
+    // or four that make whole groups, count as one row (ResNet-50 at batch 64 9782 -> 9632 us, its 1x1 layers 3 to 7 %).  From
+    // 128 channels and 192 pixels on, where the patch sums go by the list of pixels in any case (launch_patch_sums), up to the
+    // 1024 pixels a row may have there.
     if (allow_subsample && allow_fold && pd->g.KH == 1 && pd->g.KW == 1 && pd->g.sh == 1 && pd->g.sw == 1 && pd->g.ph == 0 &&
         pd->g.pw == 0 && (pd->g.W & 3) != 0 && (pd->g.C & 3) == 0 && pd->g.C >= 128) {
         const int64_t pixels = (int64_t)pd->g.H * pd->g.W;
@@ -1567,7 +1568,8 @@ int axc_table_create(const uint16_t *host_table, axc_table **out)
     if (!host_table || !out)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
     // weight-code major: tableT[b][a] = T[(a << 8) | b], in squares that the first-level cache holds by row and by column, and
-    // the two flipped copies by whole vectors (us a table with its upload, same machine: entry by entry 143 for the first alone, 181 for three; 42)
+    // the two flipped copies by whole vectors (us a table with its upload, on one machine: entry by entry 143 for the first
+    // alone, 181 for three; 42)
     const size_t entries = (size_t)kTableRows * 256, used = 65536;   // row 256: the null weight's, zeros
     std::vector<uint16_t> t(3 * entries);
     uint16_t *const T = t.data(), *const F = T + entries, *const S = F + entries;

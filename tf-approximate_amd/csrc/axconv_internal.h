@@ -148,8 +148,8 @@ struct MxPlan {
 
 // Quantized input with its padding written out, as lutgemm_mx_kernel reads it: dwords [n][Hp][C4][Wp], pixel (h, w) in
 // row h + row0, column w + col0.  The rows and columns in front of an image double as those behind the one before it,
-// so row0 and col0 are the larger of the two paddings (or one column more: padded_layout); behind the last image follow row0 more rows and, where there is
-// column padding too, one for the columns behind the last of those.  Without padding (and always for the other kernels)
+// so row0 and col0 are the larger of the two paddings (or one column more: padded_layout); behind the last image follow row0
+// more rows and, where there is column padding too, one for the columns behind the last of those.  Without padding (and always for the other kernels)
 // Hp = H, Wp = W, row0 = col0 = 0, and one row follows the last image.
 struct XqLayout {
     int Hp, Wp, row0, col0;
