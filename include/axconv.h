@@ -154,6 +154,11 @@ int axc_conv2d_matrix_plan(const axc_conv2d_desc *desc, int32_t plan[8]);
  * exchanged: the plan's pixels are then the layer's output columns, and its columns the output pixels.  A launch whose
  * workspace lacks room runs in another form or one of the other kernels, with the same results. */
 int axc_conv2d_matrix_rows(const axc_conv2d_desc *desc, int32_t *rows);
+/* Layers of few lookups run as ONE launch instead, which takes them from the raw tensors to the outputs (the queries above
+ * then say what would run them otherwise, and what the workspace query counts is asked for all the same).  fake_quant: 1 for
+ * the layer entry point, 0 for the op.  plan = { 1 or 0 (then the rest is 0 too), output pixels of a tile, columns of a tile,
+ * filter elements of a chunk, chunks, row tiles, column tiles, workgroups }.  Codes entry points never run that way. */
+int axc_conv2d_direct_plan(const axc_conv2d_desc *desc, int fake_quant, int32_t plan[8]);
 /* Pins the tile width the planner uses (16, 32 or 64 columns; 0 = its own choice, the default), process-wide, for
  * tests and timing of the wider-tile kernel variants.  The environment variable AXC_TILE_COLUMNS gives the initial
  * value and is read once, when the library is loaded.  Like axc_set_preexpand it is process-wide; a workspace query and
@@ -170,7 +175,8 @@ int axc_set_tile_columns(int columns);
 int axc_set_preexpand(int mode);
 /* Pins what axc_conv2d_matrix_rows reports: 0 = the planner decides (the default), 1 = pre-expanded rows only (layers that
  * those do not suit run the other kernels), 2 = rows made by the kernel itself wherever it can, 3 = the same with the operands
- * exchanged; process-wide, for tests and timing; a workspace query and the launch it is for must see the same value.
+ * exchanged, 4 = whole layers in one launch wherever it can (axc_conv2d_direct_plan), else as 2; process-wide, for tests and
+ * timing; a workspace query and the launch it is for must see the same value.
  * Results do not depend on it.  No counterpart in the reference. */
 int axc_set_matrix_rows(int mode);
 /* The wavefronts of the kernels that plan code 2 and axc_conv2d_matrix_plan stand for wait for each other by polling counters,
@@ -257,7 +263,9 @@ int axc_conv2d_codes_acc_i32(const axc_table *table, const axc_conv2d_desc *desc
 /* Per-kernel timing with HIP events recorded on the launch stream.  While enabled, every kernel the
  * launch calls enqueue is bracketed by two events; axc_profile_read synchronizes them and returns the
  * accumulated milliseconds and launch count per kernel name since the last reset.  A launch out of pre-expanded rows is
- * entered as lutgemm_px, and as lutgemm_mx too where the matrix cores make its sums. */
+ * entered as lutgemm_px, and as lutgemm_mx too where the matrix cores make its sums.  While the timers run, layers are
+ * launched part by part, so that every part has its time: those of axc_conv2d_direct_plan too, unless axc_set_matrix_rows pins
+ * them (then they are entered as direct). */
 int axc_profile_enable(int enable);
 int axc_profile_reset(void);
 int axc_profile_read(int index, char *name, size_t name_bytes, double *total_ms, int64_t *launches);

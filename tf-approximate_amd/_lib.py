@@ -56,6 +56,7 @@ SYMBOLS = [
     ("axc_conv2d_workspace_bytes", ctypes.c_int, [_desc, ctypes.POINTER(_sz)]),
     ("axc_conv2d_tile_plan", ctypes.c_int, [_desc, ctypes.POINTER(ctypes.c_int32)]),
     ("axc_conv2d_matrix_plan", ctypes.c_int, [_desc, ctypes.POINTER(ctypes.c_int32)]),
+    ("axc_conv2d_direct_plan", ctypes.c_int, [_desc, ctypes.c_int, ctypes.POINTER(ctypes.c_int32)]),
     ("axc_conv2d_matrix_rows", ctypes.c_int, [_desc, ctypes.POINTER(ctypes.c_int32)]),
     ("axc_set_tile_columns", ctypes.c_int, [ctypes.c_int]),
     ("axc_set_preexpand", ctypes.c_int, [ctypes.c_int]),

@@ -10,7 +10,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libaxconv_hip.so")
 SOURCES = ["axconv_api.hip", "lutgemm_kernel.hip", "lutgemm_px_kernel.hip", "lutgemm_mx_kernel.hip",
-           "lutgemm_mx_expand_kernel.hip", "prepass_kernels.hip", "depthwise_kernel.hip"]
+           "lutgemm_mx_expand_kernel.hip", "direct_kernel.hip", "prepass_kernels.hip", "depthwise_kernel.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -211,6 +211,45 @@ struct MxParams {
     uint32_t wq_bytes;
 };
 
+// ---- direct_kernel.hip: a whole layer of few lookups in one launch ----
+constexpr int kDirectThreads = 1024, kDirectWaves = kDirectThreads / 64;
+constexpr int kDirectGatherWaves = 8;          // of which this many look up
+constexpr int kDirectItems = 2;                // quads of filter elements of pixels, and of columns, a thread fetches at a time
+constexpr int kDirectMaxItems = kDirectItems * (kDirectWaves - kDirectGatherWaves - 2) * 64;   // of a chunk that is not the only one
+constexpr int kDirectLdsBytes = 163840;        // the table and 32 KiB for everything else
+constexpr int kDirectBufferBytes = kDirectLdsBytes - kTableBytes - 3 * 64 * 4 - 2 * 64 * 4;   // both buffers of a chunk
+constexpr int kDirectPixels[] = {16, 32, 64};  // pixels of a tile
+constexpr int kDirectMaxColumns = 64;
+constexpr int kDirectColumns[] = {1, 2, 3, 4, 6, 8};   // columns of a wavefront: the kernel's variants
+
+struct DirectPlan {
+    int pt, ct;            // pixels and columns of a tile
+    int ncw, wc, wc_log;   // columns of a wavefront that looks up, and how many wavefronts side by side make the tile's
+    int kc, kl, chunks;    // filter elements of a chunk and of a lane in it; chunks over the whole K
+    int buffer_bytes;
+    int n_row_tiles, n_col_tiles, grid;
+    float us;              // what the planner's model expects of the launch; 0: the layer does not suit the kernel
+};
+
+struct DirectDiv {         // as MxDiv, but whole = 2^32 - 1 and mul = 0 where the divisor is one
+    uint32_t mul, shift, whole;
+};
+
+struct DirectParams {
+    DirectPlan plan;
+    const float *x, *f, *bias;
+    const uint16_t *tableT;
+    float *out_f;
+    int32_t *out_i;
+    const LayerQuant *lq_dev;
+    TensorQuant in_q, flt_q;
+    float s1xs2, m1, m2, k_m1xm2;
+    int relu;
+    uint32_t x_bytes, f_bytes;
+    int M, K, H, W, C, KW, Co, OH, OW, sh, sw, dh, dw, ph, pw;
+    DirectDiv div_ow, div_oh, div_c, div_kw, div_kq, div_ct;   // kq: quads of a chunk
+};
+
 struct DepthwiseParams {
     int N, H, W, C, KH, KW, OH, OW, sh, sw, dh, dw, ph, pw;
     int64_t M;
@@ -361,6 +400,7 @@ hipError_t launch_swap_epilogue(const DenseParams &p, const int32_t *partials, i
                                 int32_t *out_i, hipStream_t stream);
 hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream);          // out of pre-expanded rows
 hipError_t launch_dense_mx_expand(const MxParams &p, hipStream_t stream);   // plan.expand
+hipError_t launch_direct(const DirectParams &p, hipStream_t stream);
 hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials, float *out_f, int32_t *out_i,
                                   hipStream_t stream);
 // tf1 AxConv2D: what the zero points add to the sums of products, per output pixel and per output column; and the pass

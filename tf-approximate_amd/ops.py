@@ -334,7 +334,7 @@ def conv2d_tile_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding="S
 
 def conv2d_matrix_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding="SAME", dilations=(1, 1, 1, 1)):
     """How the kernel whose sums the matrix cores make cuts a layer on the current device, as a dict; None for a layer
-    that does not run it."""
+    that does not run it.  (Layers that conv2d_direct_plan names run that way instead.)"""
     lib = _lib.load()
     desc = make_desc(tuple(input_shape), tuple(filter_shape), list(strides), padding, (), "NHWC", list(dilations), 8)
     plan = (ctypes.c_int32 * 8)()
@@ -349,6 +349,19 @@ def conv2d_matrix_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding=
     return dict(zip(keys, [int(v) for v in plan[1:]]), own_rows=rows.value - 1)
 
 
+def conv2d_direct_plan(input_shape, filter_shape, strides=(1, 1, 1, 1), padding="SAME", dilations=(1, 1, 1, 1), layer=False):
+    """How a layer that runs as one launch on the current device is cut, as a dict; None for one that does not.  layer: as
+    the layer call runs it, not the op."""
+    lib = _lib.load()
+    desc = make_desc(tuple(input_shape), tuple(filter_shape), list(strides), padding, (), "NHWC", list(dilations), 8)
+    plan = (ctypes.c_int32 * 8)()
+    _check(lib.axc_conv2d_direct_plan(ctypes.byref(desc), int(layer), plan))
+    if not plan[0]:
+        return None
+    keys = ("pixels_per_tile", "columns_per_tile", "elements_per_chunk", "chunks", "row_tiles", "column_tiles", "workgroups")
+    return dict(zip(keys, [int(v) for v in plan[1:]]))
+
+
 def set_tile_columns(columns):
     """Pins the dense kernel's tile width (16 / 32 / 64 columns; 0 = the planner's choice) for the whole process."""
     _check(_lib.load().axc_set_tile_columns(int(columns)))
@@ -361,7 +374,8 @@ def set_preexpand(mode):
 
 def set_matrix_rows(mode):
     """Rows of the kernel whose sums the matrix cores make: 0 = the planner's choice, 1 = pre-expanded ones only, 2 = made
-    by the kernel itself wherever it can, 3 = the same with the operands exchanged."""
+    by the kernel itself wherever it can, 3 = the same with the operands exchanged, 4 = whole layers in one launch wherever
+    possible."""
     _check(_lib.load().axc_set_matrix_rows(int(mode)))
 
 
