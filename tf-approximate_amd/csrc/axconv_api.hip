@@ -7,6 +7,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstdlib>
 #include <map>
@@ -998,8 +999,8 @@ void prepare_mx(PreparedDense *pd, int forms)
 // quarter (stride 2) of the pixels to quantize and sum.  Callers with a padding origin of their own (`pads`: rows and columns)
 // get the layer as given.  mx_mode: which forms of lutgemm_mx_kernel may run the layer.  allow_fold: images of a 1x1 layer may
 // count as one row.
-int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
-                  int px_mode = kPxModeGlobal, int mx_mode = kMxAny, bool allow_fold = true)
+int compute_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads, int element_bytes, int px_mode, int mx_mode,
+                  bool allow_fold)
 {
     const bool allow_subsample = pads == nullptr;
     const bool allow_flat = allow_subsample;   // both are for callers that leave the padding origin to the library
@@ -1093,6 +1094,50 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
         g_forced_nt.load(std::memory_order_relaxed) == 0)
         prepare_mx(pd, mx_mode);
     pd->ws = dense_workspace(pd->g, pd->plan, pd->mx ? &pd->mxp : nullptr, pd->lay, sub_bytes, pd->flat_row_bytes);
+    return AXC_OK;
+}
+
+// The same, looked up: a call asks for it at least twice (workspace, launch), and working it out takes 2 to 3 us of host time,
+// several plans among it.  The key is all that it depends on: the descriptor, the arguments, the pinned forms and the device's
+// compute units.
+int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
+                  int px_mode = kPxModeGlobal, int mx_mode = kMxAny, bool allow_fold = true)
+{
+    if (!desc)
+        return compute_dense(desc, pd, pads, element_bytes, px_mode, mx_mode, allow_fold);
+    typedef std::array<int64_t, 36> Key;
+    Key key{};
+    size_t n = 0;
+    for (int i = 0; i < 4; ++i) {
+        key[n++] = desc->input_shape[i];
+        key[n++] = desc->filter_shape[i];
+        key[n++] = desc->strides[i];
+        key[n++] = desc->dilations[i];
+    }
+    for (int i = 0; i < 8; ++i)
+        key[n++] = desc->explicit_paddings[i];
+    for (const int v : {desc->padding, desc->data_format, desc->num_bits, pads ? 1 : 0, pads ? pads[0] : 0, pads ? pads[1] : 0,
+                        element_bytes * 2 + (allow_fold ? 1 : 0), px_mode * 8 + mx_mode,
+                        g_forced_nt.load(std::memory_order_relaxed), g_px_mode.load(std::memory_order_relaxed),
+                        g_mx_rows.load(std::memory_order_relaxed), device_cus()})
+        key[n++] = v;
+    static std::mutex mu;
+    static std::map<Key, PreparedDense> cache;
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        const auto it = cache.find(key);
+        if (it != cache.end()) {
+            *pd = it->second;
+            return AXC_OK;
+        }
+    }
+    const int rc = compute_dense(desc, pd, pads, element_bytes, px_mode, mx_mode, allow_fold);
+    if (rc != AXC_OK)
+        return rc;
+    std::lock_guard<std::mutex> lock(mu);
+    if (cache.size() >= 1024)
+        cache.clear();
+    cache[key] = *pd;
     return AXC_OK;
 }
 

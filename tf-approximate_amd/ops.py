@@ -112,10 +112,10 @@ class TruthTable:
 _workspaces = {}
 
 
-def _workspace(device, nbytes):
+def _workspace(device, stream, nbytes):
     """Scratch memory of a call, cached per (device, current stream): calls issued on one stream run in order and
     may share it; calls on different streams may overlap and must not."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, stream)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
@@ -124,13 +124,49 @@ def _workspace(device, nbytes):
 
 
 def _scalar(v):
+    if type(v) is float:
+        return v
     if torch.is_tensor(v):
         return float(v.item())
     return float(v)
 
 
-def _stream_ptr(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+# The current stream's handle; the public way makes a Stream object of it first, which takes 2 us.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(device):
+    return _raw_stream(device.index) if _raw_stream else torch.cuda.current_stream(device).cuda_stream
+
+
+def _launch(device, fn, *args):
+    """fn(*args) with `device` current: entering a device's context takes longer than all else here."""
+    if torch.cuda.current_device() == device.index:
+        rc = fn(*args)
+    else:
+        with torch.cuda.device(device):
+            rc = fn(*args)
+    if rc != _lib.OK:
+        _check(rc)
+
+
+class _Layer:
+    """What a call needs to know of its shapes and attributes: made once for each, never changed."""
+
+    def __init__(self, desc, depthwise):
+        dims = conv2d_geometry(desc)
+        self.desc = desc
+        self.ref = ctypes.byref(desc)
+        self.columns = dims.in_depth if depthwise else dims.out_depth
+        self.out_shape = (dims.batch, int(dims.out_rows), int(dims.out_cols), self.columns)
+        self.depthwise = depthwise
+
+    def workspace(self, lib, device, stream):
+        """Asked for on every call: what it has to hold depends on the forms that are pinned."""
+        nbytes = ctypes.c_size_t()
+        fn = lib.axc_depthwise_conv2d_workspace_bytes if self.depthwise else lib.axc_conv2d_workspace_bytes
+        _check(fn(self.ref, ctypes.byref(nbytes)))
+        return _workspace(device, stream, nbytes.value)
 
 
 def _require_device_f32(t, what):
@@ -155,6 +191,7 @@ class ApproxConv2DWithMinMaxVars:
         self.dilations = list(dilations)
         self.depthwise = depthwise
         self.table = mul_map_file if isinstance(mul_map_file, TruthTable) else TruthTable(mul_map_file, num_bits)
+        self._layers = {}
         # attr checks the reference performs at construction (InitApproxConv2DParameters)
         make_desc((1, 1, 1, 1), (1, 1, 1, 1), self.strides, self.padding, self.explicit_paddings,
                   self.data_format, self.dilations, self.num_bits)
@@ -167,26 +204,31 @@ class ApproxConv2DWithMinMaxVars:
         depth = dims.in_depth if self.depthwise else dims.out_depth
         return (dims.batch, int(dims.out_rows), int(dims.out_cols), depth)
 
+    def _layer(self, input, filter):
+        key = (input.shape, filter.shape, tuple(self.strides), self.num_bits, self.padding, tuple(self.explicit_paddings),
+               self.data_format, tuple(self.dilations), self.depthwise)
+        layer = self._layers.get(key)
+        if layer is None:
+            layer = _Layer(self._desc(input, filter), self.depthwise)
+            if len(self._layers) >= 256:
+                self._layers.clear()
+            self._layers[key] = layer
+        return layer
+
     def _run(self, input, filter, mins, acc_i32):
         lib = _lib.load()
         input = _require_device_f32(input, "input")
         filter = _require_device_f32(filter, "filter")
-        desc = self._desc(input, filter)
-        dims = conv2d_geometry(desc)
-        nbytes = ctypes.c_size_t()
-        ws_fn = lib.axc_depthwise_conv2d_workspace_bytes if self.depthwise else lib.axc_conv2d_workspace_bytes
-        _check(ws_fn(ctypes.byref(desc), ctypes.byref(nbytes)))
-        ws = _workspace(input.device, nbytes.value)
-        out = torch.empty(self._out_shape(dims), dtype=torch.int32 if acc_i32 else torch.float32,
-                          device=input.device)
+        layer, device = self._layer(input, filter), input.device
+        stream = _stream(device)
+        ws = layer.workspace(lib, device, stream)
+        out = torch.empty(layer.out_shape, dtype=torch.int32 if acc_i32 else torch.float32, device=device)
         if self.depthwise:
             fn = lib.axc_depthwise_conv2d_minmax_acc_i32 if acc_i32 else lib.axc_depthwise_conv2d_minmax
         else:
             fn = lib.axc_conv2d_minmax_acc_i32 if acc_i32 else lib.axc_conv2d_minmax
-        with torch.cuda.device(input.device):
-            _check(fn(self.table.handle, ctypes.byref(desc), input.data_ptr(), filter.data_ptr(),
-                      *[_scalar(m) for m in mins], out.data_ptr(), ws.data_ptr(), ws.numel(),
-                      _stream_ptr(input.device)))
+        _launch(device, fn, self.table.handle, layer.ref, input.data_ptr(), filter.data_ptr(), *[_scalar(m) for m in mins],
+                out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         return out
 
     def __call__(self, input, filter, input_min, input_max, filter_min, filter_max, bias=None, activation=None):
@@ -199,24 +241,19 @@ class ApproxConv2DWithMinMaxVars:
         lib = _lib.load()
         input = _require_device_f32(input, "input")
         filter = _require_device_f32(filter, "filter")
-        desc = self._desc(input, filter)
-        dims = conv2d_geometry(desc)
-        out_shape = self._out_shape(dims)
+        layer, device = self._layer(input, filter), input.device
         if bias is not None:
             bias = _require_device_f32(bias, "bias")
-            if bias.numel() != out_shape[3]:
+            if bias.numel() != layer.columns:
                 raise InvalidArgumentError("bias must have one value per output channel")
-        nbytes = ctypes.c_size_t()
-        ws_fn = lib.axc_depthwise_conv2d_workspace_bytes if self.depthwise else lib.axc_conv2d_workspace_bytes
-        _check(ws_fn(ctypes.byref(desc), ctypes.byref(nbytes)))
-        ws = _workspace(input.device, nbytes.value)
-        out = torch.empty(out_shape, dtype=torch.float32, device=input.device)
-        fn = lib.axc_depthwise_conv2d_minmax_bias_act if self.depthwise else lib.axc_conv2d_minmax_bias_act
-        with torch.cuda.device(input.device):
-            _check(fn(self.table.handle, ctypes.byref(desc), input.data_ptr(), filter.data_ptr(),
-                      *[_scalar(m) for m in (input_min, input_max, filter_min, filter_max)],
-                      bias.data_ptr() if bias is not None else None, 1 if activation == "relu" else 0,
-                      out.data_ptr(), ws.data_ptr(), ws.numel(), _stream_ptr(input.device)))
+        stream = _stream(device)
+        ws = layer.workspace(lib, device, stream)
+        out = torch.empty(layer.out_shape, dtype=torch.float32, device=device)
+        _launch(device, lib.axc_depthwise_conv2d_minmax_bias_act if self.depthwise else lib.axc_conv2d_minmax_bias_act,
+                self.table.handle, layer.ref, input.data_ptr(), filter.data_ptr(),
+                _scalar(input_min), _scalar(input_max), _scalar(filter_min), _scalar(filter_max),
+                bias.data_ptr() if bias is not None else None, 1 if activation == "relu" else 0,
+                out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         return out
 
     def accumulators(self, input, filter, input_min, input_max, filter_min, filter_max):
@@ -247,19 +284,13 @@ class FakeApproxConv2D:
             bias = _require_device_f32(bias, "bias")
             if bias.numel() != (kernel.shape[2] if self.depthwise else kernel.shape[3]):
                 raise InvalidArgumentError("bias must have one value per output channel")
-        desc = self.op._desc(inputs, kernel)
-        dims = conv2d_geometry(desc)
-        nbytes = ctypes.c_size_t()
-        ws_fn = lib.axc_depthwise_conv2d_workspace_bytes if self.depthwise else lib.axc_conv2d_workspace_bytes
-        _check(ws_fn(ctypes.byref(desc), ctypes.byref(nbytes)))
-        ws = _workspace(inputs.device, nbytes.value)
-        out = torch.empty(self.op._out_shape(dims), dtype=torch.float32, device=inputs.device)
-        fn = lib.axc_fake_approx_depthwise_conv2d if self.depthwise else lib.axc_fake_approx_conv2d
-        with torch.cuda.device(inputs.device):
-            _check(fn(self.op.table.handle, ctypes.byref(desc), inputs.data_ptr(),
-                                              kernel.data_ptr(), bias.data_ptr() if bias is not None else None,
-                                              self.activation, out.data_ptr(), ws.data_ptr(), ws.numel(),
-                                              _stream_ptr(inputs.device)))
+        layer, device = self.op._layer(inputs, kernel), inputs.device
+        stream = _stream(device)
+        ws = layer.workspace(lib, device, stream)
+        out = torch.empty(layer.out_shape, dtype=torch.float32, device=device)
+        _launch(device, lib.axc_fake_approx_depthwise_conv2d if self.depthwise else lib.axc_fake_approx_conv2d,
+                self.op.table.handle, layer.ref, inputs.data_ptr(), kernel.data_ptr(),
+                bias.data_ptr() if bias is not None else None, self.activation, out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         return out
 
 
@@ -303,18 +334,15 @@ def ax_conv2d(input, filter, min_input, max_input, min_filter, max_filter, strid
     if not input.is_cuda or not filter.is_cuda:
         raise InvalidArgumentError("input and filter must be tensors on the GPU")
     input, filter = input.contiguous(), filter.contiguous()
-    desc = make_desc(tuple(input.shape), tuple(filter.shape), list(strides), padding, (), "NHWC", (1, 1, 1, 1), 8)
-    dims = conv2d_geometry(desc)
-    nbytes = ctypes.c_size_t()
-    _check(lib.axc_conv2d_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)))
-    ws = _workspace(input.device, nbytes.value)
-    out = torch.empty((dims.batch, int(dims.out_rows), int(dims.out_cols), dims.out_depth), dtype=torch.int32,
-                      device=input.device)
+    layer = _Layer(make_desc(tuple(input.shape), tuple(filter.shape), list(strides), padding, (), "NHWC", (1, 1, 1, 1), 8), False)
+    device = input.device
+    stream = _stream(device)
+    ws = layer.workspace(lib, device, stream)
+    out = torch.empty(layer.out_shape, dtype=torch.int32, device=device)
     off_in = float_to_quantized_unclamped_quint8(0.0, min_input, max_input)
     off_f = float_to_quantized_unclamped_quint8(0.0, min_filter, max_filter)
-    with torch.cuda.device(input.device):
-        _check(lib.axc_axconv2d_quint8(table.handle, ctypes.byref(desc), input.data_ptr(), filter.data_ptr(), off_in, off_f,
-                                       out.data_ptr(), ws.data_ptr(), ws.numel(), _stream_ptr(input.device)))
+    _launch(device, lib.axc_axconv2d_quint8, table.handle, layer.ref, input.data_ptr(), filter.data_ptr(), off_in, off_f,
+            out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
     lo, hi = quantization_range_for_multiplication(min_input, max_input, min_filter, max_filter)
     return out, lo, hi
 
@@ -425,7 +453,7 @@ def quantize(values, vmin, vmax):
     codes = torch.empty(values.shape, dtype=torch.uint8, device=values.device)
     with torch.cuda.device(values.device):
         _check(_lib.load().axc_quantize(values.data_ptr(), values.numel(), float(vmin), float(vmax),
-                                        codes.data_ptr(), _stream_ptr(values.device)))
+                                        codes.data_ptr(), _stream(values.device)))
     return codes
 
 
@@ -437,17 +465,13 @@ def conv2d_codes_acc_i32(table, input_codes, filter_codes, input_zero_code, stri
         raise InvalidArgumentError("codes must be uint8")
     input_codes = input_codes.contiguous()
     filter_codes = filter_codes.contiguous()
-    desc = make_desc(tuple(input_codes.shape), tuple(filter_codes.shape), strides, padding, (), "NHWC", dilations)
-    dims = conv2d_geometry(desc)
-    nbytes = ctypes.c_size_t()
-    _check(lib.axc_conv2d_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)))
-    ws = _workspace(input_codes.device, nbytes.value)
-    out = torch.empty((dims.batch, int(dims.out_rows), int(dims.out_cols), dims.out_depth), dtype=torch.int32,
-                      device=input_codes.device)
-    with torch.cuda.device(input_codes.device):
-        _check(lib.axc_conv2d_codes_acc_i32(table.handle, ctypes.byref(desc), input_codes.data_ptr(),
-                                            filter_codes.data_ptr(), int(input_zero_code), out.data_ptr(),
-                                            ws.data_ptr(), ws.numel(), _stream_ptr(input_codes.device)))
+    layer = _Layer(make_desc(tuple(input_codes.shape), tuple(filter_codes.shape), strides, padding, (), "NHWC", dilations), False)
+    device = input_codes.device
+    stream = _stream(device)
+    ws = layer.workspace(lib, device, stream)
+    out = torch.empty(layer.out_shape, dtype=torch.int32, device=device)
+    _launch(device, lib.axc_conv2d_codes_acc_i32, table.handle, layer.ref, input_codes.data_ptr(), filter_codes.data_ptr(),
+            int(input_zero_code), out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
     return out
 
 
