@@ -1364,7 +1364,20 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             AXC_HIP(launch_patch_sums(input, g, tq_in, lq_dev, psum, stream, pd.lay, xq, &quantized_by_patch_sums, &job,
                                       &filter_done, 0, &px_done));
     }
-    if (swap) {
+    // tf1 op (codes in, int32 out: neither patch nor filter sums of floats): the terms of its zero points, in their place
+    int32_t *const pixel_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(psum) : nullptr;
+    int32_t *const column_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(fsum) : nullptr;
+    bool codes_done = false;
+    if (codes_mode && mx && !swap && !flat && !g_prof_enabled.load(std::memory_order_relaxed)) {   // (the timers: part by part)
+        AXC_HIP(launch_codes_prep(input_codes, filter_codes, g, pd.lay, zp4, xq, *mx, wq, table->dev_tableT, px_rows,
+                                  tf1_offset_filter != nullptr, input_zero_code, tf1_offset_filter ? *tf1_offset_filter : 0,
+                                  pixel_term, column_term, stream, &codes_done));
+        if (codes_done)
+            filter_done = px_done = true;
+    }
+    if (codes_done) {
+        // nothing left
+    } else if (swap) {
         if (!filter_done && out_f && !codes_mode) {
             ProfScope ps("filter_pack", stream);   // the filter's sums
             AXC_HIP(launch_filter_pack(filter, filter_codes, g, pd.plan, mx, tq_f, lq_dev, wq, fsum, stream));
@@ -1394,10 +1407,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
                                    (out_f && !codes_mode) ? fsum : nullptr, stream, table->dev_tableT, px_rows, &px_done));
     }
 
-    // tf1 op (codes in, int32 out: neither patch nor filter sums of floats): the terms of its zero points, in their place
-    int32_t *const pixel_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(psum) : nullptr;
-    int32_t *const column_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(fsum) : nullptr;
-    if (tf1_offset_filter) {
+    if (tf1_offset_filter && !codes_done) {
         ProfScope ps("axconv_terms", stream);
         AXC_HIP(launch_axconv_terms(input_codes, filter_codes, g, input_zero_code, *tf1_offset_filter, pixel_term, column_term,
                                     stream));

@@ -407,6 +407,12 @@ hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials,
 // that adds them to finished sums (lutgemm_mx_kernel does so as it stores)
 hipError_t launch_axconv_terms(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,
                                int offset_filter, int32_t *pixel_term, int32_t *column_term, hipStream_t stream);
+// All three at once for lutgemm_mx_kernel's layers given as codes (*done = false: not for this one; nothing was launched):
+// relayout, filter packing or rows, and with `terms` those of the zero points.
+hipError_t launch_codes_prep(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, const XqLayout &lay, uint32_t zp4,
+                             uint32_t *xq, const MxPlan &mx, uint16_t *wq, const uint16_t *tableT, uint16_t *rows, bool terms,
+                             int offset_input, int offset_filter, int32_t *pixel_term, int32_t *column_term, hipStream_t stream,
+                             bool *done);
 hipError_t launch_axconv_correction(const ConvGeom &g, const int32_t *pixel_term, const int32_t *column_term, int32_t *out,
                                     hipStream_t stream);
 hipError_t launch_fill_u32(uint32_t *dst, int64_t n, uint32_t value, hipStream_t stream);

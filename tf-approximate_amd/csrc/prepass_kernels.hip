@@ -1,6 +1,7 @@
 // Pre-pass kernels: quantize + relayout of the input, filter quantize/pack/sums, flat quantize.
 #include "axconv_internal.h"
 #include "px_expand.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace axc {
@@ -786,18 +787,18 @@ __global__ void __launch_bounds__(1024) patch_sums_smallc_kernel(const float *__
 // Same relayout for caller-supplied codes (uint8 NHWC).
 // A workgroup turns 1024 dwords, Q channel quads of 1024 / Q pixels: read along the channels of a pixel, written along the
 // pixels of a quad (a thread for all quads of a pixel wrote and read 4 bytes per line: 1x82x82x350 70 us).
+// 256 threads of a workgroup make block (bx, by) of gx x gy; `tile`: Q * (1024 / Q + 1) dwords of LDS.
 template <int Q>
-__global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__restrict__ codes, int64_t pixels,
-                                                              int N, int H, int W, int C, int C4, const XqLayout lay,
-                                                              uint32_t zp4, uint32_t *__restrict__ xq)
+__device__ __forceinline__ void codes_relayout_body(const int t, const int64_t bx, const int by, const int64_t gx, const int gy,
+                                                    uint32_t *__restrict__ tile, const uint8_t *__restrict__ codes,
+                                                    int64_t pixels, int N, int H, int W, int C, int C4, const XqLayout &lay,
+                                                    uint32_t zp4, uint32_t *__restrict__ xq)
 {
-    constexpr int P = 1024 / Q;
-    __shared__ uint32_t tile[Q][P + 1];
-    const int t = threadIdx.x;
-    xq_fill_padding(xq, lay, N, H, C4, zp4, ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + t,
-                    (int64_t)gridDim.x * gridDim.y * 256);
-    const int64_t pix0 = (int64_t)blockIdx.x * P;
-    const int q0 = (int)blockIdx.y * Q;
+    constexpr int P = 1024 / Q, kPitch = P + 1;
+    if (bx < gx)
+        xq_fill_padding(xq, lay, N, H, C4, zp4, (by * gx + bx) * 256 + t, gx * gy * 256);
+    const int64_t pix0 = bx * P;
+    const int q0 = by * Q;
     const bool dwords = (C & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3) == 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -814,7 +815,7 @@ __global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__re
                     v |= (c + e < C ? (uint32_t)src[e] : 0u) << (8 * e);
             }
         }
-        tile[q][p] = ((v >> 2) & 0x3f3f3f3fu) | ((v & 0x03030303u) << 6);   // phys_row of every byte
+        tile[q * kPitch + p] = ((v >> 2) & 0x3f3f3f3fu) | ((v & 0x03030303u) << 6);   // phys_row of every byte
     }
     __syncthreads();
 #pragma unroll
@@ -823,9 +824,22 @@ __global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__re
         const int64_t pix = pix0 + p;
         if (pix < pixels && q0 + q < C4) {
             const int64_t nh = pix / W;
-            xq[xq_row_nh(lay, nh, H, C4) + (int64_t)(q0 + q) * lay.Wp + (pix - nh * W)] = tile[q][p];
+            xq[xq_row_nh(lay, nh, H, C4) + (int64_t)(q0 + q) * lay.Wp + (pix - nh * W)] = tile[q * kPitch + p];
         }
     }
+}
+
+template <int Q>
+constexpr int codes_relayout_lds() { return Q * (1024 / Q + 1) * 4; }
+
+template <int Q>
+__global__ void __launch_bounds__(256) codes_relayout_kernel(const uint8_t *__restrict__ codes, int64_t pixels,
+                                                              int N, int H, int W, int C, int C4, const XqLayout lay,
+                                                              uint32_t zp4, uint32_t *__restrict__ xq)
+{
+    __shared__ uint32_t tile[codes_relayout_lds<Q>() / 4];
+    codes_relayout_body<Q>((int)threadIdx.x, blockIdx.x, (int)blockIdx.y, gridDim.x, (int)gridDim.y, tile, codes, pixels, N, H, W, C,
+                           C4, lay, zp4, xq);
 }
 
 // Filter pre-pass: quantize (tf2/src/approx_nn_conv_kernels.cpp:243, hoisted out of the GEMM loop)
@@ -1769,18 +1783,15 @@ __device__ __forceinline__ uint32_t sum_of_bytes(const uint8_t *__restrict__ src
 
 // Workgroups below `filter_blocks` make column terms, the others pixel terms of `rows_out` output rows each.
 template <int V>
-__global__ void __launch_bounds__(kAxSumThreads) axconv_terms_kernel(const uint8_t *__restrict__ codes,
-                                                                     const uint8_t *__restrict__ fcodes, const ConvGeom g,
-                                                                     const int rows_out, const int filter_blocks,
-                                                                     const uint32_t offset_input,
-                                                                     const uint32_t offset_filter,
-                                                                     uint32_t *__restrict__ pixel_term,
-                                                                     uint32_t *__restrict__ column_term)
+__device__ __forceinline__ void axconv_terms_body(const int block, uint32_t *__restrict__ ax_lds,
+                                                  const uint8_t *__restrict__ codes, const uint8_t *__restrict__ fcodes,
+                                                  const ConvGeom &g, const int rows_out, const int filter_blocks,
+                                                  const uint32_t offset_input, const uint32_t offset_filter,
+                                                  uint32_t *__restrict__ pixel_term, uint32_t *__restrict__ column_term)
 {
-    extern __shared__ uint32_t ax_lds[];
     const int t = (int)threadIdx.x;
-    if ((int)blockIdx.x < filter_blocks) {
-        const int cl = t % kAxSumCols, slice = t / kAxSumCols, col = (int)blockIdx.x * kAxSumCols + cl;
+    if (block < filter_blocks) {
+        const int cl = t % kAxSumCols, slice = t / kAxSumCols, col = block * kAxSumCols + cl;
         uint32_t s = 0;
         if (col < g.Co)
 #pragma unroll 8
@@ -1796,7 +1807,7 @@ __global__ void __launch_bounds__(kAxSumThreads) axconv_terms_kernel(const uint8
         return;
     }
     const int blocks_per_image = (g.OH + rows_out - 1) / rows_out;
-    const int b = (int)blockIdx.x - filter_blocks, n = b / blocks_per_image;
+    const int b = block - filter_blocks, n = b / blocks_per_image;
     const int oh0 = (b - n * blocks_per_image) * rows_out;
     const int rows = (g.OH - oh0 < rows_out ? g.OH - oh0 : rows_out);
     const int ih0 = oh0 * g.sh - g.ph, rows_in = (rows - 1) * g.sh + (g.KH - 1) * g.dh + 1;
@@ -1838,6 +1849,20 @@ __global__ void __launch_bounds__(kAxSumThreads) axconv_terms_kernel(const uint8
     }
 }
 
+template <int V>
+__global__ void __launch_bounds__(kAxSumThreads) axconv_terms_kernel(const uint8_t *__restrict__ codes,
+                                                                     const uint8_t *__restrict__ fcodes, const ConvGeom g,
+                                                                     const int rows_out, const int filter_blocks,
+                                                                     const uint32_t offset_input,
+                                                                     const uint32_t offset_filter,
+                                                                     uint32_t *__restrict__ pixel_term,
+                                                                     uint32_t *__restrict__ column_term)
+{
+    extern __shared__ uint32_t ax_lds[];
+    axconv_terms_body<V>((int)blockIdx.x, ax_lds, codes, fcodes, g, rows_out, filter_blocks, offset_input, offset_filter, pixel_term,
+                         column_term);
+}
+
 // The same pixel terms, one thread per pixel: for images of which the rows under one output row do not fit the LDS.
 __global__ void __launch_bounds__(256) axconv_pixel_terms_kernel(const uint8_t *__restrict__ codes, ConvGeom g,
                                                                  const uint32_t offset_input, const uint32_t offset_filter,
@@ -1876,13 +1901,17 @@ __global__ void __launch_bounds__(256) axconv_correct_kernel(uint32_t *__restric
     out[i] += pixel_term[m] + column_term[i - m * Co];
 }
 
-hipError_t launch_axconv_terms(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,
-                               int offset_filter, int32_t *pixel_term, int32_t *column_term, hipStream_t stream)
+// How axconv_terms_body is launched for a layer: output rows per workgroup (about a thousand workgroups, at most 32 KiB of LDS;
+// one row may take 64 KiB), and the width of its loads where a pixel is whole chunks and the tensor begins on one.
+struct AxTermsPlan {
+    int rows, filter_blocks, v;
+    unsigned pixel_blocks;   // 0: the rows under one output row do not fit the LDS
+    size_t lds;
+};
+static AxTermsPlan axconv_terms_plan(const uint8_t *codes, const ConvGeom &g)
 {
-    const uint32_t oi = (uint32_t)offset_input, of = (uint32_t)offset_filter;
-    uint32_t *const pt = reinterpret_cast<uint32_t *>(pixel_term), *const ct = reinterpret_cast<uint32_t *>(column_term);
-    const int filter_blocks = (g.Co + kAxSumCols - 1) / kAxSumCols;
-    // output rows per workgroup: about a thousand workgroups, at most 32 KiB of LDS; one row may take 64 KiB
+    AxTermsPlan p;
+    p.filter_blocks = (g.Co + kAxSumCols - 1) / kAxSumCols;
     const int64_t under = (int64_t)(g.KH - 1) * g.dh + 1;
     auto lds_of = [&](int64_t rows) { return ((rows - 1) * g.sh + under) * g.W * 4; };
     int64_t rows = (int64_t)g.N * g.OH / 1024;
@@ -1890,18 +1919,137 @@ hipError_t launch_axconv_terms(const uint8_t *codes, const uint8_t *fcodes, cons
     while (rows > 1 && lds_of(rows) > kAxSumLdsBytes / 2)
         rows = (rows + 1) / 2;
     const bool in_lds = lds_of(rows) <= kAxSumLdsBytes && (int64_t)g.C * g.W * ((rows - 1) * g.sh + under) < (1 << 30) &&
-                        (int64_t)g.N * g.OH + filter_blocks < ((int64_t)1 << 31);
-    const unsigned pixel_blocks = in_lds ? (unsigned)((int64_t)g.N * ((g.OH + rows - 1) / rows)) : 0u;
-    size_t lds = kAxSumThreads * 4;
-    if (in_lds && (size_t)lds_of(rows) > lds)
-        lds = (size_t)lds_of(rows);
-    // wide loads where a pixel is whole chunks and the tensor begins on one
-    const int v = (g.C % 16 == 0 && ((uintptr_t)codes & 15) == 0) ? 16 : (g.C % 4 == 0 && ((uintptr_t)codes & 3) == 0) ? 4 : 1;
-    auto kernel = v == 16 ? axconv_terms_kernel<16> : v == 4 ? axconv_terms_kernel<4> : axconv_terms_kernel<1>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)filter_blocks + pixel_blocks), dim3(kAxSumThreads), lds, stream, codes, fcodes, g,
-                       (int)rows, filter_blocks, oi, of, pt, ct);
-    if (!in_lds)
+                        (int64_t)g.N * g.OH + p.filter_blocks < ((int64_t)1 << 31);
+    p.rows = (int)rows;
+    p.pixel_blocks = in_lds ? (unsigned)((int64_t)g.N * ((g.OH + rows - 1) / rows)) : 0u;
+    p.lds = kAxSumThreads * 4;
+    if (in_lds && (size_t)lds_of(rows) > p.lds)
+        p.lds = (size_t)lds_of(rows);
+    p.v = (g.C % 16 == 0 && ((uintptr_t)codes & 15) == 0) ? 16 : (g.C % 4 == 0 && ((uintptr_t)codes & 3) == 0) ? 4 : 1;
+    return p;
+}
+
+hipError_t launch_axconv_terms(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, int offset_input,
+                               int offset_filter, int32_t *pixel_term, int32_t *column_term, hipStream_t stream)
+{
+    const uint32_t oi = (uint32_t)offset_input, of = (uint32_t)offset_filter;
+    uint32_t *const pt = reinterpret_cast<uint32_t *>(pixel_term), *const ct = reinterpret_cast<uint32_t *>(column_term);
+    const AxTermsPlan plan = axconv_terms_plan(codes, g);
+    auto kernel = plan.v == 16 ? axconv_terms_kernel<16> : plan.v == 4 ? axconv_terms_kernel<4> : axconv_terms_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)plan.filter_blocks + plan.pixel_blocks), dim3(kAxSumThreads), plan.lds, stream, codes,
+                       fcodes, g, plan.rows, plan.filter_blocks, oi, of, pt, ct);
+    if (!plan.pixel_blocks)
         hipLaunchKernelGGL(axconv_pixel_terms_kernel, dim3(blocks_for(g.M, 256)), dim3(256), 0, stream, codes, g, oi, of, pt);
+    return hipGetLastError();
+}
+
+// All that lutgemm_mx_kernel needs of a layer given as codes, in one launch: the filter's pre-expanded rows or packed codes
+// (first: they take longest), the terms of the zero points (integer op), the input's codes in its layout.  One behind the other
+// they were 8, 5 and 7 us, of which each is mostly a launch and a round trip to memory: integer op 3x3 32->64 @32x32x128 77 -> 69.
+struct CodesPrep {
+    const uint8_t *codes, *fcodes;
+    uint32_t *xq;
+    uint16_t *wq, *rows;
+    const uint16_t *tableT;
+    uint32_t *pixel_term, *column_term;
+    ConvGeom g;
+    XqLayout lay;
+    int64_t pixels;
+    int mx_fills;
+    int expand_blocks, pack_blocks, terms_blocks, relayout_x, relayout_y;
+    int rows_out, filter_blocks;
+    uint32_t zp4, offset_input, offset_filter;
+};
+template <int V, int Q>
+__global__ void __launch_bounds__(kAxSumThreads) codes_prep_kernel(const CodesPrep p)
+{
+    extern __shared__ uint32_t cp_lds[];
+    int block = (int)blockIdx.x;
+    const ConvGeom &g = p.g;
+    const TensorQuant none = {};
+    if (block < p.expand_blocks) {
+        px_expand_own_codes<kAxSumThreads / 4>(block, nullptr, p.fcodes, g.KH * g.KW, g.C, g.C4, g.Co, none, p.tableT, p.rows,
+                                               p.mx_fills);
+        return;
+    }
+    block -= p.expand_blocks;
+    if (block < p.pack_blocks) {
+        mx_pack_unit((int64_t)block * kAxSumThreads + threadIdx.x, p.mx_fills, nullptr, p.fcodes, g.KH * g.KW, g.C, g.C4, g.Co, none,
+                     p.wq);
+        return;
+    }
+    block -= p.pack_blocks;
+    if (block < p.terms_blocks) {
+        axconv_terms_body<V>(block, cp_lds, p.codes, p.fcodes, g, p.rows_out, p.filter_blocks, p.offset_input, p.offset_filter,
+                             p.pixel_term, p.column_term);
+        return;
+    }
+    block -= p.terms_blocks;
+    // two blocks of 256 threads side by side (of a last one on its own the other finds no pixels)
+    const int half = (int)threadIdx.x >> 8, pairs = (p.relayout_x + 1) / 2;
+    codes_relayout_body<Q>((int)threadIdx.x & 255, 2 * (int64_t)(block % pairs) + half, block / pairs, p.relayout_x, p.relayout_y,
+                           cp_lds + half * (codes_relayout_lds<Q>() / 4), p.codes, p.pixels, g.N, g.H, g.W, g.C, g.C4, p.lay, p.zp4,
+                           p.xq);
+}
+
+hipError_t launch_codes_prep(const uint8_t *codes, const uint8_t *fcodes, const ConvGeom &g, const XqLayout &lay, uint32_t zp4,
+                             uint32_t *xq, const MxPlan &mx, uint16_t *wq, const uint16_t *tableT, uint16_t *rows, bool terms,
+                             int offset_input, int offset_filter, int32_t *pixel_term, int32_t *column_term, hipStream_t stream,
+                             bool *done)
+{
+    *done = false;
+    const int Q = g.C4 <= 4 ? 4 : g.C4 <= 8 ? 8 : 16;
+    const int64_t pixels = (int64_t)g.N * g.H * g.W, row_fills = (int64_t)mx.n_col_tiles * mx.fills;
+    AxTermsPlan plan = {0, 0, 16, 0u, 0};
+    if (terms) {
+        plan = axconv_terms_plan(codes, g);
+        if (!plan.pixel_blocks)
+            return hipSuccess;
+    }
+    if (!mx.expand && (size_t)row_fills * kPxFillBytes > ((size_t)512 << 20))   // (launch_filter_pack's bound)
+        return hipSuccess;
+    CodesPrep p = {};
+    p.codes = codes;
+    p.fcodes = fcodes;
+    p.xq = xq;
+    p.wq = wq;
+    p.rows = rows;
+    p.tableT = tableT;
+    p.pixel_term = reinterpret_cast<uint32_t *>(pixel_term);
+    p.column_term = reinterpret_cast<uint32_t *>(column_term);
+    p.g = g;
+    p.lay = lay;
+    p.pixels = pixels;
+    p.mx_fills = mx.fills;
+    const int64_t relayout_x = (pixels + 1024 / Q - 1) / (1024 / Q), relayout_y = (g.C4 + Q - 1) / Q;
+    const int64_t expand = mx.expand ? 0 : row_fills * (256 / (kAxSumThreads / 4)), pack = mx.expand ? (row_fills * 16 + kAxSumThreads - 1) / kAxSumThreads : 0;
+    const int64_t terms_blocks = (int64_t)plan.filter_blocks + plan.pixel_blocks;
+    const int64_t blocks = expand + pack + terms_blocks + (relayout_x + 1) / 2 * relayout_y;
+    if (blocks >= (int64_t)1 << 31)
+        return hipSuccess;
+    p.expand_blocks = (int)expand;
+    p.pack_blocks = (int)pack;
+    p.terms_blocks = (int)terms_blocks;
+    p.relayout_x = (int)relayout_x;
+    p.relayout_y = (int)relayout_y;
+    p.rows_out = plan.rows;
+    p.filter_blocks = plan.filter_blocks;
+    p.zp4 = zp4;
+    p.offset_input = (uint32_t)offset_input;
+    p.offset_filter = (uint32_t)offset_filter;
+    const size_t expand_lds = expand ? (size_t)px_expand_stage_dwords<kAxSumThreads / 4>() * 4 + 256 : 0;
+    const size_t lds = std::max(std::max(expand_lds, plan.lds), (size_t)2 * 16 * (1024 / 16 + 1) * 4);   // (Q = 16: the most)
+    auto of_q = [&](auto v) {
+        constexpr int V = decltype(v)::value;
+        return Q == 4 ? codes_prep_kernel<V, 4> : Q == 8 ? codes_prep_kernel<V, 8> : codes_prep_kernel<V, 16>;
+    };
+    auto kernel = plan.v == 16 ? of_q(std::integral_constant<int, 16>()) : plan.v == 4 ? of_q(std::integral_constant<int, 4>())
+                                                                                       : of_q(std::integral_constant<int, 1>());
+    const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(kernel), kAxSumLdsBytes);
+    if (e != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kAxSumThreads), lds, stream, p);
+    *done = true;
     return hipGetLastError();
 }
 
