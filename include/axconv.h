@@ -113,6 +113,22 @@ int axc_fake_approx_conv2d(const axc_table *table, const axc_conv2d_desc *desc, 
 int axc_fake_approx_depthwise_conv2d(const axc_table *table, const axc_conv2d_desc *desc, const float *input,
                                      const float *filter, const float *bias, int activation, float *output,
                                      void *workspace, size_t workspace_bytes, void *stream);
+/* The same two calls one behind the other: a call whose input another such call has just made need not read the whole tensor
+ * once more to find its smallest and largest value.  output: AXC_RANGE_BYTES of device memory (8-byte aligned) that the call
+ * fills with what it saw of its outputs as it stored them, where the kernel that it runs can (output_written says so, when the
+ * call returns); input: what the call that made the input tensor filled.  Either may be null.  Results do not depend on it. */
+#define AXC_RANGE_BYTES 32768
+typedef struct axc_layer_ranges {
+    const void *input;
+    void *output;
+    int32_t output_written;
+} axc_layer_ranges;
+int axc_fake_approx_conv2d_ranged(const axc_table *table, const axc_conv2d_desc *desc, const float *input,
+                                  const float *filter, const float *bias, int activation, float *output,
+                                  axc_layer_ranges *ranges, void *workspace, size_t workspace_bytes, void *stream);
+int axc_fake_approx_depthwise_conv2d_ranged(const axc_table *table, const axc_conv2d_desc *desc, const float *input,
+                                            const float *filter, const float *bias, int activation, float *output,
+                                            axc_layer_ranges *ranges, void *workspace, size_t workspace_bytes, void *stream);
 
 /* The tf1 integer op AxConv2D (tf1/axqconv/axqconv.cc:66-94 registration, :113-278 ReferenceAxConvFunctor,
  * :286-441 AxQuantizedConv2DOp): quint8 input and filter codes in, qint32 out,

@@ -34,6 +34,13 @@ class ConvDims(ctypes.Structure):
             "out_rows", "out_cols", "pad_rows_before", "pad_rows_after", "pad_cols_before", "pad_cols_after")]
 
 
+RANGE_BYTES = 32768
+
+
+class LayerRanges(ctypes.Structure):
+    _fields_ = [("input", ctypes.c_void_p), ("output", ctypes.c_void_p), ("output_written", ctypes.c_int32)]
+
+
 class QuantProps(ctypes.Structure):
     _fields_ = [(n, ctypes.c_float) for n in (
         "input_scale", "input_inv_scale", "input_offset", "filter_scale", "filter_inv_scale", "filter_offset",
@@ -72,6 +79,10 @@ SYMBOLS = [
     ("axc_conv2d_minmax_static", ctypes.c_int, [_vp, _desc, _vp, _vp, _f, _f, _f, _f, _vp, _vp]),
     ("axc_fake_approx_conv2d", ctypes.c_int, [_vp, _desc, _vp, _vp, _vp, ctypes.c_int, _vp, _vp, _sz, _vp]),
     ("axc_fake_approx_depthwise_conv2d", ctypes.c_int, [_vp, _desc, _vp, _vp, _vp, ctypes.c_int, _vp, _vp, _sz, _vp]),
+    ("axc_fake_approx_conv2d_ranged", ctypes.c_int,
+     [_vp, _desc, _vp, _vp, _vp, ctypes.c_int, _vp, ctypes.POINTER(LayerRanges), _vp, _sz, _vp]),
+    ("axc_fake_approx_depthwise_conv2d_ranged", ctypes.c_int,
+     [_vp, _desc, _vp, _vp, _vp, ctypes.c_int, _vp, ctypes.POINTER(LayerRanges), _vp, _sz, _vp]),
     ("axc_axconv2d_quint8", ctypes.c_int, [_vp, _desc, _vp, _vp, ctypes.c_int32, ctypes.c_int32, _vp, _vp, _sz, _vp]),
     ("axc_table_tune_weights", ctypes.c_int, [_vp, _vp]),
     ("axc_quint8_zero_point", ctypes.c_int, [_f, _f, ctypes.POINTER(ctypes.c_int32)]),

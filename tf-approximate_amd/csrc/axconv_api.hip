@@ -1259,7 +1259,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
               float in_min, float in_max, float f_min, float f_max, float *out_f, int32_t *out_i,
               void *workspace, size_t workspace_bytes, void *stream_v, bool layer_mode = false,
               const float *bias = nullptr, int activation = AXC_ACT_NONE, const int *pad_before_override = nullptr,
-              const int32_t *tf1_offset_filter = nullptr)
+              const int32_t *tf1_offset_filter = nullptr, axc_layer_ranges *ranges = nullptr)
 {
     if (!table || !desc)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
@@ -1324,7 +1324,7 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         lq_dev = reinterpret_cast<LayerQuant *>(ws + pd.ws.layer_off + align_up((size_t)4 * kMinMaxBlocks * sizeof(float)));
         const ConvGeom &gf = pd.g_full;
         AXC_HIP(launch_layer_quant(input, (int64_t)gf.N * gf.H * gf.W * gf.C, filter, (int64_t)g.K * g.Co, g.K, partials,
-                                   lq_dev, stream));
+                                   lq_dev, stream, ranges ? static_cast<const float *>(ranges->input) : nullptr));
     }
     if (!codes_mode && !pad_before_override) {
         const DirectPlan direct = choose_direct(pd, layer_mode);
@@ -1577,6 +1577,10 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             m.out_f = nullptr;
             m.out_i = part;
         }
+        if (ranges && ranges->output && out_f && mx_reports_range(*mx, m.linear != 0, g.Co)) {
+            m.range = static_cast<float *>(ranges->output);
+            ranges->output_written = 1;
+        }
         {
             ProfScope ps("lutgemm_mx", stream, mx->expand ? nullptr : "lutgemm_px");
             AXC_HIP(mx->expand ? launch_dense_mx_expand(m, stream) : launch_dense_mx(m, stream));
@@ -1671,7 +1675,7 @@ DepthwiseWorkspace depthwise_workspace(int taps, int C)
 int run_depthwise(const axc_table *table, const axc_conv2d_desc *desc, const float *input, const float *filter,
                   float in_min, float in_max, float f_min, float f_max, float *out_f, int32_t *out_i,
                   void *workspace, size_t workspace_bytes, void *stream_v, bool layer_mode = false,
-                  const float *bias = nullptr, int activation = AXC_ACT_NONE)
+                  const float *bias = nullptr, int activation = AXC_ACT_NONE, axc_layer_ranges *ranges = nullptr)
 {
     if (!table || !desc)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
@@ -1717,7 +1721,8 @@ int run_depthwise(const axc_table *table, const axc_conv2d_desc *desc, const flo
         float *partials = reinterpret_cast<float *>(ws + dws.layer_off);
         lq_dev = reinterpret_cast<LayerQuant *>(ws + dws.layer_off + align_up((size_t)4 * kMinMaxBlocks * sizeof(float)));
         AXC_HIP(launch_layer_quant(input, (int64_t)dm.batch * dm.input_rows * dm.input_cols * C, filter,
-                                   (int64_t)taps * C, taps, partials, lq_dev, stream));
+                                   (int64_t)taps * C, taps, partials, lq_dev, stream,
+                                   ranges ? static_cast<const float *>(ranges->input) : nullptr));
     }
     {
         ProfScope ps("depthwise_filter", stream);
@@ -1740,6 +1745,11 @@ int run_depthwise(const axc_table *table, const axc_conv2d_desc *desc, const flo
     p.lq_dev = lq_dev;
     p.bias = bias;
     p.relu = activation == AXC_ACT_RELU ? 1 : 0;
+    p.range = nullptr;
+    if (ranges && ranges->output && out_f && depthwise_reports_range(p)) {
+        p.range = static_cast<float *>(ranges->output);
+        ranges->output_written = 1;
+    }
     const int cus = device_cus();
     const int64_t blocks_needed = (M * C + kBlockThreads - 1) / kBlockThreads;
     const int grid = (int)(blocks_needed < cus ? blocks_needed : cus);
@@ -1906,6 +1916,40 @@ int axc_fake_approx_depthwise_conv2d(const axc_table *table, const axc_conv2d_de
         return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
     return run_depthwise(table, desc, input, filter, 0.0f, 0.0f, 0.0f, 0.0f, output, nullptr, workspace,
                          workspace_bytes, stream, true, bias, activation);
+}
+
+static int check_ranges(axc_layer_ranges *ranges)
+{
+    if (!ranges)
+        return AXC_OK;
+    ranges->output_written = 0;
+    if ((((uintptr_t)ranges->input | (uintptr_t)ranges->output) & 7) != 0)
+        return fail(AXC_INVALID_ARGUMENT, "ranges must be 8-byte aligned");
+    return AXC_OK;
+}
+
+int axc_fake_approx_conv2d_ranged(const axc_table *table, const axc_conv2d_desc *desc, const float *input,
+                                  const float *filter, const float *bias, int activation, float *output,
+                                  axc_layer_ranges *ranges, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!output)
+        return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
+    if (int rc = check_ranges(ranges))
+        return rc;
+    return run_dense(table, desc, input, filter, nullptr, nullptr, 0, 0.0f, 0.0f, 0.0f, 0.0f, output, nullptr, workspace,
+                     workspace_bytes, stream, true, bias, activation, nullptr, nullptr, ranges);
+}
+
+int axc_fake_approx_depthwise_conv2d_ranged(const axc_table *table, const axc_conv2d_desc *desc, const float *input,
+                                            const float *filter, const float *bias, int activation, float *output,
+                                            axc_layer_ranges *ranges, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!output)
+        return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
+    if (int rc = check_ranges(ranges))
+        return rc;
+    return run_depthwise(table, desc, input, filter, 0.0f, 0.0f, 0.0f, 0.0f, output, nullptr, workspace,
+                         workspace_bytes, stream, true, bias, activation, ranges);
 }
 
 int axc_axconv2d_quint8(const axc_table *table, const axc_conv2d_desc *desc, const uint8_t *input,

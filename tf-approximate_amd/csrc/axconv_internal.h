@@ -124,6 +124,8 @@ struct DenseParams {
     uint32_t *wait_error;
 };
 
+constexpr int kRangePairs = AXC_RANGE_BYTES / 8; // (smallest, largest) of a tensor as one call leaves them to the next
+
 // ---- lutgemm_mx_kernel.hip: lookups summed by the matrix cores ----
 constexpr int kMxThreads = 256;                // four wavefronts, one per SIMD, 512 registers each
 constexpr int kMxWaves = kMxThreads / 64;
@@ -209,7 +211,14 @@ struct MxParams {
     const uint16_t *wq;    // plan.expand: filter codes [column tile][fill][filter element 0..15][column 0..7], and the table
     const uint16_t *tableF;  // with the top bit of every byte flipped, filter-code major
     uint32_t wq_bytes;
+    float *range;          // not null (mx_reports_range): kRangePairs pairs, smallest and largest output
 };
+// Launches that can report the range of their outputs: tall tiles, which layers of many outputs have, in the simple store form.
+constexpr int kMxRangeUnits = 10;
+inline bool mx_reports_range(const MxPlan &plan, const bool linear, const int co)
+{
+    return plan.units >= kMxRangeUnits && !plan.swap && plan.k_splits == 1 && linear && (co & 3) == 0;
+}
 
 // ---- direct_kernel.hip: a whole layer of few lookups in one launch ----
 constexpr int kDirectThreads = 1024, kDirectWaves = kDirectThreads / 64;
@@ -265,7 +274,9 @@ struct DepthwiseParams {
     const float *bias;           // not null: added per channel after the epilogue
     int relu;                    // 1: max(x, 0) last
     int stagger_sleeps;          // s_sleep(127) periods by which every second group of workgroups starts late (0: none)
+    float *range;                // not null (depthwise_reports_range): kRangePairs pairs, smallest and largest output
 };
+bool depthwise_reports_range(const DepthwiseParams &p);
 
 // Row permutation of the expanded table: logical activation code a lives in physical row
 // (a >> 2) | ((a & 3) << 6), so that the four codes one lane transposes land in rows of
@@ -362,8 +373,9 @@ hipError_t launch_patch_sums(const float *x, const ConvGeom &g, const TensorQuan
                              const FilterJob *filter_job = nullptr, bool *filter_done = nullptr,
                              int flat_row_bytes = 0,   // > 0: a fused xq is written in the flat layout
                              bool *px_done = nullptr);
+// input_range: kRangePairs (smallest, largest) pairs of the input, which then is not read
 hipError_t launch_layer_quant(const float *input, int64_t n_input, const float *filter, int64_t n_filter, int K,
-                              float *partials, LayerQuant *lq_dev, hipStream_t stream);
+                              float *partials, LayerQuant *lq_dev, hipStream_t stream, const float *input_range = nullptr);
 constexpr int kMinMaxBlocks = 2048;   // partial (min, max) pairs per tensor in launch_layer_quant's scratch
 // out[n][oh][ow][:] = in[n][oh * sh][ow * sw][:] for tensors of element_bytes-wide elements (C per pixel)
 hipError_t launch_subsample(const void *in, int element_bytes, int N, int H, int W, int C, int sh, int sw, int OH, int OW,

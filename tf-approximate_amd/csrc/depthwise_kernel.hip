@@ -126,7 +126,8 @@ __device__ __forceinline__ dw_rsrc_t dw_make_rsrc(const void *base, uint32_t byt
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
 }
 
-template <int S, int R, bool OUT_I32, bool FQ, bool EPI>
+// RANGE: the launch reports the smallest and the largest of its outputs, a pair per wavefront.
+template <int S, int R, bool OUT_I32, bool FQ, bool EPI, bool RANGE = false>
 __global__ void __launch_bounds__(kBlockThreads) depthwise_lut3x3_kernel(const DepthwiseParams p, const int seg_len,
                                                                           const int nseg, const int wgs_per_group,
                                                                           const int group_slots)
@@ -139,8 +140,12 @@ __global__ void __launch_bounds__(kBlockThreads) depthwise_lut3x3_kernel(const D
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cl = lane & (kDwChannels - 1), half = lane >> 5;
     const int slot = (int)blockIdx.x / wgs_per_group, member = (int)blockIdx.x - slot * wgs_per_group;
-    if (slot >= group_slots)
+    if (slot >= group_slots)   // (the grid is wgs_per_group * group_slots: never)
         return;
+    float lo = INFINITY, hi = -INFINITY;
+    if (RANGE && blockIdx.x == 0)   // pairs that no wavefront of the grid writes below
+        for (int i = (int)gridDim.x * kWaves + tid; i < kRangePairs; i += kBlockThreads)
+            *reinterpret_cast<float2 *>(p.range + 2 * i) = make_float2(INFINITY, -INFINITY);
     TensorQuant q = dw_input_quant(p);
     q.fq = FQ ? 1u : 0u;                                // known at compile time: no branch per value
     const DwEpilogue ep = dw_epilogue_consts(p);
@@ -283,7 +288,13 @@ __global__ void __launch_bounds__(kBlockThreads) depthwise_lut3x3_kernel(const D
                         float v = __fsub_rn(t4, ep.k_m1xm2);
                         if (EPI)
                             v = __fadd_rn(v, bias);
-                        outw = __float_as_uint(has_relu ? fmaxf(v, 0.0f) : v);
+                        v = has_relu ? fmaxf(v, 0.0f) : v;
+                        if (RANGE) {   // what is not stored counts as NaN: as nothing
+                            const float r = (int)ooff[rr] < 0 ? __builtin_nanf("") : v;
+                            lo = fminf(lo, r);
+                            hi = fmaxf(hi, r);
+                        }
+                        outw = __float_as_uint(v);
                     }
                     // streamed past the caches, which the input rows neighbouring bands share need
                     __builtin_amdgcn_raw_buffer_store_b32(outw, o_rsrc, (int)ooff[rr], (int)ocol, 2);
@@ -298,6 +309,14 @@ __global__ void __launch_bounds__(kBlockThreads) depthwise_lut3x3_kernel(const D
                         step(k + decltype(ph)::value, ph);
                 });
         }
+    }
+    if (RANGE) {
+#pragma unroll
+        for (int step = 32; step > 0; step >>= 1) {
+            lo = fminf(lo, __shfl_xor(lo, step));
+            hi = fmaxf(hi, __shfl_xor(hi, step));
+        }
+        *reinterpret_cast<float2 *>(p.range + 2 * ((int)blockIdx.x * kWaves + wave)) = make_float2(lo, hi);   // (by every lane the same)
     }
 }
 
@@ -488,6 +507,12 @@ static hipError_t launch_window(const DepthwiseParams &p, bool out_i32, hipStrea
                                      wgs_per_group, group_slots);
 }
 
+bool depthwise_reports_range(const DepthwiseParams &p)
+{
+    return device_cus() * kWaves <= kRangePairs /* a pair per wavefront */ && p.dh == 1 && p.dw == 1 && p.sh == p.sw && (p.sw == 1 || p.sw == 2) && p.KH == 3 && p.KW == 3 && p.lq_dev &&
+           (int64_t)p.N * p.H * p.W * p.C * 4 < 0x7fffffffll && p.M * p.C * 4 < 0x7fffffffll;
+}
+
 hipError_t launch_depthwise(const DepthwiseParams &p, bool out_i32, int grid, hipStream_t stream)
 {
     // the window kernels address input and output with 32-bit byte offsets and keep the top of that range free
@@ -533,11 +558,12 @@ hipError_t launch_depthwise(const DepthwiseParams &p, bool out_i32, int grid, hi
             return (per_wg + kWaves - 1) / kWaves * (length + 3);
         });
         const int g3 = wgs_per_group * group_slots;
-#define AXC_DW_LAUNCH_AS(S_, R_, I32_, FQ_, EPI_)                                                                     \
-    launch_with_lds(depthwise_lut3x3_kernel<S_, R_, I32_, FQ_, EPI_>, g3, kDwLdsBytes, stream, p, seg.length, seg.count, \
+#define AXC_DW_LAUNCH_AS(S_, R_, I32_, FQ_, ...)                                                                     \
+    launch_with_lds(depthwise_lut3x3_kernel<S_, R_, I32_, FQ_, __VA_ARGS__>, g3, kDwLdsBytes, stream, p, seg.length, seg.count, \
                     wgs_per_group, group_slots)
 #define AXC_DW_LAUNCH(S_, R_)                                                                                        \
     (out_i32    ? AXC_DW_LAUNCH_AS(S_, R_, true, false, false)                                                           \
+     : p.range  ? AXC_DW_LAUNCH_AS(S_, R_, false, true, true, true)                                                      \
      : p.lq_dev ? AXC_DW_LAUNCH_AS(S_, R_, false, true, true)                                                            \
      : epi      ? AXC_DW_LAUNCH_AS(S_, R_, false, false, true)                                                           \
                 : AXC_DW_LAUNCH_AS(S_, R_, false, false, false))

@@ -40,7 +40,9 @@ constexpr uint32_t kMxCb = 2 * kPxFillBytes;
 // Behind that the values the wavefronts' pixels add (patch sums, or the zero-point terms of integer outputs): a dword per
 // pixel of the tile, 256 bytes per unit.
 constexpr uint32_t kMxPixelValues = kMxCb + 32;
-constexpr int mx_lds_bytes(const int units) { return (int)kMxPixelValues + kMxWaves * units * 256; }
+// ... and behind those the smallest and the largest output of every lane so far, for launches that report them.
+constexpr uint32_t mx_range_at(const int units) { return kMxPixelValues + (uint32_t)(kMxWaves * units) * 256u; }
+constexpr int mx_lds_bytes(const int units, const bool range = false) { return (int)mx_range_at(units) + (range ? kMxThreads * 8 : 0); }
 constexpr uint32_t kMxWaveBytes = kPxFillBytes / kMxWaves;   // a wavefront's share of a fill
 constexpr int kMxBlockCols = 8;   // column tiles (of 8) that the workgroups of an XCD walk side by side
 
@@ -61,6 +63,8 @@ __device__ __forceinline__ int mx_lane()
     return lane;
 }
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f32x2 *mx_lds_range;
 typedef __attribute__((address_space(3))) uint32_t *mx_lds_u32;   // from an LDS address (dynamic LDS starts at 0)
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t mx_u32x4 __attribute__((ext_vector_type(4)));
@@ -175,11 +179,25 @@ __device__ __forceinline__ void mx_x_store(const i32x16 (&land)[4], const uint32
     }
 }
 
+// The smallest and the largest of the wavefront's outputs, where the next layer's call looks for them.
+__device__ __forceinline__ void mx_store_range(float *const to, const mx_lds_range range, const int wave)
+{
+    f32x2 r = *range;
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1) {
+        r[0] = fminf(r[0], __shfl_xor(r[0], step));
+        r[1] = fmaxf(r[1], __shfl_xor(r[1], step));
+    }
+    *(f32x2 *)(to + 2 * (blockIdx.x * kMxWaves + wave)) = r;   // (by every lane the same)
+}
+
 // SIMPLE: output rows of whole groups of four pixels (p.linear) and columns in fours.  Its stores need no branch: their
 // descriptor ends behind the tile's last unit, and lanes beyond the last column start at an offset that no descriptor
 // reaches (2^31; 24 * 256 pixels of at most 2^18 bytes stay below 2^32).  An instantiation of its own, because the sums
 // leave no registers for both forms side by side (of U = 2, whose stores are few, the compiler makes none).
-template <int U, bool VEC, bool SIMPLE, bool EXPAND>
+// RANGE: the launch reports the smallest and the largest of its float outputs (p.range); an instantiation of its own, because
+// with these stores beside the others the compiler spills.
+template <int U, bool VEC, bool SIMPLE, bool EXPAND, bool RANGE = false>
 __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParams p)
 {
     fetch_arguments<sizeof(MxParams)>();
@@ -188,6 +206,15 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
 
     if (threadIdx.x < 8)
         ((mx_lds_u32)(lds_mx + kMxCb))[threadIdx.x] = 0u;
+    // (the lane's place is worked out again wherever it is needed: the fill loop leaves no register for it)
+    const auto range_of = [&]() __attribute__((always_inline)) { return (mx_lds_range)(uintptr_t)mx_range_at(U) + (wave * 64 + mx_lane()); };
+    if constexpr (RANGE) {
+        *range_of() = f32x2{__builtin_inff(), -__builtin_inff()};
+        // pairs that no wavefront of the grid writes below
+        if (blockIdx.x == 0)
+            for (int i = (int)(gridDim.x * kMxWaves + threadIdx.x); i < kRangePairs; i += kMxThreads)
+                *(f32x2 *)(p.range + 2 * i) = f32x2{__builtin_inff(), -__builtin_inff()};
+    }
     __syncthreads();   // the only barrier of the kernel
 
     const int n_col = p.plan.n_col_tiles * p.plan.k_splits, n_row = p.plan.n_row_tiles;
@@ -224,8 +251,11 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         tile_end = ntiles;
         tile_step = G;
     }
-    if (tile_first >= tile_end)
+    if (tile_first >= tile_end) {
+        if constexpr (RANGE)
+            mx_store_range(p.range, range_of(), wave);
         return;
+    }
     const uint32_t wofs = EXPAND ? 0u : (uint32_t)wave * kMxWaveBytes;
     // expanding: this lane's filter codes of the fill whose entries are loaded next; and those of the fill stored next
     constexpr uint32_t kCodesAhead = 3;   // fills by which the loop loads filter codes ahead
@@ -479,6 +509,8 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         // kInts: int32 sums; kRelu: the activation
         auto store_tile = [&](auto ints_t, auto relu_t) __attribute__((always_inline)) {
             constexpr bool kInts = decltype(ints_t)::value, kRelu = decltype(relu_t)::value;
+            float lo = __builtin_inff(), hi = -__builtin_inff();
+            const bool relu = p.relu != 0;
             constexpr int kAhead = 6;   // units whose values are read together
 #pragma unroll
             for (int u0 = 0; u0 < U; u0 += kAhead) {
@@ -492,6 +524,8 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
 #pragma unroll
                 for (int k = 0; k < kAhead; ++k) {
                     const int u = u0 + k;
+                    if constexpr (RANGE && U > 20)   // (or the scheduler joins the sums of many units ahead of their turn, and spills)
+                        __builtin_amdgcn_sched_barrier(0);
                     if (u >= U || (!SIMPLE && u * kMxWaves + wave >= p.plan.units_per_tile))
                         continue;
                     const i32x16 &a = acc[u < U ? u : 0];
@@ -520,7 +554,19 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                             for (int e = 0; e < 4; ++e) {
                                 float v = __fadd_rn(__fmul_rn((float)(int32_t)d[e], e_s1xs2), t1);
                                 v = __fadd_rn(__fsub_rn(__fadd_rn(v, t3[e]), e_km), bias[e]);
-                                d[e] = __float_as_uint(kRelu ? fmaxf(v, 0.0f) : v);
+                                if constexpr (RANGE)   // (one form: of two side by side the compiler joins all sums first, and spills)
+                                    d[e] = __float_as_uint(relu ? fmaxf(v, 0.0f) : v);
+                                else
+                                    d[e] = __float_as_uint(kRelu ? fmaxf(v, 0.0f) : v);
+                            }
+                            if constexpr (RANGE) {   // what is not stored counts as NaN: as nothing
+                                const bool there = at[jp] < (uint32_t)out_bytes;
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const float v = there && (SIMPLE || whole || col0 + e < p.Co) ? __uint_as_float(d[e]) : __builtin_nanf("");
+                                    lo = fminf(lo, v);
+                                    hi = fmaxf(hi, v);
+                                }
                             }
                         }
                         if (SIMPLE) {
@@ -536,27 +582,34 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                     }
                 }
             }
+            if constexpr (RANGE) {
+                const mx_lds_range range = range_of();
+                const f32x2 r = *range;
+                *range = f32x2{fminf(r[0], lo), fmaxf(r[1], hi)};
+            }
         };
         using yes = std::true_type;
         using no = std::false_type;
-        if (ints)
+        if (!RANGE && ints)
             store_tile(yes(), no());
-        else if (p.relu)
+        else if (!RANGE && p.relu)
             store_tile(no(), yes());
         else
             store_tile(no(), no());
         asm volatile("" ::: "memory");   // the values are read before the next tile's are fetched into their place
     }
+    if constexpr (RANGE)
+        mx_store_range(p.range, range_of(), wave);
 }
 
-template <int U, bool VEC, bool SIMPLE, bool EXPAND>
+template <int U, bool VEC, bool SIMPLE, bool EXPAND, bool RANGE = false>
 static hipError_t launch_mx_one(const MxParams &p, hipStream_t stream)
 {
-    auto kernel = lutgemm_mx_kernel<U, VEC, SIMPLE, EXPAND>;
-    const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(kernel), mx_lds_bytes(U), true);
+    auto kernel = lutgemm_mx_kernel<U, VEC, SIMPLE, EXPAND, RANGE>;
+    const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(kernel), mx_lds_bytes(U, RANGE), true);
     if (e != hipSuccess)
         return e;
-    hipLaunchKernelGGL(kernel, dim3(p.plan.grid), dim3(kMxThreads), mx_lds_bytes(U), stream, p);
+    hipLaunchKernelGGL(kernel, dim3(p.plan.grid), dim3(kMxThreads), mx_lds_bytes(U, RANGE), stream, p);
     return hipGetLastError();
 }
 
@@ -564,6 +617,10 @@ template <int U, bool EXPAND>
 static hipError_t launch_mx_units(const MxParams &p, hipStream_t stream)
 {
     const bool vec = p.pitch == 4, simple = p.linear && (p.Co & 3) == 0;
+    if constexpr (U >= kMxRangeUnits) {
+        if (p.range)   // (where mx_reports_range says so)
+            return vec ? launch_mx_one<U, true, true, EXPAND, true>(p, stream) : launch_mx_one<U, false, true, EXPAND, true>(p, stream);
+    }
     if constexpr (U > 2) {
         if (simple)
             return vec ? launch_mx_one<U, true, true, EXPAND>(p, stream) : launch_mx_one<U, false, true, EXPAND>(p, stream);

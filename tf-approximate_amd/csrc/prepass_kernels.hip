@@ -1693,20 +1693,29 @@ __device__ void tensor_quant_device(float mn, float mx, TensorQuant *t, int *zer
     *zero_point = zp;
 }
 
-// Stage 2: one workgroup folds the partial pairs of both tensors and writes the layer's constants.
-__global__ void __launch_bounds__(256) layer_quant_kernel(const float *__restrict__ partials, int n_in, int n_flt,
+// Stage 2: one workgroup folds the partial pairs of both tensors and writes the layer's constants.  n_whole > 0: of the filter
+// not pairs but its floats themselves, which are few.
+__global__ void __launch_bounds__(256) layer_quant_kernel(const float *__restrict__ in_pairs, int n_in,
+                                                           const float *__restrict__ flt, int n_flt, int n_whole,
                                                            int K, LayerQuant *__restrict__ out)
 {
     __shared__ float red[4][256];
     float v[4] = {INFINITY, -INFINITY, INFINITY, -INFINITY};
+    const float2 *const pairs = reinterpret_cast<const float2 *>(in_pairs);
+#pragma unroll 8
     for (int i = threadIdx.x; i < n_in; i += 256) {
-        v[0] = fminf(v[0], partials[2 * i]);
-        v[1] = fmaxf(v[1], partials[2 * i + 1]);
+        const float2 p = pairs[i];
+        v[0] = fminf(v[0], p.x);
+        v[1] = fmaxf(v[1], p.y);
     }
-    const float *pf = partials + 2 * kMinMaxBlocks;
     for (int i = threadIdx.x; i < n_flt; i += 256) {
-        v[2] = fminf(v[2], pf[2 * i]);
-        v[3] = fmaxf(v[3], pf[2 * i + 1]);
+        v[2] = fminf(v[2], flt[2 * i]);
+        v[3] = fmaxf(v[3], flt[2 * i + 1]);
+    }
+#pragma unroll 8
+    for (int i = threadIdx.x; i < n_whole; i += 256) {
+        v[2] = fminf(v[2], flt[i]);
+        v[3] = fmaxf(v[3], flt[i]);
     }
     for (int k = 0; k < 4; ++k)
         red[k][threadIdx.x] = v[k];
@@ -1735,16 +1744,23 @@ __global__ void __launch_bounds__(256) layer_quant_kernel(const float *__restric
 }
 
 hipError_t launch_layer_quant(const float *input, int64_t n_input, const float *filter, int64_t n_filter, int K,
-                              float *partials, LayerQuant *lq_dev, hipStream_t stream)
+                              float *partials, LayerQuant *lq_dev, hipStream_t stream, const float *input_range)
 {
     auto blocks = [](int64_t n) {
         const int64_t b = (n + 256 * 32 - 1) / (256 * 32);
         return (int)(b < 1 ? 1 : (b > kMinMaxBlocks ? kMinMaxBlocks : b));
     };
-    const int b_in = blocks(n_input), b_f = blocks(n_filter);
+    float *const flt_pairs = partials + 2 * kMinMaxBlocks;
+    if (input_range && n_filter <= 16384) {   // nothing that a second launch would be worth
+        hipLaunchKernelGGL(layer_quant_kernel, dim3(1), dim3(256), 0, stream, input_range, kRangePairs, filter, 0, (int)n_filter, K,
+                           lq_dev);
+        return hipGetLastError();
+    }
+    const int b_in = input_range ? 0 : blocks(n_input), b_f = blocks(n_filter);
     hipLaunchKernelGGL(minmax_partial_kernel, dim3(b_in + b_f), dim3(256), 0, stream, input, n_input, b_in, filter,
                        n_filter, partials);
-    hipLaunchKernelGGL(layer_quant_kernel, dim3(1), dim3(256), 0, stream, partials, b_in, b_f, K, lq_dev);
+    hipLaunchKernelGGL(layer_quant_kernel, dim3(1), dim3(256), 0, stream, input_range ? input_range : partials,
+                       input_range ? kRangePairs : b_in, flt_pairs, b_f, 0, K, lq_dev);
     return hipGetLastError();
 }
 

@@ -91,6 +91,11 @@ class ApproxNetwork:
                 self.ops[i] = ops.ApproxConv2DWithMinMaxVars([1, spec.stride, spec.stride, 1], 8, self.table, "SAME",
                                                              depthwise=spec.depthwise)
 
+        # convolutions whose output another one reads before the name stands for something else
+        self.feeds = {i for i, step in enumerate(program) if step[0] == "conv" and any(
+            later[0] == "conv" and later[2] == step[1]
+            for later in program[i + 1:next((j + 1 for j in range(i + 1, len(program)) if program[j][1] == step[1]), len(program))])}
+
     def conv_count(self):
         return len(self.ops)
 
@@ -102,6 +107,7 @@ class ApproxNetwork:
         """Returns (output tensor, total approximate MACs).  With a list as `trace`, every convolution appends
         (spec, input, filter, (min/max x4), raw output) as host arrays, for layer-by-layer checks."""
         t = {"input": x}
+        seen = {}   # fused_layers: what the call that made a tensor reported of its range
         macs = 0
         for i, step in enumerate(self.program):
             kind, dst = step[0], step[1]
@@ -109,7 +115,7 @@ class ApproxNetwork:
                 src, spec = t[step[2]], step[3]
                 w = self.weights[i]
                 if self.fused_layers:
-                    y = self.ops[i](src, w)
+                    y, seen[dst] = self.ops[i].call_in_turn(src, w, None, seen.get(step[2]), i in self.feeds)
                     if trace is not None:
                         trace.append((spec, src.cpu().numpy(), w.cpu().numpy(), None, y.cpu().numpy()))
                     macs += spec.macs(y.shape[1], y.shape[2], y.shape[0])
@@ -129,8 +135,10 @@ class ApproxNetwork:
                 macs += spec.macs(y.shape[1], y.shape[2], y.shape[0])
                 t[dst] = y
             elif kind == "add_relu":
+                seen[dst] = None
                 t[dst] = add_relu(t[step[2]], t[step[3]])
             elif kind == "maxpool":
+                seen[dst] = None
                 nchw = t[step[2]].permute(0, 3, 1, 2)
                 t[dst] = torch.nn.functional.max_pool2d(nchw, 3, 2, 1).permute(0, 2, 3, 1).contiguous()
             else:

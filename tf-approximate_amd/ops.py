@@ -277,6 +277,12 @@ class FakeApproxConv2D:
         self.activation = 1 if activation == "relu" else 0
 
     def __call__(self, inputs, kernel, bias=None):
+        return self.call_in_turn(inputs, kernel, bias, None, False)[0]
+
+    def call_in_turn(self, inputs, kernel, bias=None, input_range=None, want_range=True):
+        """The call, for a program that makes one layer's output the next one's input: (output, range).  `range` is what
+        the call saw of its outputs' smallest and largest value, for the input_range of a call on that very output, which
+        then need not read the tensor to find them; None where the kernel that ran does not report it."""
         lib = _lib.load()
         inputs = _require_device_f32(inputs, "input")
         kernel = _require_device_f32(kernel, "filter")
@@ -288,10 +294,18 @@ class FakeApproxConv2D:
         stream = _stream(device)
         ws = layer.workspace(lib, device, stream)
         out = torch.empty(layer.out_shape, dtype=torch.float32, device=device)
-        _launch(device, lib.axc_fake_approx_depthwise_conv2d if self.depthwise else lib.axc_fake_approx_conv2d,
-                self.op.table.handle, layer.ref, inputs.data_ptr(), kernel.data_ptr(),
-                bias.data_ptr() if bias is not None else None, self.activation, out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
-        return out
+        args = (self.op.table.handle, layer.ref, inputs.data_ptr(), kernel.data_ptr(),
+                bias.data_ptr() if bias is not None else None, self.activation, out.data_ptr())
+        if input_range is None and not want_range:
+            _launch(device, lib.axc_fake_approx_depthwise_conv2d if self.depthwise else lib.axc_fake_approx_conv2d,
+                    *args, ws.data_ptr(), ws.numel(), stream)
+            return out, None
+        seen = torch.empty(_lib.RANGE_BYTES // 4, dtype=torch.float32, device=device) if want_range else None
+        ranges = _lib.LayerRanges(None if input_range is None else input_range.data_ptr(),
+                                  None if seen is None else seen.data_ptr(), 0)
+        _launch(device, lib.axc_fake_approx_depthwise_conv2d_ranged if self.depthwise else lib.axc_fake_approx_conv2d_ranged,
+                *args, ctypes.byref(ranges), ws.data_ptr(), ws.numel(), stream)
+        return out, seen if ranges.output_written else None
 
 
 # ---- tf1 AxConv2D (tf1/axqconv/axqconv.cc) ----------------------------------------------------------------------
