@@ -843,7 +843,7 @@ size_t xq_bytes_of(const ConvGeom &g, const XqLayout &l, int flat_row_bytes)
 inline size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct DenseWorkspace {
-    size_t sub_off, xq_off, psum_off, wq_off, fsum_off, layer_off, part_off, px_off, px_bytes;
+    size_t sub_off, xq_off, planes_off, psum_off, wq_off, fsum_off, layer_off, part_off, px_off, px_bytes;
     size_t total;        // everything, the pre-expanded rows (last) included
     size_t total_no_px;  // what a launch needs that does without them
 };
@@ -851,7 +851,7 @@ struct DenseWorkspace {
 // sub_bytes: room for the pixels a strided 1x1 filter reads, gathered into a dense tensor (see prepare_dense).  mx: the
 // plan of lutgemm_mx_kernel where the layer runs that one, else null.
 DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, const MxPlan *mx, const XqLayout &lay,
-                               size_t sub_bytes, int flat_row_bytes)
+                               size_t sub_bytes, int flat_row_bytes, size_t planes_bytes)
 {
     const bool swap = mx && mx->swap;
     const SwapPack sp = swap_pack_of(g);
@@ -860,6 +860,7 @@ DenseWorkspace dense_workspace(const ConvGeom &g, const DensePlan &plan, const M
     w.sub_off = off; off += align_up(sub_bytes);
     w.xq_off = off;
     off += align_up(swap ? (size_t)sp.quads * sp.pitch * 4 + 16 : xq_bytes_of(g, lay, flat_row_bytes));   // + the zero-point row(s)
+    w.planes_off = off; off += align_up(planes_bytes);
     w.psum_off = off; off += align_up((size_t)g.M * 4); // patch sums: one float per output pixel
     w.wq_off = off;
     off += align_up(!mx ? (size_t)plan.n_col_tiles * plan.fills * 64 * 2
@@ -896,9 +897,26 @@ struct PreparedDense {
     bool mx;             // the layer runs lutgemm_mx_kernel, cut as mxp says (plan then only describes the other kernels)
     MxPlan mxp;
     XqLayout lay;
+    bool planes;         // lutgemm_mx_kernel reads its activations tap column by tap column (see planes_ok)
     DenseWorkspace ws;
     bool empty;
 };
+
+// Strided layers of lutgemm_mx_kernel.  At a stride four neighbouring output pixels of a row are no neighbouring dwords of xq: four
+// loads a group, and a fill at U = 13 takes 3.5 us where one load makes 2.1.  So a pass copies xq into a plane per tap column,
+// [image row][tap column][quad][output column] - what the column reads, OW wide, KW / stride of xq's size - which one load reads
+// as it reads stride 1.  prepare_mx takes it where the models of both loads say that it saves more than the pass, 4 us and its
+// bytes at 4 TB/s, costs.  Launch of the kernel without / pass + launch with, us: 3x3/2 128->128 @57x57x64 292 / 22 + 203, 256->256
+// @28x28x64 369 / 13 + 221, 512->512 @14x14x64 366 / 14 + 212; whole op 5x5/(1,2) 162->35 @12x12x10 75 / 46, 3x3/2 80->232
+// @56x56x27 182 / 137, 7x2/(1,2) 32->376 @72x8x7 40.1 / 39.2.  Of 43 random strided layers 19 take it, none is slower for it.
+bool planes_ok(const ConvGeom &g, const XqLayout &lay, const int flat_row_bytes)
+{
+    return !flat_row_bytes && g.sw > 1 && ((int64_t)g.N * lay.Hp + lay.row0) * g.KW * g.C4 * g.OW * 4 + 16 < (int64_t)1 << 31;
+}
+size_t planes_bytes_of(const ConvGeom &g, const XqLayout &lay)
+{
+    return ((size_t)g.N * lay.Hp + lay.row0) * g.KW * g.C4 * g.OW * 4 + 16;
+}
 
 // Decides whether the layer runs lutgemm_mx_kernel, and whether out of pre-expanded rows or of rows that it makes itself:
 // what the cost models, fitted to the launch times of each, say is fastest.  Whole op, us, pre-expanded / own rows / other
@@ -909,27 +927,32 @@ struct PreparedDense {
 // per weight and reading them back outweighs making them anew in every tile.  Over 240 random layers, each timed in every
 // form, the choice is 1.7 % above the fastest.
 enum { kMxNone, kMxOwnRows, kMxRows, kMxAny };   // which forms may run the layer (own rows: operands exchanged too)
-void prepare_mx(PreparedDense *pd, int forms)
+// planes: the layer's activations by tap columns, whatever that costs being in the answer: cycles of the form that was taken.
+double prepare_mx_form(PreparedDense *pd, int forms, bool planes)
 {
+    constexpr double kNone = 1e30;
     const ConvGeom &g = pd->g;
     const XqLayout lay = padded_layout(g, pd->flat_row_bytes > 0);
     const size_t padded = xq_bytes_of(g, lay, pd->flat_row_bytes), plain = xq_bytes_of(g, plain_layout(g), pd->flat_row_bytes);
     if (padded >= ((size_t)1 << 31) || padded > plain + plain / 2 + 65536)   // padding larger than the image: not worth it
-        return;
+        return kNone;
     if (g.M >= ((int64_t)1 << 31) - 4096 || g.Co > 65536)   // pixel numbers and a tile's output offsets in 31 bits
-        return;
+        return kNone;
+    if (planes && !planes_ok(g, lay, pd->flat_row_bytes))
+        return kNone;
     // Pixels of a group that do not exist are read too, up to three pitches behind the input by a scalar offset, which a
     // descriptor's bounds check need not cover: that must still be the workspace (a fill of rows, 64 KiB, lies behind, and
     // without those the layer entry point's 4 * kMinMaxBlocks floats).
-    const int64_t pitch = (int64_t)g.sw * (pd->flat_row_bytes ? g.C : 4);
+    const int64_t pitch = planes ? 4 : (int64_t)g.sw * (pd->flat_row_bytes ? g.C : 4);
     if (3 * pitch > 65536)
-        return;
+        return kNone;
     const int64_t quads = (int64_t)pd->gk.KH * pd->gk.KW * pd->gk.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
     const int64_t fills = (quads + kMxFillQuads - 1) / kMxFillQuads;
     const MxLoads loads = pitch == 4 ? MxLoads::kOne : pd->flat_row_bytes && pitch <= 16 ? MxLoads::kFourClose : MxLoads::kFour;
     const MxPlans plans = make_mx_plans(g, quads, groups, loads, device_cus());
     const MxPlan &own = plans.own, &rows = plans.rows, &swap = plans.swap;
     const double us = 1e-6 * device_clock_hz();
+    const double pass = planes ? (4.0 + (double)(padded + planes_bytes_of(g, lay)) / 4e6) * us : 0.0;
     // Rows beyond some 20 MB for few pixels take 0.19 to 0.23 us a MB of pre-pass where the plan says 0.143 (pre-pass without
     // and with them, us: 5x5 448->48 @28x28x5, 275 MB, 65 / 129; 3x3 864->80 @14x14x41, 320 MB, 113 / 178; 5x5 64->776
     // @13x13x45, 636 MB, 17 / 138): 0.07 more.  Channel counts below 64 that are no multiple of four have a patch-sum kernel of
@@ -946,11 +969,13 @@ void prepare_mx(PreparedDense *pd, int forms)
     if (mode == 3 && swap.units) {
         pd->mx = true;
         pd->mxp = swap;
-        return;
+        return swap.cost;
     }
+    double mine = pass + (expand ? own.cost : rows.cost + slow_rows);
     if (mode == 1) {
-        if (!rows_ok || (pd->plan.px ? rows.cost > pd->plan.cost : rows.cost + slow_rows > pd->plan.cost * 0.98))
-            return;
+        mine = pass + rows.cost + slow_rows;
+        if (!rows_ok || (pd->plan.px ? mine - slow_rows > pd->plan.cost : mine > pd->plan.cost * 0.98))
+            return kNone;
         expand = false;
     } else if (mode == 0) {
         // Outputs that are many for few fills are bound by their stores.  The vector-ALU kernels' leave at 3.0 TB/s at best where
@@ -961,15 +986,15 @@ void prepare_mx(PreparedDense *pd, int forms)
         // MB, 324 / 221, and 10->976 @139x139x10, 754 MB, 466 / 246, which came here while this kernel had no bound.
         const double bytes = (double)g.M * g.Co * 4.0, store = bytes > 256e6 ? bytes / 2.0e6 * us : 0.0;
         const double store_other = bytes / ((g.Co & 3) ? 0.65e6 : (g.Co & 15) ? 1.3e6 : 3.0e6) * us;
-        const double own_cost = std::max((double)own.cost, store);
+        const double own_cost = std::max((double)own.cost, store) + pass;
         // What the plan of pre-expanded rows leaves out: a K split is a little cheaper, and under short chains of patch sums
         // the first 10 MB of rows delay the launch that carries them (pre-pass without and with rows, us: 1x1 64->256
         // @56x56x9, 8 MB, 9.0 / 14.9; 1x1 128->512 @28x28x9, 34 MB, 8.5 / 23.4; but 3x3 64->64 @8x8x128, 19 MB, 12.0 / 14.3).
         // (and loads a few bytes apart are cheaper than planned)
-        const double rows_cost = std::max(rows.cost * (loads == MxLoads::kFourClose ? 0.85 : 1.0) + slow_rows, store) +
+        const double rows_cost = std::max(rows.cost * (loads == MxLoads::kFourClose ? 0.85 : 1.0) + slow_rows, store) + pass +
                                  (1.5 + (g.K <= 256 ? 0.35e-6 : 0.0) * std::min(rows_bytes, 10e6) - (rows.k_splits > 1 ? 2.6 : 0.0)) * us;
         expand = own_ok && (!rows_ok || own_cost < rows_cost);
-        const double mine = expand ? own_cost : rows_ok ? rows_cost : 1e30;
+        mine = expand ? own_cost : rows_ok ? rows_cost : kNone;
         // The vector-ALU kernels' model is low against this one's (compute_plan leaves out what a launch costs), less so for one or
         // two fills and few outputs in whole lines (1x1 18->144 @80x80x8 40 us here, 31 there, predicted 16.6 and 14.7).
         const double left_out = fills <= 2 && (g.Co & 15) == 0 && bytes < 60e6 ? 2.5 : 5.0;
@@ -980,17 +1005,27 @@ void prepare_mx(PreparedDense *pd, int forms)
         if (swap.units && swap_cost < std::min(mine, other)) {
             pd->mx = true;
             pd->mxp = swap;
-            return;
+            return swap_cost;
         }
         if (mine > other)
-            return;
+            return kNone;
     }
     if (!expand && !rows_ok)
-        return;
+        return kNone;
     const MxPlan &plan = expand ? own : rows;
     pd->mx = true;
     pd->mxp = plan;
     pd->lay = lay;
+    pd->planes = planes;
+    return mine;
+}
+
+void prepare_mx(PreparedDense *pd, int forms, bool allow_planes)
+{
+    PreparedDense with = *pd;
+    const double without = prepare_mx_form(pd, forms, false);
+    if (allow_planes && pd->g.sw > 1 && !(pd->mx && pd->mxp.swap) && prepare_mx_form(&with, forms, true) < without && with.planes)
+        *pd = with;
 }
 
 // A 1x1 filter with a stride only ever reads every stride-th pixel, and never needs padding: the op equals the 1x1
@@ -1000,11 +1035,12 @@ void prepare_mx(PreparedDense *pd, int forms)
 // get the layer as given.  mx_mode: which forms of lutgemm_mx_kernel may run the layer.  allow_fold: images of a 1x1 layer may
 // count as one row.
 int compute_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads, int element_bytes, int px_mode, int mx_mode,
-                  bool allow_fold)
+                  bool allow_fold, bool allow_planes)
 {
     const bool allow_subsample = pads == nullptr;
     const bool allow_flat = allow_subsample;   // both are for callers that leave the padding origin to the library
     pd->mx = false;
+    pd->planes = false;
     pd->mxp = MxPlan{};
     pd->lay = XqLayout{};
     int rc = geometry(desc, &pd->dims);
@@ -1092,8 +1128,9 @@ int compute_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     pd->lay = plain_layout(pd->g);
     if (mx_mode != kMxNone && px_mode == kPxModeGlobal && g_px_mode.load(std::memory_order_relaxed) == 0 &&
         g_forced_nt.load(std::memory_order_relaxed) == 0)
-        prepare_mx(pd, mx_mode);
-    pd->ws = dense_workspace(pd->g, pd->plan, pd->mx ? &pd->mxp : nullptr, pd->lay, sub_bytes, pd->flat_row_bytes);
+        prepare_mx(pd, mx_mode, allow_planes);
+    pd->ws = dense_workspace(pd->g, pd->plan, pd->mx ? &pd->mxp : nullptr, pd->lay, sub_bytes, pd->flat_row_bytes,
+                             pd->planes ? planes_bytes_of(pd->g, pd->lay) : 0);
     return AXC_OK;
 }
 
@@ -1101,10 +1138,10 @@ int compute_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
 // several plans among it.  The key is all that it depends on: the descriptor, the arguments, the pinned forms and the device's
 // compute units.
 int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
-                  int px_mode = kPxModeGlobal, int mx_mode = kMxAny, bool allow_fold = true)
+                  int px_mode = kPxModeGlobal, int mx_mode = kMxAny, bool allow_fold = true, bool allow_planes = true)
 {
     if (!desc)
-        return compute_dense(desc, pd, pads, element_bytes, px_mode, mx_mode, allow_fold);
+        return compute_dense(desc, pd, pads, element_bytes, px_mode, mx_mode, allow_fold, allow_planes);
     typedef std::array<int64_t, 36> Key;
     Key key{};
     size_t n = 0;
@@ -1117,7 +1154,7 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
     for (int i = 0; i < 8; ++i)
         key[n++] = desc->explicit_paddings[i];
     for (const int v : {desc->padding, desc->data_format, desc->num_bits, pads ? 1 : 0, pads ? pads[0] : 0, pads ? pads[1] : 0,
-                        element_bytes * 2 + (allow_fold ? 1 : 0), px_mode * 8 + mx_mode,
+                        element_bytes * 4 + (allow_fold ? 1 : 0) + (allow_planes ? 2 : 0), px_mode * 8 + mx_mode,
                         g_forced_nt.load(std::memory_order_relaxed), g_px_mode.load(std::memory_order_relaxed),
                         g_mx_rows.load(std::memory_order_relaxed), device_cus()})
         key[n++] = v;
@@ -1131,7 +1168,7 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
             return AXC_OK;
         }
     }
-    const int rc = compute_dense(desc, pd, pads, element_bytes, px_mode, mx_mode, allow_fold);
+    const int rc = compute_dense(desc, pd, pads, element_bytes, px_mode, mx_mode, allow_fold, allow_planes);
     if (rc != AXC_OK)
         return rc;
     std::lock_guard<std::mutex> lock(mu);
@@ -1161,10 +1198,16 @@ int prepare_dense_for(const axc_conv2d_desc *desc, size_t workspace_bytes, const
     size_t least = SIZE_MAX;
     for (bool fold : {true, false}) {
         for (int mx_mode : {kMxAny, kMxOwnRows, kMxRows, kMxNone}) {   // (rows: no K split where the others' sums do not fit)
-            const int rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, mx_mode, fold);
+            int rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, mx_mode, fold);
             if (rc != AXC_OK)
                 return rc;
             least = std::min(least, pd->ws.total_no_px);
+            if (pd->planes && workspace_bytes < pd->ws.total) {   // the same without the planes' room
+                rc = prepare_dense(desc, pd, pads, element_bytes, kPxModeGlobal, mx_mode, fold, false);
+                if (rc != AXC_OK)
+                    return rc;
+                least = std::min(least, pd->ws.total_no_px);
+            }
             if (!pd->mx || workspace_bytes >= pd->ws.total)
                 break;
         }
@@ -1516,6 +1559,13 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         m.plan = *mx;
         m.xq = xq;
         m.xq_bytes = (uint32_t)xq_bytes_of(g, pd.lay, pd.flat_row_bytes);
+        if (pd.planes) {
+            uint32_t *const planes = reinterpret_cast<uint32_t *>(ws + pd.ws.planes_off);
+            m.xq = planes;
+            m.xq_bytes = (uint32_t)planes_bytes_of(g, pd.lay);
+            ProfScope ps("split_columns", stream);
+            AXC_HIP(launch_split_columns(xq, g, pd.lay, planes, stream));
+        }
         m.rows = px_rows;
         m.rows_bytes = (uint32_t)pd.ws.px_bytes;
         m.wq = wq;
@@ -1544,15 +1594,16 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         m.div_oh = mx_div((uint32_t)g.OH);
         m.div_c4 = mx_div((uint32_t)gk.C4);
         m.div_kw = mx_div((uint32_t)gk.KW);
-        const uint32_t row = flat ? (uint32_t)pd.flat_row_bytes : (uint32_t)g.C4 * (uint32_t)pd.lay.Wp * 4u;
-        m.pitch = flat ? (uint32_t)(g.sw * g.C) : (uint32_t)g.sw * 4u;
-        m.origin = (uint32_t)(pd.lay.row0 - g.ph) * row + (flat ? 0u : (uint32_t)(pd.lay.col0 - g.pw) * 4u);
+        const uint32_t columns = pd.planes ? (uint32_t)g.OW : (uint32_t)pd.lay.Wp;   // of a row of one quad
+        const uint32_t row = flat ? (uint32_t)pd.flat_row_bytes : (uint32_t)g.C4 * columns * 4u * (pd.planes ? (uint32_t)g.KW : 1u);
+        m.pitch = flat ? (uint32_t)(g.sw * g.C) : pd.planes ? 4u : (uint32_t)g.sw * 4u;
+        m.origin = (uint32_t)(pd.lay.row0 - g.ph) * row + (flat || pd.planes ? 0u : (uint32_t)(pd.lay.col0 - g.pw) * 4u);
         m.img_step = (uint32_t)pd.lay.Hp * row;
         m.orow_step = (uint32_t)g.sh * row;
         m.group_step = 4u * m.pitch;
         m.kh_step = (uint32_t)g.dh * row;
-        m.kw_step = (uint32_t)g.dw * 4u;   // (the flat layout has one tap per filter row)
-        m.quad_step = flat ? 4u : (uint32_t)pd.lay.Wp * 4u;
+        m.quad_step = flat ? 4u : columns * 4u;
+        m.kw_step = pd.planes ? (uint32_t)g.C4 * m.quad_step : (uint32_t)g.dw * 4u;   // (the flat layout has one tap per filter row)
         m.c4 = gk.C4;
         m.kw = gk.KW;
         // four quads on = `taps` whole taps and dq quads

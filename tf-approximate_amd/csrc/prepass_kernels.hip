@@ -2633,6 +2633,34 @@ hipError_t launch_codes_relayout(const uint8_t *codes, const ConvGeom &g, const 
     return hipGetLastError();
 }
 
+// xq by tap columns: plane kw of an image row holds, quad after quad, the dwords that output columns 0 .. OW - 1 read under tap
+// column kw.  A workgroup copies a plane of a row (rows: of all images with their padding, and those behind the last one that a
+// filter reaches).  Bound by memory: 57x57x64 of 32 quads under three columns, 27 MB in and 39 out, 21.6 us, 3.0 TB/s of what has
+// to move; the second and third read of a row come from L2.
+__global__ void __launch_bounds__(256) split_columns_kernel(const uint32_t *__restrict__ xq, const int row_dwords, const int Wp,
+                                                            const int C4, const int KW, const int OW, const int stride,
+                                                            const int dilation, const int first, uint32_t *__restrict__ planes)
+{
+    const int row = (int)(blockIdx.x / (uint32_t)KW), kw = (int)blockIdx.x - row * KW;
+    const uint32_t *const src = xq + (int64_t)row * row_dwords + first + kw * dilation;
+    uint32_t *const dst = planes + (int64_t)blockIdx.x * (C4 * OW);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < C4 * OW; i += 256) {
+        const int q = (int)((uint32_t)i / (uint32_t)OW), ow = i - q * OW;
+        dst[i] = src[q * Wp + ow * stride];
+    }
+}
+
+hipError_t launch_split_columns(const uint32_t *xq, const ConvGeom &g, const XqLayout &lay, uint32_t *planes, hipStream_t stream)
+{
+    const int64_t blocks = ((int64_t)g.N * lay.Hp + lay.row0) * g.KW;
+    if (blocks <= 0 || blocks >= (int64_t)1 << 31)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(split_columns_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, xq, g.C4 * lay.Wp, lay.Wp, g.C4, g.KW, g.OW,
+                       g.sw, g.dw, lay.col0 - g.pw, planes);
+    return hipGetLastError();
+}
+
 hipError_t launch_filter_pack(const float *filter, const uint8_t *filter_codes, const ConvGeom &g,
                               const DensePlan &plan, const MxPlan *mx, const TensorQuant &tq, const LayerQuant *lq_dev, uint16_t *wq,
                               float *fsum, hipStream_t stream, const uint16_t *tableT, uint16_t *px_rows, bool *px_done)
