@@ -943,8 +943,9 @@ double prepare_mx_form(PreparedDense *pd, int forms, bool planes)
     // Pixels of a group that do not exist are read too, up to three pitches behind the input by a scalar offset, which a
     // descriptor's bounds check need not cover: that must still be the workspace (a fill of rows, 64 KiB, lies behind, and
     // without those the layer entry point's 4 * kMinMaxBlocks floats).
-    const int64_t pitch = planes ? 4 : (int64_t)g.sw * (pd->flat_row_bytes ? g.C : 4);
-    if (3 * pitch > 65536)
+    // (By tap columns the pitch is 4 whatever the stride; no layer comes here for that alone.)
+    const int64_t apart = (int64_t)g.sw * (pd->flat_row_bytes ? g.C : 4), pitch = planes ? 4 : apart;
+    if (3 * apart > 65536)
         return kNone;
     const int64_t quads = (int64_t)pd->gk.KH * pd->gk.KW * pd->gk.C4, groups = (int64_t)g.N * g.OH * ((g.OW + 3) / 4);
     const int64_t fills = (quads + kMxFillQuads - 1) / kMxFillQuads;
@@ -963,7 +964,7 @@ double prepare_mx_form(PreparedDense *pd, int forms, bool planes)
     const double rows_bytes = (double)rows.n_col_tiles * rows.fills * 65536.0;
     const double slow_rows = std::max(0.0, rows_bytes - 22e6) * ((g.C & 3) && (g.C < 64 || mode == 1) ? 0.2e-6 : 0.07e-6) * us;
     const bool rows_ok = forms != kMxOwnRows && rows.units && rows_bytes <= (double)kPxMaxBytes;
-    const bool own_ok = own.units && 3 * pitch <= (int64_t)(4 * kMinMaxBlocks * sizeof(float)) &&
+    const bool own_ok = own.units && 3 * apart <= (int64_t)(4 * kMinMaxBlocks * sizeof(float)) &&
                         (int64_t)own.n_col_tiles * own.fills * kMxCodeBytes < ((int64_t)1 << 31);
     bool expand = own_ok;
     if (mode == 3 && swap.units) {
