@@ -230,6 +230,17 @@ int axc_depthwise_conv2d_minmax_bias_act(const axc_table *table, const axc_conv2
                                          const float *bias, int activation,
                                          float *output, void *workspace, size_t workspace_bytes, void *stream);
 
+/* axc_conv2d_minmax_bias_act with another tensor added before the activation, as a residual network adds one to a
+ * convolution's output: activation((op + bias) + addend), each step rounded on its own.  No counterpart in the reference.
+ * addend: the output's shape, no overlap with it.  The activation keeps NaN here (s > 0 ? s : s == s ? 0 : s), as the
+ * elementwise pass that this call saves does.  The sum is made where the outputs are, or in a pass of its own behind kernels
+ * that do not take it along. */
+int axc_conv2d_minmax_bias_add_act(const axc_table *table, const axc_conv2d_desc *desc,
+                                   const float *input, const float *filter,
+                                   float input_min, float input_max, float filter_min, float filter_max,
+                                   const float *bias, const float *addend, int activation,
+                                   float *output, void *workspace, size_t workspace_bytes, void *stream);
+
 /* axc_conv2d_minmax for callers that cannot allocate or own a workspace (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The workspace is a fixed array of
  * axc_conv2d_static_workspace_limit() bytes (32 MiB) inside the library's device image, one copy per GPU, held

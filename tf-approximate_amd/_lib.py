@@ -72,6 +72,7 @@ SYMBOLS = [
     ("axc_depthwise_conv2d_workspace_bytes", ctypes.c_int, [_desc, ctypes.POINTER(_sz)]),
     ("axc_conv2d_minmax", ctypes.c_int, [_vp, _desc, _vp, _vp] + _launch_tail),
     ("axc_depthwise_conv2d_minmax", ctypes.c_int, [_vp, _desc, _vp, _vp] + _launch_tail),
+    ("axc_conv2d_minmax_bias_add_act", ctypes.c_int, [_vp, _desc, _vp, _vp, _f, _f, _f, _f, _vp, _vp, ctypes.c_int, _vp, _vp, _sz, _vp]),
     ("axc_conv2d_minmax_bias_act", ctypes.c_int, [_vp, _desc, _vp, _vp, _f, _f, _f, _f, _vp, ctypes.c_int, _vp, _vp, _sz, _vp]),
     ("axc_depthwise_conv2d_minmax_bias_act", ctypes.c_int,
      [_vp, _desc, _vp, _vp, _f, _f, _f, _f, _vp, ctypes.c_int, _vp, _vp, _sz, _vp]),

@@ -1252,14 +1252,15 @@ DirectPlan choose_direct(const PreparedDense &pd, const bool fake_quant)
 }
 
 DirectParams direct_params(const ConvGeom &g, const DirectPlan &plan, const axc_table *table, const axc_quant_props &qp,
-                           const LayerQuant *lq_dev, const float *input, const float *filter, const float *bias, int activation,
-                           float *out_f, int32_t *out_i)
+                           const LayerQuant *lq_dev, const float *input, const float *filter, const float *bias,
+                           const float *addend, int activation, float *out_f, int32_t *out_i)
 {
     DirectParams d = {};
     d.plan = plan;
     d.x = input;
     d.f = filter;
     d.bias = bias;
+    d.addend = addend;
     d.tableT = table->dev_tableT;
     d.out_f = out_f;
     d.out_i = out_i;
@@ -1303,7 +1304,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
               float in_min, float in_max, float f_min, float f_max, float *out_f, int32_t *out_i,
               void *workspace, size_t workspace_bytes, void *stream_v, bool layer_mode = false,
               const float *bias = nullptr, int activation = AXC_ACT_NONE, const int *pad_before_override = nullptr,
-              const int32_t *tf1_offset_filter = nullptr, axc_layer_ranges *ranges = nullptr)
+              const int32_t *tf1_offset_filter = nullptr, axc_layer_ranges *ranges = nullptr,
+              const float *addend = nullptr)
 {
     if (!table || !desc)
         return fail(AXC_INVALID_ARGUMENT, "null argument");
@@ -1341,6 +1343,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         // a fill kernel rather than hipMemsetAsync: callers may capture the stream into a graph
         AXC_HIP(launch_fill_u32(out_i ? reinterpret_cast<uint32_t *>(out_i) : reinterpret_cast<uint32_t *>(out_f), n, 0u,
                                 stream));
+        if (addend)
+            AXC_HIP(launch_add(out_f, addend, n, activation == AXC_ACT_RELU, stream));
         return AXC_OK;
     }
     // a workspace without room for the pre-expanded rows still serves: the layer then runs without them
@@ -1374,7 +1378,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
         const DirectPlan direct = choose_direct(pd, layer_mode);
         if (direct.us > 0.0f) {
             ProfScope ps("direct", stream);
-            AXC_HIP(launch_direct(direct_params(pd.g_full, direct, table, qp, lq_dev, input, filter, bias, activation, out_f, out_i),
+            AXC_HIP(launch_direct(direct_params(pd.g_full, direct, table, qp, lq_dev, input, filter, bias, addend, activation,
+                                                out_f, out_i),
                                   stream));
             return AXC_OK;
         }
@@ -1479,7 +1484,13 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     p.zp4 = zp4;
     p.lq_dev = lq_dev;
     p.bias = bias;
+    p.addend = addend;
     p.relu = activation == AXC_ACT_RELU ? 1 : 0;
+    // the sum with `addend`, and the activation behind it, where the launch that makes the outputs does not take them along
+    auto add = [&]() {
+        ProfScope ps("add", stream);
+        return launch_add(out_f, addend, g.M * g.Co, activation == AXC_ACT_RELU, stream);
+    };
     {
         const int64_t step = 64 * (kDenseWaves / 2), ohow = (int64_t)g.OH * g.OW;
         p.step_n = (int)(step / ohow);
@@ -1633,6 +1644,11 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             m.range = static_cast<float *>(ranges->output);
             ranges->output_written = 1;
         }
+        const bool adds = addend && mx_adds(*mx, m.linear != 0, m.pitch, g.Co);
+        if (adds)
+            m.addend = addend;
+        else if (addend)
+            m.relu = 0;
         {
             ProfScope ps("lutgemm_mx", stream, mx->expand ? nullptr : "lutgemm_px");
             AXC_HIP(mx->expand ? launch_dense_mx_expand(m, stream) : launch_dense_mx(m, stream));
@@ -1641,6 +1657,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
             p.plan.k_splits = mx->k_splits;
             ProfScope ps("splitk_epilogue", stream);
             AXC_HIP(launch_splitk_epilogue(p, part, out_f, out_i, stream));
+        } else if (addend && !adds) {
+            AXC_HIP(add());
         }
         return AXC_OK;
     }
@@ -1689,6 +1707,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     if (splits) {
         p.out_f = nullptr;
         p.out_i = part;
+    } else if (addend) {
+        p.relu = 0;
     }
     if (use_px) {
         ProfScope ps("lutgemm_px", stream);
@@ -1700,6 +1720,8 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     if (splits) {
         ProfScope ps("splitk_epilogue", stream);
         AXC_HIP(launch_splitk_epilogue(p, part, out_f, out_i, stream));
+    } else if (addend) {
+        AXC_HIP(add());
     }
     if (tf1_offset_filter) {
         ProfScope ps("axconv_correction", stream);
@@ -2236,6 +2258,17 @@ int axc_conv2d_minmax_bias_act(const axc_table *table, const axc_conv2d_desc *de
         return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
     return run_dense(table, desc, input, filter, nullptr, nullptr, 0, input_min, input_max, filter_min,
                      filter_max, output, nullptr, workspace, workspace_bytes, stream, false, bias, activation);
+}
+
+int axc_conv2d_minmax_bias_add_act(const axc_table *table, const axc_conv2d_desc *desc, const float *input,
+                                   const float *filter, float input_min, float input_max, float filter_min,
+                                   float filter_max, const float *bias, const float *addend, int activation, float *output,
+                                   void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!output || !addend)
+        return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
+    return run_dense(table, desc, input, filter, nullptr, nullptr, 0, input_min, input_max, filter_min, filter_max, output,
+                     nullptr, workspace, workspace_bytes, stream, false, bias, activation, nullptr, nullptr, nullptr, addend);
 }
 
 int axc_depthwise_conv2d_minmax_bias_act(const axc_table *table, const axc_conv2d_desc *desc, const float *input,

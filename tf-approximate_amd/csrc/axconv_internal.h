@@ -103,6 +103,7 @@ struct DenseParams {
                                   // images, output rows and output columns
     const LayerQuant *lq_dev;    // not null: epilogue constants come from here instead of the four floats above
     const float *bias;           // not null: added to every output column after the epilogue
+    const float *addend;         // not null: a tensor like the output, added before the activation, by the epilogues of split sums
     int relu;                    // 1: max(x, 0) last
     int stagger_sleeps;          // s_sleep(127) periods by which group g of the workgroups starts late, times g (0: none)
     int stagger_groups;          // g = 0 .. stagger_groups - 1 in turn (2: every second group, the only form lutgemm_expand has)
@@ -212,7 +213,13 @@ struct MxParams {
     const uint16_t *tableF;  // with the top bit of every byte flipped, filter-code major
     uint32_t wq_bytes;
     float *range;          // not null (mx_reports_range): kRangePairs pairs, smallest and largest output
+    const float *addend;   // not null (mx_adds): a tensor like the output, added before the activation
 };
+// Launches that can add a tensor to their outputs: the simple store form, activations by one load.
+inline bool mx_adds(const MxPlan &plan, const bool linear, const uint32_t pitch, const int co)
+{
+    return !plan.swap && plan.k_splits == 1 && linear && pitch == 4 && (co & 3) == 0;
+}
 // Launches that can report the range of their outputs: tall tiles, which layers of many outputs have, in the simple store form.
 constexpr int kMxRangeUnits = 10;
 inline bool mx_reports_range(const MxPlan &plan, const bool linear, const int co)
@@ -250,6 +257,7 @@ struct DirectParams {
     const uint16_t *tableT;
     float *out_f;
     int32_t *out_i;
+    const float *addend;
     const LayerQuant *lq_dev;
     TensorQuant in_q, flt_q;
     float s1xs2, m1, m2, k_m1xm2;
@@ -410,6 +418,13 @@ hipError_t launch_split_columns(const uint32_t *xq, const ConvGeom &g, const XqL
 hipError_t launch_swap_pack(const float *x, const uint8_t *codes, const float *filter, const uint8_t *filter_codes,
                             const ConvGeom &g, const TensorQuant &tq_in, const TensorQuant &tq_f, const LayerQuant *lq_dev,
                             uint32_t *xq, uint16_t *wq, hipStream_t stream);
+// out = activation(out + addend), n values
+hipError_t launch_add(float *out, const float *addend, int64_t n, bool relu, hipStream_t stream);
+// max(s, 0) as the networks' residual sums have it: NaN stays, and -0 becomes 0
+__device__ __forceinline__ float sum_activation(const float s, const int relu)
+{
+    return relu && s <= 0.0f ? 0.0f : s;
+}
 hipError_t launch_swap_epilogue(const DenseParams &p, const int32_t *partials, int k_splits, int m_pitch, float *out_f,
                                 int32_t *out_i, hipStream_t stream);
 hipError_t launch_dense_mx(const MxParams &p, hipStream_t stream);          // out of pre-expanded rows

@@ -455,7 +455,7 @@ __global__ void __launch_bounds__(kDirectThreads, 1) direct_kernel(const DirectP
         }
         dk_meet();
         const dk_args p = dk_arguments();
-        const float *const bias = p->bias;
+        const float *const bias = p->bias, *const addend = p->addend;
         const LayerQuant *const lq = p->lq_dev;
         float s1xs2 = p->s1xs2, m1 = p->m1, m2 = p->m2, k_m1xm2 = p->k_m1xm2;
         if (lq) {
@@ -481,7 +481,10 @@ __global__ void __launch_bounds__(kDirectThreads, 1) direct_kernel(const DirectP
             float v = __fadd_rn(__fmul_rn((float)s, s1xs2), __fmul_rn(m2, psum[pixel]));
             v = __fsub_rn(__fadd_rn(v, __fmul_rn(m1, fsum[c])), k_m1xm2);
             v = __fadd_rn(v, bias ? bias[col] : -0.0f);   // no bias: -0.0f, which changes no value
-            p->out_f[at] = p->relu ? fmaxf(v, 0.0f) : v;
+            if (addend)
+                p->out_f[at] = sum_activation(__fadd_rn(v, addend[at]), p->relu);
+            else
+                p->out_f[at] = p->relu ? fmaxf(v, 0.0f) : v;
         }
         dk_meet();   // the next tile's geometry and chunks
     }

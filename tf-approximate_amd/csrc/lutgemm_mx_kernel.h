@@ -197,7 +197,8 @@ __device__ __forceinline__ void mx_store_range(float *const to, const mx_lds_ran
 // leave no registers for both forms side by side (of U = 2, whose stores are few, the compiler makes none).
 // RANGE: the launch reports the smallest and the largest of its float outputs (p.range); an instantiation of its own, because
 // with these stores beside the others the compiler spills.
-template <int U, bool VEC, bool SIMPLE, bool EXPAND, bool RANGE = false>
+// ADD: a tensor like the output is added before the activation (p.addend), in an instantiation of its own for the same reason.
+template <int U, bool VEC, bool SIMPLE, bool EXPAND, bool RANGE = false, bool ADD = false>
 __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParams p)
 {
     fetch_arguments<sizeof(MxParams)>();
@@ -512,6 +513,25 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
             float lo = __builtin_inff(), hi = -__builtin_inff();
             const bool relu = p.relu != 0;
             constexpr int kAhead = 6;   // units whose values are read together
+            // What is added is loaded a batch of units ahead of its use: the vector-memory counter goes down in order, so a load
+            // waits for the stores before it, here those of two batches ago.  Bound by memory (1x1 64->256 @56x56x64, 205 MB in
+            // and out, on top of the 145 us that the layer takes: batches of 4 units 72 us, of 6 93, a window of 6 units that
+            // moves on by one 81, by two 77; an elementwise pass took 118).
+            constexpr int kBatch = 4;
+            const rsrc_t add_rsrc = make_rsrc(ADD ? p.addend + m_first * p.Co : nullptr, ADD ? (uint32_t)out_bytes : 0u);
+            const float floor = relu ? 0.0f : -__builtin_inff();
+            mx_u32x4 added[ADD ? U : 1][2];
+            auto load_added = [&](const int from, const int to) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (u >= from && u < to) {
+                        const uint32_t at = at0 + (uint32_t)u * (kMxWaves * 64u) * pixel_bytes;
+                        added[u][0] = __builtin_amdgcn_raw_buffer_load_b128(add_rsrc, (int)at, 0, 0);
+                        added[u][1] = __builtin_amdgcn_raw_buffer_load_b128(add_rsrc, (int)(at + 2u * pixel_bytes), 0, 0);
+                    }
+            };
+            if constexpr (ADD)
+                load_added(0, kBatch);
 #pragma unroll
             for (int u0 = 0; u0 < U; u0 += kAhead) {
                 uint32_t ps[kAhead][2];
@@ -524,10 +544,13 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
 #pragma unroll
                 for (int k = 0; k < kAhead; ++k) {
                     const int u = u0 + k;
-                    if constexpr (RANGE && U > 20)   // (or the scheduler joins the sums of many units ahead of their turn, and spills)
+                    if constexpr ((RANGE && U > 20) || ADD)   // (or the scheduler joins the sums of many units ahead of their turn, and spills)
                         __builtin_amdgcn_sched_barrier(0);
                     if (u >= U || (!SIMPLE && u * kMxWaves + wave >= p.plan.units_per_tile))
                         continue;
+                    if constexpr (ADD)
+                        if (u % kBatch == 0)
+                            load_added(u + kBatch, u + 2 * kBatch);
                     const i32x16 &a = acc[u < U ? u : 0];
                     uint32_t at[2] = {at0 + (uint32_t)u * (kMxWaves * 64u) * pixel_bytes, 0u};
                     at[1] = at[0] + 2u * pixel_bytes;
@@ -554,7 +577,10 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
                             for (int e = 0; e < 4; ++e) {
                                 float v = __fadd_rn(__fmul_rn((float)(int32_t)d[e], e_s1xs2), t1);
                                 v = __fadd_rn(__fsub_rn(__fadd_rn(v, t3[e]), e_km), bias[e]);
-                                if constexpr (RANGE)   // (one form: of two side by side the compiler joins all sums first, and spills)
+                                if constexpr (ADD) {   // (as the elementwise pass has it: NaN stays, and no sum of -0 does)
+                                    v = __fadd_rn(v, __uint_as_float(added[u < U ? u : 0][jp][e]));
+                                    d[e] = __float_as_uint(!(v <= floor) ? v : floor);
+                                } else if constexpr (RANGE)   // (one form: of two side by side the compiler joins all sums first, and spills)
                                     d[e] = __float_as_uint(relu ? fmaxf(v, 0.0f) : v);
                                 else
                                     d[e] = __float_as_uint(kRelu ? fmaxf(v, 0.0f) : v);
@@ -590,9 +616,9 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         };
         using yes = std::true_type;
         using no = std::false_type;
-        if (!RANGE && ints)
+        if (!RANGE && !ADD && ints)
             store_tile(yes(), no());
-        else if (!RANGE && p.relu)
+        else if (!RANGE && !ADD && p.relu)
             store_tile(no(), yes());
         else
             store_tile(no(), no());
@@ -602,10 +628,10 @@ __global__ void __launch_bounds__(kMxThreads, 1) lutgemm_mx_kernel(const MxParam
         mx_store_range(p.range, range_of(), wave);
 }
 
-template <int U, bool VEC, bool SIMPLE, bool EXPAND, bool RANGE = false>
+template <int U, bool VEC, bool SIMPLE, bool EXPAND, bool RANGE = false, bool ADD = false>
 static hipError_t launch_mx_one(const MxParams &p, hipStream_t stream)
 {
-    auto kernel = lutgemm_mx_kernel<U, VEC, SIMPLE, EXPAND, RANGE>;
+    auto kernel = lutgemm_mx_kernel<U, VEC, SIMPLE, EXPAND, RANGE, ADD>;
     const hipError_t e = set_max_dynamic_lds_once(reinterpret_cast<const void *>(kernel), mx_lds_bytes(U, RANGE), true);
     if (e != hipSuccess)
         return e;
@@ -617,6 +643,8 @@ template <int U, bool EXPAND>
 static hipError_t launch_mx_units(const MxParams &p, hipStream_t stream)
 {
     const bool vec = p.pitch == 4, simple = p.linear && (p.Co & 3) == 0;
+    if (p.addend)       // (where mx_adds says so)
+        return launch_mx_one<U, true, true, EXPAND, false, true>(p, stream);
     if constexpr (U >= kMxRangeUnits) {
         if (p.range)   // (where mx_reports_range says so)
             return vec ? launch_mx_one<U, true, true, EXPAND, true>(p, stream) : launch_mx_one<U, false, true, EXPAND, true>(p, stream);

@@ -2106,7 +2106,7 @@ __global__ void __launch_bounds__(256) swap_epilogue_kernel(const int32_t *__res
                                                             int m_pitch, const float *__restrict__ psum,
                                                             const float *__restrict__ fsum, float s1xs2, float m1, float m2,
                                                             float k_m1xm2, const LayerQuant *__restrict__ lq_dev,
-                                                            const float *__restrict__ bias, int relu,
+                                                            const float *__restrict__ bias, const float *__restrict__ addend, int relu,
                                                             float *__restrict__ out_f, int32_t *__restrict__ out_i)
 {
     __shared__ int32_t turned[4][16][17];
@@ -2131,11 +2131,13 @@ __global__ void __launch_bounds__(256) swap_epilogue_kernel(const int32_t *__res
     const int ml = t >> 4, nl = t & 15, col = n0 + nl;
     const int64_t m = m0 + ml;
     const bool there = m < M && col < Co;
-    float ps = 0.0f, fs = 0.0f, bs = -0.0f;   // (adding -0 changes nothing)
+    float ps = 0.0f, fs = 0.0f, bs = -0.0f, add = 0.0f;   // (adding -0 changes nothing)
     if (there && out_f) {
         ps = psum[m];
         fs = fsum[col];
         bs = bias ? bias[col] : -0.0f;
+        if (addend)
+            add = addend[m * Co + col];
     }
     if (lq_dev) {
         s1xs2 = lq_dev->s1xs2;
@@ -2153,7 +2155,7 @@ __global__ void __launch_bounds__(256) swap_epilogue_kernel(const int32_t *__res
     }
     float r = __fadd_rn(__fmul_rn((float)a, s1xs2), __fmul_rn(m2, ps));
     r = __fadd_rn(__fsub_rn(__fadd_rn(r, __fmul_rn(m1, fs)), k_m1xm2), bs);
-    out_f[m * Co + col] = relu ? fmaxf(r, 0.0f) : r;
+    out_f[m * Co + col] = addend ? sum_activation(__fadd_rn(r, add), relu) : relu ? fmaxf(r, 0.0f) : r;
 }
 
 hipError_t launch_swap_epilogue(const DenseParams &p, const int32_t *partials, int k_splits, int m_pitch, float *out_f,
@@ -2161,7 +2163,32 @@ hipError_t launch_swap_epilogue(const DenseParams &p, const int32_t *partials, i
 {
     const dim3 grid((unsigned)((p.g.M + 15) / 16), (unsigned)((p.g.Co + 15) / 16));
     hipLaunchKernelGGL(swap_epilogue_kernel, grid, dim3(256), 0, stream, partials, k_splits, p.g.M, p.g.Co, m_pitch, p.psum,
-                       p.fsum, p.s1xs2, p.m1, p.m2, p.k_m1xm2, p.lq_dev, p.bias, p.relu, out_f, out_i);
+                       p.fsum, p.s1xs2, p.m1, p.m2, p.k_m1xm2, p.lq_dev, p.bias, p.addend, p.relu, out_f, out_i);
+    return hipGetLastError();
+}
+
+// The sum with another tensor behind the kernels that do not take it along: the vector-ALU ones, and the matrix-core kernel where
+// rows are no whole groups of four pixels, columns come in no fours or a stride is read as it is.  Bound by memory.
+__global__ void __launch_bounds__(256) add_kernel(float *__restrict__ out, const float *__restrict__ addend, const int64_t n, const int relu)
+{
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i + 4 <= n) {
+        float4 a = *reinterpret_cast<float4 *>(out + i);
+        const float4 b = *reinterpret_cast<const float4 *>(addend + i);
+        a.x = sum_activation(__fadd_rn(a.x, b.x), relu);
+        a.y = sum_activation(__fadd_rn(a.y, b.y), relu);
+        a.z = sum_activation(__fadd_rn(a.z, b.z), relu);
+        a.w = sum_activation(__fadd_rn(a.w, b.w), relu);
+        *reinterpret_cast<float4 *>(out + i) = a;
+    } else {
+        for (int64_t e = i; e < n; ++e)
+            out[e] = sum_activation(__fadd_rn(out[e], addend[e]), relu);
+    }
+}
+
+hipError_t launch_add(float *out, const float *addend, int64_t n, bool relu, hipStream_t stream)
+{
+    hipLaunchKernelGGL(add_kernel, dim3(blocks_for((n + 3) / 4, 256)), dim3(256), 0, stream, out, addend, n, relu ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -2173,7 +2200,7 @@ __global__ void __launch_bounds__(256) splitk_epilogue_kernel(const int32_t *__r
                                                                const float *__restrict__ fsum, float s1xs2, float m1,
                                                                float m2, float k_m1xm2,
                                                                const LayerQuant *__restrict__ lq_dev,
-                                                               const float *__restrict__ bias, int relu,
+                                                               const float *__restrict__ bias, const float *__restrict__ addend, int relu,
                                                                float *__restrict__ out_f,
                                                                int32_t *__restrict__ out_i)
 {
@@ -2186,6 +2213,18 @@ __global__ void __launch_bounds__(256) splitk_epilogue_kernel(const int32_t *__r
     const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
     if (i >= mc)
         return;
+    float add[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+        add[e] = 0.0f;
+    if (addend) {
+        if (V == 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(addend + i);
+            add[0] = v.x; add[1 % V] = v.y; add[2 % V] = v.z; add[3 % V] = v.w;
+        } else {
+            add[0] = addend[i];
+        }
+    }
     int32_t a[V];
 #pragma unroll
     for (int e = 0; e < V; ++e)
@@ -2217,7 +2256,9 @@ __global__ void __launch_bounds__(256) splitk_epilogue_kernel(const int32_t *__r
         r[e] = __fsub_rn(t4, k_m1xm2);
         if (bias)
             r[e] = __fadd_rn(r[e], bias[col + e]);
-        if (relu)
+        if (addend)
+            r[e] = sum_activation(__fadd_rn(r[e], add[e]), relu);
+        else if (relu)
             r[e] = fmaxf(r[e], 0.0f);
     }
     if (V == 4)
@@ -2232,11 +2273,11 @@ hipError_t launch_splitk_epilogue(const DenseParams &p, const int32_t *partials,
     const int64_t mc = p.g.M * p.g.Co;
     if ((p.g.Co & 3) == 0)
         hipLaunchKernelGGL(splitk_epilogue_kernel<4>, dim3(blocks_for(mc / 4, 256)), dim3(256), 0, stream, partials,
-                           p.plan.k_splits, mc, p.g.Co, p.psum, p.fsum, p.s1xs2, p.m1, p.m2, p.k_m1xm2, p.lq_dev, p.bias, p.relu,
+                           p.plan.k_splits, mc, p.g.Co, p.psum, p.fsum, p.s1xs2, p.m1, p.m2, p.k_m1xm2, p.lq_dev, p.bias, p.addend, p.relu,
                            out_f, out_i);
     else
         hipLaunchKernelGGL(splitk_epilogue_kernel<1>, dim3(blocks_for(mc, 256)), dim3(256), 0, stream, partials,
-                           p.plan.k_splits, mc, p.g.Co, p.psum, p.fsum, p.s1xs2, p.m1, p.m2, p.k_m1xm2, p.lq_dev, p.bias, p.relu,
+                           p.plan.k_splits, mc, p.g.Co, p.psum, p.fsum, p.s1xs2, p.m1, p.m2, p.k_m1xm2, p.lq_dev, p.bias, p.addend, p.relu,
                            out_f, out_i);
     return hipGetLastError();
 }

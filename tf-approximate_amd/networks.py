@@ -61,6 +61,10 @@ def _he_normal(rng, shape):
     return (rng.standard_normal(shape) * math.sqrt(2.0 / fan_in)).astype(np.float32)
 
 
+def _reads(step):
+    return step[2:4] if step[0] == "add_relu" else step[2:3]
+
+
 class ApproxNetwork:
     """A forward pass described as a small program over named tensors:
     ("conv", dst, src, ConvSpec) | ("add_relu", dst, a, b) | ("maxpool", dst, src)"""
@@ -96,6 +100,18 @@ class ApproxNetwork:
             later[0] == "conv" and later[2] == step[1]
             for later in program[i + 1:next((j + 1 for j in range(i + 1, len(program)) if program[j][1] == step[1]), len(program))])}
 
+        # convolutions whose output only the sum that follows them reads: what it is added to
+        self.adds = {}
+        for i, step in enumerate(program[:-1]):
+            after = program[i + 1]
+            if step[0] != "conv" or step[3].relu or step[3].depthwise or after[0] != "add_relu" or fused_layers:
+                continue
+            dst, others = step[1], [name for name in after[2:4] if name != step[1]]
+            later = [s for s in program[i + 2:]]
+            again = next((j for j, s in enumerate(later) if s[1] == dst and dst not in _reads(s)), len(later))
+            if len(others) == 1 and (after[1] == dst or not any(dst in _reads(s) for s in later[:again])):
+                self.adds[i] = others[0]
+
     def conv_count(self):
         return len(self.ops)
 
@@ -109,8 +125,11 @@ class ApproxNetwork:
         t = {"input": x}
         seen = {}   # fused_layers: what the call that made a tensor reported of its range
         macs = 0
+        added = -1
         for i, step in enumerate(self.program):
             kind, dst = step[0], step[1]
+            if i == added:
+                continue
             if kind == "conv":
                 src, spec = t[step[2]], step[3]
                 w = self.weights[i]
@@ -125,7 +144,11 @@ class ApproxNetwork:
                     lo, hi = torch.aminmax(src)
                     wlo, whi = torch.aminmax(w)
                     self.ranges[i] = (float(lo), float(hi), float(wlo), float(whi))
-                if trace is not None or not self.fuse_relu:
+                other = t.get(self.adds[i]) if i in self.adds and trace is None and self.fuse_relu else None
+                if other is not None and other.shape == self.ops[i].output_shape(src, w):
+                    y = self.ops[i].call_and_add(src, w, *self.ranges[i], other, activation="relu")
+                    added, dst = i + 1, self.program[i + 1][1]
+                elif trace is not None or not self.fuse_relu:
                     y = self.ops[i](src, w, *self.ranges[i])
                     if trace is not None:
                         trace.append((spec, src.cpu().numpy(), w.cpu().numpy(), self.ranges[i], y.cpu().numpy()))

@@ -256,6 +256,31 @@ class ApproxConv2DWithMinMaxVars:
                 out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
         return out
 
+    def output_shape(self, input, filter):
+        return self._layer(input, filter).out_shape
+
+    def call_and_add(self, input, filter, input_min, input_max, filter_min, filter_max, addend, activation=None):
+        """The op, a tensor like its output added to it, and the activation behind that: as a residual network's sum, which
+        needs no pass of its own then.  The activation keeps NaN, as the networks' elementwise pass does."""
+        if activation not in (None, "relu"):
+            raise InvalidArgumentError("activation must be None or 'relu'")
+        if self.depthwise:
+            raise UnimplementedError("call_and_add: dense layers only")
+        lib = _lib.load()
+        input = _require_device_f32(input, "input")
+        filter = _require_device_f32(filter, "filter")
+        addend = _require_device_f32(addend, "addend")
+        layer, device = self._layer(input, filter), input.device
+        if tuple(addend.shape) != layer.out_shape:
+            raise InvalidArgumentError("addend must have the output's shape %s" % (layer.out_shape,))
+        stream = _stream(device)
+        ws = layer.workspace(lib, device, stream)
+        out = torch.empty(layer.out_shape, dtype=torch.float32, device=device)
+        _launch(device, lib.axc_conv2d_minmax_bias_add_act, self.table.handle, layer.ref, input.data_ptr(), filter.data_ptr(),
+                _scalar(input_min), _scalar(input_max), _scalar(filter_min), _scalar(filter_max), None, addend.data_ptr(),
+                1 if activation == "relu" else 0, out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+        return out
+
     def accumulators(self, input, filter, input_min, input_max, filter_min, filter_max):
         """int32 sums of table entries before the epilogue (parity entry point)."""
         return self._run(input, filter, (input_min, input_max, filter_min, filter_max), True)
