@@ -1349,9 +1349,9 @@ __device__ __forceinline__ void patch_sums_flat_body(const float *__restrict__ x
 // C dependent adds per pixel is what takes the time, and memory latency has to stay off it.  A workgroup takes
 // `pixels` (8 or 16) consecutive pixels, so that even a few thousand pixels spread over all CUs, and walks their
 // channels in passes of kDeepChunk: all threads load a pass kDeepAhead passes ahead of its use (16 bytes per lane,
-// a wavefront fetches 1 KiB of one pixel), quantize it into the code layout when xq is given and store it into
-// one half of an LDS stage [pixel][channel]; meanwhile one lane per pixel extends its sum from the other half,
-// its 16-byte LDS reads a batch of 32 channels ahead of the adds.  One barrier per pass.  Loads, stores and LDS
+// a wavefront fetches 1 KiB of one pixel) and store it into one half of an LDS stage [pixel][channel]; meanwhile one
+// lane per pixel extends its sum from the other half, its 16-byte LDS reads a batch of 32 channels ahead of the adds,
+// and the other wavefronts write that half's codes when xq is given.  One barrier per pass.  Loads, stores and LDS
 // reads are unconditional (indices clamped, zeros stored beyond C) to keep the loop body straight-line code for
 // the compiler's count of loads in flight: a store then waits for its own pass only.
 constexpr int kDeepChunk = 256, kDeepPitch = kDeepChunk + 4, kDeepAhead = 3, kDeepThreads = 512;
@@ -1379,18 +1379,37 @@ __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x
     const bool loader = t < kDeepThreads;
     const int npass = (g.C + kDeepChunk - 1) / kDeepChunk;
     const float *src[kDeepPer];
-    uint32_t xq_idx[kDeepPer];
-    bool px_ok[kDeepPer];
 #pragma unroll
     for (int k = 0; k < kDeepPer; ++k) {
         const int px = px0 + k * PSTEP;
-        px_ok[k] = loader && px < npx;
         const int64_t m = m0 + (px < npx ? px : npx - 1);
-        const int64_t nh = m / g.W;
-        const int w = (int)(m - nh * g.W);
-        xq_idx[k] = (uint32_t)(xq_row_nh(lay, nh, g.H, g.C4) + (int64_t)q * lay.Wp + w);
         src[k] = x + m * g.C;
     }
+    // The codes go out of LDS, a pixel a lane: a quad's codes of neighbouring pixels lie side by side in xq, those of
+    // neighbouring quads a row apart - 4 runs of 64 bytes a store where the registers that the floats came in made 64 of
+    // four (launch, us, before / now: 1024 channels @14x14x64 31.4 / 24.8, 512 @28x28x16 18.9 / 14.9, 2048 @7x7x64 20.2 / 17.7;
+    // 32 pixels a workgroup 28.0, 17.2, 17.1).
+    constexpr int kCodeThreads = kDeepThreads - 64, kCodeStep = kCodeThreads / PIXELS;
+    const int code_t = t - 64, code_px = code_t & (PIXELS - 1), code_q0 = code_t / PIXELS;
+    const bool code_ok = xq && code_t >= 0 && code_t < kCodeThreads && code_px < npx;
+    uint32_t code_idx = 0;            // dword index in xq of (that pixel, quad 0)
+    {
+        const int64_t m = m0 + (code_ok ? code_px : 0), nh = m / g.W;
+        code_idx = (uint32_t)(xq_row_nh(lay, nh, g.H, g.C4) + (m - nh * g.W));
+    }
+    auto codes = [&](const int pass) {
+        const float *const half = stage + (pass & 1) * (kDeepMaxPixels * kDeepPitch) + code_px * kDeepPitch;
+        const int first = pass * QUADS, left = g.C4 - first < QUADS ? g.C4 - first : QUADS;
+        if (code_ok)
+            for (int qq = code_q0; qq < left; qq += kCodeStep) {
+                const float4 f = *reinterpret_cast<const float4 *>(half + qq * 4);
+                xq[code_idx + (uint32_t)(first + qq) * (uint32_t)lay.Wp] =
+                    phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
+                    (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
+                    (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
+                    (phys_row(quantize_code(f.w, qt.offset, qt.inv_scale)) << 24);
+            }
+    };
     float4 v[kDeepAhead][kDeepPer];
     auto issue = [&](float4(&dst)[kDeepPer], int pass) {
         const int c = pass * kDeepChunk + q * 4;
@@ -1410,28 +1429,21 @@ __device__ __forceinline__ void patch_sums_deep_body(const float *__restrict__ x
                 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (loader && px < kDeepMaxPixels)
                 *reinterpret_cast<float4 *>(&half[px * kDeepPitch + q * 4]) = f;
-            if (xq && px_ok[k] && c_ok)
-                xq[xq_idx[k] + (uint32_t)(pass * (kDeepChunk / 4)) * (uint32_t)lay.Wp] =
-                    phys_row(quantize_code(f.x, qt.offset, qt.inv_scale)) |
-                    (phys_row(quantize_code(f.y, qt.offset, qt.inv_scale)) << 8) |
-                    (phys_row(quantize_code(f.z, qt.offset, qt.inv_scale)) << 16) |
-                    (phys_row(quantize_code(f.w, qt.offset, qt.inv_scale)) << 24);
         }
     };
 #pragma unroll
     for (int u = 0; u < kDeepAhead; ++u)
         issue(v[u], u);
     store(v[0], 0);
-    if (kDeepAhead < npass)
-        issue(v[0], kDeepAhead);
+    issue(v[0], kDeepAhead);
     __syncthreads();
     float s = 0.0f;
     __builtin_amdgcn_s_setprio(3);   // the chain is the critical path: its wavefront issues ahead of the others on its SIMD
     constexpr int kBatch = 8, kBatches = QUADS / kBatch; // 16-byte reads per batch; batches per pass
     auto pass_step = [&](const int p, float4(&next)[kDeepPer]) {
         store(next, p + 1);
-        if (p + 1 + kDeepAhead < npass)
-            issue(next, p + 1 + kDeepAhead);
+        codes(p);
+        issue(next, p + 1 + kDeepAhead);
         if (t < kDeepMaxPixels && p < npass) {
             const float4 *const row =
                 reinterpret_cast<const float4 *>(stage + (p & 1) * (kDeepMaxPixels * kDeepPitch) + t * kDeepPitch);
