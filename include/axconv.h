@@ -116,7 +116,9 @@ int axc_fake_approx_depthwise_conv2d(const axc_table *table, const axc_conv2d_de
 /* The same two calls one behind the other: a call whose input another such call has just made need not read the whole tensor
  * once more to find its smallest and largest value.  output: AXC_RANGE_BYTES of device memory (8-byte aligned) that the call
  * fills with what it saw of its outputs as it stored them, where the kernel that it runs can (output_written says so, when the
- * call returns); input: what the call that made the input tensor filled.  Either may be null.  Results do not depend on it. */
+ * call returns); input: what the call that made the input tensor filled, which must not have been written to since: the call
+ * takes the range as it stands and reads AXC_RANGE_BYTES of it.  Either may be null.  With that, results are those of the
+ * calls above. */
 #define AXC_RANGE_BYTES 32768
 typedef struct axc_layer_ranges {
     const void *input;

@@ -69,3 +69,50 @@ def test_kernels_that_do_not_report(pkg):
     x, f = torch.randn((1, 9, 9, 16), device="cuda:0"), torch.randn((3, 3, 16, 8), device="cuda:0")
     y, seen = layer.call_in_turn(x, f)
     assert seen is None and torch.equal(y, layer(x, f))
+
+
+def _reported(pkg):
+    """(layer, its output, the range reported with it)"""
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(9)
+    x = torch.randn((16, 56, 56, 32), device="cuda:0", generator=gen)
+    f = torch.randn((1, 1, 32, 100), device="cuda:0", generator=gen)
+    layer = pkg.ops.FakeApproxConv2D((1, 1), pkg.ops.TruthTable(pkg.synth.table_noisy(2)), "SAME")
+    pkg.ops.set_matrix_rows(1)
+    try:
+        y, seen = layer.call_in_turn(x, f)
+    finally:
+        pkg.ops.set_matrix_rows(0)
+    assert seen is not None
+    return layer, y, seen
+
+
+def test_a_range_is_that_of_one_tensor_as_it_was(pkg):
+    """Inputs that the range is not of, or no longer of, are read; the one that it is of is not."""
+    layer, y, seen = _reported(pkg)
+    f = torch.randn((1, 1, 100, 24), device="cuda:0")
+    other = y * 3.0
+    assert torch.equal(layer.call_in_turn(other, f, None, seen, False)[0], layer(other, f))
+    assert torch.equal(layer.call_in_turn(y.clone(), f, None, seen.clone(), False)[0], layer(y, f))
+    seen.view(-1, 2)[:, 1] *= 2.0        # a range that the tensor does not have: what shows that it is taken
+    taken = layer.call_in_turn(y, f, None, seen, False)[0]
+    assert not torch.equal(taken, layer(y, f))
+    for change in (lambda: y.relu_(), lambda: y.view(-1).mul_(0.25), lambda: y[3].add_(100.0)):
+        change()
+        assert torch.equal(layer.call_in_turn(y, f, None, seen, False)[0], layer(y, f))
+
+
+def test_ranges_in_inference_mode(pkg):
+    with torch.inference_mode():
+        layer, y, seen = _reported(pkg)
+        f = torch.randn((1, 1, 100, 24), device="cuda:0")
+        y.mul_(0.5)
+        assert torch.equal(layer.call_in_turn(y, f, None, seen, False)[0], layer(y, f))
+
+
+def test_what_no_range_can_be_is_refused(pkg):
+    layer, y, seen = _reported(pkg)
+    f = torch.randn((1, 1, 100, 24), device="cuda:0")
+    for bad in (seen.cpu(), seen.double(), seen[:-2], seen.view(2, -1).t(), seen.data_ptr(), [0.0, 1.0]):
+        with pytest.raises(pkg.InvalidArgumentError):
+            layer.call_in_turn(y, f, None, bad, False)

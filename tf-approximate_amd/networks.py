@@ -134,7 +134,8 @@ class ApproxNetwork:
                 src, spec = t[step[2]], step[3]
                 w = self.weights[i]
                 if self.fused_layers:
-                    y, seen[dst] = self.ops[i].call_in_turn(src, w, None, seen.get(step[2]), i in self.feeds)
+                    # (nothing writes to a tensor between the call that made it and the one that reads it)
+                    y, seen[dst] = self.ops[i]._run(src, w, None, seen.get(step[2]), i in self.feeds)
                     if trace is not None:
                         trace.append((spec, src.cpu().numpy(), w.cpu().numpy(), None, y.cpu().numpy()))
                     macs += spec.macs(y.shape[1], y.shape[2], y.shape[0])
@@ -158,7 +159,7 @@ class ApproxNetwork:
                 macs += spec.macs(y.shape[1], y.shape[2], y.shape[0])
                 t[dst] = y
             elif kind == "add_relu":
-                seen[dst] = None
+                seen[dst] = seen[step[2]] = None   # (without the JIT the sum is made in its first operand)
                 t[dst] = add_relu(t[step[2]], t[step[3]])
             elif kind == "maxpool":
                 seen[dst] = None

@@ -6,6 +6,7 @@ Tensors are torch tensors on a ROCm device (torch is only the owner of device me
 stream); all arithmetic happens in libaxconv_hip.so.
 """
 import ctypes
+import weakref
 
 import numpy as np
 
@@ -286,6 +287,11 @@ class ApproxConv2DWithMinMaxVars:
         return self._run(input, filter, (input_min, input_max, filter_min, filter_max), True)
 
 
+def _version(t):
+    """How often torch has seen the tensor's memory written to; None where it does not count."""
+    return None if t.is_inference() else t._version
+
+
 class FakeApproxConv2D:
     """The reference's Keras layer around the op (FakeApproxConv2D.call,
     tf2/python/keras/layers/fake_approx_convolutional.py:223-261) as one device-side call: min/max of the batch
@@ -302,12 +308,33 @@ class FakeApproxConv2D:
         self.activation = 1 if activation == "relu" else 0
 
     def __call__(self, inputs, kernel, bias=None):
-        return self.call_in_turn(inputs, kernel, bias, None, False)[0]
+        return self._run(inputs, kernel, bias, None, False)[0]
 
     def call_in_turn(self, inputs, kernel, bias=None, input_range=None, want_range=True):
         """The call, for a program that makes one layer's output the next one's input: (output, range).  `range` is what
         the call saw of its outputs' smallest and largest value, for the input_range of a call on that very output, which
-        then need not read the tensor to find them; None where the kernel that ran does not report it."""
+        then need not read the tensor to find them; None where the kernel that ran does not report it.
+
+        With any other input, or one that torch knows to have been written to since, the call finds the range itself; so it
+        does for outputs made under torch.inference_mode(), whose changes torch does not count.  Writes that torch does not
+        see (through data_ptr() or .data) are the caller's to mind."""
+        if input_range is not None:
+            inputs = _require_device_f32(inputs, "input")
+            if not torch.is_tensor(input_range) or input_range.device != inputs.device:
+                raise InvalidArgumentError("input_range must be a tensor on the input's GPU")
+            if (input_range.dtype != torch.float32 or not input_range.is_contiguous() or
+                    input_range.numel() * 4 < _lib.RANGE_BYTES):
+                raise InvalidArgumentError("input_range must be what call_in_turn returned")
+            of, version = getattr(input_range, "_range_of", (None, None))
+            if version is None or of() is not inputs or _version(inputs) != version:
+                input_range = None
+        out, seen = self._run(inputs, kernel, bias, input_range, want_range)
+        if seen is not None:
+            seen._range_of = weakref.ref(out), _version(out)
+        return out, seen
+
+    def _run(self, inputs, kernel, bias, input_range, want_range):
+        """call_in_turn for a caller that knows input_range to be that of `inputs` as they are."""
         lib = _lib.load()
         inputs = _require_device_f32(inputs, "input")
         kernel = _require_device_f32(kernel, "filter")
