@@ -564,23 +564,24 @@ DensePlan make_plan(const ConvGeom &g, int cus, int px_mode = kPxModeGlobal)
     struct Key {
         int taps, c4, co, cus, forced, px_mode;
         int64_t m;
+        double clock_hz;
         bool operator<(const Key &o) const
         {
-            return std::tie(taps, c4, co, cus, forced, px_mode, m) <
-                   std::tie(o.taps, o.c4, o.co, o.cus, o.forced, o.px_mode, o.m);
+            return std::tie(taps, c4, co, cus, forced, px_mode, m, clock_hz) <
+                   std::tie(o.taps, o.c4, o.co, o.cus, o.forced, o.px_mode, o.m, o.clock_hz);
         }
     };
     static std::mutex mu;
     static std::map<Key, DensePlan> cache;
     const Key key{g.KH * g.KW, g.C4, g.Co, cus, g_forced_nt.load(std::memory_order_relaxed),
-                  px_mode == kPxModeGlobal ? g_px_mode.load(std::memory_order_relaxed) : px_mode, g.M};
+                  px_mode == kPxModeGlobal ? g_px_mode.load(std::memory_order_relaxed) : px_mode, g.M, device_clock_hz()};
     {
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end())
             return it->second;
     }
-    const DensePlan plan = compute_plan(g, cus, key.forced, key.px_mode, device_clock_hz());
+    const DensePlan plan = compute_plan(g, cus, key.forced, key.px_mode, key.clock_hz);
     std::lock_guard<std::mutex> lock(mu);
     if (cache.size() >= 4096)
         cache.clear();
@@ -712,21 +713,23 @@ MxPlans make_mx_plans(const ConvGeom &g, int64_t quads, int64_t groups, MxLoads 
     struct Key {
         int64_t quads, groups, m;
         int k, co, loads, cus;
+        double clock_hz;
         bool operator<(const Key &o) const
         {
-            return std::tie(quads, groups, m, k, co, loads, cus) < std::tie(o.quads, o.groups, o.m, o.k, o.co, o.loads, o.cus);
+            return std::tie(quads, groups, m, k, co, loads, cus, clock_hz) <
+                   std::tie(o.quads, o.groups, o.m, o.k, o.co, o.loads, o.cus, o.clock_hz);
         }
     };
     static std::mutex mu;
     static std::map<Key, MxPlans> cache;
-    const Key key{quads, groups, g.M, g.K, g.Co, (int)loads, cus};
+    const double clock_hz = device_clock_hz();
+    const Key key{quads, groups, g.M, g.K, g.Co, (int)loads, cus, clock_hz};
     {
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find(key);
         if (it != cache.end())
             return it->second;
     }
-    const double clock_hz = device_clock_hz();
     const MxPlans plans = {compute_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, false, false, cus, clock_hz),
                            compute_mx_plan(quads, g.Co, groups, g.M * g.Co, loads, true, false, cus, clock_hz),
                            compute_swap_plan(g, cus, clock_hz)};
@@ -1137,13 +1140,13 @@ int compute_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
 
 // The same, looked up: a call asks for it at least twice (workspace, launch), and working it out takes 2 to 3 us of host time,
 // several plans among it.  The key is all that it depends on: the descriptor, the arguments, the pinned forms and the device's
-// compute units.
+// compute units and clock.
 int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pads = nullptr, int element_bytes = 4,
                   int px_mode = kPxModeGlobal, int mx_mode = kMxAny, bool allow_fold = true, bool allow_planes = true)
 {
     if (!desc)
         return compute_dense(desc, pd, pads, element_bytes, px_mode, mx_mode, allow_fold, allow_planes);
-    typedef std::array<int64_t, 36> Key;
+    typedef std::array<int64_t, 37> Key;
     Key key{};
     size_t n = 0;
     for (int i = 0; i < 4; ++i) {
@@ -1159,6 +1162,7 @@ int prepare_dense(const axc_conv2d_desc *desc, PreparedDense *pd, const int *pad
                         g_forced_nt.load(std::memory_order_relaxed), g_px_mode.load(std::memory_order_relaxed),
                         g_mx_rows.load(std::memory_order_relaxed), device_cus()})
         key[n++] = v;
+    key[n++] = (int64_t)device_clock_hz();
     static std::mutex mu;
     static std::map<Key, PreparedDense> cache;
     {
