@@ -197,6 +197,11 @@ int axc_set_preexpand(int mode);
  * timing; a workspace query and the launch it is for must see the same value.
  * Results do not depend on it.  No counterpart in the reference. */
 int axc_set_matrix_rows(int mode);
+/* Launches that do the work of several: the whole layers of axc_conv2d_direct_plan, and what precedes the lookups of layers
+ * given as codes.  0 = where the planner says so, except while the timers run (the default), 1 = while they run too, under the
+ * names direct and codes_prep, -1 = never: every layer runs as it would without them, also under the timers.  Process-wide, for
+ * tests and timing; neither the workspace query nor the results depend on it.  No counterpart in the reference. */
+int axc_set_merged_launches(int mode);
 /* The wavefronts of the kernels that plan code 2 and axc_conv2d_matrix_plan stand for wait for each other by polling counters,
  * every wait a bounded number of polls (the default, 2^20 of ~150 cycles each, is far beyond any legitimate wait).  A wait that runs out ends
  * the launch early - every wavefront leaves the kernel, nothing hangs - and the NEXT launch call on that GPU returns
@@ -293,8 +298,8 @@ int axc_conv2d_codes_acc_i32(const axc_table *table, const axc_conv2d_desc *desc
  * launch calls enqueue is bracketed by two events; axc_profile_read synchronizes them and returns the
  * accumulated milliseconds and launch count per kernel name since the last reset.  A launch out of pre-expanded rows is
  * entered as lutgemm_px, and as lutgemm_mx too where the matrix cores make its sums.  While the timers run, layers are
- * launched part by part, so that every part has its time: those of axc_conv2d_direct_plan too, unless axc_set_matrix_rows pins
- * them (then they are entered as direct). */
+ * launched part by part, so that every part has its time; axc_set_merged_launches(1) has them time the launches of a call
+ * without timers, and axc_set_matrix_rows(4) those of axc_conv2d_direct_plan. */
 int axc_profile_enable(int enable);
 int axc_profile_reset(void);
 int axc_profile_read(int index, char *name, size_t name_bytes, double *total_ms, int64_t *launches);

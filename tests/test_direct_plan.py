@@ -14,6 +14,8 @@ def ops(pkg):
         pkg.ops.set_matrix_rows(0)
         pkg.ops.set_preexpand(0)
         pkg.ops.set_tile_columns(0)
+        pkg.ops.set_merged_launches(0)
+        pkg.ops.profile_enable(False)
 
 
 def test_small_layers_take_it_and_large_ones_do_not(ops):
@@ -36,6 +38,26 @@ def test_pinned_forms_do_without(ops):
     ops.set_preexpand(0)
     ops.set_tile_columns(32)
     assert ops.conv2d_direct_plan(xs, fs) is None
+
+
+def test_merged_launches(ops):
+    """Pinned off, layers run as they would without; with the timers on only where that is asked for."""
+    xs, fs = (1, 32, 32, 16), (3, 3, 16, 32)
+    plan, without = ops.conv2d_direct_plan(xs, fs), (ops.conv2d_matrix_plan(xs, fs), ops.conv2d_tile_plan(xs, fs))
+    ops.profile_enable(True)
+    assert ops.conv2d_direct_plan(xs, fs) is None
+    ops.set_merged_launches(1)
+    assert ops.conv2d_direct_plan(xs, fs) == plan
+    ops.profile_enable(False)
+    assert ops.conv2d_direct_plan(xs, fs) == plan
+    ops.set_merged_launches(-1)
+    assert ops.conv2d_direct_plan(xs, fs) is None
+    assert (ops.conv2d_matrix_plan(xs, fs), ops.conv2d_tile_plan(xs, fs)) == without
+    ops.set_matrix_rows(4)
+    assert ops.conv2d_direct_plan(xs, fs) is None
+    for mode in (-2, 2):
+        with pytest.raises(ValueError):
+            ops.set_merged_launches(mode)
 
 
 @pytest.mark.parametrize("seed", range(4))

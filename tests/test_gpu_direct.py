@@ -131,3 +131,30 @@ def test_tensors_that_begin_at_any_float(pkg, direct):
     with direct():
         got = op(x, f, *MM)
     _same(got, op(x, f, *MM))
+
+
+@pytest.mark.parametrize("mode,launched", [(0, False), (1, True), (-1, False)])
+def test_what_the_timers_time(pkg, mode, launched):
+    """A small layer, and one given as codes, as a call without timers runs them (1) or part by part."""
+    ops = pkg.ops
+    table = ops.TruthTable(pkg.synth.table_noisy(2))
+    x, f = torch.rand((1, 16, 16, 16), device="cuda:0"), torch.rand((3, 3, 16, 20), device="cuda:0") - 0.5
+    codes, weights = (torch.randint(0, 256, s, dtype=torch.uint8, device="cuda:0") for s in ((7, 8, 8, 64), (1, 1, 64, 100)))
+    op = pkg.ApproxConv2DWithMinMaxVars([1, 1, 1, 1], 8, table, "SAME")
+
+    def run():
+        return op(x, f, *MM), ops.conv2d_codes_acc_i32(table, codes, weights, 3)
+    want = run()
+    ops.set_merged_launches(mode)
+    ops.profile_enable(True)
+    ops.profile_reset()
+    try:
+        got = run()
+        names = set(ops.profile_read())
+    finally:
+        ops.profile_enable(False)
+        ops.set_merged_launches(0)
+    for g, w in zip(got, want):
+        _same(g, w)
+    assert ("direct" in names) == launched and ("patch_sums" in names or "patch_sums_flat" in names) != launched, names
+    assert ("codes_prep" in names) == launched and ("codes_relayout" in names) != launched, names

@@ -68,6 +68,7 @@ SYMBOLS = [
     ("axc_set_tile_columns", ctypes.c_int, [ctypes.c_int]),
     ("axc_set_preexpand", ctypes.c_int, [ctypes.c_int]),
     ("axc_set_matrix_rows", ctypes.c_int, [ctypes.c_int]),
+    ("axc_set_merged_launches", ctypes.c_int, [ctypes.c_int]),
     ("axc_set_wait_limit", ctypes.c_int, [ctypes.c_uint32]),
     ("axc_depthwise_conv2d_workspace_bytes", ctypes.c_int, [_desc, ctypes.POINTER(_sz)]),
     ("axc_conv2d_minmax", ctypes.c_int, [_vp, _desc, _vp, _vp] + _launch_tail),

@@ -448,6 +448,14 @@ std::atomic<int> g_px_mode{[] {
 // kernels), 2 = its own wherever it can make them, 3 = with its operands exchanged wherever it can.  Set by
 // axc_set_matrix_rows.
 std::atomic<int> g_mx_rows{0};
+// Launches that do the work of several (direct_kernel, codes_prep_kernel): 0 = where the planner says so and no timers run, 1 =
+// while they run too, -1 = never.  Set by axc_set_merged_launches.
+std::atomic<int> g_merged{0};
+bool merged_launches()
+{
+    const int mode = g_merged.load(std::memory_order_relaxed);
+    return mode > 0 || (mode == 0 && !g_prof_enabled.load(std::memory_order_relaxed));   // (the timers' users want the parts' times)
+}
 constexpr size_t kPxMaxBytes = (size_t)2 << 30;     // most memory a layer's pre-expanded rows may take
 // Rows up to this size stay in the memory-side cache between the launch that writes them and the one that reads
 // them; larger sets are read from memory, and the cost model is less sure of them: they must promise a gain.
@@ -1242,8 +1250,7 @@ DirectPlan choose_direct(const PreparedDense &pd, const bool fake_quant)
     if (mode != 4 && (mode != 0 || g_px_mode.load(std::memory_order_relaxed) != 0 || g_forced_nt.load(std::memory_order_relaxed) != 0))
         return DirectPlan{};
     const ConvGeom &g = pd.g_full;
-    // (the timers' users want the parts' times: no parts, no times)
-    if (mode == 0 && (g_prof_enabled.load(std::memory_order_relaxed) || (double)g.M * g.Co * g.K > 4e8))
+    if (g_merged.load(std::memory_order_relaxed) < 0 || (mode == 0 && (!merged_launches() || (double)g.M * g.Co * g.K > 4e8)))
         return DirectPlan{};
     const DirectPlan plan = make_direct_plan(g, fake_quant, device_cus());
     if (mode == 4)
@@ -1421,12 +1428,15 @@ int run_dense(const axc_table *table, const axc_conv2d_desc *desc, const float *
     int32_t *const pixel_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(psum) : nullptr;
     int32_t *const column_term = tf1_offset_filter ? reinterpret_cast<int32_t *>(fsum) : nullptr;
     bool codes_done = false;
-    if (codes_mode && mx && !swap && !flat && !g_prof_enabled.load(std::memory_order_relaxed)) {   // (the timers: part by part)
+    if (codes_mode && mx && !swap && !flat && merged_launches()) {
+        ProfScope ps("codes_prep", stream);
         AXC_HIP(launch_codes_prep(input_codes, filter_codes, g, pd.lay, zp4, xq, *mx, wq, table->dev_tableT, px_rows,
                                   tf1_offset_filter != nullptr, input_zero_code, tf1_offset_filter ? *tf1_offset_filter : 0,
                                   pixel_term, column_term, stream, &codes_done));
         if (codes_done)
             filter_done = px_done = true;
+        else
+            ps.ev.reset();
     }
     if (codes_done) {
         // nothing left
@@ -2284,6 +2294,14 @@ int axc_depthwise_conv2d_minmax_bias_act(const axc_table *table, const axc_conv2
         return fail(AXC_INVALID_ARGUMENT, "null tensor pointer");
     return run_depthwise(table, desc, input, filter, input_min, input_max, filter_min, filter_max, output,
                          nullptr, workspace, workspace_bytes, stream, false, bias, activation);
+}
+
+int axc_set_merged_launches(int mode)
+{
+    if (mode < -1 || mode > 1)
+        return fail(AXC_INVALID_ARGUMENT, "merged launches mode must be 0 (planner's choice), 1 (while the timers run too) or -1 (never)");
+    g_merged.store(mode, std::memory_order_relaxed);
+    return AXC_OK;
 }
 
 int axc_conv2d_static_workspace_limit(size_t *bytes)

@@ -473,6 +473,12 @@ def set_matrix_rows(mode):
     _check(_lib.load().axc_set_matrix_rows(int(mode)))
 
 
+def set_merged_launches(mode):
+    """Launches that do the work of several (layers that conv2d_direct_plan names; what precedes the lookups of layers given as
+    codes): 0 = where the planner says so, except while the timers run, 1 = while they run too, -1 = never."""
+    _check(_lib.load().axc_set_merged_launches(int(mode)))
+
+
 def set_wait_limit(polls):
     """Polls a wavefront of the barrier-free LUT-GEMM kernel makes in one wait before it gives up (tests of the
     report; the default is 2**20)."""
