@@ -80,3 +80,18 @@ def test_tiles_fit_the_kernel(ops, seed):
         # of a chunk that is not the only one a copying thread holds two quads of either kind
         assert chunks == 1 or max(pt, ct) * kc // 4 <= 2 * 384
         assert pt * ct * 4 <= LDS_BESIDE_THE_TABLE
+
+
+# input, filter, stride, padding: layers of 2e8 products and more that the model of the other kernels puts too high
+SLOWER = [
+    ((30, 12, 3, 431), (3, 3, 431, 260), 1, "VALID"),          # 95 us as one launch, 75 with exchanged operands
+    ((17, 11, 11, 65), (7, 7, 65, 257), 1, "VALID"),           # 103, 83
+    ((3, 48, 2, 539), (7, 1, 539, 332), 1, "SAME"),           # 92, 75
+    ((1, 20, 20, 457), (3, 3, 457, 270), 1, "VALID"),          # 102, 82
+    ((10, 5, 6, 479), (3, 3, 479, 285), 1, "SAME"),            # 106, 85 with rows of its own
+]
+
+
+@pytest.mark.parametrize("xs,fs,stride,padding", SLOWER)
+def test_large_layers_that_another_kernel_runs_faster(ops, xs, fs, stride, padding):
+    assert ops.conv2d_direct_plan(xs, fs, (1, stride, stride, 1), padding) is None

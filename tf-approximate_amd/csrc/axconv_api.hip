@@ -1242,15 +1242,20 @@ int prepare_dense_for(const axc_conv2d_desc *desc, size_t workspace_bytes, const
 
 // Whether the layer, prepared as the other kernels would run it, runs direct_kernel instead: us = 0 where not.  What the others
 // take beside the planner's estimate of their lookups - the pre-pass, a chain of K adds in it, an epilogue of its own - was fitted
-// to the same 520 layers (mean error 11 %); with a margin of 8 % none of them takes more than 3 % longer than before, and all
-// together, up to 2e8 lookups each, 0.59 of the time (geometric mean; 0.3 at 1e5 lookups, 0.5 at 2e7, 0.8 at 6e7).
+// to the same 520 layers (mean error 11 %).  A margin of 8 %; of 18 % beyond 1.6e8 products where the other kernels make 192
+// columns and more, exchange operands or add on the vector ALUs, which that model puts too high (3x3 431->260 @12x3x30, us: 90
+// expected, 75 taken, 95 in one launch; of 427 layers beyond 1.6e8 with the one margin 48 took more than 3 % longer than the other
+// kernels).  Of 2 694 random layers of up to 4e8 products that come here 23 take more than 3 % longer (at most 1.23 of the time, all
+// but one of them beyond 6e7); all together 0.56 of the time (geometric mean; 0.41 below 1e6, 0.52 to 6e7, 0.69 to 1.6e8, 0.56
+// beyond).  Nothing larger was compared.
 DirectPlan choose_direct(const PreparedDense &pd, const bool fake_quant)
 {
     const int mode = g_mx_rows.load(std::memory_order_relaxed);
     if (mode != 4 && (mode != 0 || g_px_mode.load(std::memory_order_relaxed) != 0 || g_forced_nt.load(std::memory_order_relaxed) != 0))
         return DirectPlan{};
     const ConvGeom &g = pd.g_full;
-    if (g_merged.load(std::memory_order_relaxed) < 0 || (mode == 0 && (!merged_launches() || (double)g.M * g.Co * g.K > 4e8)))
+    const double products = (double)g.M * g.Co * g.K;
+    if (g_merged.load(std::memory_order_relaxed) < 0 || (mode == 0 && (!merged_launches() || products > 4e8)))
         return DirectPlan{};
     const DirectPlan plan = make_direct_plan(g, fake_quant, device_cus());
     if (mode == 4)
@@ -1259,7 +1264,8 @@ DirectPlan choose_direct(const PreparedDense &pd, const bool fake_quant)
     const double lookups = pd.mx ? pd.mxp.cost / us : pd.plan.cost / us * 1.06 + 2.7;
     const bool splits = (pd.mx ? pd.mxp.k_splits : pd.plan.k_splits) > 1;
     const double others = 4.3 + 1.38 * lookups + 5.6e-3 * g.K - (splits ? 3.0 : 0.0) - (pd.mx && pd.mxp.swap ? 4.3 : 0.0) + ((g.C & 3) ? 3.1 : 0.0);
-    return plan.us < 0.92 * others ? plan : DirectPlan{};
+    const bool low = products > 1.6e8 && (!pd.mx || pd.mxp.swap || g.Co >= 192);
+    return plan.us < (low ? 0.82 : 0.92) * others ? plan : DirectPlan{};
 }
 
 DirectParams direct_params(const ConvGeom &g, const DirectPlan &plan, const axc_table *table, const axc_quant_props &qp,
