@@ -65,6 +65,7 @@ def test_sum_where_the_outputs_are(pkg, xs, fs, stride, rows, px, names, activat
     assert torch.equal(addend.view(-1)[3::109], -y.view(-1)[3::109])
 
 
+@pytest.mark.usefixtures("launches")
 def test_networks_sum_in_the_layers(pkg):
     """A network's forward pass with its sums in the layers' calls, and with a pass of its own for each."""
     from tf_approximate_amd import networks

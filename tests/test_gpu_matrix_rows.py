@@ -121,6 +121,7 @@ def test_sums_and_outputs_equal_the_expanding_kernel(pkg, oracle, own_rows, case
     _compare(pkg, oracle, own_rows, case)
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", [c[:5] for c in test_gpu_matrix_sums.CASES], ids=_id)
 def test_the_cases_of_pre_expanded_rows_as_planned(pkg, oracle, case):
     """The cases chosen for the heights of the kernel that reads pre-expanded rows, in the form that the planner picks."""
@@ -160,6 +161,7 @@ FOLDED = [
 ]
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("case", FOLDED, ids=_id)
 def test_rows_of_whole_images(pkg, oracle, own_rows, case, mode):

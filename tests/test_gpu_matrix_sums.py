@@ -121,6 +121,7 @@ def test_every_tile_height_is_covered(pkg):
     assert {_plan(pkg, c)["units_per_wavefront"] for c in CASES} >= {2, 3, 4, 6, 8, 10, 13, 16, 20, 25}
 
 
+@pytest.mark.usefixtures("launches")
 def test_layer_entry_and_integer_op(pkg, oracle):
     """Ranges found on the device (zero point and constants read from memory) and the tf1 op with its own padding
     origin, which may be negative, against the oracle."""

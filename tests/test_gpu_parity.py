@@ -64,6 +64,7 @@ def _check(pkg, oracle, table, x, f, mm, strides, padding, dil, fast=False, dept
     return y, acc
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", SMALL, ids=[str(i) for i in range(len(SMALL))])
 @pytest.mark.parametrize("tname", ["random", "asymmetric", "exact"])
 def test_dense_vs_reference_order_oracle(pkg, oracle, case, tname):
@@ -74,6 +75,7 @@ def test_dense_vs_reference_order_oracle(pkg, oracle, case, tname):
     _check(pkg, oracle, table, x, f, mm, strides, padding, dil)
 
 
+@pytest.mark.usefixtures("launches")
 def test_config1_both_tables_and_committed_vectors(pkg, oracle, golden_dir):
     z = np.load(os.path.join(golden_dir, "config1_oracle.npz"))
     mm = tuple(float(v) for v in z["minmax"])
@@ -134,6 +136,7 @@ MEDIUM = [
 ]
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", MEDIUM, ids=[str(i) for i in range(len(MEDIUM))])
 def test_dense_medium_vs_oracle(pkg, oracle, case):
     xs, fs, strides = case
@@ -141,6 +144,7 @@ def test_dense_medium_vs_oracle(pkg, oracle, case):
     _check(pkg, oracle, pkg.synth.table_uniform_error(11), x, f, MM, strides, "SAME", (1, 1), fast=True)
 
 
+@pytest.mark.usefixtures("launches")
 def test_he_normal_weights_with_tensor_minmax(pkg, oracle):
     """The Keras wrapper's policy: min/max are the tensors' own extrema (fake_approx_convolutional.py:233-242)."""
     rng = np.random.default_rng(5)
@@ -151,6 +155,7 @@ def test_he_normal_weights_with_tensor_minmax(pkg, oracle):
     _check(pkg, oracle, pkg.synth.table_noisy(7), x, f, (in_min, in_max, f_min, f_max), (1, 1), "SAME", (1, 1), fast=True)
 
 
+@pytest.mark.usefixtures("launches")
 def test_off_grid_inputs_quantize_like_the_reference(pkg, oracle):
     """Inputs that were not fake-quantized (but lie inside the range) still go through the same
     three-rounding quantize expression, so codes and sums stay bit-exact."""
@@ -160,6 +165,7 @@ def test_off_grid_inputs_quantize_like_the_reference(pkg, oracle):
     _check(pkg, oracle, pkg.synth.table_random(4), x, f, MM, (1, 1), "SAME", (1, 1))
 
 
+@pytest.mark.usefixtures("launches")
 def test_zero_range_tensors(pkg, oracle):
     """min == max == 0 gives scale = inv_scale = offset = 0 (approx_ops_types.h:142-151): every code is 0."""
     x = np.zeros((1, 6, 6, 4), np.float32)
@@ -191,6 +197,7 @@ def test_quantize_entry_point(pkg, oracle):
         assert codes[-3] == 0 and codes[-2] == 255 and codes[-1] == 0      # NaN -> 0, +inf -> 255, -inf -> 0
 
 
+@pytest.mark.usefixtures("launches")
 def test_codes_entry_point(pkg, oracle):
     from tf_approximate_amd import ops
     rng = np.random.default_rng(8)
@@ -234,6 +241,7 @@ def test_depthwise_vs_oracle(pkg, oracle, case, k):
     _check(pkg, oracle, pkg.synth.table_truncated(k), x, f, MM, strides, padding, (1, 1), depthwise=True)
 
 
+@pytest.mark.usefixtures("launches")
 def test_inverted_residual_block(pkg, oracle):
     """1x1 expand (x6) -> depthwise 3x3 -> 1x1 project, each layer against the oracle."""
     rng = np.random.default_rng(2)
@@ -279,6 +287,7 @@ def test_error_paths_on_device(pkg):
     assert rc == 1 and b"workspace too small" in lib.axc_last_error()
 
 
+@pytest.mark.usefixtures("launches")
 def test_non_default_stream(pkg, oracle):
     case = pkg.synth.config1(seed=4)
     table = pkg.synth.table_noisy(7)
@@ -294,6 +303,7 @@ def test_non_default_stream(pkg, oracle):
     assert refimpl.linf_rel(y.cpu().numpy(), y_ref) <= TOL
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("name", ["cifar", "inverted_residual_s2"])
 def test_network_layers_vs_oracle(pkg, oracle, name):
     """Every convolution of a small synthetic network, checked on the tensors the network itself produced."""
@@ -349,6 +359,7 @@ LAYER_CASES = [
 ]
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", LAYER_CASES, ids=[str(i) for i in range(len(LAYER_CASES))])
 def test_fake_approx_conv2d_layer_vs_composition(pkg, oracle, case):
     """The fused layer entry point against its definition: numpy min/max, host fake quantization of both tensors,
@@ -376,6 +387,7 @@ def test_fake_approx_conv2d_layer_vs_composition(pkg, oracle, case):
     assert refimpl.linf_rel(y, y_ref) <= TOL
 
 
+@pytest.mark.usefixtures("launches")
 def test_fake_approx_conv2d_layer_ties_and_clamp_edges(pkg, oracle):
     """Fake quantization on the device at exact half-way points and at both ends of the range.  The tensors' own
     min/max are (0, 255) and (-64, 63.5), so the scales are 1 and 0.5, every float operation is exact and the
@@ -441,6 +453,7 @@ def test_fake_approx_depthwise_layer_vs_composition(pkg, oracle, case):
     assert refimpl.linf_rel(y, y_ref) <= TOL
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", LAYER_CASES + DW_LAYER, ids=[str(i) for i in range(len(LAYER_CASES) + len(DW_LAYER))])
 def test_op_with_fused_bias_and_activation_vs_oracle(pkg, oracle, case):
     """axc_conv2d_minmax_bias_act / axc_depthwise_conv2d_minmax_bias_act with ranges given by the caller: the oracle's
@@ -473,6 +486,7 @@ def test_op_with_fused_bias_and_activation_vs_oracle(pkg, oracle, case):
         assert np.array_equal(y, y_plain)
 
 
+@pytest.mark.usefixtures("launches")
 def test_fake_approx_conv2d_layer_strided_1x1_takes_minmax_of_the_whole_input(pkg, oracle):
     """A strided 1x1 layer reads a quarter of its input, but the layer's min / max are those of the whole tensor
     (fake_approx_convolutional.py:233-236): the extremes sit on pixels the filter never touches."""
@@ -492,6 +506,7 @@ def test_fake_approx_conv2d_layer_strided_1x1_takes_minmax_of_the_whole_input(pk
     assert rc == 0 and y.shape == y_ref.shape and refimpl.linf_rel(y, y_ref) <= TOL
 
 
+@pytest.mark.usefixtures("launches")
 def test_fake_approx_conv2d_layer_all_zero_input(pkg):
     """min == max == 0 for the input: every quantization constant of that tensor is 0 (approx_ops_types.h:142-151)."""
     dev = gpu_util.dev()
@@ -510,6 +525,7 @@ AXCONV_TF1 = [
 ]
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", AXCONV_TF1, ids=[str(i) for i in range(len(AXCONV_TF1))])
 def test_tf1_axconv2d_vs_reference_functor(pkg, oracle, case):
     from tf_approximate_amd import ops
@@ -530,6 +546,7 @@ def test_tf1_axconv2d_vs_reference_functor(pkg, oracle, case):
     assert lo < 0 < hi
 
 
+@pytest.mark.usefixtures("launches")
 def test_hip_graph_capture_and_replays(pkg):
     """The op and the layer entry point allocate nothing and record no memset nodes: a captured graph of a small
     network replays to the eager result every time, with eager work and synchronisation between the replays."""
@@ -558,6 +575,7 @@ def test_hip_graph_capture_and_replays(pkg):
             torch.cuda.synchronize()
 
 
+@pytest.mark.usefixtures("launches")
 def test_concurrent_host_threads_through_the_c_abi(pkg, oracle):
     """Two host threads drive the C ABI at the same time: one table, but a stream, a workspace and an output per
     thread (what the header promises to support).  Each thread alternates two layer shapes for a few hundred calls;

@@ -49,8 +49,20 @@ def _tensors(case, seed):
     return x, f, xd, torch.from_numpy(f).to("cuda:0")
 
 
+def _assert_patch_sums_run(pkg, call):
+    """The timers name what a call without merged launches runs (conftest.launches)."""
+    pkg.ops.profile_enable(True)
+    pkg.ops.profile_reset()
+    try:
+        call()
+        names = set(pkg.ops.profile_read())
+    finally:
+        pkg.ops.profile_enable(False)
+    assert names & {"patch_sums", "patch_sums_flat"} and "direct" not in names, names
+
+
 @pytest.mark.parametrize("case", CASES, ids=_id)
-def test_float_outputs_bit_equal(pkg, oracle, case):
+def test_float_outputs_bit_equal(pkg, oracle, case, launches):
     print("case", _id(case), flush=True)
     stride, padding = case[4], case[5]
     x, f, xd, fd = _tensors(case, sum(case[0]))
@@ -60,15 +72,20 @@ def test_float_outputs_bit_equal(pkg, oracle, case):
     assert rc == 0
     assert np.array_equal(op.accumulators(xd, fd, *mm).cpu().numpy(), acc)
     assert np.array_equal(op(xd, fd, *mm).cpu().numpy(), y)     # the same sums in the same order: no tolerance needed
+    if launches == "part_by_part":
+        _assert_patch_sums_run(pkg, lambda: op(xd, fd, *mm))
 
 
 @pytest.mark.parametrize("case", [CASES[0], CASES[3], CASES[4], CASES[8]], ids=_id)
-def test_layer_call_equals_the_op_on_fake_quantized_tensors(pkg, case):
+def test_layer_call_equals_the_op_on_fake_quantized_tensors(pkg, case, launches):
     """The padding quads must not be fake-quantized: zero is not on the grid."""
     _, _, xd, fd = _tensors(case, 7)
     stride, padding = case[4], case[5]
     table = pkg.ops.TruthTable(pkg.synth.table_noisy(5))
-    y = pkg.ops.FakeApproxConv2D((stride, stride), table, padding)(xd, fd)
+    layer = pkg.ops.FakeApproxConv2D((stride, stride), table, padding)
+    y = layer(xd, fd)
+    if launches == "part_by_part":
+        _assert_patch_sums_run(pkg, lambda: layer(xd, fd))
     lo, hi, flo, fhi = (float(v) for v in (xd.min(), xd.max(), fd.min(), fd.max()))
     fq = pkg.fake_quant.fake_quant_with_min_max_vars
     op = pkg.ApproxConv2DWithMinMaxVars([1, stride, stride, 1], 8, table, padding)

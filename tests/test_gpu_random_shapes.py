@@ -27,6 +27,7 @@ def _random_case(rng):
     return (n, h, w, c), (kh, kw, c, co), (sh, sw), (dh, dw), padding, mm
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("seed", range(48))
 def test_random_layer_vs_oracle(pkg, oracle, seed):
     rng = np.random.default_rng(1000 + seed)
@@ -41,6 +42,7 @@ def test_random_layer_vs_oracle(pkg, oracle, seed):
     assert refimpl.linf_rel(y, y_ref) <= 1e-5, (xs, fs, strides, dil, padding)
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("seed", range(12))
 def test_random_layer_entry_point_vs_composition(pkg, oracle, seed):
     """The same for the layer entry point (off-grid inputs: the fused fake quantization has real work to do)."""
@@ -76,6 +78,7 @@ EXTREMES = [
 ]
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", EXTREMES, ids=[str(i) for i in range(len(EXTREMES))])
 def test_extreme_shapes_vs_oracle(pkg, oracle, case):
     xs, fs, strides, dil, padding = case
@@ -102,6 +105,7 @@ WIDE_ROWS = [
 ]
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("case", WIDE_ROWS, ids=[str(i) for i in range(len(WIDE_ROWS))])
 def test_wide_rows_of_many_channels_vs_oracle(pkg, oracle, case):
     xs, fs, strides, dil, padding = case
@@ -169,6 +173,7 @@ def _sweep_case(seed):
     return xs, fs, strides, dil, padding, mm, dw
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("block", range(5))
 def test_random_sweep_slice_vs_oracle(pkg, oracle, block):
     """150 fixed-seed cases of the sweep (30 per test), dense and depthwise, whole outputs against the oracle."""

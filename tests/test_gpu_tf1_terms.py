@@ -11,6 +11,7 @@ import gpu_util
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.usefixtures("launches")
 @pytest.mark.parametrize("xs,fs,stride,padding,shift", [
     ((2, 9, 11, 16), (3, 3, 20), 1, "SAME", 0),       # 16-byte loads
     ((2, 9, 11, 16), (3, 3, 20), 1, "SAME", 4),       # ... which this tensor does not begin on
