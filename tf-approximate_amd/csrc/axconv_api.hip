@@ -919,7 +919,8 @@ struct PreparedDense {
 // as it reads stride 1.  prepare_mx takes it where the models of both loads say that it saves more than the pass, 4 us and its
 // bytes at 4 TB/s, costs.  Launch of the kernel without / pass + launch with, us: 3x3/2 128->128 @57x57x64 292 / 22 + 203, 256->256
 // @28x28x64 369 / 13 + 221, 512->512 @14x14x64 366 / 14 + 212; whole op 5x5/(1,2) 162->35 @12x12x10 75 / 46, 3x3/2 80->232
-// @56x56x27 182 / 137, 7x2/(1,2) 32->376 @72x8x7 40.1 / 39.2.  Of 43 random strided layers 19 take it, none is slower for it.
+// @56x56x27 182 / 137, 7x2/(1,2) 32->376 @72x8x7 40.1 / 39.2.  160 random strided layers of more than 4e8 lookups take 0.89 of the
+// time without (geometric mean), two of them, dilated ones, more than 3 % longer (1.04 and 1.08).
 bool planes_ok(const ConvGeom &g, const XqLayout &lay, const int flat_row_bytes)
 {
     return !flat_row_bytes && g.sw > 1 && ((int64_t)g.N * lay.Hp + lay.row0) * g.KW * g.C4 * g.OW * 4 + 16 < (int64_t)1 << 31;

@@ -411,10 +411,10 @@ bool px_free_running(const DensePlan &plan, int taps);   // the plan runs lutgem
 hipError_t launch_mx_expand_rows(const float *filter, const uint8_t *filter_codes, const ConvGeom &g, const MxPlan &plan,
                                  const TensorQuant &tq, const LayerQuant *lq_dev, const uint16_t *tableT, uint16_t *rows,
                                  hipStream_t stream);
-// mx->swap, where no other launch has done it: both operands packed, from floats or codes; and the pass behind the LUT-GEMM,
-// which adds the K splits' [Co][M] sums (rows of m_pitch), turns them and applies the op's epilogue
 // xq by tap columns, [image row][tap column][quad][output column], for lutgemm_mx_kernel at a stride
 hipError_t launch_split_columns(const uint32_t *xq, const ConvGeom &g, const XqLayout &lay, uint32_t *planes, hipStream_t stream);
+// mx->swap, where no other launch has done it: both operands packed, from floats or codes; and the pass behind the LUT-GEMM,
+// which adds the K splits' [Co][M] sums (rows of m_pitch), turns them and applies the op's epilogue
 hipError_t launch_swap_pack(const float *x, const uint8_t *codes, const float *filter, const uint8_t *filter_codes,
                             const ConvGeom &g, const TensorQuant &tq_in, const TensorQuant &tq_f, const LayerQuant *lq_dev,
                             uint32_t *xq, uint16_t *wq, hipStream_t stream);

@@ -9,10 +9,10 @@ forward pass from layer lists, random He-normal weights and synthetic inputs:
     resnet50       ResNet-50 shaped: 7x7/2 stem, bottlenecks 1x1 / 3x3 / 1x1, stage widths 256/512/1024/2048
     inverted_residual  MobileNetV2-style block: 1x1 expand (x6), depthwise 3x3 (stride 1 or 2), 1x1 project
 
-Only the convolutions run through the library (with the ReLU that directly follows one fused into its store);
-residual adds with their ReLU (one elementwise kernel built by torch.cuda.jiterator, or torch's add and relu where
-that is not available) and the max-pool are torch glue.  The
-min/max of every layer input and filter are taken from the tensors in a calibration pass (the Keras wrapper's
+Only the convolutions run through the library, with the ReLU that directly follows one fused into its store and, where ranges are
+calibrated, a residual add and its ReLU in the call of the convolution in front of it.  Other residual adds with their ReLU (one
+elementwise kernel built by torch.cuda.jiterator, or torch's add and relu where that is not available) and the max-pool are torch
+glue.  The min/max of every layer input and filter are taken from the tensors in a calibration pass (the Keras wrapper's
 policy) and then held fixed, so the timed pass has no host synchronisation.
 """
 import math
