@@ -79,3 +79,27 @@ def test_networks_sum_in_the_layers(pkg):
         adds, net.adds = net.adds, {}
         want = net.forward(x)
         assert got[1] == want[1] and torch.equal(got[0].view(torch.int32), want[0].view(torch.int32))
+
+
+@pytest.mark.parametrize("xs,fs,stride,rows,px,names", [CASES[i] for i in (0, 2, 4, 5, 7, 10, 12)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else None)
+def test_an_addend_that_begins_at_any_float(pkg, xs, fs, stride, rows, px, names):
+    print("case", xs, fs, stride, rows, px, flush=True)
+    ops = pkg.ops
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(sum(xs))
+    x = torch.rand(xs, device="cuda:0", generator=gen) * 2 - 1
+    f = torch.rand(fs, device="cuda:0", generator=gen) - 0.5
+    op = ops.ApproxConv2DWithMinMaxVars([1, stride, stride, 1], 8, ops.TruthTable(pkg.synth.table_random(4)), "SAME")
+    ops.set_preexpand(px)
+    ops.set_matrix_rows(rows)
+    try:
+        y = op(x, f, *MM)
+        for off in (1, 2, 3):
+            addend = torch.randn(y.numel() + off, device="cuda:0", generator=gen)[off:].view(y.shape)
+            assert addend.is_contiguous() and addend.data_ptr() % 16 == 4 * off
+            got = op.call_and_add(x, f, *MM, addend)
+            assert torch.equal(got.view(torch.int32), (y + addend).view(torch.int32))
+    finally:
+        ops.set_matrix_rows(0)
+        ops.set_preexpand(0)
